@@ -2008,9 +2008,69 @@ __global__ __launch_bounds__(kFusedThreads) void block_fused_kernel(const coda_b
   }
 }
 
-// Rotate a full ring into time order: slot s <- slot (head + s) % W.
+// Rotate a full ring into time order, in place: slot s <- slot (head + s) % W.
+// A workgroup takes all W slots of one column strip (kRotPieces 16-byte
+// pieces of every row) of one (sequence, head)'s K or V plane: it holds the
+// strip in registers (NP pieces a thread), waits for every load, and stores
+// it rotated; strips don't meet, so nothing goes through memory twice.
+// Bound by one load and one store round trip: at B = 1 (7B shape, 1 MiB) 64
+// workgroups, ~5 us, where one workgroup a (sequence, head) copying 2-byte
+// elements to scratch and back took 126 us; 64-byte strips keep whole
+// half-lines (narrower strips split them, wider ones leave fewer workgroups).
+static constexpr int kRotPieces = 4;
+template <int NP>
+__global__ __launch_bounds__(256) void ring_rotate_kernel(const coda_bank_desc s, int head, int row_pieces) {
+  const int pair = blockIdx.x, W = s.W, Lbuf = s.W + s.Me + s.Ms;
+  const int strip = blockIdx.y >> 1, is_v = blockIdx.y & 1;
+  uint4* plane = (uint4*)(is_v ? s.v_buf : s.k_buf) + (int64_t)pair * Lbuf * row_pieces + strip * kRotPieces;
+  const int n = W * kRotPieces;
+  uint4 r[NP];
+#pragma unroll
+  for (int k = 0; k < NP; ++k) {
+    const int i = min((int)threadIdx.x + 256 * k, n - 1);
+    int src = head + i / kRotPieces;
+    src = src >= W ? src - W : src;
+    r[k] = plane[(int64_t)src * row_pieces + i % kRotPieces];
+  }
+  // the gates of the sequence, one workgroup of its first head
+  const bool gates = blockIdx.y == 0 && pair % s.Hkv == 0;
+  constexpr int NG = (NP + kRotPieces - 1) / kRotPieces;
+  float* g = s.g_recent + (int64_t)(pair / s.Hkv) * W;
+  float gr[NG];
+  if (gates) {
+#pragma unroll
+    for (int k = 0; k < NG; ++k) {
+      int src = head + min((int)threadIdx.x + 256 * k, W - 1);
+      gr[k] = g[src >= W ? src - W : src];
+    }
+  }
+  // every load of the workgroup has landed before its first store: the
+  // values are used here (which waits for this thread's), then the barrier
+#pragma unroll
+  for (int k = 0; k < NP; ++k) asm volatile("" ::"v"(r[k].x), "v"(r[k].w));
+  if (gates) {
+#pragma unroll
+    for (int k = 0; k < NG; ++k) asm volatile("" ::"v"(gr[k]));
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NP; ++k) {
+    const int i = threadIdx.x + 256 * k;
+    if (i < n) plane[(int64_t)(i / kRotPieces) * row_pieces + i % kRotPieces] = r[k];
+  }
+  if (gates) {
+#pragma unroll
+    for (int k = 0; k < NG; ++k) {
+      const int i = threadIdx.x + 256 * k;
+      if (i < W) g[i] = gr[k];
+    }
+  }
+}
+// The same for rings past the strips' registers (W > kRotMaxW) or planes
+// that are not 16-byte aligned: through scratch, a workgroup a (sequence, head).
+static constexpr int kRotMaxW = 2048;
 template <typename T, int DH>
-__global__ __launch_bounds__(256) void ring_rotate_kernel(const coda_bank_desc s, int head, T* tmp, float* gtmp) {
+__global__ __launch_bounds__(256) void ring_rotate_scratch_kernel(const coda_bank_desc s, int head, T* tmp, float* gtmp) {
   const int h = blockIdx.x, b = blockIdx.y;
   const int W = s.W, Lbuf = s.W + s.Me + s.Ms;
   T* kb = (T*)s.k_buf + ((int64_t)b * s.Hkv + h) * Lbuf * DH;
@@ -2626,12 +2686,24 @@ extern "C" int coda_ring_rotate(const coda_bank_desc* s, int ring_head, void* wo
   hipStream_t st = (hipStream_t)stream;
   const size_t tmp_bytes = (size_t)s->B * s->Hkv * s->W * s->Dh * 2 * esz;
   float* gtmp = (float*)((char*)workspace + tmp_bytes);
+  if (s->W <= kRotMaxW && ((uintptr_t)s->k_buf | (uintptr_t)s->v_buf) % 16 == 0) {
+    // rows of Dh * esz bytes are whole strips of 64
+    const int row_pieces = (int)(s->Dh * esz / 16);
+    const dim3 grid((unsigned)(s->B * s->Hkv), 2 * (row_pieces / kRotPieces));
+    const int np = (s->W * kRotPieces + 255) / 256;
+    if (np <= 2) hipLaunchKernelGGL((ring_rotate_kernel<2>), grid, dim3(256), 0, st, *s, ring_head, row_pieces);
+    else if (np <= 4) hipLaunchKernelGGL((ring_rotate_kernel<4>), grid, dim3(256), 0, st, *s, ring_head, row_pieces);
+    else if (np <= 8) hipLaunchKernelGGL((ring_rotate_kernel<8>), grid, dim3(256), 0, st, *s, ring_head, row_pieces);
+    else hipLaunchKernelGGL((ring_rotate_kernel<kRotMaxW * kRotPieces / 256>), grid, dim3(256), 0, st, *s, ring_head,
+                            row_pieces);
+    return check_launch("ring_rotate");
+  }
   const dim3 grid(s->Hkv, s->B);
   const bool bf = s->dtype == CODA_BF16;
 #define CODA_ROT(DH)                                                                                      \
-  if (bf) hipLaunchKernelGGL((ring_rotate_kernel<bf16_t, DH>), grid, dim3(256), 0, st, *s, ring_head,   \
+  if (bf) hipLaunchKernelGGL((ring_rotate_scratch_kernel<bf16_t, DH>), grid, dim3(256), 0, st, *s, ring_head,   \
                              (bf16_t*)workspace, gtmp);                                                 \
-  else hipLaunchKernelGGL((ring_rotate_kernel<float, DH>), grid, dim3(256), 0, st, *s, ring_head,       \
+  else hipLaunchKernelGGL((ring_rotate_scratch_kernel<float, DH>), grid, dim3(256), 0, st, *s, ring_head,       \
                           (float*)workspace, gtmp);
   switch (s->Dh) {
     case 32: CODA_ROT(32) break;
