@@ -287,12 +287,83 @@ __global__ __launch_bounds__(256) void decode_bank_kernel(const coda_bank_desc s
 }
 
 // ------------------------------------------------------------ block plan
-// One wave per (chunk, sequence); lane 0 runs the libstdc++-order selection
-// on the chunk's evicted gates staged in LDS.  Gates of the virtual
-// sequence S = [initial ring (time order) | g_seq].
+// One wave per (chunk, sequence) runs the libstdc++-order selection on the
+// chunk's evicted gates staged in LDS.  Gates of the virtual sequence
+// S = [initial ring (time order) | g_seq].
 struct PlanGeom {
   int W, L, block, Lr0, ring_head, kE, kS, doE, doS, Kmax, B;
 };
+
+// sel::partition_unguarded over a[first, last) against the pivot a[pv], by a
+// whole wave, with the same swaps.  The left scan of the serial form stops at
+// elements not before the pivot, the right scan at elements the pivot is not
+// before; neither scan meets a swapped element before the scans cross.  So
+// with the left stops L_0 < L_1 < .. and the right stops R_0 > R_1 > .. of
+// the range as it stands, swap j exchanges L_j and R_j for the m first j with
+// L_j < R_j, and the cut is the next left stop: L_m, or R_{m-1} (which the
+// last swap made one) where that comes first.  lpos / rpos: LDS lists of the
+// stops, both ascending.
+__device__ __forceinline__ int wave_partition(sel::Item<float>* a, int first, int last, int pv,
+                                              const sel::Before<float>& before, uint16_t* lpos, uint16_t* rpos,
+                                              int lane) {
+  const sel::Item<float> p = a[pv];
+  const uint64_t below = (1ull << lane) - 1;
+  int nl = 0, nr = 0;
+  for (int base = first; base < last; base += 64) {
+    const int i = base + lane;
+    const sel::Item<float> x = a[min(i, last - 1)];
+    const bool sl = i < last && !before(x, p), sr = i < last && !before(p, x);
+    const uint64_t bl = __builtin_amdgcn_ballot_w64(sl), br = __builtin_amdgcn_ballot_w64(sr);
+    if (sl) lpos[nl + __popcll(bl & below)] = (uint16_t)i;
+    if (sr) rpos[nr + __popcll(br & below)] = (uint16_t)i;
+    nl += __popcll(bl);
+    nr += __popcll(br);
+  }
+  __syncthreads();
+  int m = 0;
+  for (int base = 0;; base += 64) {
+    const int j = base + lane;
+    const bool in = j < nl && j < nr;
+    const int l = lpos[in ? j : 0], r = rpos[in ? nr - 1 - j : 0];
+    const bool sw = in && l < r;
+    const int cnt = __popcll(__builtin_amdgcn_ballot_w64(sw));
+    if (sw) sel::swap_items(a, l, r);
+    m += cnt;
+    if (cnt < 64) break;
+  }
+  const int lm = m < nl ? lpos[m] : INT_MAX, rm = m > 0 ? rpos[nr - m] : INT_MAX;
+  __syncthreads();
+  return min(lm, rm);
+}
+
+// sel::nth_element over a[0, n) by a whole wave: the same sequence of
+// partitions; the depth limit's heap select and the last insertion sort
+// (at most 3 elements) stay on lane 0.
+__device__ __forceinline__ void wave_nth_element(sel::Item<float>* a, int nth, int n, const sel::Before<float>& before,
+                                                 uint16_t* lpos, uint16_t* rpos, int lane) {
+  if (n == 0 || nth == n) return;
+  int first = 0, last = n, depth = sel::floor_log2(n) * 2;
+  while (last - first > 3) {
+    if (depth == 0) {
+      if (lane == 0) {
+        sel::heap_select(a, first, nth + 1, last, before);
+        sel::swap_items(a, first, nth);
+      }
+      return;
+    }
+    --depth;
+    if (lane == 0) sel::median_to_first(a, first, first + 1, first + (last - first) / 2, last - 1, before);
+    __syncthreads();
+    const int cut = wave_partition(a, first + 1, last, first, before, lpos, rpos, lane);
+    if (cut <= nth) first = cut;
+    else last = cut;
+  }
+  if (lane == 0) sel::insertion_sort(a, first, last, before);
+}
+
+// Bound by the chain of dependent LDS passes: about 2 log2(n / K) partitions
+// of the range left.  The selection on one lane took 81 us for 8 chunks of
+// 256 tokens and 189 us for chunks of 1024, every LDS access waited for.
 
 __global__ __launch_bounds__(64) void block_plan_kernel(const float* __restrict__ g_ring,
                                                         const float* __restrict__ g_seq, int64_t g_sb,
@@ -328,7 +399,13 @@ __global__ __launch_bounds__(64) void block_plan_kernel(const float* __restrict_
     items[i] = sel::Item<float>{g, (int64_t)i};
   }
   __syncthreads();
-  if (threadIdx.x == 0) sel::topk_order<float>(items, n_ev, K, true, false);
+  // (the choice of sel::topk_order, sorted = false)
+  if (K * 64 <= n_ev) {
+    if (threadIdx.x == 0) sel::topk_order<float>(items, n_ev, K, true, false);
+  } else if (K > 0) {
+    uint16_t* lpos = reinterpret_cast<uint16_t*>(items + p.block);
+    wave_nth_element(items, K - 1, n_ev, sel::Before<float>{true}, lpos, lpos + p.block, (int)threadIdx.x);
+  }
   __syncthreads();
   for (int i = threadIdx.x; i < K; i += 64) out[i] = (int32_t)items[i].i;
 }
@@ -2262,8 +2339,10 @@ extern "C" int coda_block_plan(const float* g_ring, int ring_head, int ring_fill
   CODA_REQUIRE(K_eff <= Kmax, "coda_block_plan: Kmax %d below candidate count %d", Kmax, K_eff);
   const int n_chunks = (L + block_size - 1) / block_size;
   if (B == 0 || n_chunks == 0 || (!do_exact && !do_summary)) return CODA_OK;
-  const size_t lds = sizeof(sel::Item<float>) * (size_t)block_size;
-  CODA_REQUIRE(lds <= 64 * 1024, "coda_block_plan: block_size %d too large (max 4096)", block_size);
+  CODA_REQUIRE(block_size <= 4096, "coda_block_plan: block_size %d too large (max 4096)", block_size);
+  const size_t lds = (sizeof(sel::Item<float>) + 2 * sizeof(uint16_t)) * (size_t)block_size;
+  const int rc = lds_limit<block_plan_kernel>(lds, "coda_block_plan");
+  if (rc) return rc;
   PlanGeom p{W, L, block_size, ring_filled, ring_head, k_exact, k_summary, do_exact, do_summary, Kmax, B};
   hipLaunchKernelGGL(block_plan_kernel, dim3(n_chunks, B), dim3(64), lds, (hipStream_t)stream, g_ring, g_seq,
                      g_sb, p, plan);
