@@ -23,7 +23,7 @@
 //                    noise) sharing every K/V fragment; K/V tiles of 64
 //                    keys are staged through LDS once per workgroup.
 //                    MFMA-bound.
-//   attn_generic     fp32 (VALU): config-C1-sized problems and tests.
+//   attn_f32         fp32, 16 query rows a workgroup on the fp32 MFMA.
 //
 // MFMA fragment layouts (wave64, l = lane, n = l % 16, g4 = l / 16):
 //   v_mfma_f32_16x16x32_bf16 A[m=n][k=8*g4+j], B[k=8*g4+j][col=n], j<8
@@ -35,7 +35,9 @@
 #include "bank_ops.h"
 #include "common.h"
 
+#include <algorithm>
 #include <atomic>
+#include <climits>
 #include <cstring>
 
 #include <math.h>
@@ -188,14 +190,6 @@ __device__ __forceinline__ void stage_queries(const coda_attn_desc& a, int b, in
   }
 }
 
-// Key visibility for query qi at key index kidx in [0, Lp + Lb).
-__device__ __forceinline__ bool key_visible(const coda_attn_desc& a, int b, int qi, int kidx) {
-  if (kidx < a.Lp) return a.allowed ? (a.allowed[(int64_t)b * a.al_sb + kidx] != 0) : true;
-  const int j = kidx - a.Lp;
-  if (j >= a.Lb) return false;
-  return !a.causal || j <= qi + (a.causal == 2 ? 0 : a.Lb - a.Lq);
-}
-
 template <typename T>
 __device__ __forceinline__ const T* key_ptr(const coda_attn_desc& a, int b, int hk, int kidx,
                                             bool value) {
@@ -256,132 +250,6 @@ __device__ __forceinline__ void diff_norm_w(float (&y)[NV], const float (&os)[NV
   for (int i = 0; i < NV; ++i) y[i] = act[i] ? E::rnd(E::rnd(y[i] * r) * w[i]) : 0.f;
 }
 
-// ------------------------------------------------------------ fp32 / VALU
-// Workgroup = (query qi, KV head, batch); rows = 2 streams x G heads.
-template <typename T, int DH>
-__global__ __launch_bounds__(256) void attn_generic(const coda_attn_desc a) {
-  using E = Elt<T>;
-  constexpr int KT = 256, RMAX = 16;
-  __shared__ float qs[RMAX][DH];
-  __shared__ float sc[RMAX][KT];
-  __shared__ float red_alpha[RMAX];
-  __shared__ float m_run[RMAX], l_run[RMAX];
-  const int qi = blockIdx.x, hk = blockIdx.y, b = blockIdx.z;
-  const int G = a.H / a.Hkv, R = 2 * G;
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const float scale = (a.sm_scale > 0.f ? a.sm_scale : rsqrtf((float)DH));
-
-  for (int i = t; i < R * (DH / 8); i += 256) {
-    const int r = i / (DH / 8), c = i % (DH / 8);
-    const int s = r / G, g = r % G;
-    float x[8];
-    prep_q8<T>(a, b, hk * G + g, qi, c * 8, s, x);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) qs[r][c * 8 + j] = x[j];
-  }
-  if (t < RMAX) { m_run[t] = -INFINITY; l_run[t] = 0.f; }
-  constexpr int TPR = 256 / DH;                 // threads per row group
-  constexpr int RPT = (RMAX + TPR - 1) / TPR;   // rows per thread
-  const int dcol = t % DH, rg = t / DH;
-  float o[RPT];
-#pragma unroll
-  for (int i = 0; i < RPT; ++i) o[i] = 0.f;
-  __syncthreads();
-
-  const int Lk = a.Lp + a.Lb;
-  for (int k0 = 0; k0 < Lk; k0 += KT) {
-    const int kidx = k0 + t;
-    if (kidx < Lk) {
-      const T* kr = key_ptr<T>(a, b, hk, kidx, false);
-      float acc[RMAX];
-#pragma unroll
-      for (int r = 0; r < RMAX; ++r) acc[r] = 0.f;
-      for (int d = 0; d < DH; d += 8) {
-        float kx[8];
-        load8<T>(kr + d, kx);
-#pragma unroll
-        for (int r = 0; r < RMAX; ++r) {
-          if (r < R) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) acc[r] = fmaf(qs[r][d + j], kx[j], acc[r]);
-          }
-        }
-      }
-      const bool vis = key_visible(a, b, qi, kidx);
-      for (int r = 0; r < R; ++r) sc[r][t] = vis ? acc[r] * scale : -INFINITY;
-    } else {
-      for (int r = 0; r < R; ++r) sc[r][t] = -INFINITY;
-    }
-    __syncthreads();
-    for (int r = wv; r < R; r += 4) {
-      float mx = -INFINITY;
-      for (int i = lane; i < KT; i += 64) mx = fmaxf(mx, sc[r][i]);
-      mx = wave_max(mx);
-      const float mold = m_run[r];
-      const float mnew = fmaxf(mold, mx);
-      const float muse = (mnew == -INFINITY) ? 0.f : mnew;
-      float ps = 0.f;
-      for (int i = lane; i < KT; i += 64) {
-        const float p = expf(sc[r][i] - muse);
-        sc[r][i] = p;
-        ps += p;
-      }
-      ps = wave_sum(ps);
-      if (lane == 0) {
-        const float al = expf(mold - muse);
-        red_alpha[r] = al;
-        l_run[r] = l_run[r] * al + ps;
-        m_run[r] = mnew;
-      }
-    }
-    __syncthreads();
-    const int kn = min(KT, Lk - k0);
-#pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-      const int r = rg + i * TPR;
-      if (r < R) o[i] *= red_alpha[r];
-    }
-    for (int kk = 0; kk < kn; ++kk) {
-      const float v = E::ld(key_ptr<T>(a, b, hk, k0 + kk, true)[dcol]);
-#pragma unroll
-      for (int i = 0; i < RPT; ++i) {
-        const int r = rg + i * TPR;
-        if (r < R) o[i] = fmaf(sc[r][kk], v, o[i]);
-      }
-    }
-    __syncthreads();
-  }
-  // normalise into qs (reused as the output staging buffer)
-#pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-    const int r = rg + i * TPR;
-    if (r < R) qs[r][dcol] = l_run[r] > 0.f ? o[i] / l_run[r] : 0.f;
-  }
-  __syncthreads();
-  // epilogue: wave per head of the group
-  constexpr int NV = (DH + 63) / 64;
-  for (int g = wv; g < G; g += 4) {
-    const int h = hk * G + g;
-    float os[NV], on[NV], y[NV];
-    bool act[NV];
-    int dd[NV];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int d = lane + 64 * i;
-      act[i] = d < DH;
-      dd[i] = act[i] ? d : 0;
-      os[i] = act[i] ? qs[g][dd[i]] : 0.f;
-      on[i] = act[i] ? qs[G + g][dd[i]] : 0.f;
-    }
-    const float lam = E::ld(((const T*)a.lam)[b * a.lam_sb + h * a.lam_sh + qi * a.lam_sl]);
-    diff_norm<T, NV>(y, os, on, act, lam, (const T*)a.rms_w, dd, a.eps, DH, true, 0, 0);
-    T* orow = (T*)a.out + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_sl;
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
-      if (act[i]) orow[dd[i]] = E::st(y[i]);
-  }
-}
-
 // ------------------------------------------------------------ MFMA helpers
 __device__ __forceinline__ f32x4 mfma_k32(const bf16x8_t& a, const bf16x8_t& b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -438,12 +306,9 @@ __device__ __forceinline__ void store_vt(char* base, int kg, int d0, const uint4
 }
 
 // ------------------------------------------------------------ decode rows
-// Workgroup = (split, KV head, batch); 4 waves take 16-key tiles in turn.
-// Partial (m, l, O) of the 4 waves merge in LDS; with nsplit > 1 each
-// workgroup leaves its merged partial in `ws` for attn_rows_merge.
 // Workgroup = (split, KV head, batch); 4 attention waves take 16-key tiles
 // in turn and merge their partial (m, l, O) in LDS; with nsplit > 1 each
-// workgroup leaves its merged partial in `ws` for attn_rows_merge.
+// workgroup leaves its merged partial in `ws` for attn_merge.
 template <int DH>
 __global__ __launch_bounds__(256) void attn_rows_bf16(const coda_attn_desc a, int keys_per_split, float* ws) {
   constexpr int NC = DH / 32, NM = DH / 16, NW = 4;
@@ -742,55 +607,78 @@ __global__ __launch_bounds__(256) void attn_rows_bf16(const coda_attn_desc a, in
   }
 }
 
-// Merge the per-split partials of attn_rows_bf16 and apply the epilogue.
-template <int DH>
-__global__ __launch_bounds__(256) void attn_rows_merge(const coda_attn_desc a, int nsplit,
-                                                       const float* ws) {
-  const int hk = blockIdx.x, b = blockIdx.y;
-  const int G = a.H / a.Hkv, GL = G * a.Lq;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const float* base = ws + (((int64_t)b * a.Hkv + hk) * nsplit) * 16 * (DH + 2);
-  constexpr int NV = (DH + 63) / 64;
-  for (int orow = wv; orow < GL; orow += 4) {
-    const int g = orow / a.Lq, qi = orow % a.Lq, h = hk * G + g;
-    float os[NV], on[NV], y[NV];
-    bool act[NV];
-    int dd[NV];
-    float M[2] = {-INFINITY, -INFINITY}, L[2] = {0.f, 0.f};
-    for (int s = 0; s < 2; ++s) {
-      const int r = s * GL + orow;
-      for (int sp = 0; sp < nsplit; ++sp) M[s] = fmaxf(M[s], base[(sp * 16 + r) * (DH + 2)]);
-      const float Mu = M[s] == -INFINITY ? 0.f : M[s];
-      for (int sp = 0; sp < nsplit; ++sp) {
-        const float* pr = base + (sp * 16 + r) * (DH + 2);
-        L[s] += pr[1] * exp2f(pr[0] - Mu);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int d = lane + 64 * i;
-      act[i] = d < DH;
-      dd[i] = act[i] ? d : 0;
-      float acc[2] = {0.f, 0.f};
-      for (int s = 0; s < 2; ++s) {
-        const int r = s * GL + orow;
-        const float Mu = M[s] == -INFINITY ? 0.f : M[s];
-        for (int sp = 0; sp < nsplit; ++sp) {
-          const float* pr = base + (sp * 16 + r) * (DH + 2);
-          acc[s] += pr[2 + dd[i]] * exp2f(pr[0] - Mu);
-        }
-        acc[s] = L[s] > 0.f ? acc[s] / L[s] : 0.f;
-      }
-      os[i] = act[i] ? acc[0] : 0.f;
-      on[i] = act[i] ? acc[1] : 0.f;
-    }
-    const float lam = bf2f(((const bf16_t*)a.lam)[b * a.lam_sb + h * a.lam_sh + qi * a.lam_sl]);
-    diff_norm<bf16_t, NV>(y, os, on, act, lam, (const bf16_t*)a.rms_w, dd, a.eps, DH, true, 0, 0);
-    bf16_t* orow_p = (bf16_t*)a.out + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_sl;
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
-      if (act[i]) orow_p[dd[i]] = f2bf(y[i]);
+// Merge the per-split partials of attn_rows_bf16 / attn_f32 and apply the
+// epilogue: a workgroup per output row (query tile, head, query), since the
+// work is a few dependent round trips and little else.  The row's two streams
+// take their maxima and sums over the splits on 128 threads each, then 256 /
+// DH groups of threads sum the splits' channels.  Partials are [pair][tile]
+// [split][16 rows][m, l, O(DH)], row st * GL + orow of a tile of qt queries,
+// GL = G * qt, orow = g * qt + query.  (4096 keys, 32 pairs, 16 splits: 30 us
+// with a workgroup a pair that walked the splits one after the other.)
+static constexpr int kMaxSplits = 512;
+template <typename T, int DH>
+__global__ __launch_bounds__(256) void attn_merge(const coda_attn_desc a, int qt, int nsplit, const float* ws) {
+  using E = Elt<T>;
+  constexpr int NG = 256 / DH, NV = (DH + 63) / 64;
+  __shared__ float wts[2][kMaxSplits], red[4], acc_lds[2][NG][DH];
+  const int G = a.H / a.Hkv, GL = G * qt, ntile = gridDim.x / GL;
+  const int tile = blockIdx.x / GL, orow = blockIdx.x % GL;
+  const int g = orow / qt, qi = tile * qt + orow % qt;
+  if (qi >= a.Lq) return;
+  const int b = blockIdx.y / a.Hkv, hk = blockIdx.y % a.Hkv, h = hk * G + g;
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const float* base = ws + ((int64_t)blockIdx.y * ntile + tile) * nsplit * 16 * (DH + 2);
+  const int st = t >> 7, rs = st * GL + orow;
+  float M = -INFINITY;
+  for (int sp = t & 127; sp < nsplit; sp += 128) M = fmaxf(M, base[(sp * 16 + rs) * (DH + 2)]);
+  M = wave_max(M);
+  if (lane == 0) red[wv] = M;
+  __syncthreads();
+  M = fmaxf(red[2 * st], red[2 * st + 1]);
+  const float Mu = M == -INFINITY ? 0.f : M;
+  float L = 0.f;
+  for (int sp = t & 127; sp < nsplit; sp += 128) {
+    const float* pr = base + (sp * 16 + rs) * (DH + 2);
+    const float w = exp2f(pr[0] - Mu);
+    wts[st][sp] = w;
+    L += pr[1] * w;
   }
+  L = wave_sum(L);
+  __syncthreads();
+  if (lane == 0) red[wv] = L;
+  const int d = t % DH, gq = t / DH;
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const float* pr = base + (s * GL + orow) * (DH + 2) + 2 + d;
+    float acc = 0.f;
+#pragma unroll 4
+    for (int sp = gq; sp < nsplit; sp += NG) acc += pr[sp * 16 * (DH + 2)] * wts[s][sp];
+    acc_lds[s][gq][d] = acc;
+  }
+  __syncthreads();
+  if (wv > 0) return;
+  float o[2][NV], y[NV];
+  bool act[NV];
+  int dd[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    act[i] = lane + 64 * i < DH;
+    dd[i] = act[i] ? lane + 64 * i : 0;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const float Ls = red[2 * s] + red[2 * s + 1];
+      float acc = 0.f;
+#pragma unroll
+      for (int k = 0; k < NG; ++k) acc += acc_lds[s][k][dd[i]];
+      o[s][i] = act[i] && Ls > 0.f ? acc / Ls : 0.f;
+    }
+  }
+  const float lam = E::ld(((const T*)a.lam)[b * a.lam_sb + h * a.lam_sh + qi * a.lam_sl]);
+  diff_norm<T, NV>(y, o[0], o[1], act, lam, (const T*)a.rms_w, dd, a.eps, DH, true, 0, 0);
+  T* orow_p = (T*)a.out + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_sl;
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+    if (act[i]) orow_p[dd[i]] = E::st(y[i]);
 }
 
 // ------------------------------------------------------------ gfx950 helpers
@@ -916,6 +804,213 @@ __device__ __forceinline__ void unpack4(const uint2& u, float x[4]) {
 }
 
 // ------------------------------------------------------------ fused decode step
+// ------------------------------------------------------------ fp32
+// attn_f32: a workgroup takes 16 query rows (both streams of the G heads of
+// qt = 16 / 2G queries) of one (KV head, sequence) and a share of the keys;
+// its NW waves take 16-key tiles in turn and merge in LDS.  Products on the
+// fp32 matrix instruction (16x16x4: an fp32 multiply-add per term, like fmaf,
+// at twice the vector rate), S^T = K Q^T and O^T = V^T P^T, so that S^T's
+// result is P^T's operand as it stands:
+//   K   lane (n, g4) channels 16 i + 4 g4 .. + 4 of key n (16-byte loads)
+//   V   lane (n, g4) channels VW n .. + VW of keys 4 g4 + j, VW = DH / 16:
+//       output row m of product mt is channel VW m + mt
+// K and V go from memory to operands in registers, two tiles in flight.
+// Bound by the matrix pipe and by what each CU reads of K and V through L2
+// (16 rows reuse a key); many small workgroups, since the shapes of this
+// path are small.  At the 512-wide 8-head layer (head_dim 64, 256 queries,
+// 640 keys): 15.9 us a chunk, 9 us a decode token; one query a workgroup on
+// the vector units took 239 and 92 us.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+template <int DH, int NW>
+__global__ __launch_bounds__(NW * 64) void attn_f32(const coda_attn_desc a, int qt, int nsplit, int keys_per_split,
+                                                    float* ws) {
+  constexpr int NC = DH / 16, NM = DH / 16, VW = DH / 16, NV = (DH + 63) / 64;
+  extern __shared__ __attribute__((aligned(16))) char f32_smem[];
+  float(*red_o)[16][DH + 4] = reinterpret_cast<float(*)[16][DH + 4]>(f32_smem);  // [NW]; queries in [0] before
+  __shared__ float red_m[NW][16], red_l[NW][16];
+  __shared__ uint8_t al_lds[kMaxRowsPrefix];
+  const int tile = blockIdx.x / nsplit, split = blockIdx.x % nsplit, hk = blockIdx.y, b = blockIdx.z;
+  const int G = a.H / a.Hkv, GL = G * qt, q0 = tile * qt;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 15, g4 = lane >> 4;
+  const float scale = (a.sm_scale > 0.f ? a.sm_scale : rsqrtf((float)DH)) * kLog2e;
+  // keys [kbeg, kend) of this split, cut at the last key any row sees:
+  // prefix tiles over [kbeg, pe), then block tiles from bs0, 16 keys each
+  const int coff = a.causal == 2 ? 0 : a.Lb - a.Lq;
+  const int q_last = min(q0 + qt, a.Lq) - 1;
+  const int lk = a.Lp + (a.causal ? max(0, min(a.Lb, q_last + coff + 1)) : a.Lb);
+  const int kbeg = split * keys_per_split, kend = min(lk, kbeg + keys_per_split);
+  const int pe = min(kend, a.Lp), bs0 = max(kbeg, a.Lp);
+  const int n1 = kbeg < pe ? (pe - kbeg + 15) / 16 : 0, n2 = bs0 < kend ? (kend - bs0 + 15) / 16 : 0;
+  const int n_tiles = n1 + n2, nt_w = (n_tiles + NW - 1) / NW;
+  const float* kp = (const float*)a.kp + b * a.p_sb + hk * a.p_sh;
+  const float* vp = (const float*)a.vp + b * a.p_sb + hk * a.p_sh;
+  const float* kb = (const float*)a.kb + b * a.b_sb + hk * a.b_sh;
+  const float* vb = (const float*)a.vb + b * a.b_sb + hk * a.b_sh;
+  // this wave's i-th tile is t = wv + i * NW (past the end: the last one
+  // again, masked out); rows past the source re-read its last row
+  auto issue = [&](int i, f4u (&kf)[NC], float (&vf)[4][VW]) {
+    const int t = min(wv + i * NW, n_tiles - 1);
+    const bool pre = t < n1;
+    const int r0 = pre ? kbeg + 16 * t : bs0 - a.Lp + 16 * (t - n1), last = (pre ? a.Lp : a.Lb) - 1;
+    const float* ks = pre ? kp : kb;
+    const float* vs = pre ? vp : vb;
+    const int64_t sl = pre ? a.p_sl : a.b_sl;
+    const float* kr = ks + min(r0 + n, last) * sl + 4 * g4;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) kf[c] = *reinterpret_cast<const f4u*>(kr + 16 * c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float* vr = vs + min(r0 + 4 * g4 + j, last) * sl + VW * n;
+      if constexpr (VW == 2) {
+        const f2u u = *reinterpret_cast<const f2u*>(vr);
+        vf[j][0] = u[0];
+        vf[j][1] = u[1];
+      } else {
+#pragma unroll
+        for (int q = 0; q < VW / 4; ++q) {
+          const f4u u = *reinterpret_cast<const f4u*>(vr + 4 * q);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) vf[j][4 * q + e] = u[e];
+        }
+      }
+    }
+  };
+  f4u kf0[NC], kf1[NC];
+  float vf0[4][VW], vf1[4][VW];
+  if (n_tiles > 0) issue(0, kf0, vf0);
+  // queries (roped, rotated) and the prefix's visibility bytes to LDS
+  for (int i = threadIdx.x; i < 16 * (DH / 8); i += NW * 64) {
+    const int r = i / (DH / 8), d0 = i % (DH / 8) * 8, rem = r % GL, qi = q0 + rem % qt;
+    float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (r < 2 * GL && qi < a.Lq) prep_q8<float>(a, b, hk * G + rem / qt, qi, d0, r / GL, x);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) red_o[0][r][d0 + j] = x[j];
+  }
+  for (int i = threadIdx.x; i < a.Lp; i += NW * 64) al_lds[i] = a.allowed ? a.allowed[(int64_t)b * a.al_sb + i] : (uint8_t)1;
+  __syncthreads();
+  f32x4 qf[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) qf[c] = *reinterpret_cast<const f32x4*>(&red_o[0][n][16 * c + 4 * g4]);
+  const int row_lim = a.causal ? q0 + n % GL % qt + coff : INT_MAX;  // last block key row n sees
+  // visibility of keys 4 g4 + j of this wave's i-th tile for query row n
+  auto tile_mask = [&](int i) {
+    const int t = wv + i * NW;
+    if (t >= n_tiles) return 0;
+    const bool pre = t < n1;
+    const int kt = pre ? kbeg + 16 * t : bs0 + 16 * (t - n1), hi = pre ? pe : kend;
+    int m4 = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int kk = kt + 4 * g4 + j;
+      const bool ok = kk < hi && (pre ? al_lds[min(kk, a.Lp - 1)] != 0 : kk - a.Lp <= row_lim);
+      m4 |= (int)ok << j;
+    }
+    return m4;
+  };
+  float m_i = -INFINITY, l_i = 0.f;
+  f32x4 o[NM];
+#pragma unroll
+  for (int i = 0; i < NM; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto consume = [&](const f4u (&kf)[NC], const float (&vf)[4][VW], int vmask) {
+    if (__builtin_amdgcn_ballot_w64(vmask != 0) == 0) return;
+    f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c][e], qf[c][e], s, 0, 0, 0);
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) tmax = fmaxf(tmax, (vmask >> j) & 1 ? s[j] * scale : -INFINITY);
+    tmax = xmax32(xmax16(tmax));
+    const float mnew = fmaxf(m_i, tmax), muse = mnew == -INFINITY ? 0.f : mnew;
+    const bool grow = __builtin_amdgcn_ballot_w64(mnew != m_i) != 0;
+    const float alpha = fast_exp2(m_i - muse);
+    float p[4];
+    l_i *= alpha;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      p[j] = (vmask >> j) & 1 ? fast_exp2(fmaf(s[j], scale, -muse)) : 0.f;
+      l_i += p[j];  // this lane's share of the row's sum
+    }
+    m_i = mnew;
+    if (grow) {
+#pragma unroll
+      for (int mt = 0; mt < NM; ++mt) o[mt] *= alpha;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int mt = 0; mt < NM; ++mt) o[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[j][mt], p[j], o[mt], 0, 0, 0);
+  };
+  for (int i = 0; i < nt_w; i += 2) {
+    issue(i + 1, kf1, vf1);
+    consume(kf0, vf0, tile_mask(i));
+    if (i + 1 >= nt_w) break;
+    issue(i + 2, kf0, vf0);
+    consume(kf1, vf1, tile_mask(i + 1));
+  }
+  // merge the waves
+  l_i = xsum32(xsum16(l_i));
+  __syncthreads();  // (the queries were read)
+  if (g4 == 0) {
+    red_m[wv][n] = m_i;
+    red_l[wv][n] = l_i;
+  }
+#pragma unroll
+  for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+    for (int mt = 0; mt < NM; ++mt) red_o[wv][n][VW * (4 * g4 + jj) + mt] = o[mt][jj];
+  __syncthreads();
+  float* part = ws + (((int64_t)(b * a.Hkv + hk) * (gridDim.x / nsplit) + tile) * nsplit + split) * 16 * (DH + 2);
+  for (int orow = wv; orow < GL; orow += NW) {
+    const int h = hk * G + orow / qt, qi = q0 + orow % qt;
+    if (qi >= a.Lq) continue;
+    float acc[2][NV], M[2], L[2], y[NV];
+    bool act[NV];
+    int dd[NV];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int r = s * GL + orow;
+      M[s] = -INFINITY;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) M[s] = fmaxf(M[s], red_m[w][r]);
+      const float Mu = M[s] == -INFINITY ? 0.f : M[s];
+      L[s] = 0.f;
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        act[i] = lane + 64 * i < DH;
+        dd[i] = act[i] ? lane + 64 * i : 0;
+        acc[s][i] = 0.f;
+      }
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float f = fast_exp2(red_m[w][r] - Mu);
+        L[s] += red_l[w][r] * f;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) acc[s][i] += red_o[w][r][dd[i]] * f;
+      }
+      if (nsplit > 1) {  // partial row r: [m, l, O(DH)], unnormalised
+        float* pr = part + r * (DH + 2);
+        if (lane < 2) pr[lane] = lane ? L[s] : M[s];
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+          if (act[i]) pr[2 + dd[i]] = acc[s][i];
+      }
+#pragma unroll
+      for (int i = 0; i < NV; ++i) acc[s][i] = act[i] && L[s] > 0.f ? acc[s][i] / L[s] : 0.f;
+    }
+    if (nsplit > 1) continue;
+    const float lam = ((const float*)a.lam)[b * a.lam_sb + h * a.lam_sh + qi * a.lam_sl];
+    diff_norm<float, NV>(y, acc[0], acc[1], act, lam, (const float*)a.rms_w, dd, a.eps, DH, true, 0, 0);
+    float* orow_p = (float*)a.out + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_sl;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      if (act[i]) orow_p[dd[i]] = y[i];
+  }
+}
+
 static constexpr int kFusedMaxBank = 256;  // exact + summary slots of the fused step
 // decode_step_bf16: one workgroup per (KV head hk, sequence b) runs the
 // whole decode step of that pair once the ring is full (the same work as
@@ -2558,6 +2653,18 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
 }
 
 // ------------------------------------------------------------ host side
+// compute units of the current device (read once per device)
+static int device_cus() {
+  static std::atomic<int> cus[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cus[dev].load(std::memory_order_relaxed);
+  if (n <= 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cus[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
 static int rows_nsplit(const coda_attn_desc* d) {
   const int Lk = d->Lp + d->Lb;
   const int pairs = d->B * d->Hkv;
@@ -2566,6 +2673,28 @@ static int rows_nsplit(const coda_attn_desc* d) {
   const int max_ns = (Lk + 63) / 64;
   ns = ns < max_ns ? ns : max_ns;
   return ns < 1 ? 1 : ns;
+}
+
+// attn_f32's launch: 16-row query tiles; 8 waves a workgroup where the tiles
+// fill the CUs at most twice, and the keys over several workgroups where they
+// leave CUs idle, each with at least four tiles a wave (a decode token over
+// 384 keys: two workgroups a head and the merge 8.9 + 4.1 us, one launch 9 us)
+struct F32Shape {
+  int qt, ntile, nw, nsplit, per;
+};
+static F32Shape f32_shape(const coda_attn_desc* d, int cus) {
+  F32Shape f;
+  f.qt = std::max(1, 8 / (d->H / d->Hkv));
+  f.ntile = (d->Lq + f.qt - 1) / f.qt;
+  const int64_t wgs = (int64_t)f.ntile * d->Hkv * d->B;
+  const int Lk = d->Lp + d->Lb;
+  f.nw = wgs <= 2 * cus ? 8 : 4;
+  const int64_t want = wgs > 0 ? std::min<int64_t>(std::min<int64_t>(cus / wgs, Lk / (64 * f.nw)),
+                                                   kMaxSplits) : 1;
+  f.per = ((Lk + (int)std::max<int64_t>(want, 1) - 1) / (int)std::max<int64_t>(want, 1) + 15) / 16 * 16;
+  f.per = std::max(f.per, 16);
+  f.nsplit = std::max(1, (Lk + f.per - 1) / f.per);
+  return f;
 }
 
 static bool use_rows(const coda_attn_desc* d) {
@@ -2611,6 +2740,9 @@ extern "C" int coda_attn_workspace_bytes(const coda_attn_desc* d, size_t* bytes)
   if (use_rows(d)) {
     const int ns = rows_nsplit(d);
     if (ns > 1) *bytes = (size_t)d->B * d->Hkv * ns * 16 * (d->Dh + 2) * sizeof(float);
+  } else if (d->dtype == CODA_F32) {
+    const F32Shape f = f32_shape(d, device_cus());
+    if (f.nsplit > 1) *bytes = (size_t)d->B * d->Hkv * f.ntile * f.nsplit * 16 * (d->Dh + 2) * sizeof(float);
   }
   return CODA_OK;
 }
@@ -2636,18 +2768,6 @@ static int launch_f3_nw(const coda_attn_desc* d, hipStream_t st, int G, const Ch
   hipLaunchKernelGGL((attn_f3_bf16<DH, NW, QM, TB, NS>), dim3(nblk * npairs, cg.n > 0 ? cg.n : 1), dim3(NW * 64),
                      lds, st, *d, NQ, nblk, npairs, cg);
   return check_launch("attn_f3_bf16");
-}
-// compute units of the current device (read once per device)
-static int device_cus() {
-  static std::atomic<int> cus[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cus[dev].load(std::memory_order_relaxed);
-  if (n <= 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cus[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
 }
 // 4-wave workgroups with two tile stages (two a CU) for G <= 4 (a 4-wave
 // workgroup still holds every head of its KV head), except a one-launch grid
@@ -2679,12 +2799,34 @@ static int launch_f3(const coda_attn_desc* d, hipStream_t st, int G, const Chunk
   if (d->q_noise && !d->rope_cos) return launch_f3_qm<DH, 2, false>(d, st, G, cg);
   return launch_f3_qm<DH, 3, false>(d, st, G, cg);
 }
+template <typename T, int DH>
+static int launch_merge(const coda_attn_desc* d, hipStream_t st, int qt, int ntile, int nsplit) {
+  hipLaunchKernelGGL((attn_merge<T, DH>), dim3(ntile * (d->H / d->Hkv) * qt, d->Hkv * d->B), dim3(256), 0, st, *d, qt,
+                     nsplit, (const float*)d->workspace);
+  return check_launch("attn_merge");
+}
 template <int DH>
 static int launch_attn(const coda_attn_desc* d, hipStream_t st) {
   const int G = d->H / d->Hkv;
   if (d->dtype == CODA_F32) {
-    hipLaunchKernelGGL((attn_generic<float, DH>), dim3(d->Lq, d->Hkv, d->B), dim3(256), 0, st, *d);
-    return check_launch("attn_generic<f32>");
+    const F32Shape f = f32_shape(d, device_cus());
+    if (f.nsplit > 1) {
+      const size_t need = (size_t)d->B * d->Hkv * f.ntile * f.nsplit * 16 * (DH + 2) * sizeof(float);
+      if (!d->workspace || d->workspace_bytes < need)
+        return fail(CODA_ESMALL, "coda_diff_attn_fwd: workspace %zu < %zu bytes", d->workspace_bytes, need);
+    }
+    const size_t lds = (size_t)f.nw * 16 * (DH + 4) * sizeof(float);
+    const dim3 grid(f.ntile * f.nsplit, d->Hkv, d->B);
+    int rc;
+    if (f.nw == 8) {
+      if ((rc = lds_limit<attn_f32<DH, 8>>(lds, "coda_diff_attn_fwd"))) return rc;
+      hipLaunchKernelGGL((attn_f32<DH, 8>), grid, dim3(512), lds, st, *d, f.qt, f.nsplit, f.per, (float*)d->workspace);
+    } else {
+      hipLaunchKernelGGL((attn_f32<DH, 4>), grid, dim3(256), lds, st, *d, f.qt, f.nsplit, f.per, (float*)d->workspace);
+    }
+    rc = check_launch("attn_f32");
+    if (rc || f.nsplit <= 1) return rc;
+    return launch_merge<float, DH>(d, st, f.qt, f.ntile, f.nsplit);
   }
   if (use_rows(d)) {
     const int ns = rows_nsplit(d);
@@ -2701,9 +2843,7 @@ static int launch_attn(const coda_attn_desc* d, hipStream_t st) {
                        (float*)d->workspace);
     int rc = check_launch("attn_rows_bf16");
     if (rc || ns_eff <= 1) return rc;
-    hipLaunchKernelGGL((attn_rows_merge<DH>), dim3(d->Hkv, d->B), dim3(256), 0, st, *d, ns_eff,
-                       (const float*)d->workspace);
-    return check_launch("attn_rows_merge");
+    return launch_merge<bf16_t, DH>(d, st, d->Lq, 1, ns_eff);
   }
   if constexpr (DH >= 64) {
     if ((G == 8 || G == 4 || G == 2 || G == 1) && flash_offsets_fit(d)) return launch_f3<DH>(d, st, G);
