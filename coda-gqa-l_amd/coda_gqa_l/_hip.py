@@ -122,6 +122,9 @@ _SIGS = {
     "coda_ring_rotate": (_i32, [ctypes.POINTER(BankDesc), _i32, _vp, ctypes.c_size_t, _vp]),
     "coda_unit_rows": (_i32, [_i32, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _i32, _i32, _vp]),
     "coda_project": (_i32, [ctypes.POINTER(ProjDesc), _vp]),
+    "coda_project_rows": (_i32, [ctypes.POINTER(ProjDesc), _vp]),
+    "coda_linear_rows": (_i32, [_i32, _vp, _i64, _i32, _vp, _i32, _i32, _vp, _vp, _i64, _vp]),
+    "coda_rows_pack": (_i32, [_i32, _vp, _i32, _i32, _i64, _vp, _vp]),
     "coda_project_workspace_bytes": (_i32, [ctypes.POINTER(ProjDesc), ctypes.POINTER(ctypes.c_size_t)]),
     "coda_topk_order_host": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp]),
     # the reference's typed epilogue symbols (void, errors in coda_last_error)

@@ -301,8 +301,8 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, nn.Module):
         float32 biases (zero for a linear without one) and the weights'
         layout code for coda_project, per parameter version; with half-split
         RoPE each k head's rows are reordered to the pairs (i, i + Dh/2) on
-        adjacent rows.  Where the row kernel serves D the weights are kept in
-        its fragment tiles (coda_project_pack, layout 1), else row-major (0)."""
+        adjacent rows.  On a HIP device the weights are kept in the row
+        kernel's fragment tiles (coda_rows_pack, layout 1)."""
         lins = (self.q_proj, self.k_proj, self.v_proj, self.lambda_proj, self.write_proj)
         ps = [t for lin in lins for t in (lin.weight, lin.bias) if t is not None]
         tag = tuple((t._version, t.data_ptr(), t.dtype, t.device) for t in ps) + (self.rope_interleaved,
@@ -333,17 +333,55 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, nn.Module):
             b = torch.cat([b, torch.zeros((-b.numel()) % 4, device=dev)])
             w = w.contiguous()
             layout = 0
-            if dtype == torch.bfloat16 and w.is_cuda:
-                n_feat, D = w.shape
-                wt = torch.empty((-(-n_feat // 64) * 64, D), dtype=dtype, device=dev)
-                rc = _hip.lib().coda_project_pack(w.data_ptr(), n_feat, D, D, wt.data_ptr(), _hip.stream_of(wt))
-                if rc == _hip.CODA_OK:
-                    w, layout = wt, 1
-                elif rc != _hip.CODA_EUNSUP:
-                    _hip.check(rc)
+            if w.is_cuda:
+                w, layout = self._rows_tiles(w), 1
         val = (w, b.contiguous(), layout)
         cache[("proj", dtype)] = (tag, val)
         return val
+
+    @staticmethod
+    def _rows_tiles(w: torch.Tensor) -> torch.Tensor:
+        """(n, D) weights in the row kernel's fragment tiles (coda_rows_pack)."""
+        n, D = w.shape
+        wt = torch.empty((-(-n // 64) * 64, D), dtype=w.dtype, device=w.device)
+        _hip.check(_hip.lib().coda_rows_pack(_hip.dtype_code(w.dtype), w.data_ptr(), n, D, w.stride(0), wt.data_ptr(),
+                                             _hip.stream_of(wt)))
+        return wt
+
+    @staticmethod
+    def _plain_call(x: torch.Tensor, *lins: nn.Module) -> bool:
+        """Whether calling these modules on x is no more than their matrix
+        product: nn.Linear in x's dtype, no hooks, no autocast, no gradient."""
+        if torch.is_autocast_enabled(x.device.type) or nn.modules.module._has_any_global_hook():
+            return False
+        grad = torch.is_grad_enabled()
+        if grad and x.requires_grad:
+            return False
+        for m in lins:
+            if type(m) is not nn.Linear or m.weight.dtype != x.dtype or m._forward_hooks or m._forward_pre_hooks or \
+                    grad and m.weight.requires_grad:
+                return False
+        return True
+
+    def _out_rows(self, heads: torch.Tensor) -> torch.Tensor:
+        """o_proj of decode-shaped heads (B, L, H*Dh): at most 32 token rows
+        through the row kernel (bf16 4096 x 4096: 8.1 us at 1 row and 11.1 at
+        32 against 12.0 and 12.4 for the library's GEMM, which is ahead at 64
+        with 12.8 against 14.5; and a shorter way through the host)."""
+        B, L, K = heads.shape
+        o = self.o_proj
+        if B * L > 32 or K % 64 or heads.dtype not in (torch.bfloat16, torch.float32) or \
+                not self._plain_call(heads, o) or not heads.is_contiguous():
+            return o(heads)
+        w = self._derived("o_rows", o.weight, heads.dtype, lambda: self._rows_tiles(o.weight.detach().contiguous()))
+        b = None
+        if o.bias is not None:
+            b = self._derived("o_bias", o.bias, heads.dtype, lambda: o.bias.detach().float().contiguous())
+        y = torch.empty((B, L, o.out_features), dtype=heads.dtype, device=heads.device)
+        _hip.check(_hip.lib().coda_linear_rows(
+            _hip.dtype_code(heads.dtype), heads.data_ptr(), K, B * L, w.data_ptr(), o.out_features, K, _hip.ptr(b),
+            y.data_ptr(), o.out_features, _hip.stream_of(heads)))
+        return y
 
     def _proj_desc(self, x: torch.Tensor, M: int, L: int, cos: torch.Tensor, sin: torch.Tensor):
         d = _hip.ProjDesc()
@@ -354,10 +392,19 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, nn.Module):
         return d
 
     def _fused_front_ok(self, x: torch.Tensor) -> bool:
-        """Whether coda_project serves x: bf16, at most 64 token rows, D a
-        multiple of 64, head_dim a multiple of 4."""
+        """Whether coda_project_rows serves x: D a multiple of 64, head_dim a
+        multiple of 4, and few token rows.  bf16: at most 64, or 128 (5 library
+        GEMMs with their sigmoids and RoPE take 103 us at 10305 x 8192 and 128
+        rows, the one launch 53); fp32: at most 32 (at 64 the library's GEMMs
+        are ahead)."""
         B, L, D = x.shape
-        return x.dtype == torch.bfloat16 and B * L <= 64 and D % 64 == 0 and self.head_dim % 4 == 0
+        if D % 64 or self.head_dim % 4:
+            return False
+        if x.dtype == torch.bfloat16 and B * L <= 64:
+            return True
+        most = 128 if x.dtype == torch.bfloat16 else 32 if x.dtype == torch.float32 else 0
+        return B * L <= most and self._plain_call(x, self.q_proj, self.k_proj, self.v_proj, self.lambda_proj,
+                                                  self.write_proj)
 
     def _front(self, x: torch.Tensor, p0: int, fused: bool = False):
         """Projections of x (B, L, D) at positions p0 ..: q (B,H,L,Dh)
@@ -378,8 +425,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, nn.Module):
         if fused:
             if not self._fused_front_ok(x):
                 raise NotImplementedError(
-                    "the fused projection front end serves bf16 inputs of at most 64 token rows (decode); many "
-                    "rows take the torch linears: a many-row fused form (an in-place epilogue over a library GEMM, "
+                    "the fused projection front end serves few token rows (decode: bf16 128, fp32 32); many rows take the torch linears: a many-row fused form (an in-place epilogue over a library GEMM, "
                     "q / k / v / lambda as strided views of its output) faulted the GPU in a full-size run with no "
                     "cause shown, and was removed")
             cos, sin = self._rope_rows(p0, L, x.device, x.dtype)
@@ -408,7 +454,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, nn.Module):
                 if ws is None or ws.numel() < nb[key]:
                     ws = cache[str(x.device)] = torch.empty(nb[key], dtype=torch.uint8, device=x.device)
             d.workspace, d.workspace_bytes = _hip.ptr(ws), nb[key]
-            _hip.check(_hip.lib().coda_project(d, _hip.stream_of(x)))
+            _hip.check(_hip.lib().coda_project_rows(d, _hip.stream_of(x)))
             return (q.view(B, L, H, Dh).permute(0, 2, 1, 3), k.permute(0, 2, 1, 3),
                     v.view(B, L, Hkv, Dh).permute(0, 2, 1, 3), g, lam.permute(0, 2, 1), cos, sin)
         cos, sin = self.rope(seq_len=L, offset=p0, device=x.device, dtype=x.dtype)
@@ -506,7 +552,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, nn.Module):
                 # one launch for q / k (roped) / v / lambda / gate
                 q, k_new, v_new, g, lam, cos, sin = self._front(x, q_pos, fused=True)
                 heads = self.decode_step_core(q, k_new, v_new, g.reshape(B), lam, state, cos, sin, k_roped=True)
-                return self.o_proj(heads.view(B, 1, self.num_heads * self.head_dim)), state
+                return self._out_rows(heads.view(B, 1, self.num_heads * self.head_dim)), state
             # the raw k projection: the step ropes it with the query's tables
             cos, sin = self.rope(seq_len=1, offset=q_pos, device=x.device, dtype=x.dtype)
             k_raw, v_new = self._project_kv_raw(x)
@@ -520,10 +566,10 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, nn.Module):
 
     def _step_fast(self, x: torch.Tensor, st: CoDAGQALandmarkStatePerf2) -> Optional[torch.Tensor]:
         """A steady-state decode step (full ring, fixed bank sizes, no
-        metrics or traces, bf16 decode-shaped input) from descriptors and
+        metrics or traces, decode-shaped input) from descriptors and
         buffers cached per state: per token the host sets the input and
-        RoPE-row pointers, makes two library calls (coda_project, then
-        coda_decode_step on its outputs) and the o_proj GEMM.  Returns None
+        RoPE-row pointers, makes two library calls (coda_project_rows,
+        then coda_decode_step on its outputs) and o_proj.  Returns None
         when the general path must run; the cache is rebuilt whenever a
         parameter, the state's tensors (object, storage or in-place version)
         or the batch changes."""
@@ -565,7 +611,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, nn.Module):
         fp["record_pos"] = pos + 1 if routed.value else -1
         # the general path's carried-record tag no longer matches this state
         self.__dict__["_route_tag"] = None
-        return self.o_proj(fp["heads_flat"])
+        return self._out_rows(fp["heads_flat"])
 
     def _param_key(self) -> tuple:
         """Identity and in-place version of every parameter of the layer and
@@ -636,7 +682,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, nn.Module):
               "keep": (keep, q, k, v, lam, g, heads, w, b, pws, ws, ct, sn, eta, self._rms_weight(dt)),
               "k_ptr": k.data_ptr(), "v_ptr": v.data_ptr(), "k_sb": Fk, "k_sh": Dh, "g_ptr": g.data_ptr(),
               "ws_ptr": _hip.ptr(ws), "ws_bytes": nb.value, "routed": routed, "routed_ref": ctypes.byref(routed),
-              "record_pos": routed_pos, "project": L_.coda_project, "step": L_.coda_decode_step,
+              "record_pos": routed_pos, "project": L_.coda_project_rows, "step": L_.coda_decode_step,
               "heads_flat": heads.view(B, 1, H * Dh)}
         self.__dict__["_fast"] = fp
         return fp

@@ -52,6 +52,19 @@ inline int lds_limit(size_t lds, const char* who) {
   return CODA_OK;
 }
 
+// compute units of the current device (read once per device)
+inline int device_cus() {
+  static std::atomic<int> cus[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cus[dev].load(std::memory_order_relaxed);
+  if (n <= 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cus[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
 // ----------------------------------------------------------------- types
 typedef uint16_t bf16_t;  // raw bfloat16 bits
 

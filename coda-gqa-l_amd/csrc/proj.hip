@@ -13,198 +13,220 @@
 // is packed with each pair (i, i + Dh/2) on adjacent weight rows).
 #include "common.h"
 
+#include <climits>
 
 namespace coda {
 
 typedef __bf16 pbf16x8_t __attribute__((ext_vector_type(8)));
 typedef float pf32x4 __attribute__((ext_vector_type(4)));
-typedef float pf32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t pu32x4 __attribute__((ext_vector_type(4)));
 
-static constexpr int kProjKT = 64;        // k per LDS stage
-static constexpr int kProjPitch = 72;     // LDS row pitch (bf16): 144 bytes, conflict-free fragment reads
+// dword 3 of a raw buffer resource on gfx9 (32-bit data format, no swizzle)
+static constexpr int kProjBufWord3 = 0x00020000;
+static constexpr int kProjKT = 64;        // D of coda_project: whole multiples
 
 __device__ __forceinline__ float proj_sigmoid(float x) { return 1.f / (1.f + expf(-x)); }
+
+// Four consecutive elements to memory: one 8-byte (bf16) or 16-byte (fp32,
+// any 4-byte address) store
+typedef float pf4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void proj_put4(bf16_t* p, const pf32x4& v) {
+  using E = Elt<bf16_t>;
+  uint2 w;
+  w.x = (uint32_t)E::st(v[0]) | ((uint32_t)E::st(v[1]) << 16);
+  w.y = (uint32_t)E::st(v[2]) | ((uint32_t)E::st(v[3]) << 16);
+  *reinterpret_cast<uint2*>(p) = w;
+}
+__device__ __forceinline__ void proj_put4(float* p, const pf32x4& v) { *reinterpret_cast<pf4u*>(p) = v; }
 
 // Epilogue of features f .. f + 3 (f a multiple of 4) of token row m:
 // the fp32 accumulators plus bias, rounded and routed to q / k (RoPE) / v /
 // lambda / gate
-__device__ __forceinline__ void proj_store4(const coda_proj_desc& d, int f, int m, pf32x4 v) {
-  using E = Elt<bf16_t>;
-  const int Fq = d.H * d.Dh, Fk = d.Hkv * d.Dh, half = d.Dh / 2;
-  const int o_k = Fq, o_v = Fq + Fk, o_l = Fq + 2 * Fk, o_g = o_l + d.H;
-  if (f + 3 < o_l) {  // q / k / v: the linear's bias (zero where it has none)
-    const float4 bb = *reinterpret_cast<const float4*>(d.bias + f);
-    v[0] += bb.x;
-    v[1] += bb.y;
-    v[2] += bb.z;
-    v[3] += bb.w;
+template <typename T>
+struct FrontEpilogue {
+  coda_proj_desc d;
+  __device__ __forceinline__ void operator()(int f, int m, pf32x4 v) const {
+    using E = Elt<T>;
+    const int Fq = d.H * d.Dh, Fk = d.Hkv * d.Dh, half = d.Dh / 2;
+    const int o_k = Fq, o_v = Fq + Fk, o_l = Fq + 2 * Fk, o_g = o_l + d.H;
+    if (f + 3 < o_l) {  // q / k / v: the linear's bias (zero where it has none)
+      const float4 bb = *reinterpret_cast<const float4*>(d.bias + f);
+      v[0] += bb.x;
+      v[1] += bb.y;
+      v[2] += bb.z;
+      v[3] += bb.w;
+    }
+    if (f + 3 < o_k) {  // q
+      proj_put4((T*)d.q + (int64_t)m * d.q_sm + f, v);
+    } else if (f >= o_k && f + 3 < o_v) {  // k: two RoPE pairs
+      const int kf = f - o_k, hk = kf / d.Dh, c = kf % d.Dh, prow = m % d.L;
+      const bool inter = d.rope_interleaved != 0;
+      const T* cs = (const T*)d.rope_cos;
+      const T* sn = (const T*)d.rope_sin;
+      T* krow = (T*)d.k + (int64_t)m * d.k_sm + (int64_t)hk * d.Dh;
+      float r[4];
+#pragma unroll
+      for (int pp = 0; pp < 2; ++pp) {
+        const int p = c / 2 + pp;  // pair index
+        const float cc = E::ld(cs[(int64_t)prow * half + p]), ss = E::ld(sn[(int64_t)prow * half + p]);
+        rope_pair_t<T>(E::rnd(v[2 * pp]), E::rnd(v[2 * pp + 1]), cc, ss, inter, r[2 * pp], r[2 * pp + 1]);
+      }
+      if (inter) {
+        proj_put4(krow + c, pf32x4{r[0], r[1], r[2], r[3]});
+      } else {  // packed pairs (p, p + half): channels c/2, c/2 + 1 and the same + half
+        const int p = c / 2;
+        krow[p] = E::st(r[0]);
+        krow[p + 1] = E::st(r[2]);
+        krow[p + half] = E::st(r[1]);
+        krow[p + half + 1] = E::st(r[3]);
+      }
+    } else if (f >= o_v && f + 3 < o_l) {  // v
+      proj_put4((T*)d.v + (int64_t)m * d.v_sm + (f - o_v), v);
+    } else {  // lambda / write gate, one feature at a time
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        const int ff = f + rr;
+        if (ff < o_l || ff >= o_g + (d.gate ? 1 : 0)) continue;
+        const float lin = E::rnd(v[rr] + d.bias[ff]);
+        const float sg = E::rnd(proj_sigmoid(lin));
+        if (ff < o_g) ((T*)d.lam)[(int64_t)m * d.lam_sm + (ff - o_l)] = E::st(sg);
+        else d.g[m] = sg;
+      }
+    }
   }
-  if (f + 3 < o_k) {  // q
-    uint2 w;
-    w.x = (uint32_t)E::st(v[0]) | ((uint32_t)E::st(v[1]) << 16);
-    w.y = (uint32_t)E::st(v[2]) | ((uint32_t)E::st(v[3]) << 16);
-    *reinterpret_cast<uint2*>((bf16_t*)d.q + (int64_t)m * d.q_sm + f) = w;
-  } else if (f >= o_k && f + 3 < o_v) {  // k: two RoPE pairs
-    const int kf = f - o_k, hk = kf / d.Dh, c = kf % d.Dh, prow = m % d.L;
-    const bool inter = d.rope_interleaved != 0;
-    const bf16_t* cs = (const bf16_t*)d.rope_cos;
-    const bf16_t* sn = (const bf16_t*)d.rope_sin;
-    bf16_t* krow = (bf16_t*)d.k + (int64_t)m * d.k_sm + (int64_t)hk * d.Dh;
-    float r[4];
+  // no gate column: the gate is 1
+  __device__ __forceinline__ void once(int t) const {
+    if (!d.gate && t < d.M) d.g[t] = 1.f;
+  }
+};
+
+// Epilogue of a plain linear layer: out = acc + bias, one rounding
+template <typename T>
+struct LinearEpilogue {
+  T* out;
+  const float* bias;  // or null
+  int64_t o_sm;
+  int n_feat;
+  __device__ __forceinline__ void operator()(int f, int m, pf32x4 v) const {
+    T* row = out + (int64_t)m * o_sm;
 #pragma unroll
-    for (int pp = 0; pp < 2; ++pp) {
-      const int p = c / 2 + pp;  // pair index
-      const float cc = E::ld(cs[(int64_t)prow * half + p]), ss = E::ld(sn[(int64_t)prow * half + p]);
-      rope_pair_t<bf16_t>(E::rnd(v[2 * pp]), E::rnd(v[2 * pp + 1]), cc, ss, inter, r[2 * pp], r[2 * pp + 1]);
-    }
-    if (inter) {
-      uint2 w;
-      w.x = (uint32_t)E::st(r[0]) | ((uint32_t)E::st(r[1]) << 16);
-      w.y = (uint32_t)E::st(r[2]) | ((uint32_t)E::st(r[3]) << 16);
-      *reinterpret_cast<uint2*>(krow + c) = w;
-    } else {  // packed pairs (p, p + half): channels c/2, c/2 + 1 and the same + half
-      const int p = c / 2;
-      *reinterpret_cast<uint32_t*>(krow + p) = (uint32_t)E::st(r[0]) | ((uint32_t)E::st(r[2]) << 16);
-      *reinterpret_cast<uint32_t*>(krow + p + half) = (uint32_t)E::st(r[1]) | ((uint32_t)E::st(r[3]) << 16);
-    }
-  } else if (f >= o_v && f + 3 < o_l) {  // v
-    uint2 w;
-    w.x = (uint32_t)E::st(v[0]) | ((uint32_t)E::st(v[1]) << 16);
-    w.y = (uint32_t)E::st(v[2]) | ((uint32_t)E::st(v[3]) << 16);
-    *reinterpret_cast<uint2*>((bf16_t*)d.v + (int64_t)m * d.v_sm + (f - o_v)) = w;
-  } else {  // lambda / write gate, one feature at a time
+    for (int e = 0; e < 4; ++e) v[e] += bias && f + e < n_feat ? bias[f + e] : 0.f;
+    if (f + 3 < n_feat) {
+      proj_put4(row + f, v);
+    } else {
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-      const int ff = f + rr;
-      if (ff < o_l || ff >= o_g + (d.gate ? 1 : 0)) continue;
-      const float lin = E::rnd(v[rr] + d.bias[ff]);
-      const float sg = E::rnd(proj_sigmoid(lin));
-      if (ff < o_g) ((bf16_t*)d.lam)[(int64_t)m * d.lam_sm + (ff - o_l)] = E::st(sg);
-      else d.g[m] = sg;
+      for (int e = 0; e < 4; ++e)
+        if (f + e < n_feat) row[f + e] = Elt<T>::st(v[e]);
     }
+  }
+  __device__ __forceinline__ void once(int) const {}
+};
+
+// Few token rows (M <= 128): the weights are the traffic.  A workgroup owns
+// 16 RB features over all of K: its 8 waves split K and stream their weight
+// rows and the token rows of that range straight from memory into MFMA
+// fragments, one 16 x 16 accumulator per 16 features and 16 tokens; the
+// partials meet in LDS and are summed in wave order (deterministic), then
+// the epilogue.  No workspace, no cross-workgroup exchange.  Weights cross
+// HBM once; the token rows are read by every workgroup from L2.
+// K goes in pairs of 64-byte steps: a lane's two 16-byte pieces of a row
+// come from the two halves of one 128-byte line, requested back to back.
+// Measured (bf16, weights not in cache): 6184 x 4096 M = 1 12.5 us, M = 16
+// 14.1 us (4.0 / 3.6 TB/s), 4096 x 4096 M = 1 8.1 us (the library 12.0),
+// 10305 x 8192 M = 1 30.4 us (5.5 TB/s).
+// TILED: W in fragment tiles (coda_project_pack), where the operand of row
+// block fb at k-step ks is the KiB at (fb D/32 + ks) 512 elements (bf16),
+// lane l's 16 bytes at 16 l; else row-major with row stride w_sm.
+template <typename T>
+__device__ __forceinline__ pf32x4 rows_mfma(const pu32x4& a, const pu32x4& b, pf32x4 c) {
+  if constexpr (sizeof(T) == 2) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(pbf16x8_t, a), __builtin_bit_cast(pbf16x8_t, b),
+                                                   c, 0, 0, 0);
+  } else {
+    const pf32x4 x = __builtin_bit_cast(pf32x4, a), y = __builtin_bit_cast(pf32x4, b);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], y[e], c, 0, 0, 0);
+    return c;
   }
 }
-
-// Workgroup tile: NTF features x MTT tokens; WF x WT waves, wave tile
-// (NTF / WF) x (MTT / WT) in 16 x 16 MFMA blocks.  K staged through LDS in
-// kProjKT slices, double-buffered through registers.
-template <int NTF, int MTT, int WF, int WT>
-__global__ __launch_bounds__(64 * WF * WT) void proj_gemm_bf16(const coda_proj_desc d, int n_feat) {
-  using E = Elt<bf16_t>;
-  constexpr int NT = 64 * WF * WT;
-  constexpr int BF = NTF / WF / 16, BT = MTT / WT / 16;
-  constexpr int ROWS = NTF + MTT, CH = kProjKT / 8, PER = ROWS * CH / NT;
-  static_assert(ROWS * CH % NT == 0, "whole 16-byte pieces per thread");
-  extern __shared__ __attribute__((aligned(16))) bf16_t proj_lds[];  // [2][ROWS * kProjPitch]
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int wf = wv % WF, wt = wv / WF;
-  const int f0 = blockIdx.x * NTF, m0 = blockIdx.y * MTT;
-  const bf16_t* W = (const bf16_t*)d.w;
-  const bf16_t* X = (const bf16_t*)d.x;
-  // this thread's pieces: row r of the stage (features first, then
-  // tokens), 16-byte chunk c; rows past the matrices read row 0 / M - 1
-  const bf16_t* src[PER];
-  int dst[PER];
+// waves whose partials meet in LDS at once: all 8, or 4 after the upper 4
+// have handed theirs to the lower 4
+template <int MT, int RB>
+struct RowsLds {
+  static constexpr int kWaves = RB * MT <= 8 ? 8 : 4;
+  static constexpr size_t kBytes = (size_t)kWaves * RB * MT * 64 * sizeof(pf32x4);
+};
+// The waves' partials (accumulators of 16 features x 16 tokens each), summed in
+// wave order, and the epilogue
+template <int MT, int RB, typename Epi>
+__device__ __forceinline__ void rows_finish(pf32x4 (&acc)[RB][MT], char* smem, int n_feat, int M, const Epi& epi) {
+  pf32x4* part = reinterpret_cast<pf32x4*>(smem);
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), f0 = blockIdx.x * 16 * RB;
+  constexpr int NWv = RowsLds<MT, RB>::kWaves;
+  if constexpr (NWv == 4) {
+    if (wv >= 4)
 #pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    const int i = t + u * NT, r = i / CH, c = i % CH;
-    if (r < NTF) {
-      const int f = min(f0 + r, n_feat - 1);
-      src[u] = W + (int64_t)f * d.D + 8 * c;
-    } else {
-      const int m = min(m0 + r - NTF, d.M - 1);
-      src[u] = X + (int64_t)m * d.x_sm + 8 * c;
-    }
-    dst[u] = r * kProjPitch + 8 * c;
-  }
-  uint4 reg[PER];
-  auto load = [&](int kb) {
+      for (int i = 0; i < RB; ++i)
 #pragma unroll
-    for (int u = 0; u < PER; ++u) reg[u] = *reinterpret_cast<const uint4*>(src[u] + kb * kProjKT);
-  };
-  auto store = [&](int buf) {
+        for (int j = 0; j < MT; ++j) part[(((wv - 4) * RB + i) * MT + j) * 64 + lane] = acc[i][j];
+    __syncthreads();
+    if (wv < 4)
 #pragma unroll
-    for (int u = 0; u < PER; ++u) *reinterpret_cast<uint4*>(&proj_lds[buf * ROWS * kProjPitch + dst[u]]) = reg[u];
-  };
-  pf32x4 acc[BF][BT];
+      for (int i = 0; i < RB; ++i)
 #pragma unroll
-  for (int i = 0; i < BF; ++i)
-#pragma unroll
-    for (int j = 0; j < BT; ++j) acc[i][j] = pf32x4{0.f, 0.f, 0.f, 0.f};
-  const int r16 = lane & 15, kq = lane >> 4;
-  const int nk = d.D / kProjKT;
-  load(0);
-  store(0);
-  __syncthreads();
-  for (int kb = 0; kb < nk; ++kb) {
-    if (kb + 1 < nk) load(kb + 1);
-    const bf16_t* L = proj_lds + (kb & 1) * ROWS * kProjPitch;
-#pragma unroll
-    for (int s = 0; s < kProjKT / 32; ++s) {
-      pbf16x8_t a[BF], b[BT];
-#pragma unroll
-      for (int i = 0; i < BF; ++i)
-        a[i] = *reinterpret_cast<const pbf16x8_t*>(L + ((wf * BF + i) * 16 + r16) * kProjPitch + 32 * s + 8 * kq);
-#pragma unroll
-      for (int j = 0; j < BT; ++j)
-        b[j] = *reinterpret_cast<const pbf16x8_t*>(L + (NTF + (wt * BT + j) * 16 + r16) * kProjPitch + 32 * s +
-                                                   8 * kq);
-#pragma unroll
-      for (int i = 0; i < BF; ++i)
-#pragma unroll
-        for (int j = 0; j < BT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-    if (kb + 1 < nk) store((kb + 1) & 1);
+        for (int j = 0; j < MT; ++j) acc[i][j] += part[((wv * RB + i) * MT + j) * 64 + lane];
     __syncthreads();
   }
-  // ---- epilogue: lane holds features fb + 4 g4 .. + 3 of token tb + (lane & 15)
+  if (wv < NWv)
 #pragma unroll
-  for (int j = 0; j < BT; ++j) {
-    const int m = m0 + (wt * BT + j) * 16 + r16;
-    if (m >= d.M) continue;
+    for (int i = 0; i < RB; ++i)
 #pragma unroll
-    for (int i = 0; i < BF; ++i) proj_store4(d, f0 + (wf * BF + i) * 16 + 4 * kq, m, acc[i][j]);
+      for (int j = 0; j < MT; ++j) part[((wv * RB + i) * MT + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  if (blockIdx.x == 0) epi.once(t);
+  // item 64 (MT i + j) + l: features f0 + 16 i + 4 (l / 16) .. + 3 of token
+  // 16 j + l % 16
+  for (int item = t; item < 64 * MT * RB; item += 512) {
+    const int ij = item >> 6, l = item & 63;
+    pf32x4 sum = part[ij * 64 + l];
+#pragma unroll
+    for (int w = 1; w < NWv; ++w) sum += part[(w * RB * MT + ij) * 64 + l];
+    const int m = 16 * (ij % MT) + (l & 15), f = f0 + 16 * (ij / MT) + 4 * (l >> 4);
+    if (m < M && f < n_feat) epi(f, m, sum);
   }
-  if (!d.gate && blockIdx.x == 0)
-    for (int m = m0 + t; m < min(d.M, m0 + MTT); m += NT) d.g[m] = 1.f;
 }
 
-// Few token rows (M <= 64): the weights are the traffic.  A workgroup owns
-// 16 features over all of K: wave w of 8 takes k in [w K/8, (w + 1) K/8)
-// and streams its 16 weight rows and the token rows of that range straight
-// from memory into MFMA fragments (16 bytes per lane and k-step, LA steps
-// ahead), one 16 x 16 accumulator per 16 tokens; the 8 partials meet in LDS
-// and are summed in wave order (deterministic), then the epilogue runs on
-// 64 MT lanes.  No workspace, no cross-workgroup exchange.  Weights cross
-// HBM once; the token rows (at most 512 KiB) are read by every workgroup
-// from L2.
-static constexpr int kRowsLA = 4;  // k-steps of loads in flight ahead of the products
-// RB row blocks of 16 features per wave: the token rows a wave loads feed
-// RB products each.  TILED: W in fragment tiles (coda_project_pack), where
-// the operand of row block fb at k-step ks is the KiB at (fb D/32 + ks) 512
-// elements, lane l's 16 bytes at 8 l; else row-major with row stride w_sm.
-template <int NS, int MT, int RB, bool TILED>
-__device__ __forceinline__ void rows_partial(const bf16_t* __restrict__ W, int64_t w_sm, int n_feat,
-                                             const bf16_t* __restrict__ X, int64_t x_sm, int M, int f0,
-                                             pf32x4* part) {
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6, r16 = lane & 15, kq = lane >> 4;
-  const int k0 = wv * (NS * 32) + 8 * kq;
-  const bf16_t* wr[RB];
-  // element step between k-steps: 32 columns, or one tile
-  constexpr int WS = TILED ? 512 : 32;
+template <typename T, int MT, int RB, bool TILED, typename Epi>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void proj_rows(
+    const T* __restrict__ W, int64_t w_sm, int n_feat, int D, const T* __restrict__ X, int64_t x_sm, int M,
+    const Epi epi) {
+  extern __shared__ __attribute__((aligned(16))) char rows_smem[];
+  // pairs of k-steps in flight ahead of the products
+  constexpr int LP = RB * MT <= 3 ? 4 : RB * MT <= 12 ? 2 : 1;
+  const int f0 = blockIdx.x * 16 * RB;
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), r16 = lane & 15, kq = lane >> 4;
+  const int pairs = D * (int)sizeof(T) / 128, p0 = pairs * wv / 8, np = pairs * (wv + 1) / 8 - p0;
+  // byte addresses of this lane's first piece of pair 0; WP / WH: bytes from
+  // a pair to the next, from its first half to its second
+  constexpr int WP = TILED ? 2048 : 128, WH = TILED ? 1024 : 64;
+  const char* wr[RB];
 #pragma unroll
   for (int i = 0; i < RB; ++i)
-    wr[i] = TILED ? W + ((int64_t)(f0 / 16 + i) * (8 * NS) + wv * NS) * 512 + 8 * lane
-                  : W + (int64_t)min(f0 + 16 * i + r16, n_feat - 1) * w_sm + k0;
-  const bf16_t* xr[MT];
+    wr[i] = TILED ? (const char*)W + ((int64_t)min(f0 / 16 + i, (n_feat + 15) / 16 - 1) * pairs + p0) * 2048 + 16 * lane
+                  : (const char*)(W + (int64_t)min(f0 + 16 * i + r16, n_feat - 1) * w_sm) + 128 * p0 + 16 * kq;
+  const char* xr[MT];
 #pragma unroll
-  for (int j = 0; j < MT; ++j) xr[j] = X + (int64_t)min(16 * j + r16, M - 1) * x_sm + k0;
-  pbf16x8_t a[kRowsLA][RB], b[kRowsLA][MT];
-  auto load = [&](int s) {
+  for (int j = 0; j < MT; ++j) xr[j] = (const char*)(X + (int64_t)min(16 * j + r16, M - 1) * x_sm) + 128 * p0 + 16 * kq;
+  pu32x4 a[LP][RB][2], b[LP][MT][2];
+  auto load = [&](int u, int p) {
 #pragma unroll
-    for (int i = 0; i < RB; ++i) a[s % kRowsLA][i] = *reinterpret_cast<const pbf16x8_t*>(wr[i] + WS * s);
+    for (int i = 0; i < RB; ++i)
 #pragma unroll
-    for (int j = 0; j < MT; ++j) b[s % kRowsLA][j] = *reinterpret_cast<const pbf16x8_t*>(xr[j] + 32 * s);
+      for (int h = 0; h < 2; ++h) a[u][i][h] = *reinterpret_cast<const pu32x4*>(wr[i] + WP * p + WH * h);
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) b[u][j][h] = *reinterpret_cast<const pu32x4*>(xr[j] + 128 * p + 64 * h);
   };
   pf32x4 acc[RB][MT];
 #pragma unroll
@@ -212,110 +234,250 @@ __device__ __forceinline__ void rows_partial(const bf16_t* __restrict__ W, int64
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[i][j] = pf32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int s = 0; s < kRowsLA && s < NS; ++s) load(s);
+  for (int u = 0; u < LP; ++u)
+    if (u < np) load(u, u);
+  auto products = [&](const pu32x4 (&as)[RB][2], const pu32x4 (&bs)[MT][2]) {
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    pbf16x8_t as[RB], bs[MT];
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int i = 0; i < RB; ++i) as[i] = a[s % kRowsLA][i];
+      for (int i = 0; i < RB; ++i)
 #pragma unroll
-    for (int j = 0; j < MT; ++j) bs[j] = b[s % kRowsLA][j];
-    if (s + kRowsLA < NS) load(s + kRowsLA);
+        for (int j = 0; j < MT; ++j) acc[i][j] = rows_mfma<T>(as[i][h], bs[j][h], acc[i][j]);
+  };
+  int p = 0;
+  for (; p + 2 * LP <= np; p += LP) {
 #pragma unroll
-    for (int i = 0; i < RB; ++i)
-#pragma unroll
-      for (int j = 0; j < MT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as[i], bs[j], acc[i][j], 0, 0, 0);
+    for (int u = 0; u < LP; ++u) {
+      products(a[u], b[u]);
+      load(u, p + u + LP);
+    }
   }
+#pragma unroll
+  for (int u = 0; u < 2 * LP; ++u) {
+    if (p + u >= np) break;
+    products(a[u % LP], b[u % LP]);
+    if (p + u + LP < np) load(u % LP, p + u + LP);
+  }
+  rows_finish<MT, RB>(acc, rows_smem, n_feat, M, epi);
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const char* p, int nbytes) {
+  const uint64_t v = (uint64_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(((uint64_t)hi << 32) | lo), (short)0,
+                                           __builtin_amdgcn_readfirstlane(nbytes), kProjBufWord3);
+}
+// The same for 17 .. 128 rows and K in whole chunks (8 waves x CS steps of 64
+// bytes): the token rows pass through LDS.  Operand loads straight from
+// memory take 16 rows' 64-byte pieces at a power-of-two stride, a quarter of
+// the rate of contiguous ones, and with 64 rows they outweigh the weights
+// (6184 x 4096, M = 64: 23.7 us with them, 18.8 us here; 10305 x 8192, M =
+// 128: 83 against 52.7 us; 4096 x 4096, M = 32: 12.1 against 11.1 us).  Per chunk and 16
+// tokens a wave loads its own part of the rows as CS * 64 contiguous bytes a
+// row into registers (two such slabs in flight), writes it to its LDS slab
+// and reads the operands back; 16-byte pieces are swizzled by the row, so
+// writes and reads spread over the banks.  The slab is the wave's alone and
+// LDS serves a wave in order: no barrier.  The next chunk's weights load
+// while this chunk's products run.  Same sums in the same order as proj_rows.
+template <typename T, int MT, int RB, int CS, typename Epi>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void proj_rows_lds(
+    const T* __restrict__ W, int n_feat, int D, const T* __restrict__ X, int64_t x_sm, int M, const Epi epi) {
+  extern __shared__ __attribute__((aligned(16))) char rows_smem[];
+  constexpr int RBY = CS * 64, PCS = RBY / 16, NI = 16 * PCS / 64, RPI = 64 / PCS;  // row bytes, pieces; loads a slab, rows a load
+  const int f0 = blockIdx.x * 16 * RB;
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), r16 = lane & 15, kq = lane >> 4;
+  const int steps = D * (int)sizeof(T) / 64, nc = steps / (8 * CS), s0 = nc * CS * wv;
+  char* slab = rows_smem + wv * 16 * RBY;
+  // weights and token rows through raw buffer resources: 32-bit offsets, and
+  // token rows past the last read 0 without touching memory
+  const int nfb = (n_feat + 15) / 16;
+  const __amdgpu_buffer_rsrc_t rw = rows_rsrc((const char*)W + (int64_t)(f0 / 16) * steps * 1024, RB * steps * 1024);
+  const __amdgpu_buffer_rsrc_t rx = rows_rsrc((const char*)X, (int)(((M - 1) * x_sm + D) * (int)sizeof(T)));
+  int wo[RB];
+#pragma unroll
+  for (int i = 0; i < RB; ++i) wo[i] = (min(f0 / 16 + i, nfb - 1) - f0 / 16) * steps * 1024 + s0 * 1024;
+  const int lr = lane / PCS, lp = lane % PCS, xrow = (int)x_sm * (int)sizeof(T);
+  const int xo = 64 * s0 + 16 * lp + lr * xrow;
+  pu32x4 a0[CS][RB], a1[CS][RB], x0[NI], x1[NI];
+  auto load_w = [&](pu32x4 (&w)[CS][RB], int c) {
+#pragma unroll
+    for (int s = 0; s < CS; ++s)
+#pragma unroll
+      for (int i = 0; i < RB; ++i)
+        w[s][i] = __builtin_amdgcn_raw_buffer_load_b128(rw, 16 * lane, wo[i] + (c * CS + s) * 1024, 0);
+  };
+  // slab (chunk c, tokens 16 j ..)
+  auto load_x = [&](pu32x4 (&v)[NI], int c, int j) {
+    const int cb = xo + c * RBY;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, cb + (16 * j + RPI * i) * xrow, 0, 0);
+  };
+  pf32x4 acc[RB][MT];
 #pragma unroll
   for (int i = 0; i < RB; ++i)
 #pragma unroll
-    for (int j = 0; j < MT; ++j) part[((wv * RB + i) * MT + j) * 64 + lane] = acc[i][j];
-  __syncthreads();
-}
-// Sum of the 8 waves' partials for (row block i, token block j, lane l) =
-// item 64 (MT i + j) + l: features f0 + 16 i + 4 (l / 16) .. + 3 of token
-// 16 j + l % 16
-template <int MT, int RB>
-__device__ __forceinline__ pf32x4 rows_sum(const pf32x4* part, int item) {
-  const int ij = item >> 6, l = item & 63;
-  pf32x4 sum = part[ij * 64 + l];
+    for (int j = 0; j < MT; ++j) acc[i][j] = pf32x4{0.f, 0.f, 0.f, 0.f};
+  auto tokens = [&](int c, int j, pu32x4 (&v)[NI], const pu32x4 (&w)[CS][RB], pf32x4 (&ac)[RB][MT]) {
 #pragma unroll
-  for (int w = 1; w < 8; ++w) sum += part[(w * RB * MT + ij) * 64 + l];
-  return sum;
+    for (int i = 0; i < NI; ++i) {
+      const int row = RPI * i + lr;
+      *reinterpret_cast<pu32x4*>(slab + row * RBY + ((lp ^ row) & (PCS - 1)) * 16) = v[i];
+    }
+    // slab j + 2 of the walk over (chunk, tokens); past the end: the last again
+    load_x(v, j + 2 < MT ? c : min(c + 1, nc - 1), (j + 2) % MT);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int s = 0; s < CS; ++s) {
+      const pu32x4 b = *reinterpret_cast<const pu32x4*>(slab + r16 * RBY + (((4 * s + kq) ^ r16) & (PCS - 1)) * 16);
+#pragma unroll
+      for (int i = 0; i < RB; ++i) ac[i][j] = rows_mfma<T>(w[s][i], b, ac[i][j]);
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  auto chunk = [&](int c, pu32x4 (&w)[CS][RB], pu32x4 (&wn)[CS][RB]) {
+    load_w(wn, min(c + 1, nc - 1));
+#pragma unroll
+    for (int j = 0; j < MT; j += 2) {
+      tokens(c, j, x0, w, acc);
+      tokens(c, j + 1, x1, w, acc);
+    }
+  };
+  static_assert(MT % 2 == 0, "slabs alternate between two register sets");
+  load_w(a0, 0);
+  load_x(x0, 0, 0);
+  load_x(x1, 0, 1);
+  int c = 0;
+  for (; c + 1 < nc; c += 2) {
+    chunk(c, a0, a1);
+    chunk(c + 1, a1, a0);
+  }
+  if (c < nc) chunk(c, a0, a1);
+  __syncthreads();
+  rows_finish<MT, RB>(acc, rows_smem, n_feat, M, epi);
 }
 
-template <int NS, int MT, int RB, bool TILED>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void proj_rows_bf16(
-    const coda_proj_desc d, int n_feat) {
-  __shared__ pf32x4 part[8 * RB * MT * 64];
-  const int f0 = blockIdx.x * 16 * RB;
-  rows_partial<NS, MT, RB, TILED>((const bf16_t*)d.w, d.D, n_feat, (const bf16_t*)d.x, d.x_sm, d.M, f0, part);
-  const int t = threadIdx.x;
-  if (!d.gate && blockIdx.x == 0 && t < d.M) d.g[t] = 1.f;
-  for (int item = t; item < 64 * MT * RB; item += 512) {
-    const pf32x4 sum = rows_sum<MT, RB>(part, item);
-    const int i = (item >> 6) / MT, j = (item >> 6) % MT, l = item & 63;
-    const int m = 16 * j + (l & 15), f = f0 + 16 * i + 4 * (l >> 4);
-    if (m < d.M && f < n_feat) proj_store4(d, f, m, sum);
+template <typename T, int MT, int RB, bool TILED, typename Epi>
+static int launch_rows_k(const T* W, int64_t w_sm, int n_feat, int D, const T* X, int64_t x_sm, int M, const Epi& epi,
+                         hipStream_t st, const char* who) {
+  constexpr size_t lds = RowsLds<MT, RB>::kBytes;
+  const int rc = lds_limit<proj_rows<T, MT, RB, TILED, Epi>>(lds, who);
+  if (rc) return rc;
+  hipLaunchKernelGGL((proj_rows<T, MT, RB, TILED, Epi>), dim3((n_feat + 16 * RB - 1) / (16 * RB)), dim3(512), lds, st, W,
+                     w_sm, n_feat, D, X, x_sm, M, epi);
+  return check_launch("proj_rows");
+}
+// Features a workgroup: the RB (1 .. 3) of the fewest 16-feature turns, ceil
+// (workgroups / CUs) * RB, and of these the largest (it reads the token rows
+// least often)
+static int rows_rb(int n_feat) {
+  const int cus = device_cus(), fb = (n_feat + 15) / 16;
+  int best = 1, turns = INT_MAX;
+  for (int rb = 1; rb <= 3; ++rb) {
+    const int n = ((fb + rb - 1) / rb + cus - 1) / cus * rb;
+    if (n <= turns) {
+      turns = n;
+      best = rb;
+    }
+  }
+  return best;
+}
+template <typename T, int MT, int RB, typename Epi>
+static int launch_rows_lds(const T* W, int n_feat, int D, const T* X, int64_t x_sm, int M, const Epi& epi,
+                           hipStream_t st, const char* who) {
+  // steps a chunk: as many as the accumulators leave registers for
+  constexpr int CS = RB * MT <= 4 ? 8 : RB * MT <= 16 ? 4 : 2;
+  constexpr size_t slabs = (size_t)8 * 16 * CS * 64;
+  constexpr size_t lds = slabs > RowsLds<MT, RB>::kBytes ? slabs : RowsLds<MT, RB>::kBytes;
+  const int rc = lds_limit<proj_rows_lds<T, MT, RB, CS, Epi>>(lds, who);
+  if (rc) return rc;
+  hipLaunchKernelGGL((proj_rows_lds<T, MT, RB, CS, Epi>), dim3((n_feat + 16 * RB - 1) / (16 * RB)), dim3(512), lds, st,
+                     W, n_feat, D, X, x_sm, M, epi);
+  return check_launch("proj_rows_lds");
+}
+template <typename T, int MT, bool TILED, typename Epi>
+static int launch_rows_mt(const T* W, int64_t w_sm, int n_feat, int D, const T* X, int64_t x_sm, int M, const Epi& epi,
+                          hipStream_t st, const char* who) {
+  if constexpr (TILED && MT > 1) {
+    // (token rows within a 31-bit offset)
+    if (D * sizeof(T) % 4096 == 0 && x_sm >= 0 && (M * x_sm + D) * (int64_t)sizeof(T) < INT_MAX) {
+      switch (rows_rb(n_feat)) {
+        case 1: return launch_rows_lds<T, MT, 1>(W, n_feat, D, X, x_sm, M, epi, st, who);
+        case 2: return launch_rows_lds<T, MT, 2>(W, n_feat, D, X, x_sm, M, epi, st, who);
+        default: return launch_rows_lds<T, MT, 3>(W, n_feat, D, X, x_sm, M, epi, st, who);
+      }
+    }
+  }
+  switch (rows_rb(n_feat)) {
+    case 1: return launch_rows_k<T, MT, 1, TILED>(W, w_sm, n_feat, D, X, x_sm, M, epi, st, who);
+    case 2: return launch_rows_k<T, MT, 2, TILED>(W, w_sm, n_feat, D, X, x_sm, M, epi, st, who);
+    default: return launch_rows_k<T, MT, 3, TILED>(W, w_sm, n_feat, D, X, x_sm, M, epi, st, who);
   }
 }
-
-template <int NS, int RB, bool TILED>
-static int launch_rows_t(const coda_proj_desc* d, int n_feat, hipStream_t st) {
-  const dim3 grid((n_feat + 16 * RB - 1) / (16 * RB));
-  if (d->M <= 16) hipLaunchKernelGGL((proj_rows_bf16<NS, 1, RB, TILED>), grid, dim3(512), 0, st, *d, n_feat);
-  else if (d->M <= 32) hipLaunchKernelGGL((proj_rows_bf16<NS, 2, RB, TILED>), grid, dim3(512), 0, st, *d, n_feat);
-  else hipLaunchKernelGGL((proj_rows_bf16<NS, 4, RB, TILED>), grid, dim3(512), 0, st, *d, n_feat);
-  return check_launch("proj_rows_bf16");
+template <typename T, bool TILED, typename Epi>
+static int launch_rows_t(const T* W, int64_t w_sm, int n_feat, int D, const T* X, int64_t x_sm, int M, const Epi& epi,
+                         hipStream_t st, const char* who) {
+  if (M <= 16) return launch_rows_mt<T, 1, TILED>(W, w_sm, n_feat, D, X, x_sm, M, epi, st, who);
+  if (M <= 32) return launch_rows_mt<T, 2, TILED>(W, w_sm, n_feat, D, X, x_sm, M, epi, st, who);
+  if (M <= 64) return launch_rows_mt<T, 4, TILED>(W, w_sm, n_feat, D, X, x_sm, M, epi, st, who);
+  return launch_rows_mt<T, 8, TILED>(W, w_sm, n_feat, D, X, x_sm, M, epi, st, who);
 }
-template <int NS, int RB>
-static int launch_rows_rb(const coda_proj_desc* d, int n_feat, hipStream_t st) {
-  return d->w_layout == 1 ? launch_rows_t<NS, RB, true>(d, n_feat, st) : launch_rows_t<NS, RB, false>(d, n_feat, st);
+template <typename T, typename Epi>
+static int launch_rows(const void* W, int64_t w_sm, int tiled, int n_feat, int D, const void* X, int64_t x_sm, int M,
+                       const Epi& epi, hipStream_t st, const char* who) {
+  return tiled ? launch_rows_t<T, true>((const T*)W, w_sm, n_feat, D, (const T*)X, x_sm, M, epi, st, who)
+               : launch_rows_t<T, false>((const T*)W, w_sm, n_feat, D, (const T*)X, x_sm, M, epi, st, who);
 }
-// 16 RB features per workgroup: RB 2 up to 16 k-steps per wave (K <= 4096),
-// RB 4 beyond (measured fastest at the 7B and 70B shapes, batch 1 .. 64)
-template <int NS>
-static int launch_rows_ns(const coda_proj_desc* d, int n_feat, hipStream_t st) {
-  return launch_rows_rb<NS, (NS <= 16 ? 2 : 4)>(d, n_feat, st);
-}
-static int launch_rows(const coda_proj_desc* d, int n_feat, hipStream_t st) {
-  switch (d->D / 256) {
-    case 2: return launch_rows_ns<2>(d, n_feat, st);
-    case 4: return launch_rows_ns<4>(d, n_feat, st);
-    case 8: return launch_rows_ns<8>(d, n_feat, st);
-    case 16: return launch_rows_ns<16>(d, n_feat, st);
-    case 32: return launch_rows_ns<32>(d, n_feat, st);
-    default: return -1;
-  }
-}
-// one thread per 16-byte piece of the tiled copy
-__global__ __launch_bounds__(256) void proj_pack_kernel(const bf16_t* __restrict__ w, int n_feat, int D, int64_t w_sm,
-                                                        bf16_t* __restrict__ out, int64_t n_pieces) {
+// one thread per 16-byte piece of the tiled copy; row_pieces: 16-byte pieces
+// of a row
+__global__ __launch_bounds__(256) void proj_pack_kernel(const char* __restrict__ w, int n_feat, int row_pieces,
+                                                        int64_t row_bytes, uint4* __restrict__ out, int64_t n_pieces) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n_pieces) return;
   const int l = (int)(i & 63), r = l & 15, q = l >> 4;
   const int64_t tile = i >> 6;
-  const int ksteps = D / 32;
+  const int ksteps = row_pieces / 4;
   const int64_t fb = tile / ksteps;
   const int ks = (int)(tile % ksteps);
   const int64_t f = fb * 16 + r;
   uint4 v = make_uint4(0u, 0u, 0u, 0u);
-  if (f < n_feat) v = *reinterpret_cast<const uint4*>(w + f * w_sm + 32 * ks + 8 * q);
-  *reinterpret_cast<uint4*>(out + 8 * i) = v;
+  if (f < n_feat) v = *reinterpret_cast<const uint4*>(w + f * row_bytes + 64 * ks + 16 * q);
+  out[i] = v;
+}
+static int launch_pack(int esz, const void* w, int n_feat, int D, int64_t w_sm, void* out, hipStream_t st) {
+  // (rows padded to a multiple of 64)
+  const int row_pieces = D * esz / 16;
+  const int64_t n_pieces = (int64_t)((n_feat + 63) / 64) * 64 * row_pieces;
+  hipLaunchKernelGGL(proj_pack_kernel, dim3((unsigned)((n_pieces + 255) / 256)), dim3(256), 0, st, (const char*)w, n_feat,
+                     row_pieces, w_sm * esz, (uint4*)out, n_pieces);
+  return check_launch("proj_pack_kernel");
 }
 
+// D of the tiled weights that coda_project_pack makes
 static bool rows_path(int D) {
   return D >= 512 && D <= 8192 && D % 256 == 0 && ((D / 256) & (D / 256 - 1)) == 0;
 }
 
-template <int NTF, int MTT, int WF, int WT>
-static int launch_proj(const coda_proj_desc* d, int n_feat, hipStream_t st) {
-  const dim3 grid((n_feat + NTF - 1) / NTF, (d->M + MTT - 1) / MTT);
-  const size_t lds = 2 * sizeof(bf16_t) * (NTF + MTT) * kProjPitch;
-  const int rc = lds_limit<proj_gemm_bf16<NTF, MTT, WF, WT>>(lds, "coda_project");
-  if (rc) return rc;
-  hipLaunchKernelGGL((proj_gemm_bf16<NTF, MTT, WF, WT>), grid, dim3(64 * WF * WT), lds, st, *d, n_feat);
-  return check_launch("proj_gemm_bf16");
+// What both front-end entries ask of a descriptor
+static int check_project(const coda_proj_desc* d, const char* who) {
+  CODA_REQUIRE(d->D > 0 && d->D % kProjKT == 0, "%s: D=%d must be a positive multiple of %d", who, d->D, kProjKT);
+  CODA_REQUIRE(d->H > 0 && d->Hkv > 0 && d->Dh > 0 && d->Dh % 4 == 0 && d->L > 0,
+               "%s: bad sizes H=%d Hkv=%d Dh=%d L=%d", who, d->H, d->Hkv, d->Dh, d->L);
+  CODA_REQUIRE(d->x && d->w && d->bias && d->rope_cos && d->rope_sin && d->q && d->k && d->v && d->lam && d->g,
+               "%s: pointer missing", who);
+  CODA_REQUIRE(((uintptr_t)d->bias % 16) == 0, "%s: bias must be 16-byte aligned", who);
+  const int pc = d->dtype == CODA_BF16 ? 8 : 4;  // elements of a 16-byte piece
+  CODA_REQUIRE(d->x_sm % pc == 0 && ((uintptr_t)d->x % 16) == 0 && ((uintptr_t)d->w % 16) == 0,
+               "%s: x / w rows must be 16-byte aligned", who);
+  CODA_REQUIRE(d->q_sm % 4 == 0 && d->k_sm % 4 == 0 && d->v_sm % 4 == 0 && ((uintptr_t)d->q % 8) == 0 &&
+                   ((uintptr_t)d->k % 8) == 0 && ((uintptr_t)d->v % 8) == 0,
+               "%s: q / k / v rows must be 8-byte aligned", who);
+  return CODA_OK;
+}
+template <typename T>
+static int run_project(const coda_proj_desc* d, hipStream_t st, const char* who) {
+  const int n_feat = d->H * d->Dh + 2 * d->Hkv * d->Dh + d->H + (d->gate ? 1 : 0);
+  return launch_rows<T>(d->w, d->D, d->w_layout, n_feat, d->D, d->x, d->x_sm, d->M, FrontEpilogue<T>{*d}, st, who);
 }
 
 }  // namespace coda
@@ -327,40 +489,62 @@ extern "C" int coda_project(const coda_proj_desc* d, void* stream) {
   CODA_REQUIRE(d->dtype == CODA_BF16, "coda_project: bf16 only");
   CODA_REQUIRE(d->M >= 0 && d->M <= 64, "coda_project: %d token rows; the front end serves decode-shaped inputs "
                "(at most 64 rows), many rows are library GEMMs", d->M);
-  CODA_REQUIRE(d->D > 0 && d->D % kProjKT == 0, "coda_project: D=%d must be a positive multiple of %d", d->D,
-               kProjKT);
-  CODA_REQUIRE(d->H > 0 && d->Hkv > 0 && d->Dh > 0 && d->Dh % 4 == 0 && d->L > 0,
-               "coda_project: bad sizes H=%d Hkv=%d Dh=%d L=%d", d->H, d->Hkv, d->Dh, d->L);
-  CODA_REQUIRE(d->x && d->w && d->bias && d->rope_cos && d->rope_sin && d->q && d->k && d->v && d->lam && d->g,
-               "coda_project: pointer missing");
-  CODA_REQUIRE(((uintptr_t)d->bias % 16) == 0, "coda_project: bias must be 16-byte aligned");
-  CODA_REQUIRE(d->x_sm % 8 == 0 && ((uintptr_t)d->x % 16) == 0 && ((uintptr_t)d->w % 16) == 0,
-               "coda_project: x / w rows must be 16-byte aligned");
-  CODA_REQUIRE(d->q_sm % 4 == 0 && d->k_sm % 4 == 0 && d->v_sm % 4 == 0 && ((uintptr_t)d->q % 8) == 0 &&
-                   ((uintptr_t)d->k % 8) == 0 && ((uintptr_t)d->v % 8) == 0,
-               "coda_project: q / k / v rows must be 8-byte aligned");
+  const int rc = check_project(d, "coda_project");
+  if (rc) return rc;
   if (d->M == 0) return CODA_OK;
-  const int n_feat = d->H * d->Dh + 2 * d->Hkv * d->Dh + d->H + (d->gate ? 1 : 0);
-  hipStream_t st = (hipStream_t)stream;
-  // K 512 .. 8192, a power of two times 256: row tiles over all of K (no
-  // workspace); else 64 x 64 tiles over K
   CODA_REQUIRE(d->w_layout == 0 || (d->w_layout == 1 && rows_path(d->D)),
                "coda_project: weight layout %d with D=%d (tiles serve the row kernel's D only)", d->w_layout, d->D);
-  if (rows_path(d->D)) return launch_rows(d, n_feat, st);
-  return launch_proj<64, 64, 4, 1>(d, n_feat, st);
+  return run_project<bf16_t>(d, (hipStream_t)stream, "coda_project");
+}
+
+extern "C" int coda_project_rows(const coda_proj_desc* d, void* stream) {
+  CODA_REQUIRE(d != nullptr, "coda_project_rows: null descriptor");
+  CODA_REQUIRE(d->dtype == CODA_BF16 || d->dtype == CODA_F32, "coda_project_rows: dtype must be CODA_F32 or CODA_BF16");
+  CODA_REQUIRE(d->M >= 0 && d->M <= 128, "coda_project_rows: %d token rows (at most 128)", d->M);
+  const int rc = check_project(d, "coda_project_rows");
+  if (rc) return rc;
+  if (d->M == 0) return CODA_OK;
+  CODA_REQUIRE(d->w_layout == 0 || d->w_layout == 1, "coda_project_rows: weight layout %d", d->w_layout);
+  return d->dtype == CODA_BF16 ? run_project<bf16_t>(d, (hipStream_t)stream, "coda_project_rows")
+                               : run_project<float>(d, (hipStream_t)stream, "coda_project_rows");
+}
+
+extern "C" int coda_linear_rows(int dtype, const void* x, int64_t x_sm, int M, const void* w, int n_feat, int D,
+                                const float* bias, void* out, int64_t o_sm, void* stream) {
+  CODA_REQUIRE(dtype == CODA_BF16 || dtype == CODA_F32, "coda_linear_rows: dtype must be CODA_F32 or CODA_BF16");
+  CODA_REQUIRE(M >= 0 && M <= 128 && n_feat > 0 && D > 0 && D % kProjKT == 0,
+               "coda_linear_rows: bad sizes M=%d n_feat=%d D=%d (at most 128 rows, D a multiple of %d)", M, n_feat, D,
+               kProjKT);
+  CODA_REQUIRE(x && w && out, "coda_linear_rows: null pointer");
+  const int pc = dtype == CODA_BF16 ? 8 : 4;
+  CODA_REQUIRE(x_sm % pc == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0,
+               "coda_linear_rows: x / w rows must be 16-byte aligned");
+  CODA_REQUIRE(o_sm % 4 == 0 && ((uintptr_t)out % 8) == 0, "coda_linear_rows: out rows must be 8-byte aligned");
+  if (M == 0) return CODA_OK;
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == CODA_BF16)
+    return launch_rows_t<bf16_t, true>((const bf16_t*)w, D, n_feat, D, (const bf16_t*)x, x_sm, M,
+                                       LinearEpilogue<bf16_t>{(bf16_t*)out, bias, o_sm, n_feat}, st,
+                                       "coda_linear_rows");
+  return launch_rows_t<float, true>((const float*)w, D, n_feat, D, (const float*)x, x_sm, M,
+                                    LinearEpilogue<float>{(float*)out, bias, o_sm, n_feat}, st, "coda_linear_rows");
+}
+
+extern "C" int coda_rows_pack(int dtype, const void* w, int n_feat, int D, int64_t w_sm, void* out, void* stream) {
+  CODA_REQUIRE(dtype == CODA_BF16 || dtype == CODA_F32, "coda_rows_pack: dtype must be CODA_F32 or CODA_BF16");
+  CODA_REQUIRE(w && out && n_feat > 0 && D > 0 && D % kProjKT == 0 && w_sm >= D, "coda_rows_pack: bad arguments");
+  const int esz = dtype == CODA_BF16 ? 2 : 4;
+  CODA_REQUIRE(w_sm * esz % 16 == 0 && ((uintptr_t)w % 16) == 0 && ((uintptr_t)out % 16) == 0,
+               "coda_rows_pack: rows must be 16-byte aligned");
+  return launch_pack(esz, w, n_feat, D, w_sm, out, (hipStream_t)stream);
 }
 
 extern "C" int coda_project_pack(const void* w, int n_feat, int D, int64_t w_sm, void* out, void* stream) {
   CODA_REQUIRE(w && out && n_feat > 0 && D > 0 && w_sm >= D, "coda_project_pack: bad arguments");
-  if (!rows_path(D)) return fail(CODA_EUNSUP, "coda_project_pack: D=%d does not take the row kernel", D);
+  if (!rows_path(D)) return fail(CODA_EUNSUP, "coda_project_pack: D=%d does not take the tiled weights", D);
   CODA_REQUIRE(w_sm % 8 == 0 && ((uintptr_t)w % 16) == 0 && ((uintptr_t)out % 16) == 0,
                "coda_project_pack: rows must be 16-byte aligned");
-  // rows padded to a multiple of 64: the row kernel reads up to 4 row
-  // blocks per workgroup past the last feature
-  const int64_t n_pieces = (int64_t)((n_feat + 63) / 64) * 4 * (D / 32) * 64;
-  hipLaunchKernelGGL(proj_pack_kernel, dim3((unsigned)((n_pieces + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                     (const bf16_t*)w, n_feat, D, w_sm, (bf16_t*)out, n_pieces);
-  return check_launch("proj_pack_kernel");
+  return launch_pack(2, w, n_feat, D, w_sm, out, (hipStream_t)stream);
 }
 
 extern "C" int coda_project_workspace_bytes(const coda_proj_desc* d, size_t* bytes) {

@@ -81,7 +81,7 @@ int coda_device_count(void);
  *   v_proj, lambda_proj + sigmoid, write_proj + sigmoid, and the RoPE of k.
  * ---------------------------------------------------------------------- */
 typedef struct {
-  int dtype;               /* CODA_BF16 */
+  int dtype;               /* CODA_BF16; coda_project_rows: CODA_F32 too */
   int M, D, L;             /* token rows, model width, tokens per sequence (table row = m % L) */
   int H, Hkv, Dh;
   int rope_interleaved;
@@ -106,14 +106,25 @@ typedef struct {
   size_t workspace_bytes;
 } coda_proj_desc;
 
-/* Decode-shaped inputs only: M <= 64 token rows (more rows: CODA_EINVAL;
- * the layer's prefill projections are library GEMMs).  D 512 .. 8192 and a
- * power of two times 256: each workgroup owns 32 features over all of K,
- * its 8 waves' K-range partials summed in LDS in wave order
- * (deterministic); the weights row-major or in fragment tiles.  Other D (a
- * multiple of 64): 64 x 64 tiles over K, row-major weights only.  No
- * workspace. */
+/* Decode-shaped inputs only: bf16, M <= 64 token rows (more rows:
+ * CODA_EINVAL).  Each workgroup owns 16 to 48 features over all of K, its 8
+ * waves' K-range partials summed in LDS in wave order (deterministic); the
+ * weights row-major, or in fragment tiles for D 512 .. 8192 and a power of
+ * two times 256.  No workspace. */
 int coda_project(const coda_proj_desc* d, void* stream);
+
+/* The same for M <= 128 token rows, CODA_F32 too (every product and sum in
+ * fp32, no rounding in between; tables, q, k, v and lam float), and fragment
+ * tiles (coda_rows_pack) for every D that is a multiple of 64. */
+int coda_project_rows(const coda_proj_desc* d, void* stream);
+
+/* out (M, n_feat; row stride o_sm) = x (M, D; row stride x_sm) W^T + bias
+ * for M <= 128 token rows: fp32 accumulation, one rounding.  w: the (n_feat,
+ * D) weights in fragment tiles (coda_rows_pack); bias: (n_feat) float32 or
+ * NULL; D a multiple of 64; rows 16-byte (x) and 8-byte (out) aligned.
+ * Replaces: o_proj of CoDAGQALandmarkPerf2.step (attention.py:538). */
+int coda_linear_rows(int dtype, const void* x, int64_t x_sm, int M, const void* w, int n_feat, int D,
+                     const float* bias, void* out, int64_t o_sm, void* stream);
 
 /* The weights of coda_project in fragment tiles (w_layout 1): for row block
  * fb of 16 rows and k-step ks of 32 columns, a 1 KiB tile at element offset
@@ -126,6 +137,11 @@ int coda_project(const coda_proj_desc* d, void* stream);
  * 8192, a power of two times 256): CODA_EUNSUP otherwise, nothing written.
  * No counterpart in the reference (its projections are nn.Linear). */
 int coda_project_pack(const void* w, int n_feat, int D, int64_t w_sm, void* out, void* stream);
+
+/* The same tiles for either dtype and every D that is a multiple of 64 (fp32:
+ * k-steps of 16 columns, element 4 (r + 16 q) + e holds W[16 fb + r][16 ks +
+ * 4 q + e], e < 4). */
+int coda_rows_pack(int dtype, const void* w, int n_feat, int D, int64_t w_sm, void* out, void* stream);
 
 /* Workspace bytes coda_project needs for this descriptor (0: the kernels
  * keep their partial sums in LDS; kept for callers that size one). */
