@@ -31,12 +31,13 @@ import torch.nn as nn
 from . import _hip, ops
 from .memory_banks import METRIC_KEYS, DeviceMetrics, MemoryBankMixin
 from .primitives import HeadwiseRMSNorm, RotaryEmbedding, apply_rope
+from .rows import RowsMixin
 from .state import CoDAGQALandmarkStatePerf2
 
 __all__ = ["CoDAGQALandmarkPerf2", "CoDAGQALandmarkStatePerf2"]
 
 
-class CoDAGQALandmarkPerf2(MemoryBankMixin, nn.Module):
+class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
     def __init__(
         self,
         *,
@@ -282,130 +283,6 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, nn.Module):
         return self._derived("rms_w", w, dtype, lambda: w.detach().to(dtype).contiguous())
 
     # ------------------------------------------------------------ projection front end
-    def _rope_rows(self, p0: int, L: int, device, dtype: torch.dtype) -> Tuple[torch.Tensor, torch.Tensor]:
-        """RoPE tables (L, Dh/2) of positions p0 .. p0 + L - 1: rows of one
-        cached table, grown by doubling; every element is the same fp32
-        product and cos / sin as in a table made for these positions alone."""
-        cache = self.__dict__.setdefault("_rope_cache", {})
-        key = (torch.device(device), dtype)
-        tab = cache.get(key)
-        need = int(p0) + int(L)
-        if tab is None or tab[0].shape[0] < need:
-            n = 1 << max(12, (need - 1).bit_length())
-            c, s_ = self.rope(seq_len=n, offset=0, device=device, dtype=dtype)
-            tab = cache[key] = (c.contiguous(), s_.contiguous())
-        return tab[0][p0:need], tab[1][p0:need]
-
-    def _proj_pack(self, dtype: torch.dtype):
-        """Packed [q | k | v | lambda | write] weights (n_feat, D) in `dtype`,
-        float32 biases (zero for a linear without one) and the weights'
-        layout code for coda_project, per parameter version; with half-split
-        RoPE each k head's rows are reordered to the pairs (i, i + Dh/2) on
-        adjacent rows.  On a HIP device the weights are kept in the row
-        kernel's fragment tiles (coda_rows_pack, layout 1)."""
-        lins = (self.q_proj, self.k_proj, self.v_proj, self.lambda_proj, self.write_proj)
-        ps = [t for lin in lins for t in (lin.weight, lin.bias) if t is not None]
-        tag = tuple((t._version, t.data_ptr(), t.dtype, t.device) for t in ps) + (self.rope_interleaved,
-                                                                                 self.write_policy)
-        cache = self.__dict__.setdefault("_derived_cache", {})
-        hit = cache.get(("proj", dtype))
-        if hit is not None and hit[0] == tag:
-            return hit[1]
-        H, Hkv, Dh = self.num_heads, self.num_kv_heads, self.head_dim
-        gate = self.write_policy != "none"
-        with torch.no_grad():
-            dev = self.q_proj.weight.device
-            wk, bk = self.k_proj.weight, self.k_proj.bias
-            if not self.rope_interleaved:
-                half = Dh // 2
-                pair = torch.stack([torch.arange(half), torch.arange(half) + half], 1).reshape(-1)
-                perm = (torch.arange(Hkv)[:, None] * Dh + pair[None]).reshape(-1).to(dev)
-                wk = wk[perm]
-                bk = bk[perm] if bk is not None else None
-            ws = [self.q_proj.weight, wk, self.v_proj.weight, self.lambda_proj.weight]
-            bt = [self.q_proj.bias, bk, self.v_proj.bias, self.lambda_proj.bias]
-            if gate:
-                ws.append(self.write_proj.weight)
-                bt.append(self.write_proj.bias)
-            w = torch.cat([t.detach() for t in ws]).to(dtype)
-            b = torch.cat([t.detach().float() if t is not None else torch.zeros(wt.shape[0], device=dev)
-                           for t, wt in zip(bt, ws)])
-            b = torch.cat([b, torch.zeros((-b.numel()) % 4, device=dev)])
-            w = w.contiguous()
-            layout = 0
-            if w.is_cuda:
-                w, layout = self._rows_tiles(w), 1
-        val = (w, b.contiguous(), layout)
-        cache[("proj", dtype)] = (tag, val)
-        return val
-
-    @staticmethod
-    def _rows_tiles(w: torch.Tensor) -> torch.Tensor:
-        """(n, D) weights in the row kernel's fragment tiles (coda_rows_pack)."""
-        n, D = w.shape
-        wt = torch.empty((-(-n // 64) * 64, D), dtype=w.dtype, device=w.device)
-        _hip.check(_hip.lib().coda_rows_pack(_hip.dtype_code(w.dtype), w.data_ptr(), n, D, w.stride(0), wt.data_ptr(),
-                                             _hip.stream_of(wt)))
-        return wt
-
-    @staticmethod
-    def _plain_call(x: torch.Tensor, *lins: nn.Module) -> bool:
-        """Whether calling these modules on x is no more than their matrix
-        product: nn.Linear in x's dtype, no hooks, no autocast, no gradient."""
-        if torch.is_autocast_enabled(x.device.type) or nn.modules.module._has_any_global_hook():
-            return False
-        grad = torch.is_grad_enabled()
-        if grad and x.requires_grad:
-            return False
-        for m in lins:
-            if type(m) is not nn.Linear or m.weight.dtype != x.dtype or m._forward_hooks or m._forward_pre_hooks or \
-                    grad and m.weight.requires_grad:
-                return False
-        return True
-
-    def _out_rows(self, heads: torch.Tensor) -> torch.Tensor:
-        """o_proj of decode-shaped heads (B, L, H*Dh): at most 32 token rows
-        through the row kernel (bf16 4096 x 4096: 8.1 us at 1 row and 11.1 at
-        32 against 12.0 and 12.4 for the library's GEMM, which is ahead at 64
-        with 12.8 against 14.5; and a shorter way through the host)."""
-        B, L, K = heads.shape
-        o = self.o_proj
-        if B * L > 32 or K % 64 or heads.dtype not in (torch.bfloat16, torch.float32) or \
-                not self._plain_call(heads, o) or not heads.is_contiguous():
-            return o(heads)
-        w = self._derived("o_rows", o.weight, heads.dtype, lambda: self._rows_tiles(o.weight.detach().contiguous()))
-        b = None
-        if o.bias is not None:
-            b = self._derived("o_bias", o.bias, heads.dtype, lambda: o.bias.detach().float().contiguous())
-        y = torch.empty((B, L, o.out_features), dtype=heads.dtype, device=heads.device)
-        _hip.check(_hip.lib().coda_linear_rows(
-            _hip.dtype_code(heads.dtype), heads.data_ptr(), K, B * L, w.data_ptr(), o.out_features, K, _hip.ptr(b),
-            y.data_ptr(), o.out_features, _hip.stream_of(heads)))
-        return y
-
-    def _proj_desc(self, x: torch.Tensor, M: int, L: int, cos: torch.Tensor, sin: torch.Tensor):
-        d = _hip.ProjDesc()
-        d.dtype, d.M, d.D, d.L = _hip.dtype_code(x.dtype), M, self.embed_dim, L
-        d.H, d.Hkv, d.Dh = self.num_heads, self.num_kv_heads, self.head_dim
-        d.rope_interleaved, d.gate = int(self.rope_interleaved), int(self.write_policy != "none")
-        d.rope_cos, d.rope_sin = cos.data_ptr(), sin.data_ptr()
-        return d
-
-    def _fused_front_ok(self, x: torch.Tensor) -> bool:
-        """Whether coda_project_rows serves x: D a multiple of 64, head_dim a
-        multiple of 4, and few token rows.  bf16: at most 64, or 128 (5 library
-        GEMMs with their sigmoids and RoPE take 103 us at 10305 x 8192 and 128
-        rows, the one launch 53); fp32: at most 32 (at 64 the library's GEMMs
-        are ahead)."""
-        B, L, D = x.shape
-        if D % 64 or self.head_dim % 4:
-            return False
-        if x.dtype == torch.bfloat16 and B * L <= 64:
-            return True
-        most = 128 if x.dtype == torch.bfloat16 else 32 if x.dtype == torch.float32 else 0
-        return B * L <= most and self._plain_call(x, self.q_proj, self.k_proj, self.v_proj, self.lambda_proj,
-                                                  self.write_proj)
-
     def _front(self, x: torch.Tensor, p0: int, fused: bool = False):
         """Projections of x (B, L, D) at positions p0 ..: q (B,H,L,Dh)
         pre-RoPE, k (B,Hkv,L,Dh) roped, v (B,Hkv,L,Dh), g (B,L) float32,
@@ -425,8 +302,8 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, nn.Module):
         if fused:
             if not self._fused_front_ok(x):
                 raise NotImplementedError(
-                    "the fused projection front end serves few token rows (decode: bf16 128, fp32 32); many rows take the torch linears: a many-row fused form (an in-place epilogue over a library GEMM, "
-                    "q / k / v / lambda as strided views of its output) faulted the GPU in a full-size run with no "
+                    "the fused projection front end serves few token rows (decode: bf16 128, fp32 32); many rows "
+                    "take the torch linears: a many-row fused form (an in-place epilogue over a library GEMM, q / k / v / lambda as strided views of its output) faulted the GPU in a full-size run with no "
                     "cause shown, and was removed")
             cos, sin = self._rope_rows(p0, L, x.device, x.dtype)
             d = self._proj_desc(x, M, L, cos, sin)

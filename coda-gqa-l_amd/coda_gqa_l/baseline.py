@@ -9,6 +9,7 @@ norm run inside one attention kernel (no repeat_kv copies, one K/V pass).
 
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Optional, Tuple
 
@@ -17,9 +18,10 @@ import torch.nn as nn
 
 from . import _hip, ops
 from .primitives import HeadwiseRMSNorm, RotaryEmbedding, apply_rope
+from .rows import RowsMixin
 
 
-class CoDAGQA(nn.Module):
+class CoDAGQA(RowsMixin, nn.Module):
     def __init__(self, *, embed_dim: int, num_heads: int, num_kv_heads: int, rope_base: float = 10_000.0,
                  lambda_init_bias: float = -6.0, theta_init: float = math.pi / 2, eps: float = 1e-6,
                  head_norm_mode: str = "full", rope_interleaved: bool = True):
@@ -81,6 +83,8 @@ class CoDAGQA(nn.Module):
         _hip.require_device(x)
         B, L, D = x.shape
         H, Hkv, Dh = self.num_heads, self.num_kv_heads, self.head_dim
+        if past_key_value is not None and self._decode_ok(x, past_key_value, is_causal):
+            return self._decode(x, *past_key_value)
         q = self.q_proj(x).view(B, L, H, Dh).permute(0, 2, 1, 3)
         k = self.k_proj(x).view(B, L, Hkv, Dh).permute(0, 2, 1, 3)
         v = self.v_proj(x).view(B, L, Hkv, Dh).permute(0, 2, 1, 3)
@@ -97,3 +101,74 @@ class CoDAGQA(nn.Module):
         # torch SDPA's is_causal aligns upper-left; with no past it is square
         heads = self.attention_core(q, k, v, lam, cos, sin, causal=2 if is_causal else 0)
         return self.o_proj(heads.view(B, L, D)), (k, v)
+
+    def _decode_ok(self, x: torch.Tensor, past: Tuple[torch.Tensor, torch.Tensor], is_causal: bool) -> bool:
+        """Whether _decode serves this call: few new tokens on top of a past,
+        no mask, bf16, at most 8 / G tokens a sequence, row-aligned K / V of
+        the layer's shape whose planes stay within the kernel's 31-bit offsets."""
+        B, L, _ = x.shape
+        k, v = past
+        if is_causal or L == 0 or x.dtype != torch.bfloat16 or k.dtype != x.dtype or v.dtype != x.dtype or \
+                2 * L * (self.num_heads // self.num_kv_heads) > 16 or self.head_dim not in (32, 64, 128):
+            return False
+        shape = (B, self.num_kv_heads, k.shape[2] if k.dim() == 4 else 0, self.head_dim)
+        st = k.stride()
+        return (tuple(k.shape) == shape and tuple(v.shape) == shape and shape[2] > 0 and v.stride() == st and
+                st[3] == 1 and not (st[0] % 8 or st[1] % 8 or st[2] % 8) and
+                0 <= st[2] and (shape[2] + L + 16) * max(st[2], self.head_dim) < 1 << 30 and
+                not (k.data_ptr() % 16 or v.data_ptr() % 16) and k.device == v.device == x.device and
+                not (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad)) and
+                self._fused_front_ok(x) and self._plain_call(x, self.q_proj, self.k_proj, self.v_proj,
+                                                             self.lambda_proj))
+
+    def _decode(self, x: torch.Tensor, k_past: torch.Tensor, v_past: torch.Tensor):
+        """forward() on top of a past for a few new tokens: one launch for the
+        projections and the RoPE of k (coda_project_rows), one for the
+        attention and the concatenated K / V (coda_attn_append, which reads
+        the past once for both), the merge of its splits, and o_proj."""
+        B, L, D = x.shape
+        H, Hkv, Dh = self.num_heads, self.num_kv_heads, self.head_dim
+        G, past, M, e = H // Hkv, k_past.shape[2], B * L, x.element_size()
+        lib, stream, dev = _hip.lib(), _hip.stream_of(x), x.device
+        xs = x if x.is_contiguous() and x.data_ptr() % 16 == 0 else x.contiguous()
+        cos, sin = self._rope_rows(past, L, dev, x.dtype)
+        th = self.theta
+        ct, st = self._derived("theta", th, x.dtype, lambda: (torch.cos(th).to(dtype=x.dtype).contiguous(),
+                                                              torch.sin(th).to(dtype=x.dtype).contiguous()))
+        w = self.head_norm.weight.detach().to(x.dtype).contiguous() if self.head_norm_mode == "full" else None
+        a = _hip.AttnDesc()
+        a.dtype = _hip.dtype_code(x.dtype)
+        a.B, a.H, a.Hkv, a.Lq, a.Dh = B, H, Hkv, L, Dh
+        # q | k | v | lambda | gate of the new tokens, then the heads, in one buffer
+        sizes = [M * D * e, M * Hkv * Dh * e, M * Hkv * Dh * e, M * H * e, M * 4]
+        at = [0]
+        for n in sizes:
+            at.append(at[-1] + -(-n // 256) * 256)
+        buf = torch.empty(at[-1], dtype=torch.uint8, device=dev)
+        heads = torch.empty((B, L, D), dtype=x.dtype, device=dev)
+        k, v = (torch.empty((B, Hkv, past + L, Dh), dtype=x.dtype, device=dev) for _ in range(2))
+        q_p, k_p, v_p, l_p, g_p = (buf.data_ptr() + o for o in at[:5])
+        d = self._proj_desc(x, M, L, cos, sin)
+        pw, pb, d.w_layout = self._proj_pack(x.dtype)
+        d.x, d.x_sm, d.w, d.bias = xs.data_ptr(), D, pw.data_ptr(), pb.data_ptr()
+        d.q, d.q_sm, d.k, d.k_sm, d.v, d.v_sm = q_p, D, k_p, Hkv * Dh, v_p, Hkv * Dh
+        d.lam, d.lam_sm, d.g = l_p, H, g_p
+        _hip.check(lib.coda_project_rows(d, stream))
+        a.q, a.q_sb, a.q_sh, a.q_sl = q_p, L * D, Dh, D
+        a.theta_cos, a.theta_sin = ct.data_ptr(), st.data_ptr()
+        a.rope_cos, a.rope_sin, a.rope_interleaved = cos.data_ptr(), sin.data_ptr(), int(self.rope_interleaved)
+        a.kp, a.vp, a.Lp = k_p, v_p, L
+        a.p_sb, a.p_sh, a.p_sl = L * Hkv * Dh, Dh, Hkv * Dh
+        a.kb, a.vb, a.Lb = k_past.data_ptr(), v_past.data_ptr(), past
+        a.b_sb, a.b_sh, a.b_sl = k_past.stride()[:3]
+        a.causal = 0
+        a.lam, a.lam_sb, a.lam_sh, a.lam_sl = l_p, L * H, 1, H
+        a.rms_w, a.eps, a.sm_scale = _hip.ptr(w), self._eps, 1.0 / math.sqrt(Dh)
+        a.out, a.o_sb, a.o_sh, a.o_sl = heads.data_ptr(), L * D, Dh, D
+        need = ctypes.c_size_t(0)
+        _hip.check(lib.coda_attn_workspace_bytes(a, need))
+        ws = torch.empty(need.value, dtype=torch.uint8, device=dev) if need.value else None
+        a.workspace, a.workspace_bytes = _hip.ptr(ws), need.value
+        _hip.check(lib.coda_attn_append(a, k.data_ptr(), v.data_ptr(), Hkv * (past + L) * Dh, (past + L) * Dh, Dh,
+                                        stream))
+        return self._out_rows(heads), (k, v)

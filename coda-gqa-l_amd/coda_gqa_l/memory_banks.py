@@ -186,20 +186,6 @@ class MemoryBankMixin:
                     t = t.to(st.k_buf.dtype)
                 setattr(st, name, t.contiguous())
 
-    def _derived(self, name: str, src: torch.Tensor, key, fn) -> torch.Tensor:
-        """Tensor derived from a parameter, recomputed only when the parameter
-        changes (in-place version counter or storage), so a decode step
-        launches no conversion kernels."""
-        cache = self.__dict__.setdefault("_derived_cache", {})
-        tag = (src._version, src.data_ptr(), src.dtype, src.device)
-        hit = cache.get((name, key))
-        if hit is not None and hit[0] == tag:
-            return hit[1]
-        with torch.no_grad():
-            val = fn()
-        cache[(name, key)] = (tag, val)
-        return val
-
     def _eta_f32(self, device, dtype: torch.dtype) -> torch.Tensor:
         """sigmoid(summary_eta_logit).to(dtype) per KV head, as float32 on the
         device (memory_banks.py:394, :902).  The sigmoid is torch's CPU op on

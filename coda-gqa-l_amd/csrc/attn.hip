@@ -309,8 +309,18 @@ __device__ __forceinline__ void store_vt(char* base, int kg, int d0, const uint4
 // Workgroup = (split, KV head, batch); 4 attention waves take 16-key tiles
 // in turn and merge their partial (m, l, O) in LDS; with nsplit > 1 each
 // workgroup leaves its merged partial in `ws` for attn_merge.
-template <int DH>
-__global__ __launch_bounds__(256) void attn_rows_bf16(const coda_attn_desc a, int keys_per_split, float* ws) {
+// APPEND: the keys and values also go to ap's buffers as they are read, the
+// block's rows first, then the prefix's: a decode step of the unbounded layer
+// (block = the past, prefix = the new tokens) makes its concatenated K / V in
+// the same pass over the past that attends to it.
+struct AppendTo {
+  bf16_t* k;
+  bf16_t* v;
+  int64_t sb, sh, sl;
+};
+template <int DH, bool APPEND>
+__global__ __launch_bounds__(256) void attn_rows_bf16(const coda_attn_desc a, int keys_per_split, float* ws,
+                                                      const AppendTo ap) {
   constexpr int NC = DH / 32, NM = DH / 16, NW = 4;
   __shared__ __attribute__((aligned(16))) char vt_smem[NW][VtLayout<DH>::kTileBytes];
   __shared__ float red_m[NW][16], red_l[NW][16];
@@ -396,6 +406,26 @@ __global__ __launch_bounds__(256) void attn_rows_bf16(const coda_attn_desc a, in
 #pragma unroll
     for (int jj = 0; jj < 4; ++jj)
       vv[jj] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rv, voff + jj * rb, 0, 0));
+  };
+  // this wave's i-th tile to the appended buffers (rows of other splits and
+  // tiles past the end excepted)
+  auto append = [&](int i, const bf16x8_t (&kf)[NC], const uint4 (&vv)[4]) {
+    const int t = wv + i * NW;
+    if (t >= n_tiles) return;
+    const bool pre = t < n1;
+    const int kt = tile_kt(t), hi = pre ? pe : kend;
+    const int64_t base = (int64_t)b * ap.sb + (int64_t)hk * ap.sh;
+    const int to = pre ? a.Lb : -a.Lp;  // key index -> row of the appended buffers
+    if (kt + n < hi) {
+      bf16_t* kr = ap.k + base + (int64_t)(kt + n + to) * ap.sl + 8 * g4;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) *reinterpret_cast<bf16x8_t*>(kr + 32 * c) = kf[c];
+    }
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {
+      const int kk = kt + 4 * kgl + jj;
+      if (vload && kk < hi) *reinterpret_cast<uint4*>(ap.v + base + (int64_t)(kk + to) * ap.sl + 8 * dcl) = vv[jj];
+    }
   };
   int row_qi = 0;
   // visibility of this lane's 4 keys (kt + 4 g4 + j) for query row n in
@@ -523,11 +553,13 @@ __global__ __launch_bounds__(256) void attn_rows_bf16(const coda_attn_desc a, in
     issue(i + 1, kf1, vv1);
     vm1 = tile_mask(i + 1);
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (APPEND) append(i, kf0, vv0);
     consume(kf0, vv0, vm0);
     if (i + 1 >= nt_w) break;
     issue(i + 2, kf0, vv0);
     vm0 = tile_mask(i + 2);
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (APPEND) append(i + 1, kf1, vv1);
     consume(kf1, vv1, vm1);
   }
   // merge the 4 attention waves
@@ -2793,6 +2825,24 @@ static int launch_merge(const coda_attn_desc* d, hipStream_t st, int qt, int nti
                      nsplit, (const float*)d->workspace);
   return check_launch("attn_merge");
 }
+template <int DH, bool APPEND>
+static int launch_rows(const coda_attn_desc* d, hipStream_t st, const AppendTo& ap) {
+  const int ns = rows_nsplit(d);
+  const int Lk = d->Lp + d->Lb;
+  int per = ((Lk + ns - 1) / ns + 15) / 16 * 16;
+  if (per < 16) per = 16;
+  const int ns_eff = Lk > 0 ? (Lk + per - 1) / per : 1;
+  if (ns_eff > 1) {
+    size_t need = (size_t)d->B * d->Hkv * ns_eff * 16 * (d->Dh + 2) * sizeof(float);
+    if (!d->workspace || d->workspace_bytes < need)
+      return fail(CODA_ESMALL, "coda_diff_attn_fwd: workspace %zu < %zu bytes", d->workspace_bytes, need);
+  }
+  hipLaunchKernelGGL((attn_rows_bf16<DH, APPEND>), dim3(ns_eff > 0 ? ns_eff : 1, d->Hkv, d->B), dim3(256), 0, st, *d, per,
+                     (float*)d->workspace, ap);
+  int rc = check_launch("attn_rows_bf16");
+  if (rc || ns_eff <= 1) return rc;
+  return launch_merge<bf16_t, DH>(d, st, d->Lq, 1, ns_eff);
+}
 template <int DH>
 static int launch_attn(const coda_attn_desc* d, hipStream_t st) {
   const int G = d->H / d->Hkv;
@@ -2816,23 +2866,7 @@ static int launch_attn(const coda_attn_desc* d, hipStream_t st) {
     if (rc || f.nsplit <= 1) return rc;
     return launch_merge<float, DH>(d, st, f.qt, f.ntile, f.nsplit);
   }
-  if (use_rows(d)) {
-    const int ns = rows_nsplit(d);
-    const int Lk = d->Lp + d->Lb;
-    int per = ((Lk + ns - 1) / ns + 15) / 16 * 16;
-    if (per < 16) per = 16;
-    const int ns_eff = Lk > 0 ? (Lk + per - 1) / per : 1;
-    if (ns_eff > 1) {
-      size_t need = (size_t)d->B * d->Hkv * ns_eff * 16 * (d->Dh + 2) * sizeof(float);
-      if (!d->workspace || d->workspace_bytes < need)
-        return fail(CODA_ESMALL, "coda_diff_attn_fwd: workspace %zu < %zu bytes", d->workspace_bytes, need);
-    }
-    hipLaunchKernelGGL((attn_rows_bf16<DH>), dim3(ns_eff > 0 ? ns_eff : 1, d->Hkv, d->B), dim3(256), 0, st, *d, per,
-                       (float*)d->workspace);
-    int rc = check_launch("attn_rows_bf16");
-    if (rc || ns_eff <= 1) return rc;
-    return launch_merge<bf16_t, DH>(d, st, d->Lq, 1, ns_eff);
-  }
+  if (use_rows(d)) return launch_rows<DH, false>(d, st, AppendTo{});
   if constexpr (DH >= 64) {
     if ((G == 8 || G == 4 || G == 2 || G == 1) && flash_offsets_fit(d)) return launch_f3<DH>(d, st, G);
   }
@@ -2871,6 +2905,32 @@ extern "C" int coda_prefill_attn_chunks(const coda_attn_desc* d, int n_chunks, i
   ChunkGeom cg{n_chunks, c_first, blk, L, W, 0, snap_stride, al_stride};
   hipStream_t st = (hipStream_t)stream;
   return w.Dh == 64 ? launch_f3<64>(&w, st, G, cg) : launch_f3<128>(&w, st, G, cg);
+}
+
+extern "C" int coda_attn_append(const coda_attn_desc* d, void* k_out, void* v_out, int64_t o_sb, int64_t o_sh,
+                                int64_t o_sl, void* stream) {
+  int rc = validate(d);
+  if (rc) return rc;
+  CODA_REQUIRE(use_rows(d) && d->causal == 0 && !d->allowed && d->Lq > 0,
+               "coda_attn_append: needs bf16, at most 8 / G queries, no mask");
+  CODA_REQUIRE(k_out && v_out && ((uintptr_t)k_out | (uintptr_t)v_out) % 16 == 0 && (o_sb | o_sh | o_sl) % 8 == 0 &&
+                   o_sl >= d->Dh,
+               "coda_attn_append: output rows must be 16-byte aligned");
+  const int64_t lim = (int64_t)1 << 30;  // elements: the kernel's 31-bit byte offsets into a plane
+  CODA_REQUIRE(d->b_sl >= 0 && d->p_sl >= 0 && (int64_t)(d->Lb + 16) * d->b_sl < lim &&
+                   (int64_t)(d->Lp + 16) * d->p_sl < lim,
+               "coda_attn_append: a (sequence, head) plane of keys beyond 2 GiB");
+  CODA_REQUIRE(((uintptr_t)d->kb | (uintptr_t)d->vb | (uintptr_t)d->kp | (uintptr_t)d->vp) % 16 == 0 &&
+                   (d->b_sb | d->b_sh | d->b_sl | d->p_sb | d->p_sh | d->p_sl) % 8 == 0,
+               "coda_attn_append: key rows must be 16-byte aligned");
+  if (d->B == 0) return CODA_OK;
+  const AppendTo ap{(bf16_t*)k_out, (bf16_t*)v_out, o_sb, o_sh, o_sl};
+  hipStream_t st = (hipStream_t)stream;
+  switch (d->Dh) {
+    case 32: return launch_rows<32, true>(d, st, ap);
+    case 64: return launch_rows<64, true>(d, st, ap);
+    default: return launch_rows<128, true>(d, st, ap);
+  }
 }
 
 extern "C" int coda_diff_attn_fwd(const coda_attn_desc* d, void* stream) {

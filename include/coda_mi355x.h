@@ -215,6 +215,16 @@ int coda_attn_workspace_bytes(const coda_attn_desc* d, size_t* bytes);
 
 int coda_diff_attn_fwd(const coda_attn_desc* d, void* stream);
 
+/* The attention of a decode step over [block = the past | prefix = the new
+ * tokens] (causal 0, no `allowed`, at most 8 / G query rows, bf16) that also
+ * writes the concatenation, block rows first, to k_out / v_out (element
+ * strides o_sb, o_sh, o_sl; 16-byte aligned rows).  Workspace as
+ * coda_attn_workspace_bytes says.
+ * Replaces: the two torch.cat and the attention of CoDAGQA.forward with
+ *   past_key_value (src/coda_gqa_l/baseline.py:113-141). */
+int coda_attn_append(const coda_attn_desc* d, void* k_out, void* v_out, int64_t o_sb, int64_t o_sh,
+                     int64_t o_sl, void* stream);
+
 /* The attention of chunks c_first .. c_first + n_chunks - 1 of a chunked
  * prefill call in one launch, from bank snapshots instead of the live state.
  * Chunk c covers queries [t0, t0 + Lq) of the call, t0 = c * blk,
