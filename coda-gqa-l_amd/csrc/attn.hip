@@ -1915,6 +1915,14 @@ __device__ __forceinline__ void lds_wait2_n(uint2& a, uint2& b) {
   asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(a), "+v"(b) : "i"(N));
 }
 
+// m = max(m, a, b) in one instruction, kept where it stands (written as
+// fmaxf, the compiler first quiets every accumulator, three instructions a
+// pair, and sinks all of it below the products it is meant to run beside).
+// a, b are results of products finished at least two products earlier.
+__device__ __forceinline__ void vmax3(float& m, float a, float b) {
+  asm volatile("v_max3_f32 %0, %0, %1, %2" : "+v"(m) : "v"(a), "v"(b));
+}
+
 template <int DH>
 struct F2Layout {
   static constexpr int KT = 64;                  // keys per tile
@@ -2596,33 +2604,34 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     {
       const uint32_t va = lds_addr(vbuf(it));
       constexpr int NPV = 4 * NDB;
-      uint2 rd[3][2];
+      // VAH reads ahead of the products (LDS latency is some three products)
+      constexpr int VAH = 5, NRD = VAH + 1;
+      uint2 rd[NRD][2];
       auto v_issue = [&](auto q_c) {
         constexpr int q = decltype(q_c)::value;
         if constexpr (q < NPV) {
           constexpr int p = q / NDB, db = q % NDB;
           constexpr int ROW0 = 16 * p * Lay::ROWB, ROW8 = ROW0 + 8 * Lay::ROWB;
-          rd[q % 3][0] = lds_read_tr16_at<ROW0>(va + v_off[db]);
-          rd[q % 3][1] = lds_read_tr16_at<ROW8>(va + v_off[db]);
+          rd[q % NRD][0] = lds_read_tr16_at<ROW0>(va + v_off[db]);
+          rd[q % NRD][1] = lds_read_tr16_at<ROW8>(va + v_off[db]);
         }
       };
-      v_issue(std::integral_constant<int, 0>{});
-      v_issue(std::integral_constant<int, 1>{});
+      static_for<VAH>([&](auto q_c) { v_issue(q_c); });
       static_for<NPV>([&](auto q_c) {
         constexpr int q = decltype(q_c)::value;
-        constexpr int p = q / NDB, db = q % NDB, b3 = q % 3;
-        lds_wait2_n<(q + 1 < NPV) ? 2 : 0>(rd[b3][0], rd[b3][1]);
+        constexpr int p = q / NDB, db = q % NDB, b3 = q % NRD;
+        constexpr int later = NPV - 1 - q < VAH - 1 ? NPV - 1 - q : VAH - 1;  // reads issued after this product's
+        lds_wait2_n<2 * later>(rd[b3][0], rd[b3][1]);
         const bf16x8_t va8 = __builtin_bit_cast(bf16x8_t, uint4{rd[b3][0].x, rd[b3][0].y, rd[b3][1].x, rd[b3][1].y});
         const uint4 pf = uint4{pw[4 * p], pw[4 * p + 1], pw[4 * p + 2], pw[4 * p + 3]};
         o[db] = mfma_32x32x16(va8, __builtin_bit_cast(bf16x8_t, pf), o[db]);
+        v_issue(std::integral_constant<int, q + VAH>{});
         constexpr int PER = 32 / NPV;
 #pragma unroll
-        for (int u = 0; u < PER; ++u) {
+        for (int u = 0; u < PER; u += 2) {
           constexpr int e0 = PER * q;
-          mx = fmaxf(mx, st[NXT][(e0 + u) >> 4][(e0 + u) & 15]);
+          vmax3(mx, st[NXT][(e0 + u) >> 4][(e0 + u) & 15], st[NXT][(e0 + u) >> 4][(e0 + u + 1) & 15]);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        v_issue(std::integral_constant<int, q + 2>{});
         __builtin_amdgcn_sched_barrier(0);
       });
     }
