@@ -573,7 +573,7 @@ __global__ __launch_bounds__(256) void attn_rows_bf16(const coda_attn_desc a, in
   __syncthreads();
 
   if (nsplit > 1) {
-    // partial row r: [m, l, O(DH)] unnormalised w.r.t. the merged max
+    // partial row r (attn_merge's layout): m, l, O(DH) unnormalised w.r.t. the merged max
     float* base = ws + ((((int64_t)b * a.Hkv + hk) * nsplit + split) * 16) * (DH + 2);
     for (int i = threadIdx.x; i < R * (DH + 2); i += blockDim.x) {
       const int r = i / (DH + 2), c = i % (DH + 2);
@@ -591,7 +591,7 @@ __global__ __launch_bounds__(256) void attn_rows_bf16(const coda_attn_desc a, in
 #pragma unroll
         for (int w = 0; w < NW; ++w) v += red_o[w][r][c - 2] * exp2f(red_m[w][r] - Mu);
       }
-      base[r * (DH + 2) + c] = v;
+      base[c < 2 ? 16 * DH + 16 * c + r : r * DH + c - 2] = v;
     }
     return;
   }
@@ -639,18 +639,92 @@ __global__ __launch_bounds__(256) void attn_rows_bf16(const coda_attn_desc a, in
   }
 }
 
-// Merge the per-split partials of attn_rows_bf16 / attn_f32 and apply the
-// epilogue: a workgroup per output row (query tile, head, query), since the
-// work is a few dependent round trips and little else.  The row's two streams
-// take their maxima and sums over the splits on 128 threads each, then 256 /
-// DH groups of threads sum the splits' channels.  Partials are [pair][tile]
-// [split][16 rows][m, l, O(DH)], row st * GL + orow of a tile of qt queries,
-// GL = G * qt, orow = g * qt + query.  (4096 keys, 32 pairs, 16 splits: 30 us
-// with a workgroup a pair that walked the splits one after the other.)
-static constexpr int kMaxSplits = 512;
-template <typename T, int DH>
-__global__ __launch_bounds__(256) void attn_merge(const coda_attn_desc a, int qt, int nsplit, const float* ws) {
+__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// Merge of the per-split partials of attn_rows_bf16, attn_f32 and attn_f3_bf16,
+// and the epilogue.  Partials are [pair][tile][split] blocks of R rows, O [R][DH]
+// then m [R], l [R]; row st * GL + orow of a tile of qt queries, GL = G * qt,
+// orow = g * qt + query.  FLASH: the epilogue of attn_f3_bf16 (fp32, the noise
+// output rounded once) instead of the eager ops' rounding.
+static constexpr int kMaxSplits = 512, kFewSplits = 64;
+template <typename T, int DH, bool FLASH>
+__device__ __forceinline__ void merge_store(const coda_attn_desc& a, int b, int h, int qi, int lane,
+                                            const float (&os)[(DH + 63) / 64], const float (&on)[(DH + 63) / 64]) {
   using E = Elt<T>;
+  constexpr int NV = (DH + 63) / 64;
+  float y[NV];
+  bool act[NV];
+  int dd[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    act[i] = lane + 64 * i < DH;
+    dd[i] = act[i] ? lane + 64 * i : 0;
+  }
+  const float lam = E::ld(((const T*)a.lam)[b * a.lam_sb + h * a.lam_sh + qi * a.lam_sl]);
+  if constexpr (FLASH) {
+    float sq = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      y[i] = fmaf(-lam, E::rnd(on[i]), os[i]);
+      sq = fmaf(y[i], y[i], sq);  // (0 past DH)
+    }
+    if (a.rms_w) {
+      const float rr = 1.0f / sqrtf(wave_sum(sq) / (float)DH + a.eps);
+#pragma unroll
+      for (int i = 0; i < NV; ++i) y[i] *= rr * E::ld(((const T*)a.rms_w)[dd[i]]);
+    }
+  } else {
+    diff_norm<T, NV>(y, os, on, act, lam, (const T*)a.rms_w, dd, a.eps, DH, true, 0, 0);
+  }
+  T* orow_p = (T*)a.out + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_sl;
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+    if (act[i]) orow_p[dd[i]] = E::st(y[i]);
+}
+
+// At most kFewSplits splits: a wave per output row, four rows a workgroup, a
+// lane per split for the weights, no barrier.  Two dependent round trips and
+// the partials' bytes (a workgroup a row and its barriers: 18 us for 8192
+// rows of two splits, about 8 here).
+template <typename T, int DH, bool FLASH>
+__global__ __launch_bounds__(256) void attn_merge_few(const coda_attn_desc a, int qt, int R, int nsplit, const float* ws) {
+  constexpr int NV = (DH + 63) / 64;
+  const int G = a.H / a.Hkv, GL = G * qt, lane = threadIdx.x & 63;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), ntile = (a.Lq + qt - 1) / qt;
+  const int tile = row / GL, orow = row % GL, g = orow / qt, qi = tile * qt + orow % qt;
+  if (tile >= ntile || qi >= a.Lq) return;
+  const int b = blockIdx.y / a.Hkv, hk = blockIdx.y % a.Hkv, blk = R * (DH + 2);
+  const float* base = ws + ((int64_t)blockIdx.y * ntile + tile) * nsplit * blk;
+  float o[2][NV];
+#pragma unroll
+  for (int st = 0; st < 2; ++st) {
+    const int rs = st * GL + orow;
+    const float* ml = base + min(lane, nsplit - 1) * blk + R * DH + rs;
+    const float mv = lane < nsplit ? ml[0] : -INFINITY, lv = ml[R];
+    const float M = wave_max(mv), Mu = M == -INFINITY ? 0.f : M;
+    const float w = fast_exp2(mv - Mu);
+    const float L = wave_sum(lane < nsplit ? lv * w : 0.f);
+    float acc[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) acc[i] = 0.f;
+#pragma unroll 8
+    for (int sp = 0; sp < nsplit; ++sp) {
+      const float f = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), sp));
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        acc[i] = fmaf(base[sp * blk + rs * DH + min(lane + 64 * i, DH - 1)], f, acc[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) o[st][i] = lane + 64 * i < DH && L > 0.f ? acc[i] / L : 0.f;
+  }
+  merge_store<T, DH, FLASH>(a, b, hk * G + g, qi, lane, o[0], o[1]);
+}
+
+// More splits (few query rows over very many keys): a workgroup per output
+// row, its two streams' maxima and sums over the splits on 128 threads each,
+// then 256 / DH groups of threads sum the splits' channels.
+template <typename T, int DH>
+__global__ __launch_bounds__(256) void attn_merge(const coda_attn_desc a, int qt, int R, int nsplit, const float* ws) {
   constexpr int NG = 256 / DH, NV = (DH + 63) / 64;
   __shared__ float wts[2][kMaxSplits], red[4], acc_lds[2][NG][DH];
   const int G = a.H / a.Hkv, GL = G * qt, ntile = gridDim.x / GL;
@@ -659,10 +733,10 @@ __global__ __launch_bounds__(256) void attn_merge(const coda_attn_desc a, int qt
   if (qi >= a.Lq) return;
   const int b = blockIdx.y / a.Hkv, hk = blockIdx.y % a.Hkv, h = hk * G + g;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const float* base = ws + ((int64_t)blockIdx.y * ntile + tile) * nsplit * 16 * (DH + 2);
-  const int st = t >> 7, rs = st * GL + orow;
+  const int st = t >> 7, rs = st * GL + orow, blk = R * (DH + 2);
+  const float* base = ws + ((int64_t)blockIdx.y * ntile + tile) * nsplit * blk;
   float M = -INFINITY;
-  for (int sp = t & 127; sp < nsplit; sp += 128) M = fmaxf(M, base[(sp * 16 + rs) * (DH + 2)]);
+  for (int sp = t & 127; sp < nsplit; sp += 128) M = fmaxf(M, base[sp * blk + R * DH + rs]);
   M = wave_max(M);
   if (lane == 0) red[wv] = M;
   __syncthreads();
@@ -670,10 +744,10 @@ __global__ __launch_bounds__(256) void attn_merge(const coda_attn_desc a, int qt
   const float Mu = M == -INFINITY ? 0.f : M;
   float L = 0.f;
   for (int sp = t & 127; sp < nsplit; sp += 128) {
-    const float* pr = base + (sp * 16 + rs) * (DH + 2);
+    const float* pr = base + sp * blk + R * DH + rs;
     const float w = exp2f(pr[0] - Mu);
     wts[st][sp] = w;
-    L += pr[1] * w;
+    L += pr[R] * w;
   }
   L = wave_sum(L);
   __syncthreads();
@@ -681,36 +755,27 @@ __global__ __launch_bounds__(256) void attn_merge(const coda_attn_desc a, int qt
   const int d = t % DH, gq = t / DH;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    const float* pr = base + (s * GL + orow) * (DH + 2) + 2 + d;
+    const float* pr = base + (s * GL + orow) * DH + d;
     float acc = 0.f;
 #pragma unroll 4
-    for (int sp = gq; sp < nsplit; sp += NG) acc += pr[sp * 16 * (DH + 2)] * wts[s][sp];
+    for (int sp = gq; sp < nsplit; sp += NG) acc += pr[sp * blk] * wts[s][sp];
     acc_lds[s][gq][d] = acc;
   }
   __syncthreads();
   if (wv > 0) return;
-  float o[2][NV], y[NV];
-  bool act[NV];
-  int dd[NV];
+  float o[2][NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    act[i] = lane + 64 * i < DH;
-    dd[i] = act[i] ? lane + 64 * i : 0;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const float Ls = red[2 * s] + red[2 * s + 1];
       float acc = 0.f;
 #pragma unroll
-      for (int k = 0; k < NG; ++k) acc += acc_lds[s][k][dd[i]];
-      o[s][i] = act[i] && Ls > 0.f ? acc / Ls : 0.f;
+      for (int k = 0; k < NG; ++k) acc += acc_lds[s][k][min(lane + 64 * i, DH - 1)];
+      o[s][i] = lane + 64 * i < DH && Ls > 0.f ? acc / Ls : 0.f;
     }
   }
-  const float lam = E::ld(((const T*)a.lam)[b * a.lam_sb + h * a.lam_sh + qi * a.lam_sl]);
-  diff_norm<T, NV>(y, o[0], o[1], act, lam, (const T*)a.rms_w, dd, a.eps, DH, true, 0, 0);
-  T* orow_p = (T*)a.out + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_sl;
-#pragma unroll
-  for (int i = 0; i < NV; ++i)
-    if (act[i]) orow_p[dd[i]] = E::st(y[i]);
+  merge_store<T, DH, false>(a, b, h, qi, lane, o[0], o[1]);
 }
 
 // ------------------------------------------------------------ gfx950 helpers
@@ -796,7 +861,6 @@ __device__ __forceinline__ int fa_vswz(int k) {
 }
 
 // v_exp_f32 (2^x; -inf -> 0)
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
   typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
@@ -1023,12 +1087,11 @@ __global__ __launch_bounds__(NW * 64) void attn_f32(const coda_attn_desc a, int 
 #pragma unroll
         for (int i = 0; i < NV; ++i) acc[s][i] += red_o[w][r][dd[i]] * f;
       }
-      if (nsplit > 1) {  // partial row r: [m, l, O(DH)], unnormalised
-        float* pr = part + r * (DH + 2);
-        if (lane < 2) pr[lane] = lane ? L[s] : M[s];
+      if (nsplit > 1) {  // partial row r, unnormalised
+        if (lane < 2) part[16 * DH + 16 * lane + r] = lane ? L[s] : M[s];
 #pragma unroll
         for (int i = 0; i < NV; ++i)
-          if (act[i]) pr[2 + dd[i]] = acc[s][i];
+          if (act[i]) part[r * DH + dd[i]] = acc[s][i];
       }
 #pragma unroll
       for (int i = 0; i < NV; ++i) acc[s][i] = act[i] && L[s] > 0.f ? acc[s][i] / L[s] : 0.f;
@@ -2016,9 +2079,11 @@ __device__ __forceinline__ coda_attn_desc chunk_view(const coda_attn_desc& a0, c
   return a;
 }
 
-template <int DH, int NW, int QM, bool TB, int NS>
+// KSPLIT: blockIdx.y takes a share of the tiles and leaves a partial for
+// attn_merge in ws.
+template <int DH, int NW, int QM, bool TB, int NS, bool KSPLIT>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void attn_f3_bf16(
-    const coda_attn_desc a_, int NQ, int nqb, int npairs, ChunkGeom cg) {
+    const coda_attn_desc a_, int NQ, int nqb, int npairs, ChunkGeom cg, float* ws) {
   const coda_attn_desc a = chunk_view<DH>(a_, cg);
   using Lay = F2Layout<DH>;
   static_assert(NS == 2 || NS == 4, "tile stages");
@@ -2071,7 +2136,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
   const int coff = a.causal == 2 ? 0 : a.Lb - a.Lq;
   const int q_hi = min(a.Lq - 1, qb * 16 * NQ + 16 * NQ - 1);
   const int klim = a.causal ? min(Lk, a.Lp + q_hi + coff + 1) : Lk;
-  const int ntile = (klim + KT - 1) / KT;
+  const int ntall = (klim + KT - 1) / KT;
+  // this workgroup's tiles [tb, ntile)
+  const int tb = KSPLIT ? (int)((int64_t)ntall * blockIdx.y / gridDim.y) : 0;
+  const int ntile = KSPLIT ? (int)((int64_t)ntall * (blockIdx.y + 1) / gridDim.y) : ntall;
 
   const bf16_t* kpb = a.Lp > 0 ? (const bf16_t*)a.kp + b * a.p_sb + hk * a.p_sh : nullptr;
   const bf16_t* vpb = a.Lp > 0 ? (const bf16_t*)a.vp + b * a.p_sb + hk * a.p_sh : nullptr;
@@ -2357,11 +2425,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     if constexpr (NS == 4) {
 #pragma unroll
       for (int t = 0; t < NS - 1; ++t)
-        if (t < ntile) tile_load(t);
+        if (tb + t < ntile) tile_load(tb + t);
     } else {
-      if (ntile > 0) tile_part(TrueC{}, FalseC{}, 0);
-      if (ntile > 1) tile_part(TrueC{}, FalseC{}, 1);
-      if (ntile > 0) tile_part(FalseC{}, TrueC{}, 0);
+      if (ntile > tb) tile_part(TrueC{}, FalseC{}, tb);
+      if (ntile > tb + 1) tile_part(TrueC{}, FalseC{}, tb + 1);
+      if (ntile > tb) tile_part(FalseC{}, TrueC{}, tb);
     }
 #pragma unroll
     for (int u = 0; u < NOWN; ++u) {
@@ -2497,14 +2565,14 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
   };
 
   // ---- S(0), masked, max folded
-  if (ntile > 0) {
+  if (ntile > tb) {
     if constexpr (NS == 4)
-      vm_wait(LPT * (min(ntile, NS - 1) - 1));
+      vm_wait(LPT * (min(ntile - tb, NS - 1) - 1));
     else
-      vm_wait(ntile > 1 ? KCW + VCW : VCW);
+      vm_wait(ntile > tb + 1 ? KCW + VCW : VCW);
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_s_barrier();
-    const uint32_t ka = lds_addr(f3_smem) + 16 * lane;
+    const uint32_t ka = lds_addr(kbuf(tb)) + 16 * lane;
     u32x4v_t kr[4];
     auto k_issue = [&](auto f_c) {
       constexpr int f = decltype(f_c)::value;
@@ -2520,7 +2588,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
       st[0][kb] = mfma_32x32x16(__builtin_bit_cast(bf16x8_t, kr[f % 4]), qf[ks], ks == 0 ? f32x16{} : st[0][kb]);
       __builtin_amdgcn_sched_barrier(0);
     });
-    mask_tile(std::integral_constant<int, 0>{}, 0, tile_mask_mode(0));
+    mask_tile(std::integral_constant<int, 0>{}, tb * KT, tile_mask_mode(tb * KT));
     float mx = st[0][0][0];
 #pragma unroll
     for (int j = 1; j < 16; ++j) mx = fmaxf(mx, st[0][0][j]);
@@ -2529,7 +2597,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     fold_max(mx);
   }
 
-  // one pipelined iteration; PAR = it % 2 selects the S registers
+  // one pipelined iteration; PAR = (it - tb) % 2 selects the S registers
   auto iteration = [&](auto par_c, int it) {
     constexpr int PAR = decltype(par_c)::value, NXT = 1 - PAR;
     const bool has_next = it + 1 < ntile;
@@ -2638,7 +2706,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     __builtin_amdgcn_s_setprio(0);
     if (has_next) fold_max(mx);
   };
-  for (int it = 0; it < ntile; it += 2) {
+  for (int it = tb; it < ntile; it += 2) {
     iteration(std::integral_constant<int, 0>{}, it);
     if (it + 1 < ntile) iteration(std::integral_constant<int, 1>{}, it + 1);
   }
@@ -2648,6 +2716,24 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
   // hands it to the signal lane l ^ 16; y = O_signal - lam rnd(O_noise),
   // then the HeadwiseRMSNorm and weight in fp32, one rounding at the store.
   const float l_tot = xsum32(l_s);
+  if constexpr (KSPLIT) {
+    // row (stream, head, query) of this tile's partial, unnormalised
+    if (qrow < a.Lq) {
+      const int nq = 16 * NQ, R = 2 * G * nq, r = strm * G * nq + g * nq + 16 * qsub + qn;
+      float* part = ws + (((int64_t)pair * nqb + qb) * gridDim.y + blockIdx.y) * R * (DH + 2);
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int jq = 0; jq < 4; ++jq)
+          *reinterpret_cast<float4*>(part + r * DH + 32 * db + 8 * jq + 4 * hl) =
+              float4{o[db][4 * jq], o[db][4 * jq + 1], o[db][4 * jq + 2], o[db][4 * jq + 3]};
+      if (hl == 0) {
+        part[R * DH + r] = m_s;
+        part[R * DH + R + r] = l_tot;
+      }
+    }
+    return;
+  }
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   const float lam = lam_lds[wv * 16 + qn];
   float y[NDB][16];
@@ -2761,21 +2847,6 @@ static int validate(const coda_attn_desc* d) {
 
 using namespace coda;
 
-extern "C" int coda_attn_workspace_bytes(const coda_attn_desc* d, size_t* bytes) {
-  int rc = validate(d);
-  if (rc) return rc;
-  CODA_REQUIRE(bytes != nullptr, "coda_attn_workspace_bytes: null out pointer");
-  *bytes = 0;
-  if (use_rows(d)) {
-    const int ns = rows_nsplit(d);
-    if (ns > 1) *bytes = (size_t)d->B * d->Hkv * ns * 16 * (d->Dh + 2) * sizeof(float);
-  } else if (d->dtype == CODA_F32) {
-    const F32Shape f = f32_shape(d, device_cus());
-    if (f.nsplit > 1) *bytes = (size_t)d->B * d->Hkv * f.ntile * f.nsplit * 16 * (d->Dh + 2) * sizeof(float);
-  }
-  return CODA_OK;
-}
-
 // the flash kernel's per-lane load offsets are 31-bit byte counts from a
 // tile's first row (or from the prefix / block start on a boundary tile)
 static bool flash_offsets_fit(const coda_attn_desc* d) {
@@ -2784,19 +2855,47 @@ static bool flash_offsets_fit(const coda_attn_desc* d) {
          (d->Lb == 0 || (d->b_sl >= 0 && ((int64_t)d->Lb + 64) * d->b_sl < lim));
 }
 
+template <typename T, int DH, bool FLASH>
+static int launch_merge_few(const coda_attn_desc* d, hipStream_t st, int qt, int R, int nsplit) {
+  const int64_t rows = (int64_t)((d->Lq + qt - 1) / qt) * (d->H / d->Hkv) * qt;
+  hipLaunchKernelGGL((attn_merge_few<T, DH, FLASH>), dim3((unsigned)((rows + 3) / 4), d->Hkv * d->B), dim3(256), 0, st, *d,
+                     qt, R, nsplit, (const float*)d->workspace);
+  return check_launch("attn_merge_few");
+}
 // pipelined 32-row flash tiles: NW waves, G heads x NW / G groups of 16
 // queries, NS tile stages; QM the query case (see attn_f3_bf16)
-template <int DH, int QM, bool TB, int NW, int NS>
-static int launch_f3_nw(const coda_attn_desc* d, hipStream_t st, int G, const ChunkGeom& cg) {
+template <int DH, int QM, bool TB, int NW, int NS, bool SPLIT>
+static int launch_f3_nw(const coda_attn_desc* d, hipStream_t st, int G, const ChunkGeom& cg, int ns) {
   const int npairs = d->B * d->Hkv;
   const int NQ = NW / G;
   const int nblk = (d->Lq + 16 * NQ - 1) / (16 * NQ);
   const size_t lds = f3_lds_bytes<DH, NS>();
-  int rc = lds_limit<attn_f3_bf16<DH, NW, QM, TB, NS>>(lds, "coda_diff_attn_fwd");
+  int rc = lds_limit<attn_f3_bf16<DH, NW, QM, TB, NS, SPLIT>>(lds, "coda_diff_attn_fwd");
   if (rc) return rc;
-  hipLaunchKernelGGL((attn_f3_bf16<DH, NW, QM, TB, NS>), dim3(nblk * npairs, cg.n > 0 ? cg.n : 1), dim3(NW * 64),
-                     lds, st, *d, NQ, nblk, npairs, cg);
-  return check_launch("attn_f3_bf16");
+  hipLaunchKernelGGL((attn_f3_bf16<DH, NW, QM, TB, NS, SPLIT>), dim3(nblk * npairs, SPLIT ? ns : cg.n > 0 ? cg.n : 1),
+                     dim3(NW * 64), lds, st, *d, NQ, nblk, npairs, cg, (float*)d->workspace);
+  rc = check_launch("attn_f3_bf16");
+  if (rc || !SPLIT) return rc;
+  return launch_merge_few<bf16_t, DH, true>(d, st, 16 * NQ, 2 * G * 16 * NQ, ns);
+}
+// Key splits of one attn_f3_bf16 launch: where its workgroups (4 waves, two a
+// CU, for G <= 4; 8 waves for G = 8) leave places free and each split keeps at
+// least 8 tiles of 64 keys on average over the query blocks.  A few workgroups
+// walk their tiles one after the other, about 1 us each: 777 queries, 4097
+// keys, 8 heads of 64 72 -> 37 us in 5 splits; 500 x 8000, 8 of 128 164 -> 62;
+// 300 x 3000, G = 8 89 -> 39.  Shorter splits don't pay for the merge: 1000
+// causal tokens 21.5 us in one, 23.4 in two; 256 x 640, 32 heads 21 and 31.
+static constexpr int kSplitTiles = 8;
+static int f3_nsplit(const coda_attn_desc* d, int cus) {
+  const int G = d->H / d->Hkv, rows = 16 * (G <= 4 ? 4 / G : 1);
+  const int64_t wgs = (int64_t)((d->Lq + rows - 1) / rows) * d->B * d->Hkv;
+  const int64_t tiles = ((int64_t)d->Lp + d->Lb - (d->causal ? d->Lq / 2 : 0)) / 64;
+  const int64_t ns = wgs > 0 ? std::min<int64_t>({(G <= 4 ? 2 : 1) * cus / wgs, tiles / kSplitTiles, 16}) : 1;
+  return ns < 1 ? 1 : (int)ns;
+}
+static size_t f3_split_bytes(const coda_attn_desc* d, int ns) {
+  const int G = d->H / d->Hkv, rows = 16 * (G <= 4 ? 4 / G : 1);
+  return (size_t)((d->Lq + rows - 1) / rows) * d->B * d->Hkv * ns * 2 * G * rows * (d->Dh + 2) * sizeof(float);
 }
 // 4-wave workgroups with two tile stages (two a CU) for G <= 4 (a 4-wave
 // workgroup still holds every head of its KV head), except a one-launch grid
@@ -2807,13 +2906,20 @@ static int launch_f3_nw(const coda_attn_desc* d, hipStream_t st, int G, const Ch
 // 4096 workgroups)
 template <int DH, int QM, bool TB>
 static int launch_f3_qm(const coda_attn_desc* d, hipStream_t st, int G, const ChunkGeom& cg) {
+  if (cg.n == 0) {
+    // (a caller's workspace too small for the splits: one launch)
+    const int ns = f3_nsplit(d, device_cus());
+    if (ns > 1 && d->workspace && d->workspace_bytes >= f3_split_bytes(d, ns) && (uintptr_t)d->workspace % 16 == 0)
+      return G <= 4 ? launch_f3_nw<DH, QM, TB, 4, 2, true>(d, st, G, cg, ns)
+                    : launch_f3_nw<DH, QM, TB, 8, 4, true>(d, st, G, cg, ns);
+  }
   if (G <= 4) {
     const int64_t rows8 = 16 * (8 / G);
     const int64_t n8 = (d->Lq + rows8 - 1) / rows8 * d->B * d->Hkv * (cg.n > 0 ? cg.n : 1);
     const int64_t cus = device_cus();
-    if (cg.n > 1 || n8 < cus || n8 >= 2 * cus) return launch_f3_nw<DH, QM, TB, 4, 2>(d, st, G, cg);
+    if (cg.n > 1 || n8 < cus || n8 >= 2 * cus) return launch_f3_nw<DH, QM, TB, 4, 2, false>(d, st, G, cg, 1);
   }
-  return launch_f3_nw<DH, QM, TB, 8, 4>(d, st, G, cg);
+  return launch_f3_nw<DH, QM, TB, 8, 4, false>(d, st, G, cg, 1);
 }
 template <int DH>
 static int launch_f3(const coda_attn_desc* d, hipStream_t st, int G, const ChunkGeom& cg = ChunkGeom{}) {
@@ -2830,7 +2936,8 @@ static int launch_f3(const coda_attn_desc* d, hipStream_t st, int G, const Chunk
 }
 template <typename T, int DH>
 static int launch_merge(const coda_attn_desc* d, hipStream_t st, int qt, int ntile, int nsplit) {
-  hipLaunchKernelGGL((attn_merge<T, DH>), dim3(ntile * (d->H / d->Hkv) * qt, d->Hkv * d->B), dim3(256), 0, st, *d, qt,
+  if (nsplit <= kFewSplits) return launch_merge_few<T, DH, false>(d, st, qt, 16, nsplit);
+  hipLaunchKernelGGL((attn_merge<T, DH>), dim3(ntile * (d->H / d->Hkv) * qt, d->Hkv * d->B), dim3(256), 0, st, *d, qt, 16,
                      nsplit, (const float*)d->workspace);
   return check_launch("attn_merge");
 }
@@ -2889,6 +2996,24 @@ static int launch_attn(const coda_attn_desc* d, hipStream_t st) {
     return fail(CODA_EUNSUP, "coda_diff_attn_fwd: G=%d with Lq=%d unsupported for bf16 tiles", G, d->Lq);
   }
   return check_launch("attn_tile_bf16");
+}
+
+extern "C" int coda_attn_workspace_bytes(const coda_attn_desc* d, size_t* bytes) {
+  int rc = validate(d);
+  if (rc) return rc;
+  CODA_REQUIRE(bytes != nullptr, "coda_attn_workspace_bytes: null out pointer");
+  *bytes = 0;
+  if (use_rows(d)) {
+    const int ns = rows_nsplit(d);
+    if (ns > 1) *bytes = (size_t)d->B * d->Hkv * ns * 16 * (d->Dh + 2) * sizeof(float);
+  } else if (d->dtype == CODA_F32) {
+    const F32Shape f = f32_shape(d, device_cus());
+    if (f.nsplit > 1) *bytes = (size_t)d->B * d->Hkv * f.ntile * f.nsplit * 16 * (d->Dh + 2) * sizeof(float);
+  } else if (d->Dh >= 64 && (d->H / d->Hkv & (d->H / d->Hkv - 1)) == 0 && flash_offsets_fit(d)) {
+    const int ns = f3_nsplit(d, device_cus());
+    if (ns > 1) *bytes = f3_split_bytes(d, ns);
+  }
+  return CODA_OK;
 }
 
 extern "C" int coda_prefill_attn_chunks(const coda_attn_desc* d, int n_chunks, int c_first, int blk, int L, int W,
