@@ -294,6 +294,13 @@ struct PlanGeom {
   int W, L, block, Lr0, ring_head, kE, kS, doE, doS, Kmax, B;
 };
 
+// LDS accesses of one wave are served in order: between a wave's own writes
+// and reads only the compiler has to be kept from moving them
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // sel::partition_unguarded over a[first, last) against the pivot a[pv], by a
 // whole wave, with the same swaps.  The left scan of the serial form stops at
 // elements not before the pivot, the right scan at elements the pivot is not
@@ -303,15 +310,14 @@ struct PlanGeom {
 // L_j < R_j, and the cut is the next left stop: L_m, or R_{m-1} (which the
 // last swap made one) where that comes first.  lpos / rpos: LDS lists of the
 // stops, both ascending.
-__device__ __forceinline__ int wave_partition(sel::Item<float>* a, int first, int last, int pv,
-                                              const sel::Before<float>& before, uint16_t* lpos, uint16_t* rpos,
-                                              int lane) {
-  const sel::Item<float> p = a[pv];
+template <typename V>
+__device__ __forceinline__ int wave_partition(sel::Item<V>* a, int first, int last, const sel::Item<V>& p,
+                                              const sel::Before<V>& before, uint16_t* lpos, uint16_t* rpos, int lane) {
   const uint64_t below = (1ull << lane) - 1;
   int nl = 0, nr = 0;
   for (int base = first; base < last; base += 64) {
     const int i = base + lane;
-    const sel::Item<float> x = a[min(i, last - 1)];
+    const sel::Item<V> x = a[min(i, last - 1)];
     const bool sl = i < last && !before(x, p), sr = i < last && !before(p, x);
     const uint64_t bl = __builtin_amdgcn_ballot_w64(sl), br = __builtin_amdgcn_ballot_w64(sr);
     if (sl) lpos[nl + __popcll(bl & below)] = (uint16_t)i;
@@ -319,7 +325,7 @@ __device__ __forceinline__ int wave_partition(sel::Item<float>* a, int first, in
     nl += __popcll(bl);
     nr += __popcll(br);
   }
-  __syncthreads();
+  wave_lds_fence();
   int m = 0;
   for (int base = 0;; base += 64) {
     const int j = base + lane;
@@ -332,14 +338,16 @@ __device__ __forceinline__ int wave_partition(sel::Item<float>* a, int first, in
     if (cnt < 64) break;
   }
   const int lm = m < nl ? lpos[m] : INT_MAX, rm = m > 0 ? rpos[nr - m] : INT_MAX;
-  __syncthreads();
+  wave_lds_fence();
   return min(lm, rm);
 }
 
 // sel::nth_element over a[0, n) by a whole wave: the same sequence of
-// partitions; the depth limit's heap select and the last insertion sort
-// (at most 3 elements) stay on lane 0.
-__device__ __forceinline__ void wave_nth_element(sel::Item<float>* a, int nth, int n, const sel::Before<float>& before,
+// partitions (the median of three read by every lane at once, swapped to the
+// front by lane 0); the depth limit's heap select and the last insertion
+// sort (at most 3 elements) stay on lane 0.
+template <typename V>
+__device__ __forceinline__ void wave_nth_element(sel::Item<V>* a, int nth, int n, const sel::Before<V>& before,
                                                  uint16_t* lpos, uint16_t* rpos, int lane) {
   if (n == 0 || nth == n) return;
   int first = 0, last = n, depth = sel::floor_log2(n) * 2;
@@ -349,16 +357,54 @@ __device__ __forceinline__ void wave_nth_element(sel::Item<float>* a, int nth, i
         sel::heap_select(a, first, nth + 1, last, before);
         sel::swap_items(a, first, nth);
       }
+      wave_lds_fence();
       return;
     }
     --depth;
-    if (lane == 0) sel::median_to_first(a, first, first + 1, first + (last - first) / 2, last - 1, before);
-    __syncthreads();
-    const int cut = wave_partition(a, first + 1, last, first, before, lpos, rpos, lane);
+    const int xi = first + 1, yi = first + (last - first) / 2, zi = last - 1;
+    const sel::Item<V> f = a[first], x = a[xi], y = a[yi], z = a[zi];
+    // (sel::median_to_first)
+    const bool xy = before(x, y), yz = before(y, z), xz = before(x, z);
+    const int pi = xy ? (yz ? yi : xz ? zi : xi) : (xz ? xi : yz ? zi : yi);
+    const sel::Item<V> p = pi == xi ? x : pi == yi ? y : z;
+    if (lane == 0) {
+      a[first] = p;
+      a[pi] = f;
+    }
+    wave_lds_fence();
+    const int cut = wave_partition(a, first + 1, last, p, before, lpos, rpos, lane);
     if (cut <= nth) first = cut;
     else last = cut;
   }
   if (lane == 0) sel::insertion_sort(a, first, last, before);
+  wave_lds_fence();
+}
+
+// sel::topk_order over a[0, n) by a whole wave.  Its sort of at most 16
+// elements is an insertion sort, which is stable: each lane counts the
+// elements that go before its own.
+template <typename V>
+__device__ __forceinline__ void wave_topk_order(sel::Item<V>* a, int n, int k, bool largest, bool sorted,
+                                                uint16_t* lpos, uint16_t* rpos, int lane) {
+  if (k == 0) return;
+  const sel::Before<V> before{largest};
+  if (k * 64 <= n || (sorted && k > 17)) {
+    if (lane == 0) sel::topk_order<V>(a, n, k, largest, sorted);
+    wave_lds_fence();
+    return;
+  }
+  wave_nth_element(a, k - 1, n, before, lpos, rpos, lane);
+  if (sorted && k > 2) {
+    const sel::Item<V> mine = a[min(lane, k - 2)];
+    int rank = 0;
+    for (int j = 0; j < k - 1; ++j) {
+      const sel::Item<V> o = a[j];
+      rank += before(o, mine) || (j < lane && !before(mine, o));
+    }
+    wave_lds_fence();
+    if (lane < k - 1) a[rank] = mine;
+    wave_lds_fence();
+  }
 }
 
 // Bound by the chain of dependent LDS passes: about 2 log2(n / K) partitions
@@ -399,12 +445,9 @@ __global__ __launch_bounds__(64) void block_plan_kernel(const float* __restrict_
     items[i] = sel::Item<float>{g, (int64_t)i};
   }
   __syncthreads();
-  // (the choice of sel::topk_order, sorted = false)
-  if (K * 64 <= n_ev) {
-    if (threadIdx.x == 0) sel::topk_order<float>(items, n_ev, K, true, false);
-  } else if (K > 0) {
+  {
     uint16_t* lpos = reinterpret_cast<uint16_t*>(items + p.block);
-    wave_nth_element(items, K - 1, n_ev, sel::Before<float>{true}, lpos, lpos + p.block, (int)threadIdx.x);
+    wave_topk_order<float>(items, n_ev, K, true, false, lpos, lpos + p.block, (int)threadIdx.x);
   }
   __syncthreads();
   for (int i = threadIdx.x; i < K; i += 64) out[i] = (int32_t)items[i].i;
@@ -1781,16 +1824,20 @@ __global__ __launch_bounds__(kFusedThreads) void block_fused_kernel(const coda_b
       }
     }
   }
-  if (Te > 0 && ties) {
-    // ties among the leading LRU keys: libstdc++'s order
-    if (t == 0) sel::topk_order<int64_t>(rk, Me, n_lru, false, true);
-    __syncthreads();
-    for (int r = t; r < n_lru; r += NT) lru[r] = (int32_t)rk[r].i;
-  }
   // sync 2; meanwhile this workgroup's share of head h's ring (every
-  // workgroup of head h has read its candidate rows before sync 1)
+  // workgroup of head h has read its candidate rows before sync 1), and, where
+  // the leading LRU keys tie (slots still unused), their order as libstdc++
+  // leaves it, on one wave (on one thread and before the sync it took 6 us of
+  // a chunk of a fresh prompt)
   const bool gave_up2 = group_sync(flags, K, me, 2 * epoch + 1, 2 * epoch + 1, spin_limit, status, &sync_gave_up,
                                    [&](int t1, int nt1) {
+    if (Te > 0 && ties && t1 < 64) {
+      // (the stop lists where the norm caches were, last read before sync 1:
+      // at least Me rows)
+      uint16_t* lpos = reinterpret_cast<uint16_t*>(fsm + L.ov);
+      wave_topk_order<int64_t>(rk, Me, n_lru, false, true, lpos, lpos + Me, t1);
+      for (int r = t1; r < n_lru; r += 64) lru[r] = (int32_t)rk[r].i;
+    }
     const int n_all = (Lr + g.blk - first) * CH;
     const int pz = (n_all + NZ - 1) / NZ, p0 = min(n_all, z * pz), p1 = min(n_all, p0 + pz);
     for (int base = p0 + t1; base < p1; base += kRingPre * nt1) {
