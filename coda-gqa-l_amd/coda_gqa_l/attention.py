@@ -652,11 +652,14 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         snapshots followed by one attention launch per group: the conditions
         of coda_prefill_attn_chunks (bf16, head_dim 64 / 128, G in {1, 2,
         4, 8}, the MFMA flash path, 31-bit per-lane key offsets) and banks
-        with candidates, so that every chunk's update is one launch."""
+        with candidates, so that every chunk's update is one launch.  With
+        mask_unused_memory False the ring's unused slots are attended to too,
+        which the grouped launch does not see: a full ring then."""
         B, H, L, Dh = q.shape
         G = H // self.num_kv_heads
         return (q.dtype == torch.bfloat16 and state.k_buf.dtype == torch.bfloat16 and Dh in (64, 128) and
                 G in (1, 2, 4, 8) and self.Me + self.Ms > 0 and min(int(block_size), L) * G > 8 and
+                (self.mask_unused_memory or state.recent_filled >= self.window) and
                 k.stride() == v.stride() and k.stride(-1) == 1 and
                 (self.window + int(block_size) + 64) * k.stride(2) < (1 << 30) and
                 (self.Me > 0 and self.exact_candidates_per_block > 0 or
