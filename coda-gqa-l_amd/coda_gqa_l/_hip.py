@@ -91,6 +91,7 @@ _SIGS = {
     "coda_diff_attn_fwd": (_i32, [ctypes.POINTER(AttnDesc), _vp]),
     "coda_attn_append": (_i32, [ctypes.POINTER(AttnDesc), _vp, _vp, _i64, _i64, _i64, _vp]),
     "coda_prefill_attn_chunks": (_i32, [ctypes.POINTER(AttnDesc), _i32, _i32, _i32, _i32, _i32, _i64, _i64, _vp]),
+    "coda_prefill_attn_chunks_f32": (_i32, [ctypes.POINTER(AttnDesc), _i32, _i32, _i32, _i32, _i32, _i64, _i64, _vp]),
     "coda_diff_epilogue_fwd": (_i32, [_i32, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _f32, _vp]),
     "coda_diff_sub_only_fwd": (_i32, [_i32, _vp, _vp, _vp, _vp, _i32, _i32, _vp]),
     "coda_rope_fwd": (_i32, [_i32, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _vp, _vp, _i32, _i32, _i32,

@@ -651,17 +651,22 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         """Whether prefill_core's chunks may run as a bank chain with
         snapshots followed by one attention launch per group: the conditions
         of coda_prefill_attn_chunks (bf16, head_dim 64 / 128, G in {1, 2,
-        4, 8}, the MFMA flash path, 31-bit per-lane key offsets) and banks
-        with candidates, so that every chunk's update is one launch.  With
-        mask_unused_memory False the ring's unused slots are attended to too,
-        which the grouped launch does not see: a full ring then."""
+        4, 8}, the MFMA flash path, 31-bit per-lane key offsets) or its fp32
+        form, and banks with candidates, so that every chunk's update is one
+        launch.  With mask_unused_memory False the ring's unused slots are
+        attended to too, which the grouped launch does not see: a full ring
+        then."""
         B, H, L, Dh = q.shape
         G = H // self.num_kv_heads
-        return (q.dtype == torch.bfloat16 and state.k_buf.dtype == torch.bfloat16 and Dh in (64, 128) and
-                G in (1, 2, 4, 8) and self.Me + self.Ms > 0 and min(int(block_size), L) * G > 8 and
+        if q.dtype == torch.bfloat16:
+            ok = Dh in (64, 128) and G in (1, 2, 4, 8) and min(int(block_size), L) * G > 8 and \
+                (self.window + int(block_size) + 64) * k.stride(2) < (1 << 30)
+        else:
+            # (one chunk alone: nothing to group)
+            ok = q.dtype == torch.float32 and Dh in (32, 64, 128) and G <= 8 and L > block_size
+        return (ok and state.k_buf.dtype == q.dtype and self.Me + self.Ms > 0 and
                 (self.mask_unused_memory or state.recent_filled >= self.window) and
                 k.stride() == v.stride() and k.stride(-1) == 1 and
-                (self.window + int(block_size) + 64) * k.stride(2) < (1 << 30) and
                 (self.Me > 0 and self.exact_candidates_per_block > 0 or
                  self.Ms > 0 and self.summary_candidates_per_block > 0))
 
@@ -681,7 +686,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         # snapshot buffers of up to 256 MiB (at most 1024 chunks), made once
         # per shape and kept: calls of any length reuse them
         per_chunk = 2 * B * Hkv * S * Dh * q.element_size()
-        cap = max(1, min(1024, (256 << 20) // max(per_chunk, 1)))
+        cap = max(1, min(1024, 65535 // max(B, 1), (256 << 20) // max(per_chunk, 1)))
         if self.pipelined_group_chunks is not None:
             cap = max(1, min(cap, int(self.pipelined_group_chunks)))
         group = min(n_chunks - c, cap)
@@ -746,8 +751,9 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
             q=q, rope_cos=rope_cos, rope_sin=rope_sin, rope_interleaved=self.rope_interleaved, theta_cos=ct,
             theta_sin=sn, k_prefix=sk[0], v_prefix=sv[0], allowed=sa[0] if self.mask_unused_memory else None,
             k_block=k, v_block=v, lam=lam, rms_weight=w, eps=self._eps, out=out.permute(0, 2, 1, 3))
-        _hip.check(_hip.lib().coda_prefill_attn_chunks(d, cb - ca, ca, blk, L, self.window, sk[0].numel(),
-                                                       sa[0].numel(), _hip.stream_of(q)))
+        lib = _hip.lib()
+        fn = lib.coda_prefill_attn_chunks if q.dtype == torch.bfloat16 else lib.coda_prefill_attn_chunks_f32
+        _hip.check(fn(d, cb - ca, ca, blk, L, self.window, sk[0].numel(), sa[0].numel(), _hip.stream_of(q)))
         # (the last grouped launch, for measurement: its chunks' snapshots
         # stay in the buffers until the next call)
         self.__dict__["_last_chunk_group"] = (ca, cb, blk, L)

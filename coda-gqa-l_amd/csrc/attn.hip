@@ -900,6 +900,43 @@ __device__ __forceinline__ void unpack4(const uint2& u, float x[4]) {
 }
 
 // ------------------------------------------------------------ fused decode step
+// Chunks of a prefill call in one launch (coda_prefill_attn_chunks):
+// y = chunk c_first + y (blockIdx.y; attn_f32: blockIdx.z / B), covering queries [t0, t0 + Lq) of the
+// call, t0 = c blk, Lq = min(blk, L - t0); its block keys are the call's
+// keys [t0 - win, t0 + Lq) with win = min(t0, W) (the ring window, in time
+// order, then the chunk itself, lower-right causal); its prefix is bank
+// snapshot y (prefix pointers and visibility bytes advanced by y strides).
+// n == 0: one chunk, as the descriptor says.
+struct ChunkGeom {
+  int n, c_first, blk, L, W, pad;
+  int64_t snap_stride;  // elements from one snapshot's K / V to the next
+  int64_t al_stride;    // bytes from one snapshot's visibility bytes to the next
+};
+template <typename T, int DH>
+__device__ __forceinline__ coda_attn_desc chunk_view(const coda_attn_desc& a0, const ChunkGeom& cg, int y) {
+  if (cg.n == 0) return a0;
+  coda_attn_desc a = a0;
+  const int64_t t0 = (int64_t)(cg.c_first + y) * cg.blk;
+  const int Lq = min(cg.blk, cg.L - (int)t0);
+  const int win = min((int)t0, cg.W);
+  using B = const T*;
+  a.q = (B)a0.q + t0 * a0.q_sl;
+  a.lam = (B)a0.lam + t0 * a0.lam_sl;
+  a.out = (T*)a0.out + t0 * a0.o_sl;
+  if (a0.rope_cos) {
+    a.rope_cos = (B)a0.rope_cos + t0 * (DH / 2);
+    a.rope_sin = (B)a0.rope_sin + t0 * (DH / 2);
+  }
+  a.kb = (B)a0.kb + (t0 - win) * a0.b_sl;
+  a.vb = (B)a0.vb + (t0 - win) * a0.b_sl;
+  a.Lq = Lq;
+  a.Lb = win + Lq;
+  a.kp = (B)a0.kp + y * cg.snap_stride;
+  a.vp = (B)a0.vp + y * cg.snap_stride;
+  if (a0.allowed) a.allowed = a0.allowed + y * cg.al_stride;
+  return a;
+}
+
 // ------------------------------------------------------------ fp32
 // attn_f32: a workgroup takes 16 query rows (both streams of the G heads of
 // qt = 16 / 2G queries) of one (KV head, sequence) and a share of the keys;
@@ -919,15 +956,17 @@ __device__ __forceinline__ void unpack4(const uint2& u, float x[4]) {
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
 template <int DH, int NW>
-__global__ __launch_bounds__(NW * 64) void attn_f32(const coda_attn_desc a, int qt, int nsplit, int keys_per_split,
-                                                    float* ws) {
+__global__ __launch_bounds__(NW * 64) void attn_f32(const coda_attn_desc a_, int qt, int nsplit,
+                                                    int keys_per_split, float* ws, const ChunkGeom cg) {
+  const coda_attn_desc a = chunk_view<float, DH>(a_, cg, blockIdx.z / a_.B);
   constexpr int NC = DH / 16, NM = DH / 16, VW = DH / 16, NV = (DH + 63) / 64;
   extern __shared__ __attribute__((aligned(16))) char f32_smem[];
   float(*red_o)[16][DH + 4] = reinterpret_cast<float(*)[16][DH + 4]>(f32_smem);  // [NW]; queries in [0] before
   __shared__ float red_m[NW][16], red_l[NW][16];
   __shared__ uint8_t al_lds[kMaxRowsPrefix];
-  const int tile = blockIdx.x / nsplit, split = blockIdx.x % nsplit, hk = blockIdx.y, b = blockIdx.z;
+  const int tile = blockIdx.x / nsplit, split = blockIdx.x % nsplit, hk = blockIdx.y, b = blockIdx.z % a.B;
   const int G = a.H / a.Hkv, GL = G * qt, q0 = tile * qt;
+  if (q0 >= a.Lq) return;  // (the last chunk of a call may be short)
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, g4 = lane >> 4;
   const float scale = (a.sm_scale > 0.f ? a.sm_scale : rsqrtf((float)DH)) * kLog2e;
@@ -2041,50 +2080,12 @@ constexpr size_t f3_lds_bytes() {
   return NS == 4 || tabs < tiles ? tiles : tabs;
 }
 
-// Chunks of a prefill call in one launch (coda_prefill_attn_chunks):
-// blockIdx.y = chunk c_first + y, covering queries [t0, t0 + Lq) of the
-// call, t0 = c blk, Lq = min(blk, L - t0); its block keys are the call's
-// keys [t0 - win, t0 + Lq) with win = min(t0, W) (the ring window, in time
-// order, then the chunk itself, lower-right causal); its prefix is bank
-// snapshot y (prefix pointers and visibility bytes advanced by y strides).
-// n == 0: one chunk, as the descriptor says.
-struct ChunkGeom {
-  int n, c_first, blk, L, W, pad;
-  int64_t snap_stride;  // elements from one snapshot's K / V to the next
-  int64_t al_stride;    // bytes from one snapshot's visibility bytes to the next
-};
-template <int DH>
-__device__ __forceinline__ coda_attn_desc chunk_view(const coda_attn_desc& a0, const ChunkGeom& cg) {
-  if (cg.n == 0) return a0;
-  coda_attn_desc a = a0;
-  const int y = blockIdx.y;
-  const int64_t t0 = (int64_t)(cg.c_first + y) * cg.blk;
-  const int Lq = min(cg.blk, cg.L - (int)t0);
-  const int win = min((int)t0, cg.W);
-  using B = const bf16_t*;
-  a.q = (B)a0.q + t0 * a0.q_sl;
-  a.lam = (B)a0.lam + t0 * a0.lam_sl;
-  a.out = (bf16_t*)a0.out + t0 * a0.o_sl;
-  if (a0.rope_cos) {
-    a.rope_cos = (B)a0.rope_cos + t0 * (DH / 2);
-    a.rope_sin = (B)a0.rope_sin + t0 * (DH / 2);
-  }
-  a.kb = (B)a0.kb + (t0 - win) * a0.b_sl;
-  a.vb = (B)a0.vb + (t0 - win) * a0.b_sl;
-  a.Lq = Lq;
-  a.Lb = win + Lq;
-  a.kp = (B)a0.kp + y * cg.snap_stride;
-  a.vp = (B)a0.vp + y * cg.snap_stride;
-  if (a0.allowed) a.allowed = a0.allowed + y * cg.al_stride;
-  return a;
-}
-
 // KSPLIT: blockIdx.y takes a share of the tiles and leaves a partial for
 // attn_merge in ws.
 template <int DH, int NW, int QM, bool TB, int NS, bool KSPLIT>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void attn_f3_bf16(
     const coda_attn_desc a_, int NQ, int nqb, int npairs, ChunkGeom cg, float* ws) {
-  const coda_attn_desc a = chunk_view<DH>(a_, cg);
+  const coda_attn_desc a = chunk_view<bf16_t, DH>(a_, cg, blockIdx.y);
   using Lay = F2Layout<DH>;
   static_assert(NS == 2 || NS == 4, "tile stages");
   static_assert(!TB || QM == 0 || QM == 1, "tables staged for the RoPE + rotation query cases");
@@ -2797,11 +2798,11 @@ static int rows_nsplit(const coda_attn_desc* d) {
 struct F32Shape {
   int qt, ntile, nw, nsplit, per;
 };
-static F32Shape f32_shape(const coda_attn_desc* d, int cus) {
+static F32Shape f32_shape(const coda_attn_desc* d, int cus, int chunks = 1) {
   F32Shape f;
   f.qt = std::max(1, 8 / (d->H / d->Hkv));
   f.ntile = (d->Lq + f.qt - 1) / f.qt;
-  const int64_t wgs = (int64_t)f.ntile * d->Hkv * d->B;
+  const int64_t wgs = (int64_t)f.ntile * d->Hkv * d->B * chunks;
   const int Lk = d->Lp + d->Lb;
   f.nw = wgs <= 2 * cus ? 8 : 4;
   const int64_t want = wgs > 0 ? std::min<int64_t>(std::min<int64_t>(cus / wgs, Lk / (64 * f.nw)),
@@ -2809,6 +2810,10 @@ static F32Shape f32_shape(const coda_attn_desc* d, int cus) {
   f.per = ((Lk + (int)std::max<int64_t>(want, 1) - 1) / (int)std::max<int64_t>(want, 1) + 15) / 16 * 16;
   f.per = std::max(f.per, 16);
   f.nsplit = std::max(1, (Lk + f.per - 1) / f.per);
+  if (chunks > 1) {  // (each chunk has keys of its own)
+    f.nsplit = 1;
+    f.per = std::max(Lk, 16);
+  }
   return f;
 }
 
@@ -2941,6 +2946,28 @@ static int launch_merge(const coda_attn_desc* d, hipStream_t st, int qt, int nti
                      nsplit, (const float*)d->workspace);
   return check_launch("attn_merge");
 }
+template <int DH>
+static int launch_f32(const coda_attn_desc* d, hipStream_t st, const ChunkGeom& cg) {
+  const int n = cg.n > 0 ? cg.n : 1;
+  F32Shape f = f32_shape(d, device_cus(), n);
+  if (f.nsplit > 1) {
+    const size_t need = (size_t)d->B * d->Hkv * f.ntile * f.nsplit * 16 * (DH + 2) * sizeof(float);
+    if (!d->workspace || d->workspace_bytes < need)
+      return fail(CODA_ESMALL, "coda_diff_attn_fwd: workspace %zu < %zu bytes", d->workspace_bytes, need);
+  }
+  const size_t lds = (size_t)f.nw * 16 * (DH + 4) * sizeof(float);
+  const dim3 grid(f.ntile * f.nsplit, d->Hkv, d->B * n);
+  int rc;
+  if (f.nw == 8) {
+    if ((rc = lds_limit<attn_f32<DH, 8>>(lds, "coda_diff_attn_fwd"))) return rc;
+    hipLaunchKernelGGL((attn_f32<DH, 8>), grid, dim3(512), lds, st, *d, f.qt, f.nsplit, f.per, (float*)d->workspace, cg);
+  } else {
+    hipLaunchKernelGGL((attn_f32<DH, 4>), grid, dim3(256), lds, st, *d, f.qt, f.nsplit, f.per, (float*)d->workspace, cg);
+  }
+  rc = check_launch("attn_f32");
+  if (rc || f.nsplit <= 1) return rc;
+  return launch_merge<float, DH>(d, st, f.qt, f.ntile, f.nsplit);
+}
 template <int DH, bool APPEND>
 static int launch_rows(const coda_attn_desc* d, hipStream_t st, const AppendTo& ap) {
   const int ns = rows_nsplit(d);
@@ -2963,24 +2990,7 @@ template <int DH>
 static int launch_attn(const coda_attn_desc* d, hipStream_t st) {
   const int G = d->H / d->Hkv;
   if (d->dtype == CODA_F32) {
-    const F32Shape f = f32_shape(d, device_cus());
-    if (f.nsplit > 1) {
-      const size_t need = (size_t)d->B * d->Hkv * f.ntile * f.nsplit * 16 * (DH + 2) * sizeof(float);
-      if (!d->workspace || d->workspace_bytes < need)
-        return fail(CODA_ESMALL, "coda_diff_attn_fwd: workspace %zu < %zu bytes", d->workspace_bytes, need);
-    }
-    const size_t lds = (size_t)f.nw * 16 * (DH + 4) * sizeof(float);
-    const dim3 grid(f.ntile * f.nsplit, d->Hkv, d->B);
-    int rc;
-    if (f.nw == 8) {
-      if ((rc = lds_limit<attn_f32<DH, 8>>(lds, "coda_diff_attn_fwd"))) return rc;
-      hipLaunchKernelGGL((attn_f32<DH, 8>), grid, dim3(512), lds, st, *d, f.qt, f.nsplit, f.per, (float*)d->workspace);
-    } else {
-      hipLaunchKernelGGL((attn_f32<DH, 4>), grid, dim3(256), lds, st, *d, f.qt, f.nsplit, f.per, (float*)d->workspace);
-    }
-    rc = check_launch("attn_f32");
-    if (rc || f.nsplit <= 1) return rc;
-    return launch_merge<float, DH>(d, st, f.qt, f.ntile, f.nsplit);
+    return launch_f32<DH>(d, st, ChunkGeom{});
   }
   if (use_rows(d)) return launch_rows<DH, false>(d, st, AppendTo{});
   if constexpr (DH >= 64) {
@@ -3039,6 +3049,31 @@ extern "C" int coda_prefill_attn_chunks(const coda_attn_desc* d, int n_chunks, i
   ChunkGeom cg{n_chunks, c_first, blk, L, W, 0, snap_stride, al_stride};
   hipStream_t st = (hipStream_t)stream;
   return w.Dh == 64 ? launch_f3<64>(&w, st, G, cg) : launch_f3<128>(&w, st, G, cg);
+}
+
+extern "C" int coda_prefill_attn_chunks_f32(const coda_attn_desc* d, int n_chunks, int c_first, int blk, int L, int W,
+                                            int64_t snap_stride, int64_t al_stride, void* stream) {
+  CODA_REQUIRE(d != nullptr, "coda_prefill_attn_chunks_f32: null descriptor");
+  CODA_REQUIRE(n_chunks > 0 && c_first >= 0 && blk > 0 && W >= 0 && L > (int64_t)(c_first + n_chunks - 1) * blk,
+               "coda_prefill_attn_chunks_f32: chunks %d .. %d of %d tokens in blocks of %d", c_first,
+               c_first + n_chunks - 1, L, blk);
+  coda_attn_desc w = *d;
+  w.Lq = blk < L ? blk : L;
+  w.Lb = W + w.Lq;
+  const int rc = validate(&w);
+  if (rc) return rc;
+  CODA_REQUIRE(w.dtype == CODA_F32 && w.causal == 1 && !w.q_noise && w.rope_cos,
+               "coda_prefill_attn_chunks_f32: needs fp32, the lower-right causal block and queries roped in-kernel");
+  CODA_REQUIRE(snap_stride >= 0 && al_stride >= 0, "coda_prefill_attn_chunks_f32: negative snapshot stride");
+  CODA_REQUIRE((int64_t)w.B * n_chunks <= 65535, "coda_prefill_attn_chunks_f32: %d sequences of %d chunks", w.B, n_chunks);
+  if (w.B == 0) return CODA_OK;
+  const ChunkGeom cg{n_chunks, c_first, blk, L, W, 0, snap_stride, al_stride};
+  hipStream_t st = (hipStream_t)stream;
+  switch (w.Dh) {
+    case 32: return launch_f32<32>(&w, st, cg);
+    case 64: return launch_f32<64>(&w, st, cg);
+    default: return launch_f32<128>(&w, st, cg);
+  }
 }
 
 extern "C" int coda_attn_append(const coda_attn_desc* d, void* k_out, void* v_out, int64_t o_sb, int64_t o_sh,

@@ -251,6 +251,10 @@ int coda_attn_append(const coda_attn_desc* d, void* k_out, void* v_out, int64_t 
 int coda_prefill_attn_chunks(const coda_attn_desc* d, int n_chunks, int c_first, int blk, int L, int W,
                              int64_t snap_stride, int64_t al_stride, void* stream);
 
+/* The same for fp32 (head_dim 32 too, any G up to 8). */
+int coda_prefill_attn_chunks_f32(const coda_attn_desc* d, int n_chunks, int c_first, int blk, int L, int W,
+                                 int64_t snap_stride, int64_t al_stride, void* stream);
+
 /* ------------------------------------------------------------------------
  * Standalone differential epilogue over rows of Dh:
  *   out = RMSNorm(sig - lam * noise) * w     (coda_diff_epilogue_fwd)
