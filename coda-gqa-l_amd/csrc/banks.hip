@@ -829,7 +829,8 @@ struct Dec {
   int32_t* idx_s;
   float* wtok;
 };
-__device__ __forceinline__ Dec dec_of(const coda_bank_desc& s, const BlockGeom& g, float* ws, int b) {
+template <typename G>
+__device__ __forceinline__ Dec dec_of(const coda_bank_desc& s, const G& g, float* ws, int b) {
   int32_t* base = reinterpret_cast<int32_t*>(ws + CODA_WS(ws_dec, s, g)) + (int64_t)b * dec_words(s.Me, g.Te, g.Ts);
   Dec d;
   d.idx_e = base;
@@ -1044,6 +1045,17 @@ __device__ __forceinline__ void st8_row(T* p, const Piece8<T> x) {
     reinterpret_cast<uint2*>(p)[1] = make_uint2(x.w[0].z, x.w[0].w);
   } else {
     st8<T>(p, x);
+  }
+}
+template <typename T>
+__device__ __forceinline__ Piece8<T> ld8_row(const T* p) {
+  if constexpr (sizeof(T) == 2) {
+    const uint2 a = reinterpret_cast<const uint2*>(p)[0], b = reinterpret_cast<const uint2*>(p)[1];
+    Piece8<T> x;
+    x.w[0] = make_uint4(a.x, a.y, b.x, b.y);
+    return x;
+  } else {
+    return ld8<T>(p);
   }
 }
 template <typename T>
@@ -1375,54 +1387,84 @@ __global__ __launch_bounds__(kApplyThreads) void block_ring_kernel(const coda_ba
 }
 
 // ------------------------------------------------------------ fused block write
-// The chunk's whole bank update in one launch when its working set fits in
-// LDS: NZ workgroups per (sequence b, head h), with the routing rows, bank
-// slots and ring pieces of head h split over them.  Workgroup (h, z, b):
-//   1. stages the raw K and V rows of the chunk's candidates for head h
-//      (the plan's first max(Te, Ts) tokens: the exact candidates are the
-//      first Te, the summary candidates the first Ts), its own bank slots,
-//      the norm caches its routing rows need, and the sequence's bank
-//      metadata (used bits, LRU stamps, candidate gates, LRU victim order);
-//   2. normalises its share of the routing rows (exact candidates z, z +
-//      NZ, ... as V rows, summary candidates z, z + NZ, ... as LF-K
-//      bands) and forms their dots with head h's norm caches (the CPU
-//      matmul order) into the workspace;
-//   -- sync 1 of the Hkv * NZ workgroups of b (meanwhile: the LRU order) --
-//   3. routes the tokens it is assigned (token i of [Te | Ts] goes to
+// The whole bank update of n >= 1 chunks in one launch when the working set
+// fits in LDS: NZ workgroups per (sequence b, head h), each with its share of
+// head h's bank slots (and their norm-cache rows) in LDS from the first chunk
+// to the last.  Workgroup (h, z, b) first stages its slots, the sequence's
+// bank metadata (used bits, LRU stamps; every workgroup keeps its own copy,
+// which all of them update alike) and normalises the first chunk's candidate
+// rows (the plan's first max(Te, Ts) tokens: the exact candidates are the
+// first Te, the summary candidates the first Ts).  Then, chunk by chunk:
+//   1. dots of every candidate's normalised row (exact: V; summary: LF-K
+//      band) with its own slots' norm rows (the CPU matmul order) into the
+//      workspace;
+//   -- sync 1 of the Hkv * NZ workgroups of b (meanwhile: the candidates' raw
+//      rows into LDS, the LRU order, the snapshot of its slots) --
+//   2. routes the tokens it is assigned (token i of [Te | Ts] goes to
 //      workgroup i mod (Hkv * NZ)): head-mean of the dots, first-occurrence
 //      argmax, published to the workspace;
-//   -- sync 2 (meanwhile: its share of head h's ring) --
-//   4. reads every token's routing, takes the exact decisions (the same
+//   -- sync 2 (meanwhile: the next chunk's candidate rows, normalised) --
+//   3. reads every token's routing, takes the exact decisions (the same
 //      serial walk, from the same values, in every workgroup) and applies
-//      them and the summary routing to its own slots of head h (exact delta
-//      write-back, summary accumulate + EMA, norm caches).
-// Workgroup (0, 0, b) (the lead) commits what the sequence shares: LRU stamps,
-// visibility bytes, ring gates, counters and the decision trace, after
-// sync 1 (every workgroup has read them by then).
+//      them and the summary routing to its own slots in LDS (exact delta
+//      write-back, summary accumulate + EMA, norm rows).
+// At the end it writes its slots, norm rows and its share of head h's ring;
+// workgroup (0, 0, b) (the lead) writes what the sequence shares.  A chunk's
+// candidates are read where they lay when the launch began: ring slots or
+// rows of the call (the ring is written once, after every read).
+//
+// What bounds it: latency, chunk after chunk (two syncs across the XCDs of
+// about 2 us each, and the serial steps between them), with 64 workgroups a
+// sequence and 8 waves each.  Hence nothing that another phase could hide
+// stands between the syncs, slots are split by owner (a split of the
+// candidates instead needs the other workgroups' updated norm rows: a third
+// sync, or a launch a chunk) and exactly what must cross goes through memory.
+// Per chunk of 256 tokens at 64 + 64 slots, 8 KV heads of 128, 4 sequences, bf16:
+// 14.3 us, where a launch a chunk (candidates split, norm caches reloaded) took
+// 27.3 with the gap to the next; 128 + 128 slots, 8 sequences: 22 against 44.
+// Of the 14.3: dots 3.0, sync 1 3.6, routing 1.6, sync 2 1.9, the decisions and
+// updates 3.8.  A launch's first staging and last writes take 8 and 6 us more.
+//
 // Sync: every workgroup of b stores (2 epoch + k) at sync k in its own
 // 64-bit flag word of the workspace and waits until all flags of b reach
-// it; the epoch is unique per launch, so no word needs clearing.  The epoch
-// of sequence b mixes the host's per-call value with a generation word of
-// b kept in the workspace's tail, which the lead workgroup advances once
-// every workgroup of b has passed sync 2 (so all of them read the same
+// it; the epoch is unique per chunk and launch, so no word needs clearing.
+// The epoch of sequence b mixes the host's per-call value with a generation
+// word of b kept in the workspace's tail, which the lead workgroup advances
+// once every workgroup of b has passed sync 2 (so all of them read the same
 // value first): a launch replayed from a captured graph, whose host value
 // is fixed, still meets its own sync words and never a stale one.  What
 // crosses a sync (dots, routing) is written and read with agent-scope
 // atomic accesses (coherent across the XCDs' L2s, no cache write-back or
 // invalidation), and a workgroup's flag is stored only after all its
-// waves' such stores have completed.  A workgroup waits on workgroups of b
-// only; they lie in one contiguous range of launch order (with whole other
-// sequences at most, at most 64 workgroups), dispatched after every earlier
-// range: one that waits never holds back one it waits for.  Waits are
-// bounded (spin_limit sleeps, about 0.1 s by default); a workgroup that
+// waves' such stores have completed.  One buffer of each kind does for every
+// chunk: dots are read before sync 2 and written after it, routing is read
+// before the next sync 1 and written after it.  A workgroup waits on
+// workgroups of b only; they lie in one contiguous range of launch order
+// (with whole other sequences at most, at most 64 workgroups), dispatched
+// after every earlier range: one that waits never holds back one it waits
+// for.  Waits are bounded (spin_limit sleeps, about 0.1 s by default, and a
+// launch takes at most kChainChunks chunks, some 3 ms); a workgroup that
 // gives up counts itself in g_block_sync_timeouts and in the workspace's
-// status word, and exits without writing any more state (the chunk's
-// update is then incomplete: the caller reads the status word and must
-// treat the state as lost).
+// status word, and exits without writing any state (the update is then
+// incomplete: the caller reads the status word and must treat the state as
+// lost).
 static constexpr int kFusedThreads = 512;
 static constexpr int kFusedMaxGroup = 64;  // Hkv * NZ: one wave polls every flag of a sequence
+static constexpr int kChainChunks = 64;
 static constexpr int kSyncSpinLimit = 1 << 20;
 static __device__ unsigned int g_block_sync_timeouts;
+
+// The chunks of one launch: n chunks of blk tokens (the last may be shorter)
+// over the L token rows the launch's K / V / gate pointers start at, from a
+// ring of ring_filled tokens with its oldest at ring_head; ke / ks the
+// candidate counts asked for, Te / Ts the largest that a chunk has; chunk
+// c's snapshot lies snap_stride elements (snap_al_stride bytes) after chunk
+// c - 1's.
+struct ChainGeom {
+  int n, L, blk, ring_head, ring_filled, Kmax, ke, ks, Te, Ts;
+  int64_t pos0;
+  int64_t b_sb, b_sh, b_sl, g_sb, snap_stride, snap_al_stride;
+};
 
 // Sync of the K workgroups of one sequence (see above).  While wave 0
 // polls, waves 1 .. hold `busy`: work that needs nothing from the other
@@ -1464,57 +1506,60 @@ __device__ __forceinline__ bool group_sync(unsigned long long* flags, int K, int
 }
 
 struct FusedLds {
-  int raw_k, raw_v, own_ek, own_ev, own_sv, own_sk, gate, used, last, rk, lru, pc, idx_e, fl_e, bv_e, bi_e, idx_s,
-      wtok, eflag, smask, scnt, sflag, knew, ov, total;
+  int raw_k, raw_v, own_ek, own_ev, own_sv, own_sk, gate, used, last, touch, emask, key, lru, pc, idx_e, bv_e, bi_e,
+      fl_e, idx_s, wtok, smask, scnt, sflag, knew, nrm_e, cnd_e, nrm_s, cnd_s, total;
 };
 __host__ __device__ __forceinline__ int al16(int x) { return (x + 15) & ~15; }
 __host__ __device__ __forceinline__ FusedLds fused_lds(int DH, int esz, int Me, int Ms, int Te, int Ts, int NZ) {
   const int TT = Te > Ts ? Te : Ts, LF = DH / 2;
   const int PE = (Me + NZ - 1) / NZ, PS = (Ms + NZ - 1) / NZ;
-  const int ne = (Te + NZ - 1) / NZ, ns = (Ts + NZ - 1) / NZ;
   FusedLds L;
   int o = 0;
-  L.raw_k = o; o += al16(TT * DH * esz);
-  L.raw_v = o; o += al16(TT * DH * esz);
-  L.own_ek = o; o += al16(PE * DH * esz);
-  L.own_ev = o; o += al16(PE * DH * esz);
-  L.own_sv = o; o += al16(PS * DH * esz);
-  L.own_sk = o; o += al16(PS * DH * esz);
-  L.gate = o; o += al16(4 * TT);
-  L.used = o; o += al16(4 * (Me + Ms));
-  L.last = o; o += al16(8 * Me);
-  L.rk = o; o += al16(16 * Me);
-  L.lru = o; o += al16(4 * Me);
-  L.pc = o; o += al16(4 * TT);
-  L.idx_e = o; o += al16(4 * Te);
-  L.fl_e = o; o += al16(4 * Te);
-  L.bv_e = o; o += al16(4 * Te);
-  L.bi_e = o; o += al16(4 * Te);
-  L.idx_s = o; o += al16(4 * Ts);
-  L.wtok = o; o += al16(4 * Ts);
-  L.eflag = o; o += al16(4 * Me);
-  L.smask = o; o += al16(8 * Ms);
-  L.scnt = o; o += al16(4 * Ms);
-  L.sflag = o; o += al16(4 * Ms);
-  L.knew = o; o += al16(4 * PS * LF);
-  L.ov = o;
-  // routing rows: head h's norm caches in the element type (widened as the
-  // dots read them) and this workgroup's normalised rows in fp32
-  L.total = o + al16(Me * (DH + 4) * esz) + al16(4 * ne * (DH + 4)) + al16(Ms * (LF + 4) * esz) +
-            al16(4 * ns * (LF + 4));
+  auto take = [&](int bytes) { const int at = o; o += al16(bytes); return at; };
+  L.raw_k = take(TT * DH * esz);
+  L.raw_v = take(TT * DH * esz);
+  L.own_ek = take(PE * DH * esz);
+  L.own_ev = take(PE * DH * esz);
+  L.own_sv = take(PS * DH * esz);
+  L.own_sk = take(PS * DH * esz);
+  L.gate = take(2 * 4 * TT);
+  L.used = take(4 * (Me + Ms));
+  L.last = take(8 * Me);
+  L.touch = take(8 * Me);  // (touch and emask together hold the Me items of a tied LRU order)
+  L.emask = take(8 * Me);
+  L.key = take(8 * Me);
+  L.lru = take(4 * Me);
+  L.pc = take(2 * 4 * TT);
+  L.idx_e = take(4 * Te);
+  L.bv_e = take(4 * Te);
+  L.bi_e = take(4 * Te);
+  L.fl_e = take(4 * Te);
+  L.idx_s = take(4 * Ts);
+  L.wtok = take(4 * Ts);
+  L.smask = take(8 * Ms);
+  L.scnt = take(4 * Ms);
+  L.sflag = take(4 * Ms);
+  L.knew = take(4 * (kFusedThreads / 64) * LF);
+  // own norm rows in the element type (widened as the dots read them), the
+  // candidates' normalised rows in fp32
+  L.nrm_e = take(PE * (DH + 4) * esz);
+  L.cnd_e = take(4 * Te * (DH + 4));
+  L.nrm_s = take(PS * (LF + 4) * esz);
+  L.cnd_s = take(4 * Ts * (LF + 4));
+  L.total = o;
   return L;
 }
 
 template <typename T, int DH>
-__global__ __launch_bounds__(kFusedThreads) void block_fused_kernel(const coda_bank_desc s, BlockGeom g, int NZ,
+__global__ __launch_bounds__(kFusedThreads) void block_fused_kernel(const coda_bank_desc s, ChainGeom g, int NZ,
                                                                     const T* kbk, const T* vbk, const float* gb,
-                                                                    const int32_t* __restrict__ plan_c, float* ws,
+                                                                    const int32_t* __restrict__ plan, float* ws,
                                                                     unsigned long long* flags_all,
                                                                     unsigned long long host_epoch,
                                                                     unsigned long long* tail, int spin_limit,
                                                                     BankSnap snap) {
   using E = Elt<T>;
-  constexpr int NV = (DH + 63) / 64, LF = DH / 2, NCOL = DH + LF, CH = DH / 8;
+  constexpr int NV = (DH + 63) / 64, LF = DH / 2, NCOL = DH + LF, CH = DH / 8, CHL = LF / 8;
   extern __shared__ __attribute__((aligned(16))) char fsm[];
   __shared__ int ties, sync_gave_up;
   // workgroup -> (sequence, head, z): workgroups are dealt round robin to
@@ -1526,268 +1571,378 @@ __global__ __launch_bounds__(kFusedThreads) void block_fused_kernel(const coda_b
   const int b = pair / s.Hkv, h = pair % s.Hkv;
   if (b >= s.B) return;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6, NT = blockDim.x, NW = NT >> 6;
-  const int W = s.W, Me = s.Me, Ms = s.Ms, Hkv = s.Hkv, Te = g.Te, Ts = g.Ts;
-  const int TT = max(Te, Ts), Lbuf = W + Me + Ms, K = Hkv * NZ, me = h * NZ + z;
+  const int W = s.W, Me = s.Me, Ms = s.Ms, Hkv = s.Hkv, TeM = g.Te, TsM = g.Ts, TM = max(TeM, TsM);
+  const int Lbuf = W + Me + Ms, K = Hkv * NZ, me = h * NZ + z;
   const bool lead = me == 0;
-  const int Ae = act_exact(s), As = act_summary(s), n_lru = min(Te, Ae);
-  const FusedLds L = fused_lds(DH, (int)sizeof(T), Me, Ms, Te, Ts, NZ);
+  const int Ae = act_exact(s), As = act_summary(s);
+  const FusedLds L = fused_lds(DH, (int)sizeof(T), Me, Ms, TeM, TsM, NZ);
   T* raw_k = reinterpret_cast<T*>(fsm + L.raw_k);    // [TT][DH] candidate K rows of head h
   T* raw_v = reinterpret_cast<T*>(fsm + L.raw_v);    // [TT][DH] candidate V rows
   T* own_ek = reinterpret_cast<T*>(fsm + L.own_ek);  // [PE][DH] own exact slots: K
   T* own_ev = reinterpret_cast<T*>(fsm + L.own_ev);  // V
   T* own_sv = reinterpret_cast<T*>(fsm + L.own_sv);  // [PS][DH] own summary slots: V
   T* own_sk = reinterpret_cast<T*>(fsm + L.own_sk);  // [PS][DH] own summary slots: K
-  float* gate = reinterpret_cast<float*>(fsm + L.gate);
   int32_t* used = reinterpret_cast<int32_t*>(fsm + L.used);
   int64_t* last = reinterpret_cast<int64_t*>(fsm + L.last);
-  sel::Item<int64_t>* rk = reinterpret_cast<sel::Item<int64_t>*>(fsm + L.rk);
+  int64_t* touch = reinterpret_cast<int64_t*>(fsm + L.touch);
+  int64_t* key = reinterpret_cast<int64_t*>(fsm + L.key);
   int32_t* lru = reinterpret_cast<int32_t*>(fsm + L.lru);
-  int32_t* pcl = reinterpret_cast<int32_t*>(fsm + L.pc);
   int32_t* idx_e = reinterpret_cast<int32_t*>(fsm + L.idx_e);
-  int32_t* fl_e = reinterpret_cast<int32_t*>(fsm + L.fl_e);
   float* bv_e = reinterpret_cast<float*>(fsm + L.bv_e);
   int32_t* bi_e = reinterpret_cast<int32_t*>(fsm + L.bi_e);
+  int32_t* fl_e = reinterpret_cast<int32_t*>(fsm + L.fl_e);
   int32_t* idx_s = reinterpret_cast<int32_t*>(fsm + L.idx_s);
   float* wtok = reinterpret_cast<float*>(fsm + L.wtok);
-  int32_t* eflag = reinterpret_cast<int32_t*>(fsm + L.eflag);
-  uint64_t* smask = reinterpret_cast<uint64_t*>(fsm + L.smask);
+  unsigned long long* emask = reinterpret_cast<unsigned long long*>(fsm + L.emask);  // tokens written to a slot
+  unsigned long long* smask = reinterpret_cast<unsigned long long*>(fsm + L.smask);
   float* scnt = reinterpret_cast<float*>(fsm + L.scnt);
   int32_t* sflag = reinterpret_cast<int32_t*>(fsm + L.sflag);
-  float* knew = reinterpret_cast<float*>(fsm + L.knew);  // [PS][LF]
-  const int le = DH + 4, lsum = LF + 4;
-  // this workgroup's routing rows: exact candidates e = z, z + NZ, ... and
-  // summary candidates z, z + NZ, ... (every workgroup forms both kinds)
-  const int ne = z < Te ? (Te - z + NZ - 1) / NZ : 0, ns = z < Ts ? (Ts - z + NZ - 1) / NZ : 0;
+  float* knew = reinterpret_cast<float*>(fsm + L.knew) + wv * LF;  // a row a wave
   // (rows of le / lsum elements: 8-byte aligned in bf16, 16-byte in fp32,
   // and 2 (bf16) or 4 (fp32) banks apart from row to row)
-  constexpr int ES = (int)sizeof(T);
-  char* ovp = fsm + L.ov;
-  T* nrm_e = reinterpret_cast<T*>(ovp);                                               // [Me][le]
-  ovp += ne > 0 ? al16(Me * le * ES) : 0;
-  float* cnd_e = reinterpret_cast<float*>(ovp);                                       // [ne][le]
-  ovp += al16(4 * ne * le);
-  T* nrm_s = reinterpret_cast<T*>(ovp);                                               // [Ms][lsum]
-  ovp += ns > 0 ? al16(Ms * lsum * ES) : 0;
-  float* cnd_s = reinterpret_cast<float*>(ovp);                                       // [ns][lsum]
+  constexpr int le = DH + 4, lsum = LF + 4;
+  T* nrm_e = reinterpret_cast<T*>(fsm + L.nrm_e);          // [PE][le]
+  float* cnd_e = reinterpret_cast<float*>(fsm + L.cnd_e);  // [Te][le]
+  T* nrm_s = reinterpret_cast<T*>(fsm + L.nrm_s);          // [PS][lsum]
+  float* cnd_s = reinterpret_cast<float*>(fsm + L.cnd_s);  // [Ts][lsum]
   // this workgroup's bank slots of head h
-  const int PE = (Me + NZ - 1) / NZ, e0 = min(Me, z * PE), e1 = min(Me, e0 + PE);
-  const int PS = (Ms + NZ - 1) / NZ, s0 = min(Ms, z * PS), s1 = min(Ms, s0 + PS);
+  const int PE = (Me + NZ - 1) / NZ, e0 = min(Me, z * PE), e1 = min(Me, e0 + PE), ne = e1 - e0;
+  const int PS = (Ms + NZ - 1) / NZ, s0 = min(Ms, z * PS), s1 = min(Ms, s0 + PS), ns = s1 - s0;
   T* kb = (T*)s.k_buf + ((int64_t)b * Hkv + h) * Lbuf * DH;
   T* vb = (T*)s.v_buf + ((int64_t)b * Hkv + h) * Lbuf * DH;
+  T* gn_e = (T*)s.exact_v_norm + (((int64_t)b * Hkv + h) * Me + e0) * DH;
+  T* gn_s = (T*)s.sum_lf_k_norm + (((int64_t)b * Hkv + h) * Ms + s0) * LF;
+  const T* kc = kbk + b * g.b_sb + h * g.b_sh;  // the call's rows of head h
+  const T* vc = vbk + b * g.b_sb + h * g.b_sh;
+  const float* gc = gb + (int64_t)b * g.g_sb;
   uint8_t* al = s.allowed + (int64_t)b * Lbuf;
-  const int32_t* pc = plan_c + (int64_t)b * g.Kmax;
   unsigned long long* flags = flags_all + (int64_t)b * K;
   // epoch of this launch for sequence b: the host value mixed with b's
   // generation word (tail[b]); tail[B] is the status word
   unsigned long long* status = tail + s.B;
   if (t == 0) sync_gave_up = 0;
   const Dec dx = dec_of(s, g, ws, b);  // exchange: idx_s [Ts], best value / slot of the exact tokens
-  const int Lr = g.ring_filled, first = max(Lr, g.n_ev), rhead = (Lr == W) ? g.ring_head : 0;
 
-  // ---- 1. staging in one batch of loads: the plan entries behind this
-  // thread's candidate pieces first, then plan, metadata, own bank slots
-  // and norm caches, then the candidate rows and gates through those plan
-  // entries (their wait covers only the entries), then every LDS store
+  // Token R counts from the ring's oldest at the launch's start: the first F0
+  // lie in the ring, the others are rows of the call.
+  const int F0 = g.ring_filled, rhead = F0 == W ? g.ring_head : 0;
+  auto ring_slot = [&](int R) __attribute__((always_inline)) {
+    const int q = rhead + R;
+    return q - (q >= W ? W : 0);
+  };
+  auto row_of = [&](const T* ring, const T* call, int R) __attribute__((always_inline)) {
+    return R < F0 ? ring + (int64_t)ring_slot(R) * DH : call + (int64_t)(R - F0) * g.b_sl;
+  };
+  // sizes of a chunk: token R of its oldest, its evictions and candidates
+  int base = 0, filled = F0, n_ev, Te, Ts;
+  auto sizes = [&](int c, int f, int& ev, int& te, int& ts) __attribute__((always_inline)) {
+    const int tok = min(g.blk, g.L - c * g.blk);
+    ev = max(0, f + tok - W);
+    te = min(g.ke, ev);
+    ts = min(g.ks, ev);
+    return f + tok - ev;
+  };
+  int filled_next = sizes(0, filled, n_ev, Te, Ts);
+
+  // Normalised rows (exact: V, all DH channels; summary: K channels [DH/2,
+  // DH)) of the candidates pcx[], eight rows a wave at a time (a task): lane
+  // 8 r + j holds channels j, j + 8, ... of row r, the accumulator j of the
+  // CPU's 2-norm, and the eight accumulators are added in order
+  // (wave_sumsq_cpu_order, whose row a wave takes eight times as long).
+  constexpr int NX = DH / 8;
+  auto n_tasks = [](int te, int ts) __attribute__((always_inline)) { return (te + 7) / 8 + (ts + 7) / 8; };
+  auto task_load = [&](const int32_t* pcx, int te, int ts, int task, T (&x)[NX]) __attribute__((always_inline)) {
+    const int nte = (te + 7) / 8;
+    const bool ex = task < nte;
+    const int R = pcx[min(8 * (ex ? task : task - nte) + (lane >> 3), (ex ? te : ts) - 1)];
+    const T* row = (ex ? row_of(vb, vc, R) : row_of(kb, kc, R) + LF) + (lane & 7);
+#pragma unroll
+    for (int k = 0; k < NX; ++k)
+      if (ex || k < NX / 2) x[k] = row[8 * k];
+  };
+  auto task_unit = [&](int te, int ts, int task, const T (&xt)[NX]) __attribute__((always_inline)) {
+    const int nte = (te + 7) / 8;
+    const bool ex = task < nte;
+    const int r = 8 * (ex ? task : task - nte) + (lane >> 3);
+    float x[NX], acc = 0.f;
+#pragma unroll
+    for (int k = 0; k < NX; ++k)
+      if (ex || k < NX / 2) {
+        x[k] = E::ld(xt[k]);
+        acc = fmaf(x[k], x[k], acc);
+      }
+    float part[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) part[q] = __shfl(acc, (lane & 56) + q, 64);
+    float ss = part[0];
+#pragma unroll
+    for (int q = 1; q < 8; ++q) ss = ss + part[q];
+    const float den = fmaxf(E::rnd(sqrtf(ss)), eps_r<T>());
+    float* out = (ex ? cnd_e + r * le : cnd_s + r * lsum) + (lane & 7);
+    if (r < (ex ? te : ts)) {
+#pragma unroll
+      for (int k = 0; k < NX; ++k)
+        if (ex || k < NX / 2) out[8 * k] = E::rnd(x[k] / den);
+    }
+  };
+  auto gate_of = [&](int R) __attribute__((always_inline)) {
+    return R < F0 ? s.g_recent + (int64_t)b * W + ring_slot(R) : gc + (R - F0);
+  };
+
+  // ---- staging in one batch of loads: plan, metadata, own bank slots and
+  // norm rows, then every LDS store
   {
     constexpr int UR = 2;  // pieces of each kind per thread and round
-    constexpr int CHL = LF / 8;
-    const int n_raw = TT * CH, n_us = Me + Ms, n_ee = (e1 - e0) * CH, n_ss = (s1 - s0) * CH;
-    const int n_ne = ne > 0 ? Me * CH : 0, n_ns = ns > 0 ? Ms * CHL : 0;
-    const int n_rnd = max(max(max(n_raw, TT), max(n_us, n_ee)), max(max(n_ss, n_ne), n_ns));
-    const T* nre = (const T*)s.exact_v_norm + ((int64_t)b * Hkv + h) * Me * DH;
-    const T* nrs = (const T*)s.sum_lf_k_norm + ((int64_t)b * Hkv + h) * Ms * LF;
-    for (int base = t; base < n_rnd; base += UR * NT) {
-      int32_t rr[UR], vpc[UR];
+    const int n_us = Me + Ms, n_ee = ne * CH, n_ss = ns * CH, n_ns = ns * CHL, tt = max(Te, Ts);
+    const int n_rnd = max(max(tt, n_us), max(n_ee, n_ss));
+    int32_t* pc = reinterpret_cast<int32_t*>(fsm + L.pc);
+    for (int i0 = t; i0 < n_rnd; i0 += UR * NT) {
+      int32_t vpc[UR];
       uint32_t vus[UR];
       int64_t vla[UR];
-      Piece8<T> vek[UR], vev[UR], vsv[UR], vsk[UR], vne[UR], vns[UR], vrk[UR], vrv[UR];
-      float vg[UR];
+      Piece8<T> vek[UR], vev[UR], vsv[UR], vsk[UR], vne[UR], vns[UR];
       // every load unconditional, from a clamped index or (an empty array)
-      // the workspace: the compiler then counts the loads in flight and
-      // waits for the plan entries alone before the candidate rows, where a
-      // load under a branch makes it wait for everything
+      // the workspace: the compiler then keeps them all in flight, where a
+      // load under a branch makes it wait
+      const T* none = reinterpret_cast<const T*>(ws);
 #pragma unroll
       for (int u = 0; u < UR; ++u) {
-        const int i = base + u * NT;
-        rr[u] = pc[min(i, n_raw - 1) / CH];
-      }
-#pragma unroll
-      for (int u = 0; u < UR; ++u) {
-        const int i = base + u * NT;
-        vpc[u] = pc[min(i, TT - 1)];
+        const int i = i0 + u * NT;
+        vpc[u] = plan[(int64_t)b * g.Kmax + min(i, tt - 1)];
         vus[u] = al[W + min(i, n_us - 1)];
         vla[u] = *(Me > 0 ? s.mem_last + (int64_t)b * Me + min(i, Me - 1) : reinterpret_cast<const int64_t*>(ws));
         {
-          const int ic = min(i, max(n_ee, 1) - 1), r = ic / CH, c = ic % CH;
-          const int64_t o = (int64_t)(W + e0 + r) * DH + 8 * c;
-          vek[u] = ld8<T>(n_ee > 0 ? kb + o : reinterpret_cast<const T*>(ws));
-          vev[u] = ld8<T>(n_ee > 0 ? vb + o : reinterpret_cast<const T*>(ws));
+          const int64_t o = (int64_t)(W + e0) * DH + 8 * min(i, max(n_ee, 1) - 1);
+          vek[u] = ld8<T>(n_ee > 0 ? kb + o : none);
+          vev[u] = ld8<T>(n_ee > 0 ? vb + o : none);
+          vne[u] = ld8<T>(n_ee > 0 ? gn_e + 8 * min(i, n_ee - 1) : none);
         }
         {
-          const int ic = min(i, max(n_ss, 1) - 1), r = ic / CH, c = ic % CH;
-          const int64_t o = (int64_t)(W + Me + s0 + r) * DH + 8 * c;
-          vsv[u] = ld8<T>(n_ss > 0 ? vb + o : reinterpret_cast<const T*>(ws));
-          vsk[u] = ld8<T>(n_ss > 0 ? kb + o : reinterpret_cast<const T*>(ws));
+          const int64_t o = (int64_t)(W + Me + s0) * DH + 8 * min(i, max(n_ss, 1) - 1);
+          vsv[u] = ld8<T>(n_ss > 0 ? vb + o : none);
+          vsk[u] = ld8<T>(n_ss > 0 ? kb + o : none);
+          vns[u] = ld8<T>(n_ns > 0 ? gn_s + 8 * min(i, n_ns - 1) : none);
         }
-        vne[u] = ld8<T>(n_ne > 0 ? nre + 8 * (int64_t)min(i, n_ne - 1) : reinterpret_cast<const T*>(ws));
-        vns[u] = ld8<T>(n_ns > 0 ? nrs + 8 * (int64_t)min(i, n_ns - 1) : reinterpret_cast<const T*>(ws));
       }
 #pragma unroll
       for (int u = 0; u < UR; ++u) {
-        const int i = base + u * NT;
-        const int c = min(i, n_raw - 1) % CH;
-        vrk[u] = ld8<T>(cand_row<T, DH>(s, g, kbk, b, h, rr[u], false) + 8 * c);
-        vrv[u] = ld8<T>(cand_row<T, DH>(s, g, vbk, b, h, rr[u], true) + 8 * c);
-        vg[u] = *cand_gate_ptr(s, g, gb, b, rr[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < UR; ++u) {
-        const int i = base + u * NT;
-        if (i < TT) pcl[i] = vpc[u];
+        const int i = i0 + u * NT;
+        if (i < tt) pc[i] = vpc[u];
         if (i < n_us) used[i] = (int32_t)(vus[u] & 0xffu);
         if (i < Me) last[i] = vla[u];
         if (i < n_ee) {
-          const int r = i / CH, c = i % CH;
-          st8<T>(own_ek + r * DH + 8 * c, vek[u]);
-          st8<T>(own_ev + r * DH + 8 * c, vev[u]);
+          st8<T>(own_ek + 8 * i, vek[u]);
+          st8<T>(own_ev + 8 * i, vev[u]);
+          st8_row<T>(nrm_e + (i / CH) * le + 8 * (i % CH), vne[u]);
         }
         if (i < n_ss) {
-          const int r = i / CH, c = i % CH;
-          st8<T>(own_sv + r * DH + 8 * c, vsv[u]);
-          st8<T>(own_sk + r * DH + 8 * c, vsk[u]);
+          st8<T>(own_sv + 8 * i, vsv[u]);
+          st8<T>(own_sk + 8 * i, vsk[u]);
         }
-        if (i < n_ne) st8_row<T>(nrm_e + (i / CH) * le + 8 * (i % CH), vne[u]);
         if (i < n_ns) st8_row<T>(nrm_s + (i / CHL) * lsum + 8 * (i % CHL), vns[u]);
-        if (i < n_raw) {
-          st8<T>(raw_k + 8 * i, vrk[u]);
-          st8<T>(raw_v + 8 * i, vrv[u]);
-          if (i % CH == 0) gate[i / CH] = vg[u];
-        }
       }
     }
   }
-  // b's generation word, first used at sync 1: loaded after the staging
-  // loop (a load pending at a loop's head is waited for there), through a
-  // lane-varying zero in the address, which keeps it in a vector register (a
-  // uniform load is copied to a scalar register, and waited for, at once)
+  // b's generation word, first used at sync 1, through a lane-varying zero in
+  // the address, which keeps it in a vector register (a uniform load is
+  // copied to a scalar register, and waited for, at once)
   const int lane0 = (int)__builtin_amdgcn_mbcnt_lo(0u, 0u);
   const unsigned long long gen_b =
       __hip_atomic_load(tail + b + lane0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
-  // LRU keys over the pre-update stamps (memory_banks.py:640-660):
-  // ascending stamps of used active slots, unused ones first
-  if (Te > 0)
-    for (int m = t; m < Me; m += NT) {
-      const bool u = used[m] != 0 && m < Ae;
-      rk[m] = sel::Item<int64_t>{u ? last[m] : kNegBig, (int64_t)m};
-    }
+  // LRU key of slot m (memory_banks.py:640-660): ascending stamps of used
+  // active slots, unused ones first
+  auto lru_key = [&](int m, bool u, int64_t at) __attribute__((always_inline)) {
+    key[m] = u && m < Ae ? at : kNegBig;
+  };
+  for (int m = t; m < Me; m += NT) lru_key(m, used[m] != 0, last[m]);
   if (t == 0) ties = 0;
-  __syncthreads();
-  // ---- 2. this workgroup's routing rows, normalised (exact: V, all DH
-  // channels; summary: K channels [DH/2, DH)), then their dots with head
-  // h's norm caches, one dot per thread (lanes over bank slots)
-  for (int r = wv; r < ne + ns; r += NW) {
-    const bool ex = r < ne;
-    const int k = ex ? r : r - ne, c = z + k * NZ;
-    float x[NV];
-    bool act[NV];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int d = lane + 64 * i;
-      act[i] = ex ? d < DH : (d >= LF && d < DH);
-      x[i] = E::ld((ex ? raw_v : raw_k)[c * DH + min(d, DH - 1)]);
-    }
-    if (ex) {
-      wave_unit<T, NV>(x, act);
-#pragma unroll
-      for (int i = 0; i < NV; ++i)
-        if (act[i]) cnd_e[k * le + lane + 64 * i] = x[i];
-    } else {
-      wave_unit<T, NV, LF>(x, act);
-#pragma unroll
-      for (int i = 0; i < NV; ++i)
-        if (act[i]) cnd_s[k * lsum + lane + 64 * i - LF] = x[i];
-    }
-  }
-  __syncthreads();
   {
-    float* dot_e = ws + ((int64_t)b * Hkv + h) * Te * Me;
-    float* dot_s = ws + CODA_WS(ws_dot_s, s, g) + ((int64_t)b * Hkv + h) * Ts * Ms;
-    const int n_e = ne * Me, n_s = ns * Ms, n_all = n_e + n_s;
-    // each dot is one serial chain (DH or DH/2 steps): the exact dots take
-    // the last n_e threads alone, the summary dots the others, so that no
-    // thread chains an exact dot after a summary one (when n_e <= NT / 2)
-    const bool split = n_e > 0 && 2 * n_e <= NT;
-    const int ns_thr = split ? NT - n_e : NT;
-    const int it0 = split ? (t >= ns_thr ? n_s + (t - ns_thr) : t) : t;
-    const int step = split ? (t >= ns_thr ? n_all : ns_thr) : NT;
-    for (int it1 = it0; it1 < (split && t < ns_thr ? n_s : n_all); it1 += step) {
-      // item order: [exact | summary] in the unsplit case, [summary | exact] in the split one
-      const int it = split ? (it1 < n_s ? n_e + it1 : it1 - n_s) : it1;
-      const bool ex = it < n_e;
-      const int k = ex ? it / Me : (it - n_e) / Ms, m = ex ? it % Me : (it - n_e) % Ms;
-      const T* rw = ex ? nrm_e + m * le : nrm_s + m * lsum;
-      const float* cd = ex ? cnd_e + k * le : cnd_s + k * lsum;
-      const int len = ex ? DH : LF;
-      float acc = 0.f;
-#pragma unroll 4
-      for (int d = 0; d < len; d += 4) {
-        const float4 rv = ld4_row<T>(rw + d);
-        const float4 cv = *reinterpret_cast<const float4*>(cd + d);
-        acc = dot_pair(acc, cv.x, rv.x, cv.y, rv.y);
-        acc = dot_pair(acc, cv.z, rv.z, cv.w, rv.w);
-      }
-      // coherent at agent scope: read by workgroups on other XCDs
-      float* o = ex ? dot_e + (int64_t)(z + k * NZ) * Me + m : dot_s + (int64_t)(z + k * NZ) * Ms + m;
-      __hip_atomic_store(o, E::rnd(acc), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int32_t* pc = reinterpret_cast<const int32_t*>(fsm + L.pc);
+    if (t < max(Te, Ts)) reinterpret_cast<float*>(fsm + L.gate)[t] = *gate_of(pc[t]);
+    for (int k = wv; k < n_tasks(Te, Ts); k += 2 * NW) {
+      T x[2][NX];
+      task_load(pc, Te, Ts, k, x[0]);
+      task_load(pc, Te, Ts, min(k + NW, n_tasks(Te, Ts) - 1), x[1]);
+      task_unit(Te, Ts, k, x[0]);
+      if (k + NW < n_tasks(Te, Ts)) task_unit(Te, Ts, k + NW, x[1]);
     }
   }
-  // sync 1; meanwhile the LRU victim order (rank of each key among all:
-  // one key per wave and pass, counted by ballots over the others)
   const unsigned long long epoch = (host_epoch + gen_b * 0x9E3779B97F4A7C15ull) & ((1ull << 62) - 1);
-  const bool gave_up1 = group_sync(flags, K, me, 2 * epoch, 2 * epoch + 1, spin_limit, status, &sync_gave_up,
-                                   [&](int t1, int nt1) {
-    if (Te > 0) {
-      const int wb = t1 >> 6, nwb = nt1 >> 6, ln = t1 & 63;
-      for (int m = wb; m < Me; m += nwb) {
-        const int64_t km = rk[m].v;
-        int lt = 0, eq = 0;
-        for (int j0 = 0; j0 < Me; j0 += 64) {
-          const int j = j0 + ln;
-          const bool in = j < Me;
-          const int64_t kj = rk[in ? j : 0].v;
-          lt += __popcll(__ballot(in && kj < km));
-          eq += __popcll(__ballot(in && kj == km && j != m));
-        }
-        if (ln == 0 && lt < n_lru) {
-          if (eq) atomicOr(&ties, 1);
-          else lru[lt] = m;
+  float* dot_e = ws + (int64_t)b * Hkv * TeM * Me;  // [h][Te][Me]
+  float* dot_s = ws + CODA_WS(ws_dot_s, s, g) + (int64_t)b * Hkv * TsM * Ms;
+
+  for (int c = 0;; ++c) {
+    const bool more = c + 1 < g.n;
+    const int TT = max(Te, Ts), n_lru = min(Te, Ae);
+    const int32_t* pc = reinterpret_cast<const int32_t*>(fsm + L.pc) + (c & 1) * TM;
+    const float* gate = reinterpret_cast<const float*>(fsm + L.gate) + (c & 1) * TM;
+    const unsigned long long val = 2 * (epoch + c);
+    // the next chunk's sizes and plan
+    int n_ev1 = 0, Te1 = 0, Ts1 = 0, filled1 = 0;
+    int32_t pn = 0;
+    if (more) {
+      filled1 = sizes(c + 1, filled_next, n_ev1, Te1, Ts1);
+      if (t < max(Te1, Ts1)) pn = plan[((int64_t)(c + 1) * s.B + b) * g.Kmax + t];
+    }
+    __syncthreads();
+    // this chunk's raw rows, in flight during the dots
+    constexpr int UC = 2;
+    const int n_raw = TT * CH;
+    Piece8<T> vk[UC], vv[UC];
+    auto raw_load = [&](int i0) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < UC; ++u) {
+        const int i = min(i0 + u * NT, n_raw - 1), R = pc[i / CH], o = 8 * (i % CH);
+        vk[u] = ld8<T>(row_of(kb, kc, R) + o);
+        vv[u] = ld8<T>(row_of(vb, vc, R) + o);
+      }
+    };
+    auto raw_store = [&](int i0) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < UC; ++u) {
+        const int i = i0 + u * NT;
+        if (i < n_raw) {
+          st8<T>(raw_k + 8 * i, vk[u]);
+          st8<T>(raw_v + 8 * i, vv[u]);
         }
       }
-    }
-    if (snap.k) {
-      // the bank slots as staged, before this chunk's update, copied out of
-      // LDS while the sync waits (a loop of stores only: inside the staging
-      // loop, with its loads, every store would be waited for)
-      const int64_t sb = ((int64_t)b * Hkv + h) * (Me + Ms) * DH;
-      const int n_ee = (e1 - e0) * CH, n_ss = (s1 - s0) * CH;
-      for (int i = t1; i < n_ee + n_ss; i += nt1) {
-        const bool ex = i < n_ee;
-        const int j = ex ? i : i - n_ee, r = j / CH, c = j % CH;
-        const int64_t row = ex ? e0 + r : Me + s0 + r;
-        st8<T>((T*)snap.k + sb + row * DH + 8 * c, ld8<T>((ex ? own_ek : own_sk) + r * DH + 8 * c));
-        st8<T>((T*)snap.v + sb + row * DH + 8 * c, ld8<T>((ex ? own_ev : own_sv) + r * DH + 8 * c));
+    };
+    raw_load(t);
+    // ---- 1. dots of every candidate with this workgroup's slots.  Each dot
+    // is one serial chain (DH or DH/2 steps); a thread takes a block of RB
+    // slots by CB candidates (their chains side by side, each row read once),
+    // as large as leaves every thread one block.  The exact dots take the
+    // last threads alone, the summary dots the others, so that no thread
+    // chains an exact dot after a summary one (when half the threads do for
+    // the exact ones).
+    {
+      // coherent at agent scope: read by workgroups on other XCDs
+      auto run = [&](auto rbc, auto cbc, const T* nrm, const float* cnd, auto lenc, int np, int nc, float* out, int M,
+                     int at, int step) __attribute__((always_inline)) {
+        constexpr int RB = decltype(rbc)::value, CB = decltype(cbc)::value, LEN = decltype(lenc)::value, ST = LEN + 4;
+        const int nr = (np + RB - 1) / RB, n = nr * ((nc + CB - 1) / CB);
+        for (int it = at; it < n; it += step) {
+          const int r0 = it % nr, c0 = CB * (it / nr);  // slots r0, r0 + nr, ..
+          float acc[RB][CB];
+#pragma unroll
+          for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int j = 0; j < CB; ++j) acc[i][j] = 0.f;
+#pragma unroll 4
+          for (int d = 0; d < LEN; d += 4) {
+            float4 rv[RB], cv[CB];
+#pragma unroll
+            for (int i = 0; i < RB; ++i) rv[i] = ld4_row<T>(nrm + min(r0 + i * nr, np - 1) * ST + d);
+#pragma unroll
+            for (int j = 0; j < CB; ++j) cv[j] = *reinterpret_cast<const float4*>(cnd + min(c0 + j, nc - 1) * ST + d);
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+              for (int j = 0; j < CB; ++j) {
+                acc[i][j] = dot_pair(acc[i][j], cv[j].x, rv[i].x, cv[j].y, rv[i].y);
+                acc[i][j] = dot_pair(acc[i][j], cv[j].z, rv[i].z, cv[j].w, rv[i].w);
+              }
+          }
+#pragma unroll
+          for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int j = 0; j < CB; ++j)
+              if (r0 + i * nr < np && c0 + j < nc)
+                __hip_atomic_store(out + (int64_t)(c0 + j) * M + r0 + i * nr, E::rnd(acc[i][j]), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+        }
+      };
+      constexpr std::integral_constant<int, 1> c1{};
+      constexpr std::integral_constant<int, 2> c2{};
+      constexpr std::integral_constant<int, 4> c4{};
+      constexpr std::integral_constant<int, DH> full{};
+      constexpr std::integral_constant<int, LF> low{};
+      float* oe = dot_e + (int64_t)h * TeM * Me + e0;
+      float* os = dot_s + (int64_t)h * TsM * Ms + s0;
+      const bool pairs_e = Te * ne > 128;
+      const int n_e = Te * (pairs_e ? (ne + 1) / 2 : ne), n_s = Ts * ns;  // exact blocks, summary dots
+      const bool split = n_e > 0 && 2 * n_e <= NT;
+      const int thr = split ? NT - n_e : NT;  // threads of the summary dots
+      if (n_e > 0 && (!split || t >= thr)) {
+        const int at = split ? t - thr : t, step = split ? n_e : NT;
+        if (pairs_e) run(c2, c1, nrm_e, cnd_e, full, ne, Te, oe, Me, at, step);
+        else run(c1, c1, nrm_e, cnd_e, full, ne, Te, oe, Me, at, step);
       }
-      if (lead)
-        for (int i = t1; i < Me + Ms; i += nt1) snap.allowed[(int64_t)b * (Me + Ms) + i] = (uint8_t)used[i];
+      if (n_s > 0 && t < thr) {
+        if (n_s <= thr) run(c1, c1, nrm_s, cnd_s, low, ns, Ts, os, Ms, t, thr);
+        else if (n_s <= 2 * thr) run(c2, c1, nrm_s, cnd_s, low, ns, Ts, os, Ms, t, thr);
+        else if (n_s <= 4 * thr) run(c2, c2, nrm_s, cnd_s, low, ns, Ts, os, Ms, t, thr);
+        else run(c4, c2, nrm_s, cnd_s, low, ns, Ts, os, Ms, t, thr);
+      }
     }
-  });
-  if (gave_up1) return;
-  // ---- 3. routing of this workgroup's tokens (token i of [Te | Ts] goes
-  // to workgroup i mod K): one wave per token
-  {
-    const float* dall_e = ws + (int64_t)b * Hkv * Te * Me;
-    const float* dall_s = ws + CODA_WS(ws_dot_s, s, g) + (int64_t)b * Hkv * Ts * Ms;
+    if (more && t < max(Te1, Ts1)) reinterpret_cast<int32_t*>(fsm + L.pc)[((c + 1) & 1) * TM + t] = base + n_ev + pn;
+    for (int i0 = t; i0 < n_raw; i0 += UC * NT) {
+      if (i0 != t) raw_load(i0);
+      raw_store(i0);
+    }
+    // the next chunk's rows and gates: loaded at sync 1, normalised at sync 2
+    const int32_t* pc1 = reinterpret_cast<const int32_t*>(fsm + L.pc) + ((c + 1) & 1) * TM;
+    const int nt1k = more ? n_tasks(Te1, Ts1) : 0;
+    constexpr int XT = sizeof(T) == 2 ? 2 : 1;  // tasks a wave ahead (fp32: registers for one)
+    T xn[XT][NX];
+    float gn = 0.f;
+    // sync 1
+    const bool gave_up1 = group_sync(flags, K, me, val, val + 1, spin_limit, status, &sync_gave_up,
+                                     [&](int t1, int nt1) __attribute__((always_inline)) {
+      for (int m = t1; m < Ms; m += nt1) smask[m] = 0;
+      const int w1 = t1 >> 6, nw1 = nt1 >> 6;
+      // the LRU victim order: the rank of each key among all, a key per wave
+      // and pass, counted by ballots (a key per lane walking all of them took
+      // 2 us at 64 keys, 4 at 128)
+      if (Te > 0) {
+        const int64_t k0 = key[min(lane, Me - 1)], k1 = key[min(64 + lane, Me - 1)];
+        for (int l0 = 0; w1 + nw1 * l0 < Me; l0 += 64) {
+          const int64_t mine = key[min(w1 + nw1 * (l0 + lane), Me - 1)];
+          for (int l = 0; l < 64; ++l) {
+            const int m = w1 + nw1 * (l0 + l);
+            if (m >= Me) break;
+            const int64_t km = (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(mine >> 32), l) << 32 |
+                                         (uint32_t)__builtin_amdgcn_readlane((int)mine, l));
+            int lt = __popcll(__ballot(lane < Me && k0 < km)) + __popcll(__ballot(64 + lane < Me && k1 < km));
+            int eq = __popcll(__ballot(lane < Me && k0 == km)) + __popcll(__ballot(64 + lane < Me && k1 == km));
+            for (int j0 = 128; j0 < Me; j0 += 64) {
+              const int64_t kj = key[min(j0 + lane, Me - 1)];
+              lt += __popcll(__ballot(j0 + lane < Me && kj < km));
+              eq += __popcll(__ballot(j0 + lane < Me && kj == km));
+            }
+            if (lt < n_lru && lane == 0) {
+              if (eq > 1) ties = 1;
+              else lru[lt] = m;
+            }
+          }
+        }
+      }
+      if (snap.k) {
+        // the bank slots before this chunk's update
+        const int64_t sb = c * g.snap_stride + ((int64_t)b * Hkv + h) * (Me + Ms) * DH;
+        const int n_ee = ne * CH, n_ss = ns * CH;
+        for (int i = t1; i < n_ee + n_ss; i += nt1) {
+          const bool ex = i < n_ee;
+          const int j = 8 * (ex ? i : i - n_ee);
+          const int64_t o = sb + (int64_t)(ex ? e0 : Me + s0) * DH + j;
+          st8<T>((T*)snap.k + o, ld8<T>((ex ? own_ek : own_sk) + j));
+          st8<T>((T*)snap.v + o, ld8<T>((ex ? own_ev : own_sv) + j));
+        }
+        if (lead)
+          for (int i = t1; i < Me + Ms; i += nt1)
+            snap.allowed[c * g.snap_al_stride + (int64_t)b * (Me + Ms) + i] = (uint8_t)used[i];
+      }
+      // (last: a load in flight is waited for at the head of a loop)
+      if (w1 < nt1k) {
+#pragma unroll
+        for (int u = 0; u < XT; ++u) task_load(pc1, Te1, Ts1, min(w1 + u * nw1, nt1k - 1), xn[u]);
+        if (t1 < max(Te1, Ts1)) gn = *gate_of(pc1[t1]);
+      }
+    });
+    if (gave_up1) return;
+    // ---- 2. routing of this workgroup's tokens (token i of [Te | Ts] goes
+    // to workgroup i mod K): one wave per token
     for (int i = me + K * wv; i < Te + Ts; i += K * NW) {
       const bool ex = i < Te;
       const int tt = ex ? i : i - Te, M = ex ? Me : Ms;
@@ -1796,8 +1951,8 @@ __global__ __launch_bounds__(kFusedThreads) void block_fused_kernel(const coda_b
       for (int m = lane; m < M; m += 64) {
         // the heads' dots 8 at a time, all in flight before the sum (kept
         // in head order: the reference's mean over heads)
-        const float* src = ex ? dall_e + (int64_t)tt * Me + m : dall_s + (int64_t)tt * Ms + m;
-        const int64_t hstride = ex ? (int64_t)Te * Me : (int64_t)Ts * Ms;
+        const float* src = ex ? dot_e + (int64_t)tt * Me + m : dot_s + (int64_t)tt * Ms + m;
+        const int64_t hstride = ex ? (int64_t)TeM * Me : (int64_t)TsM * Ms;
         float acc = 0.f;
         for (int h0 = 0; h0 < Hkv; h0 += 8) {
           float hv[8];
@@ -1823,311 +1978,355 @@ __global__ __launch_bounds__(kFusedThreads) void block_fused_kernel(const coda_b
         }
       }
     }
-  }
-  // sync 2; meanwhile this workgroup's share of head h's ring (every
-  // workgroup of head h has read its candidate rows before sync 1), and, where
-  // the leading LRU keys tie (slots still unused), their order as libstdc++
-  // leaves it, on one wave (on one thread and before the sync it took 6 us of
-  // a chunk of a fresh prompt)
-  const bool gave_up2 = group_sync(flags, K, me, 2 * epoch + 1, 2 * epoch + 1, spin_limit, status, &sync_gave_up,
-                                   [&](int t1, int nt1) {
-    if (Te > 0 && ties && t1 < 64) {
-      // (the stop lists where the norm caches were, last read before sync 1:
-      // at least Me rows)
-      uint16_t* lpos = reinterpret_cast<uint16_t*>(fsm + L.ov);
-      wave_topk_order<int64_t>(rk, Me, n_lru, false, true, lpos, lpos + Me, t1);
-      for (int r = t1; r < n_lru; r += 64) lru[r] = (int32_t)rk[r].i;
-    }
-    const int n_all = (Lr + g.blk - first) * CH;
-    const int pz = (n_all + NZ - 1) / NZ, p0 = min(n_all, z * pz), p1 = min(n_all, p0 + pz);
-    for (int base = p0 + t1; base < p1; base += kRingPre * nt1) {
-      Piece8<T> pk[kRingPre], pv[kRingPre];
-#pragma unroll
-      for (int u = 0; u < kRingPre; ++u) {
-        const int i = min(base + u * nt1, p1 - 1);
-        const int jb = first + i / CH - Lr, c = i % CH;
-        pk[u] = ld8<T>(kbk + b * g.b_sb + h * g.b_sh + (int64_t)jb * g.b_sl + 8 * c);
-        pv[u] = ld8<T>(vbk + b * g.b_sb + h * g.b_sh + (int64_t)jb * g.b_sl + 8 * c);
+    // sync 2; meanwhile the next chunk's candidate rows (the dots have read
+    // this chunk's) and, where the leading LRU keys tie (slots still
+    // unused), their order as libstdc++ leaves it, on one wave (on one
+    // thread and before the sync it took 6 us of a chunk of a fresh prompt)
+    const bool gave_up2 = group_sync(flags, K, me, val + 1, val + 2, spin_limit, status, &sync_gave_up,
+                                     [&](int t1, int nt1) __attribute__((always_inline)) {
+      if (Te > 0 && ties && t1 < 64) {
+        // (touch and emask are free until the decisions, lru until the order
+        // is known)
+        sel::Item<int64_t>* rk = reinterpret_cast<sel::Item<int64_t>*>(fsm + L.touch);
+        uint16_t* lpos = reinterpret_cast<uint16_t*>(lru);
+        for (int m = t1; m < Me; m += 64) rk[m] = sel::Item<int64_t>{key[m], (int64_t)m};
+        wave_lds_fence();
+        wave_topk_order<int64_t>(rk, Me, n_lru, false, true, lpos, lpos + Me, t1);
+        wave_lds_fence();
+        for (int r = t1; r < n_lru; r += 64) lru[r] = (int32_t)rk[r].i;
       }
+      const int w1 = t1 >> 6, nw1 = nt1 >> 6;
+      if (w1 < nt1k) {
 #pragma unroll
-      for (int u = 0; u < kRingPre; ++u) {
-        const int i = base + u * nt1;
-        if (i < p1) {
-          const int slot = (rhead + first + i / CH) % W, c = i % CH;
-          st8<T>(kb + (int64_t)slot * DH + 8 * c, pk[u]);
-          st8<T>(vb + (int64_t)slot * DH + 8 * c, pv[u]);
+        for (int u = 0; u < XT; ++u)
+          if (w1 + u * nw1 < nt1k) task_unit(Te1, Ts1, w1 + u * nw1, xn[u]);
+        for (int k = w1 + XT * nw1; k < nt1k; k += nw1) {
+          task_load(pc1, Te1, Ts1, k, xn[0]);
+          task_unit(Te1, Ts1, k, xn[0]);
+        }
+        if (t1 < max(Te1, Ts1)) reinterpret_cast<float*>(fsm + L.gate)[((c + 1) & 1) * TM + t1] = gn;
+      }
+    });
+    if (gave_up2) return;
+    // ---- 3a. every token's routing (all three loads in flight together);
+    // the summary slots' token masks
+    for (int i = t; i < TT; i += NT) {
+      const int ie = min(i, max(Te, 1) - 1), is = min(i, max(Ts, 1) - 1);
+      const int32_t fe = Te > 0 ? __hip_atomic_load(dx.fl_e + ie, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+      const int32_t xe = Te > 0 ? __hip_atomic_load(dx.idx_e + ie, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+      const int32_t xs = Ts > 0 ? __hip_atomic_load(dx.idx_s + is, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+      if (i < Te) {
+        bv_e[i] = __builtin_bit_cast(float, fe);
+        bi_e[i] = xe;
+      }
+      if (i < Ts) {
+        idx_s[i] = xs;
+        const float gt = gate[i];
+        wtok[i] = (!s.gated || gt >= s.tau_summary) ? E::rnd(gt) : 0.f;
+        if (xs >= 0 && xs < Ms) atomicOr(&smask[xs], 1ull << i);
+      }
+    }
+    __syncthreads();
+    // exact decisions (memory_banks.py:640-697) on wave 0 (at most 64
+    // tokens: lane tt takes token tt), the summary slots' weights on the
+    // other waves, side by side
+    const int sum_w0 = Te > 0 ? 1 : 0;
+    if (Te > 0 && wv == 0) {
+      // (the slots' masks and stamps of this chunk start cleared)
+      int u = 0;
+      for (int m = lane; m < Me; m += 64) {
+        u |= used[m] != 0;
+        emask[m] = 0;
+        touch[m] = kNegBig;
+      }
+      const int any_used = wave_or(u);
+      // the rank of a novel kept token (the reference's cumsum(novel & keep)
+      // - 1) from the ballot of the lanes before it
+      const uint64_t lt_mask = lane ? (~0ull >> (64 - lane)) : 0ull;
+      const int tt = lane;
+      const bool in = tt < Te;
+      const int ti = in ? tt : Te - 1;
+      const bool keep = s.gated ? (gate[ti] >= s.tau_exact) : true;
+      const float bv = bv_e[ti];
+      const bool novel = !any_used || bv < E::rnd(s.tau_novel);
+      const bool hit = any_used && bv >= E::rnd(s.tau_match);
+      const bool nk = in && novel && keep;
+      const uint64_t bal = __ballot(nk);
+      const int rank = __popcll(bal & lt_mask) + (nk ? 1 : 0) - 1;
+      const bool cap = nk && rank < Ae;
+      int idx = bi_e[ti];
+      if (cap) idx = lru[min(max(rank, 0), n_lru - 1)];
+      const bool tch = keep && (!novel || cap);
+      const bool ow = s.refresh_on_hit ? (keep && (cap || hit)) : cap;
+      if (in) {
+        idx_e[tt] = idx;
+        fl_e[tt] = (ow ? 1 : 0) | (tch ? 2 : 0);
+        // the slot's writing tokens, and the largest position of its touching
+        // ones, through LDS atomics (after this wave's clears, in its LDS order)
+        if (ow) atomicOr(&emask[idx], 1ull << tt);
+        if (tch) atomicMax(reinterpret_cast<long long*>(&touch[idx]), (long long)(g.pos0 - F0 + pc[tt]));
+      }
+      if (lead && (s.metrics || s.frustrated)) {
+        const int c_ow = __popcll(__ballot(in && ow)), c_cap = __popcll(__ballot(in && cap));
+        const int c_hit = __popcll(__ballot(in && hit && keep)), c_gated = __popcll(__ballot(in && !keep));
+        const int c_fr = __popcll(__ballot(nk && !cap));
+        if (lane == 0) {
+          if (s.metrics) {
+            atomic_add_i64(s.metrics + CODA_CNT_EXACT_OVERWRITES, c_ow);
+            atomic_add_i64(s.metrics + CODA_CNT_EXACT_FRUSTRATED, c_fr);
+            atomic_add_i64(s.metrics + CODA_CNT_EXACT_INSERTS, c_cap);
+            atomic_add_i64(s.metrics + CODA_CNT_EXACT_HITS, c_hit);
+            if (s.gated) atomic_add_i64(s.metrics + CODA_CNT_TOKENS_GATED_OUT, c_gated);
+          }
+          if (s.frustrated) atomic_add_i64(s.frustrated + 0, c_fr);
         }
       }
     }
-    // ring gates and visibility bytes of the chunk's surviving tokens
-    // (per sequence: head 0's workgroups share them)
-    if (h == 0) {
-      const int n_tok = Lr + g.blk - first;
-      const int pt = (n_tok + NZ - 1) / NZ, q0 = min(n_tok, z * pt), q1 = min(n_tok, q0 + pt);
-      for (int i = q0 + t1; i < q1; i += nt1) {
-        const int r = first + i, slot = (rhead + r) % W;
-        s.g_recent[(int64_t)b * W + slot] = gb[(int64_t)b * g.g_sb + (r - Lr)];
-        al[slot] = 1;
-      }
-    }
-  });
-  if (gave_up2) return;
-  // every workgroup of b has read gen_b (before its sync-1 flag): the next
-  // launch on this workspace takes the next generation
-  if (lead && t == 0) __hip_atomic_store(tail + b, gen_b + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  // ---- 4a. every token's routing (all three loads in flight together);
-  // exact decisions (memory_banks.py:640-697)
-  for (int i = t; i < TT; i += NT) {
-    const int ie = min(i, max(Te, 1) - 1), is = min(i, max(Ts, 1) - 1);
-    const int32_t fe = Te > 0 ? __hip_atomic_load(dx.fl_e + ie, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
-    const int32_t xe = Te > 0 ? __hip_atomic_load(dx.idx_e + ie, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
-    const int32_t xs = Ts > 0 ? __hip_atomic_load(dx.idx_s + is, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
-    if (i < Te) {
-      bv_e[i] = __builtin_bit_cast(float, fe);
-      bi_e[i] = xe;
-    }
-    if (i < Ts) {
-      idx_s[i] = xs;
-      const float gt = gate[i];
-      wtok[i] = (!s.gated || gt >= s.tau_summary) ? E::rnd(gt) : 0.f;
-    }
-  }
-  __syncthreads();
-  // exact decisions on wave 0 (at most 64 tokens: lane tt takes token tt),
-  // the summary slots' token masks on the other waves, side by side
-  const int sum_w0 = Te > 0 ? 1 : 0;  // first wave of the summary masks
-  if (Te > 0 && wv == 0) {
-    // (exact flags and touch stamps start cleared; the staged stamps are no
-    // longer read)
-    int u = 0;
-    for (int m = lane; m < Me; m += 64) {
-      u |= used[m] != 0;
-      eflag[m] = 0;
-      last[m] = kNegBig;
-    }
-    const int any_used = wave_or(u);
-    // the rank of a novel kept token (the reference's cumsum(novel & keep)
-    // - 1) from the ballot of the lanes before it
-    const uint64_t lt_mask = lane ? (~0ull >> (64 - lane)) : 0ull;
-    const int tt = lane;
-    const bool in = tt < Te;
-    const int ti = in ? tt : Te - 1;
-    const bool keep = s.gated ? (gate[ti] >= s.tau_exact) : true;
-    const float bv = bv_e[ti];
-    const bool novel = !any_used || bv < E::rnd(s.tau_novel);
-    const bool hit = any_used && bv >= E::rnd(s.tau_match);
-    const bool nk = in && novel && keep;
-    const uint64_t bal = __ballot(nk);
-    const int rank = __popcll(bal & lt_mask) + (nk ? 1 : 0) - 1;
-    const bool cap = nk && rank < Ae;
-    int idx = bi_e[ti];
-    if (cap) idx = lru[min(max(rank, 0), n_lru - 1)];
-    const bool touch = keep && (!novel || cap);
-    const bool ow = s.refresh_on_hit ? (keep && (cap || hit)) : cap;
-    if (in) {
-      idx_e[tt] = idx;
-      fl_e[tt] = (ow ? 1 : 0) | (touch ? 2 : 0);
-      // the slot's flags through LDS atomics (after this wave's clears, in
-      // its LDS order): written (an overwriting token) and touched (max
-      // position of the touching tokens)
-      if (ow) atomicOr(&eflag[idx], 1);
-      if (touch) atomicMax(reinterpret_cast<long long*>(&last[idx]), (long long)(g.pos0 - g.ring_filled + pcl[tt]));
-    }
-    if (lead && (s.metrics || s.frustrated)) {
-      const int c_ow = __popcll(__ballot(in && ow)), c_cap = __popcll(__ballot(in && cap));
-      const int c_hit = __popcll(__ballot(in && hit && keep)), c_gated = __popcll(__ballot(in && !keep));
-      const int c_fr = __popcll(__ballot(nk && !cap));
-      if (lane == 0) {
-        if (s.metrics) {
-          atomic_add_i64(s.metrics + CODA_CNT_EXACT_OVERWRITES, c_ow);
-          atomic_add_i64(s.metrics + CODA_CNT_EXACT_FRUSTRATED, c_fr);
-          atomic_add_i64(s.metrics + CODA_CNT_EXACT_INSERTS, c_cap);
-          atomic_add_i64(s.metrics + CODA_CNT_EXACT_HITS, c_hit);
-          if (s.gated) atomic_add_i64(s.metrics + CODA_CNT_TOKENS_GATED_OUT, c_gated);
-        }
-        if (s.frustrated) atomic_add_i64(s.frustrated + 0, c_fr);
-      }
-    }
-  }
-  if (wv >= sum_w0) {
-    // summary slots, 8 per wave and pass: token masks (ballots over the
-    // tokens), then lane u sums slot u's weights in token order (fp32: the
-    // scatter_add order) and sets its active / newly used flags
-    for (int m0 = 8 * (wv - sum_w0); m0 < Ms; m0 += 8 * (NW - sum_w0)) {
-      uint64_t mine = 0;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const uint64_t mk = __ballot(lane < Ts && idx_s[min(lane, max(Ts, 1) - 1)] == m0 + u);
-        if (lane == u) mine = mk;
-      }
-      const int m = m0 + lane;
-      if (lane < 8 && m < Ms) {
-        float c = 0.f;
-        for (uint64_t r = mine; r; r &= r - 1) c += wtok[__builtin_ctzll(r)];
-        c = E::rnd(c);
-        smask[m] = mine;
-        scnt[m] = c;
-        const bool active = c > 0.f;
+    if (wv >= sum_w0) {
+      // each slot's weights in token order (fp32: the scatter_add order),
+      // its active / newly used flags
+      for (int m = t - 64 * sum_w0; m < Ms; m += NT - 64 * sum_w0) {
+        float cn = 0.f;
+        for (uint64_t r = smask[m]; r; r &= r - 1) cn += wtok[__builtin_ctzll(r)];
+        cn = E::rnd(cn);
+        scnt[m] = cn;
+        const bool active = cn > 0.f;
         sflag[m] = (active ? 1 : 0) | ((active && used[Me + m] == 0) ? 2 : 0);
       }
     }
+    __syncthreads();
+    if (lead && (s.metrics || s.frustrated || s.trace)) {
+      int32_t* tr = s.trace ? s.trace + (int64_t)b * (2 * Te + Ts) : nullptr;
+      if (tr) {
+        for (int tt = t; tt < Te; tt += NT) {
+          tr[tt] = idx_e[tt];
+          tr[Te + tt] = fl_e[tt];
+        }
+        for (int tt = t; tt < Ts; tt += NT) tr[2 * Te + tt] = idx_s[tt];
+      }
+      if (Ts > 0 && wv == 0) {
+        int64_t upd = 0, ins = 0;
+        bool all_used = true, any_cnt = false;
+        for (int m0 = 0; m0 < Ms; m0 += 64) {
+          const int m = m0 + lane;
+          const int f = m < Ms ? sflag[m] : 0;
+          const bool act = m < Ms && m < As;
+          upd += __popcll(__ballot(f & 1));
+          ins += __popcll(__ballot((f >> 1) & 1));
+          all_used = all_used && __ballot(act && !(used[Me + min(m, Ms - 1)] != 0 || (f & 1))) == 0;
+          any_cnt = any_cnt || __ballot(act && (f & 1)) != 0;
+        }
+        if (lane == 0) {
+          if (s.metrics) {
+            atomic_add_i64(s.metrics + CODA_CNT_SUMMARY_UPDATES, upd);
+            if (s.overwrite_on_insert) atomic_add_i64(s.metrics + CODA_CNT_SUMMARY_INSERTS, ins);
+          }
+          if (s.frustrated) {
+            if (!all_used) atomic_add_i64(s.frustrated + 1, 1);
+            if (any_cnt) atomic_add_i64(s.frustrated + 2, 1);
+          }
+        }
+      }
+      __syncthreads();
+    }
+    // ---- 3b. the sequence's metadata after this chunk (LRU: the largest
+    // position of the touching tokens), and the next LRU keys
+    for (int m = t; m < Me; m += NT) {
+      const int64_t tm = touch[m];
+      const int64_t at = Te > 0 && tm != kNegBig ? tm : last[m];
+      const int u = Te > 0 && emask[m] ? 1 : used[m];
+      last[m] = at;
+      used[m] = u;
+      lru_key(m, u != 0, at);
+    }
+    if (Ts > 0)
+      for (int m = t; m < Ms; m += NT)
+        if (sflag[m] & 1) used[Me + m] = 1;
+    if (t == 0) ties = 0;
+    // ---- 3c. exact write-back of this workgroup's slots (memory_banks.py:
+    // 707-742): one wave per written slot, deltas summed in token order
+    if (Te > 0) {
+      int turn_e = 0;
+      for (int m0 = e0; m0 < e1; m0 += 64) {
+        uint64_t todo = __ballot(m0 + lane < e1 && emask[min(m0 + lane, e1 - 1)] != 0);
+        for (; todo; todo &= todo - 1, ++turn_e) {
+          if (turn_e % NW != wv) continue;
+          const int m = m0 + __builtin_ctzll(todo), r = m - e0;
+          float mk[NV], mv[NV], ak[NV], av[NV];
+#pragma unroll
+          for (int i = 0; i < NV; ++i) {
+            const int d = min(lane + 64 * i, DH - 1);
+            mk[i] = E::ld(own_ek[r * DH + d]);
+            mv[i] = E::ld(own_ev[r * DH + d]);
+            ak[i] = 0.f;
+            av[i] = 0.f;
+          }
+          for (uint64_t wr = emask[m]; wr; wr &= wr - 1) {
+            const int tt = __builtin_ctzll(wr);
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+              const int d = min(lane + 64 * i, DH - 1);
+              ak[i] += E::rnd(E::ld(raw_k[tt * DH + d]) - mk[i]);
+              av[i] += E::rnd(E::ld(raw_v[tt * DH + d]) - mv[i]);
+            }
+          }
+          float nv[NV];
+          bool act[NV];
+#pragma unroll
+          for (int i = 0; i < NV; ++i) {
+            const int d = lane + 64 * i;
+            act[i] = d < DH;
+            nv[i] = 0.f;
+            if (act[i]) {
+              own_ek[r * DH + d] = E::st(mk[i] + E::rnd(ak[i]));
+              nv[i] = E::rnd(mv[i] + E::rnd(av[i]));
+              own_ev[r * DH + d] = E::st(nv[i]);
+            }
+          }
+          wave_unit<T, NV>(nv, act);
+#pragma unroll
+          for (int i = 0; i < NV; ++i)
+            if (act[i]) nrm_e[r * le + lane + 64 * i] = E::st(nv[i]);
+        }
+      }
+    }
+    // ---- 3d. summary accumulate + EMA of this workgroup's slots
+    // (memory_banks.py:880-932): one wave per active slot (from the last wave
+    // down: the first ones have the exact slots), lane l taking columns l,
+    // l + 64, ... (column col < DH is V channel col, else K channel DH/2 +
+    // col - DH), all of them over the slot's tokens in token order (the fp32
+    // scatter_add order); then the slot's new LF key row through LDS and its
+    // norm row, within the wave
+    if (Ts > 0) {
+      const float eta_h = s.eta[h];
+      constexpr int NCW = (NCOL + 63) / 64;
+      int turn_s = 0;
+      for (int m0 = s0; m0 < s1; m0 += 64) {
+        uint64_t todo = __ballot(m0 + lane < s1 && (sflag[min(m0 + lane, s1 - 1)] & 1));
+        for (; todo; todo &= todo - 1, ++turn_s) {
+          if (NW - 1 - turn_s % NW != wv) continue;
+          const int m = m0 + __builtin_ctzll(todo), rl = m - s0;
+          const uint64_t msk = smask[m];
+          const float eta = (s.overwrite_on_insert && (sflag[m] & 2)) ? 1.f : eta_h;
+          const float cnt = fmaxf(scnt[m], eps_r<T>());
+          const T* tokv[NCW];
+          float a[NCW];
+#pragma unroll
+          for (int jc = 0; jc < NCW; ++jc) {
+            const int col = min(lane + 64 * jc, NCOL - 1);
+            tokv[jc] = (col < DH ? raw_v : raw_k) + (col < DH ? col : LF + (col - DH));
+          }
+          {
+            uint64_t r = msk;
+            int tt = __builtin_ctzll(r);
+            float wt = wtok[tt];
+#pragma unroll
+            for (int jc = 0; jc < NCW; ++jc) a[jc] = E::rnd(E::ld(tokv[jc][tt * DH]) * wt);
+            for (r &= r - 1; r; r &= r - 1) {
+              tt = __builtin_ctzll(r);
+              wt = wtok[tt];
+#pragma unroll
+              for (int jc = 0; jc < NCW; ++jc) a[jc] += E::rnd(E::ld(tokv[jc][tt * DH]) * wt);
+            }
+          }
+#pragma unroll
+          for (int jc = 0; jc < NCW; ++jc) {
+            const int col = lane + 64 * jc;
+            if (col >= NCOL) continue;
+            const float avg = E::rnd(E::rnd(a[jc]) / cnt);
+            if (col < DH) {
+              const float mem = E::ld(own_sv[rl * DH + col]);
+              own_sv[rl * DH + col] = E::st(mem + E::rnd(eta * E::rnd(avg - mem)));
+            } else {
+              const int d = LF + (col - DH);
+              const float mem = E::ld(own_sk[rl * DH + d]);
+              const float dk = E::rnd(E::rnd(avg * s.energy_scale) - mem);
+              const float nkv = E::rnd(mem + E::rnd(eta * dk));
+              own_sk[rl * DH + d] = E::st(nkv);
+              knew[col - DH] = nkv;  // new LF key for the norm row
+            }
+          }
+          wave_lds_fence();  // this wave's LF keys are in LDS
+          float x[NV];
+          bool act[NV];
+#pragma unroll
+          for (int i = 0; i < NV; ++i) {
+            const int dd = lane + 64 * i;
+            act[i] = dd < LF;
+            x[i] = act[i] ? knew[dd] : 0.f;
+          }
+          wave_unit<T, NV>(x, act);
+#pragma unroll
+          for (int i = 0; i < NV; ++i)
+            if (act[i]) nrm_s[rl * lsum + lane + 64 * i] = E::st(x[i]);
+        }
+      }
+    }
+    base += n_ev;
+    filled = filled_next;
+    if (!more) break;
+    filled_next = filled1;
+    n_ev = n_ev1;
+    Te = Te1;
+    Ts = Ts1;
   }
+  // every workgroup of b has read gen_b (before its first flag): the next
+  // launch on this workspace takes the next generation
+  if (lead && t == 0) __hip_atomic_store(tail + b, gen_b + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
+  // ---- 4. what the launch leaves: this workgroup's slots and norm rows,
+  {
+    const int n_ee = ne * CH, n_ss = ns * CH, n_ns = ns * CHL;
+    for (int i = t; i < n_ee; i += NT) {
+      const int64_t o = (int64_t)(W + e0) * DH + 8 * i;
+      st8<T>(kb + o, ld8<T>(own_ek + 8 * i));
+      st8<T>(vb + o, ld8<T>(own_ev + 8 * i));
+      st8<T>(gn_e + 8 * i, ld8_row<T>(nrm_e + (i / CH) * le + 8 * (i % CH)));
+    }
+    for (int i = t; i < n_ss; i += NT) {
+      const int64_t o = (int64_t)(W + Me + s0) * DH + 8 * i;
+      st8<T>(kb + o, ld8<T>(own_sk + 8 * i));
+      st8<T>(vb + o, ld8<T>(own_sv + 8 * i));
+      if (i < n_ns) st8<T>(gn_s + 8 * i, ld8_row<T>(nrm_s + (i / CHL) * lsum + 8 * (i % CHL)));
+    }
+  }
+  // the sequence's metadata,
   if (lead) {
-    if (Te > 0)
-      for (int m = t; m < Me; m += NT) {
-        if (last[m] != kNegBig) s.mem_last[(int64_t)b * Me + m] = last[m];  // LRU: max pos of the touching tokens
-        if (eflag[m]) al[W + m] = 1;
-      }
-    int32_t* tr = s.trace ? s.trace + (int64_t)b * (2 * Te + Ts) : nullptr;
-    if (tr) {
-      for (int tt = t; tt < Te; tt += NT) {
-        tr[tt] = idx_e[tt];
-        tr[Te + tt] = fl_e[tt];
-      }
-      for (int tt = t; tt < Ts; tt += NT) tr[2 * Te + tt] = idx_s[tt];
-    }
-    for (int m = t; m < Ms; m += NT)
-      if (sflag[m] & 1) al[W + Me + m] = 1;
-    if (Ts > 0 && wv == 0) {
-      // counts and flags by ballots (no shuffle chain on the lead's path)
-      int64_t upd = 0, ins = 0;
-      bool all_used = true, any_cnt = false;
-      for (int m0 = 0; m0 < Ms; m0 += 64) {
-        const int m = m0 + lane;
-        const int f = m < Ms ? sflag[m] : 0;
-        const bool act = m < Ms && m < As;
-        upd += __popcll(__ballot(f & 1));
-        ins += __popcll(__ballot((f >> 1) & 1));
-        all_used = all_used && __ballot(act && !(used[Me + min(m, Ms - 1)] != 0 || (f & 1))) == 0;
-        any_cnt = any_cnt || __ballot(act && (f & 1)) != 0;
-      }
-      if (lane == 0) {
-        if (s.metrics) {
-          atomic_add_i64(s.metrics + CODA_CNT_SUMMARY_UPDATES, upd);
-          if (s.overwrite_on_insert) atomic_add_i64(s.metrics + CODA_CNT_SUMMARY_INSERTS, ins);
-        }
-        if (s.frustrated) {
-          if (!all_used) atomic_add_i64(s.frustrated + 1, 1);
-          if (any_cnt) atomic_add_i64(s.frustrated + 2, 1);
-        }
-      }
-    }
+    for (int m = t; m < Me; m += NT) s.mem_last[(int64_t)b * Me + m] = last[m];
+    for (int m = t; m < Me + Ms; m += NT) al[W + m] = (uint8_t)used[m];
   }
-  __syncthreads();
-  // ---- 4b. exact write-back of this workgroup's slots (memory_banks.py:
-  // 707-742): one wave per written slot, deltas summed in token order
-  if (Te > 0) {
-    for (int m = e0 + wv; m < e1; m += NW) {
-      if (!eflag[m]) continue;
-      const int r = m - e0;
-      float mk[NV], mv[NV], ak[NV], av[NV];
+  // and its share of head h's ring (every candidate row and gate in the ring
+  // has been read: before sync 2); per sequence, head 0's workgroups share
+  // the ring gates and visibility bytes
+  {
+    const int total = base + filled, first = max(F0, total - W), n_tok = total - first, n_all = n_tok * CH;
+    const int pz = (n_all + NZ - 1) / NZ, p0 = min(n_all, z * pz), p1 = min(n_all, p0 + pz);
+    for (int i0 = p0 + t; i0 < p1; i0 += kRingPre * NT) {
+      Piece8<T> pk[kRingPre], pv[kRingPre];
 #pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const int d = min(lane + 64 * i, DH - 1);
-        mk[i] = E::ld(own_ek[r * DH + d]);
-        mv[i] = E::ld(own_ev[r * DH + d]);
-        ak[i] = 0.f;
-        av[i] = 0.f;
+      for (int u = 0; u < kRingPre; ++u) {
+        const int i = min(i0 + u * NT, p1 - 1);
+        const int64_t o = (int64_t)(first + i / CH - F0) * g.b_sl + 8 * (i % CH);
+        pk[u] = ld8<T>(kc + o);
+        pv[u] = ld8<T>(vc + o);
       }
-      for (int tt = 0; tt < Te; ++tt) {
-        if (idx_e[tt] != m || !(fl_e[tt] & 1)) continue;
 #pragma unroll
-        for (int i = 0; i < NV; ++i) {
-          const int d = min(lane + 64 * i, DH - 1);
-          ak[i] += E::rnd(E::ld(raw_k[tt * DH + d]) - mk[i]);
-          av[i] += E::rnd(E::ld(raw_v[tt * DH + d]) - mv[i]);
+      for (int u = 0; u < kRingPre; ++u) {
+        const int i = i0 + u * NT;
+        if (i < p1) {
+          const int64_t o = (int64_t)((rhead + first + i / CH) % W) * DH + 8 * (i % CH);
+          st8<T>(kb + o, pk[u]);
+          st8<T>(vb + o, pv[u]);
         }
       }
-      T* kr = kb + (int64_t)(W + m) * DH;
-      T* vr = vb + (int64_t)(W + m) * DH;
-      float nv[NV];
-      bool act[NV];
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const int d = lane + 64 * i;
-        act[i] = d < DH;
-        nv[i] = 0.f;
-        if (act[i]) {
-          kr[d] = E::st(mk[i] + E::rnd(ak[i]));
-          nv[i] = E::rnd(mv[i] + E::rnd(av[i]));
-          vr[d] = E::st(nv[i]);
-        }
-      }
-      wave_unit<T, NV>(nv, act);
-      T* nr = (T*)s.exact_v_norm + (((int64_t)b * Hkv + h) * Me + m) * DH;
-#pragma unroll
-      for (int i = 0; i < NV; ++i)
-        if (act[i]) nr[lane + 64 * i] = E::st(nv[i]);
     }
-  }
-  // ---- 4c. summary accumulate + EMA of this workgroup's slots
-  // (memory_banks.py:880-932): one wave per slot, lane l taking columns l,
-  // l + 64, ... (column col < DH is V channel col, else K channel
-  // DH/2 + col - DH), all of them over the slot's tokens in token order (the
-  // fp32 scatter_add order); then the slot's new LF key row through LDS and
-  // its norm-cache row, within the wave
-  if (Ts > 0) {
-    const float eta_h = s.eta[h];
-    constexpr int NCW = (NCOL + 63) / 64;
-    for (int m = s0 + wv; m < s1; m += NW) {
-      if (!(sflag[m] & 1)) continue;
-      const uint64_t msk = smask[m];
-      const float eta = (s.overwrite_on_insert && (sflag[m] & 2)) ? 1.f : eta_h;
-      const float cnt = fmaxf(scnt[m], eps_r<T>());
-      const int rl = m - s0;
-      const T* tokv[NCW];
-      float a[NCW];
-#pragma unroll
-      for (int jc = 0; jc < NCW; ++jc) {
-        const int col = min(lane + 64 * jc, NCOL - 1);
-        tokv[jc] = (col < DH ? raw_v : raw_k) + (col < DH ? col : LF + (col - DH));
+    if (h == 0) {
+      const int pt = (n_tok + NZ - 1) / NZ, q0 = min(n_tok, z * pt), q1 = min(n_tok, q0 + pt);
+      for (int i = q0 + t; i < q1; i += NT) {
+        const int slot = (rhead + first + i) % W;
+        s.g_recent[(int64_t)b * W + slot] = gc[first + i - F0];
+        al[slot] = 1;
       }
-      {
-        uint64_t r = msk;
-        int tt = __builtin_ctzll(r);
-        float wt = wtok[tt];
-#pragma unroll
-        for (int jc = 0; jc < NCW; ++jc) a[jc] = E::rnd(E::ld(tokv[jc][tt * DH]) * wt);
-        for (r &= r - 1; r; r &= r - 1) {
-          tt = __builtin_ctzll(r);
-          wt = wtok[tt];
-#pragma unroll
-          for (int jc = 0; jc < NCW; ++jc) a[jc] += E::rnd(E::ld(tokv[jc][tt * DH]) * wt);
-        }
-      }
-#pragma unroll
-      for (int jc = 0; jc < NCW; ++jc) {
-        const int col = lane + 64 * jc;
-        if (col >= NCOL) continue;
-        const float avg = E::rnd(E::rnd(a[jc]) / cnt);
-        if (col < DH) {
-          const float mem = E::ld(own_sv[rl * DH + col]);
-          vb[(int64_t)(W + Me + m) * DH + col] = E::st(mem + E::rnd(eta * E::rnd(avg - mem)));
-        } else {
-          const int d = LF + (col - DH);
-          const float mem = E::ld(own_sk[rl * DH + d]);
-          const float dk = E::rnd(E::rnd(avg * s.energy_scale) - mem);
-          const float nkv = E::rnd(mem + E::rnd(eta * dk));
-          kb[(int64_t)(W + Me + m) * DH + d] = E::st(nkv);
-          knew[rl * LF + (col - DH)] = nkv;  // new LF key for the norm cache
-        }
-      }
-      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LF keys are in LDS
-      __builtin_amdgcn_wave_barrier();
-      float x[NV];
-      bool act[NV];
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const int dd = lane + 64 * i;
-        act[i] = dd < LF;
-        x[i] = act[i] ? knew[rl * LF + dd] : 0.f;
-      }
-      wave_unit<T, NV>(x, act);
-      T* nr = (T*)s.sum_lf_k_norm + (((int64_t)b * Hkv + h) * Ms + m) * LF;
-#pragma unroll
-      for (int i = 0; i < NV; ++i)
-        if (act[i]) nr[lane + 64 * i] = E::st(x[i]);
     }
   }
 }
@@ -2421,10 +2620,10 @@ extern "C" int coda_block_workspace_bytes(const coda_bank_desc* s, int Kmax, siz
 // the process (48 bits), started from a clock-derived value so that a sync
 // word left in a reused workspace never carries the epoch of a later
 // launch (the kernel mixes in the sequence's generation word).
-static unsigned long long next_epoch() {
+static unsigned long long next_epoch(int chunks) {
   static std::atomic<unsigned long long> ep{
       (unsigned long long)std::chrono::steady_clock::now().time_since_epoch().count() * 0x9E3779B97F4A7C15ull};
-  return ep.fetch_add(1, std::memory_order_relaxed) & ((1ull << 48) - 1);
+  return ep.fetch_add((unsigned long long)chunks, std::memory_order_relaxed) & ((1ull << 48) - 1);
 }
 
 // The fused kernel runs when its LDS fits and CODA_BLOCK_FUSED is not "0"
@@ -2492,6 +2691,22 @@ static SplitShape split_shape(const coda_bank_desc* s, int Te, int Ts, int pairs
 static std::atomic<int> g_spin_limit{kSyncSpinLimit};
 
 template <typename T, int DH>
+static int launch_fused(const coda_bank_desc* s, const void* kb, const void* vb, const float* gb, const ChainGeom& g,
+                        FusedShape fs, const int32_t* plan, float* ws, unsigned long long* tail, hipStream_t st,
+                        BankSnap snap) {
+  const int rc = lds_limit<block_fused_kernel<T, DH>>(fs.lds, "coda_block_write");
+  if (rc) return rc;
+  unsigned long long* flags = reinterpret_cast<unsigned long long*>(ws + CODA_WS(ws_sync, *s, g));
+  // (sequence, head) pairs in blocks of 8, one pair per XCD (a pair beyond
+  // B * Hkv exits at once)
+  const int nwg = ((s->B * s->Hkv + 7) / 8) * 8 * fs.nz;
+  hipLaunchKernelGGL((block_fused_kernel<T, DH>), dim3(nwg), dim3(kFusedThreads), fs.lds, st, *s, g, fs.nz,
+                     (const T*)kb, (const T*)vb, gb, plan, ws, flags, next_epoch(g.n), tail,
+                     g_spin_limit.load(std::memory_order_relaxed), snap);
+  return check_launch("block_fused");
+}
+
+template <typename T, int DH>
 static int launch_block(const coda_bank_desc* s, const void* kb, const void* vb, const float* gb, BlockGeom g,
                         const int32_t* plan_c, float* ws, unsigned long long* tail, hipStream_t st,
                         BankSnap snap) {
@@ -2499,19 +2714,10 @@ static int launch_block(const coda_bank_desc* s, const void* kb, const void* vb,
   const int pairs = s->B * s->Hkv;
   if (g.n_ev > 0 && TT > 0 && fused_enabled()) {
     const FusedShape fs = fused_shape(s, (int)sizeof(T), g.Te, g.Ts, pairs);
-    const int NZ = fs.nz;
-    const size_t lds = fs.lds;
-    if (NZ > 0) {
-      int rc = lds_limit<block_fused_kernel<T, DH>>(lds, "coda_block_write");
-      if (rc) return rc;
-      unsigned long long* flags = reinterpret_cast<unsigned long long*>(ws + CODA_WS(ws_sync, *s, g));
-      // (sequence, head) pairs in blocks of 8, one pair per XCD (a pair
-      // beyond B * Hkv exits at once)
-      const int nwg = ((pairs + 7) / 8) * 8 * NZ;
-      hipLaunchKernelGGL((block_fused_kernel<T, DH>), dim3(nwg), dim3(kFusedThreads), lds, st, *s, g, NZ,
-                         (const T*)kb, (const T*)vb, gb, plan_c, ws, flags, next_epoch(), tail,
-                         g_spin_limit.load(std::memory_order_relaxed), snap);
-      return check_launch("block_fused");
+    if (fs.nz > 0) {
+      const ChainGeom cg{1, g.blk, g.blk, g.ring_head, g.ring_filled, g.Kmax, g.Te, g.Ts, g.Te, g.Ts, g.pos0,
+                         g.b_sb, g.b_sh, g.b_sl, g.g_sb, 0, 0};
+      return launch_fused<T, DH>(s, kb, vb, gb, cg, fs, plan_c, ws, tail, st, snap);
     }
   }
   if (snap.k)
@@ -2651,6 +2857,9 @@ extern "C" int coda_block_write_chain(const coda_bank_desc* s, const void* kb, c
                c_first + n_chunks - 1, L, blk);
   CODA_REQUIRE(!s->metrics && !s->frustrated && !s->trace,
                "coda_block_write_chain: metrics, frustration flags and traces need the per-chunk calls");
+  CODA_REQUIRE(ring_filled >= 0 && ring_filled <= s->W, "coda_block_write_chain: ring_filled outside [0, W]");
+  CODA_REQUIRE(ring_head >= 0 && ring_head < s->W && (ring_filled == s->W || ring_head == 0),
+               "coda_block_write_chain: bad ring head %d", ring_head);
   CODA_REQUIRE(snap_stride >= 0 && snap_al_stride >= 0, "coda_block_write_chain: negative snapshot stride");
   CODA_REQUIRE(((uintptr_t)snap_k % 16) == 0 && ((uintptr_t)snap_v % 16) == 0 &&
                    (snap_stride * (s->dtype == CODA_BF16 ? 2 : 4)) % 16 == 0,
@@ -2658,7 +2867,7 @@ extern "C" int coda_block_write_chain(const coda_bank_desc* s, const void* kb, c
   // the ring progression first: every chunk must evict and take the
   // one-launch update, else nothing is enqueued
   const size_t esz = s->dtype == CODA_BF16 ? 2 : 4;
-  int head = ring_head, filled = ring_filled;
+  int head = ring_head, filled = ring_filled, Te_max = 0, Ts_max = 0;
   for (int i = 0; i < n_chunks; ++i) {
     const int t = (c_first + i) * blk, n = blk < L - t ? blk : L - t;
     const int total = filled + n, keep = total < s->W ? total : s->W, n_ev = total - keep;
@@ -2666,6 +2875,9 @@ extern "C" int coda_block_write_chain(const coda_bank_desc* s, const void* kb, c
     const int Ts = s->Ms > 0 ? (k_summary < n_ev ? k_summary : n_ev) : 0;
     CODA_REQUIRE(n_ev > 0 && (Te > 0 || Ts > 0), "coda_block_write_chain: chunk %d evicts nothing", c_first + i);
     CODA_REQUIRE(Te <= Kmax && Ts <= Kmax, "coda_block_write_chain: Kmax %d < candidates", Kmax);
+    CODA_REQUIRE(Te >= 0 && Ts >= 0, "coda_block_write_chain: negative candidate counts");
+    Te_max = std::max(Te_max, Te);
+    Ts_max = std::max(Ts_max, Ts);
     if (!(fused_enabled() && fused_shape(s, (int)esz, Te, Ts, s->B * s->Hkv).nz > 0))
       return fail(CODA_EUNSUP, "coda_block_write_chain: chunk %d does not take the one-launch update",
                   c_first + i);
@@ -2673,25 +2885,39 @@ extern "C" int coda_block_write_chain(const coda_bank_desc* s, const void* kb, c
     if (keep == s->W) head = (head + n_ev) % s->W;
     filled = keep;
   }
-  head = ring_head;
-  filled = ring_filled;
-  for (int i = 0; i < n_chunks; ++i) {
-    const int t = (c_first + i) * blk, n = blk < L - t ? blk : L - t;
-    const int total = filled + n, keep = total < s->W ? total : s->W, n_ev = total - keep;
-    const int Te = s->Me > 0 ? (k_exact < n_ev ? k_exact : n_ev) : 0;
-    const int Ts = s->Ms > 0 ? (k_summary < n_ev ? k_summary : n_ev) : 0;
-    const char* kbc = (const char*)kb + (int64_t)t * b_sl * (int64_t)esz;
-    const char* vbc = (const char*)vb + (int64_t)t * b_sl * (int64_t)esz;
-    rc = block_write_impl(s, kbc, vbc, b_sb, b_sh, b_sl, gb + t, g_sb, n, head, filled, pos0 + (int64_t)i * blk,
-                          plan + (int64_t)(c_first + i) * s->B * Kmax, Kmax, Te, Ts, workspace, workspace_bytes,
-                          stream,
-                          BankSnap{(char*)snap_k + (int64_t)i * snap_stride * (int64_t)esz,
-                                   (char*)snap_v + (int64_t)i * snap_stride * (int64_t)esz,
-                                   snap_allowed + (int64_t)i * snap_al_stride});
-    if (rc) return rc;
-    head = filled == s->W ? head : 0;
-    if (keep == s->W) head = (head + n_ev) % s->W;
-    filled = keep;
+  const size_t need = block_ws_bytes(s, Te_max, Ts_max);
+  CODA_REQUIRE(workspace && workspace_bytes >= need, "coda_block_write_chain: workspace %zu < %zu bytes",
+               workspace_bytes, need);
+  if (s->B > 0) {
+    const FusedShape fs = fused_shape(s, (int)esz, Te_max, Ts_max, s->B * s->Hkv);
+    unsigned long long* tail = block_tail(s, workspace, workspace_bytes);
+    int hd = ring_head, fl = ring_filled;
+    for (int i = 0; i < n_chunks; i += kChainChunks) {
+      const int n = std::min(kChainChunks, n_chunks - i), t = (c_first + i) * blk;
+      const int len = std::min(L - t, n * blk);
+      const ChainGeom g{n, len, blk, hd, fl, Kmax, s->Me > 0 ? k_exact : 0, s->Ms > 0 ? k_summary : 0, Te_max, Ts_max,
+                        pos0 + (int64_t)i * blk, b_sb, b_sh, b_sl, g_sb, snap_stride, snap_al_stride};
+      const char* kbc = (const char*)kb + (int64_t)t * b_sl * (int64_t)esz;
+      const char* vbc = (const char*)vb + (int64_t)t * b_sl * (int64_t)esz;
+      const BankSnap snap{(char*)snap_k + (int64_t)i * snap_stride * (int64_t)esz,
+                          (char*)snap_v + (int64_t)i * snap_stride * (int64_t)esz,
+                          snap_allowed + (int64_t)i * snap_al_stride};
+      const int32_t* pl = plan + (int64_t)(c_first + i) * s->B * Kmax;
+#define CODA_CHAIN(D)                                                                                                \
+  rc = s->dtype == CODA_BF16                                                                                         \
+           ? launch_fused<bf16_t, D>(s, kbc, vbc, gb + t, g, fs, pl, (float*)workspace, tail, (hipStream_t)stream, snap) \
+           : launch_fused<float, D>(s, kbc, vbc, gb + t, g, fs, pl, (float*)workspace, tail, (hipStream_t)stream, snap)
+      switch (s->Dh) {
+        case 32: CODA_CHAIN(32); break;
+        case 64: CODA_CHAIN(64); break;
+        default: CODA_CHAIN(128);
+      }
+#undef CODA_CHAIN
+      if (rc) return rc;
+      const int total = fl + len;
+      if (total >= s->W) hd = ((fl == s->W ? hd : 0) + total - s->W) % s->W;
+      fl = total < s->W ? total : s->W;
+    }
   }
   ring_out[0] = head;
   ring_out[1] = filled;
