@@ -334,8 +334,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
             _hip.check(_hip.lib().coda_project_rows(d, _hip.stream_of(x)))
             return (q.view(B, L, H, Dh).permute(0, 2, 1, 3), k.permute(0, 2, 1, 3),
                     v.view(B, L, Hkv, Dh).permute(0, 2, 1, 3), g, lam.permute(0, 2, 1), cos, sin)
-        cos, sin = self.rope(seq_len=L, offset=p0, device=x.device, dtype=x.dtype)
-        cos, sin = cos.contiguous(), sin.contiguous()
+        cos, sin = self._rope_tables(p0, L, x.device, x.dtype)
         q = self._project_q(x)
         k_raw, v = self._project_kv_raw(x)
         # roped keys in the token-major layout of v, so K and V share strides

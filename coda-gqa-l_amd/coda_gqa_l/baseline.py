@@ -89,8 +89,7 @@ class CoDAGQA(RowsMixin, nn.Module):
         k = self.k_proj(x).view(B, L, Hkv, Dh).permute(0, 2, 1, 3)
         v = self.v_proj(x).view(B, L, Hkv, Dh).permute(0, 2, 1, 3)
         offset = past_key_value[0].size(2) if past_key_value is not None else 0
-        cos, sin = self.rope(seq_len=L, offset=offset, device=x.device, dtype=q.dtype)
-        cos, sin = cos.contiguous(), sin.contiguous()
+        cos, sin = self._rope_tables(offset, L, x.device, q.dtype)
         k = apply_rope(k, cos, sin, interleaved=self.rope_interleaved)
         if past_key_value is not None:
             k = torch.cat([past_key_value[0], k], dim=2)

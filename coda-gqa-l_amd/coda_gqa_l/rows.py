@@ -10,6 +10,7 @@ import torch
 import torch.nn as nn
 
 from . import _hip
+from .primitives import RotaryEmbedding
 
 
 class _Made:
@@ -62,14 +63,34 @@ class RowsMixin:
         cached table, grown by doubling; every element is the same fp32
         product and cos / sin as in a table made for these positions alone."""
         cache = self.__dict__.setdefault("_rope_cache", {})
+        made = self.__dict__.setdefault("_rope_made", {})
         key = (torch.device(device), dtype)
         tab = cache.get(key)
         need = int(p0) + int(L)
-        if tab is None or tab[0].shape[0] < need:
+        inv = self.rope.inv_freq
+        hit = made.get(key)
+        if tab is None or tab[0].shape[0] < need or hit is None or hit[0] is not inv or \
+                hit[1] != (inv._version, inv.data_ptr()):
             n = 1 << max(12, (need - 1).bit_length())
             c, s_ = self.rope(seq_len=n, offset=0, device=device, dtype=dtype)
             tab = cache[key] = (c.contiguous(), s_.contiguous())
+            made[key] = (inv, (inv._version, inv.data_ptr()), _Made(*tab) if tab[0].is_cuda else None)
+        elif hit[2] is not None:
+            hit[2].use()
         return tab[0][p0:need], tab[1][p0:need]
+
+    def _rope_tables(self, p0: int, L: int, device, dtype: torch.dtype) -> Tuple[torch.Tensor, torch.Tensor]:
+        """RoPE tables (L, Dh/2) of a prompt: rows of the cached table (made
+        for the call alone they are seven small kernels, 20 us, and 45 us of
+        host time), but for positions past 65536 (tables of at most 32 MiB
+        are kept), under capture (a graph must not hold rows of a table that
+        a later call replaces) and where self.rope is not the plain module."""
+        r = self.rope
+        if p0 + L > 65536 or type(r) is not RotaryEmbedding or r._forward_hooks or r._forward_pre_hooks or \
+                nn.modules.module._has_any_global_hook() or torch.cuda.is_current_stream_capturing():
+            c, s_ = r(seq_len=L, offset=p0, device=device, dtype=dtype)
+            return c.contiguous(), s_.contiguous()
+        return self._rope_rows(p0, L, device, dtype)
 
     def _proj_pack(self, dtype: torch.dtype):
         """Packed [q | k | v | lambda | write] weights (n_feat, D) in `dtype`,
