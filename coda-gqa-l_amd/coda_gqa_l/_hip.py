@@ -109,6 +109,8 @@ _SIGS = {
                                 _i32, _i64, _vp, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp]),
     "coda_block_write_snapshot": (_i32, [ctypes.POINTER(BankDesc), _vp, _vp, _i64, _i64, _i64, _vp, _i64, _i32, _i32,
                                          _i32, _i64, _vp, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp, _vp, _vp, _vp]),
+    "coda_block_ring_snapshot": (_i32, [ctypes.POINTER(BankDesc), _vp, _vp, _i64, _i64, _i64, _vp, _i64, _i32, _i32, _vp,
+                                        _vp, _vp, _vp]),
     "coda_project_pack": (_i32, [_vp, _i32, _i32, _i64, _vp, _vp]),
     "coda_block_write_chain": (_i32, [ctypes.POINTER(BankDesc), _vp, _vp, _i64, _i64, _i64, _vp, _i64, _i32, _i32, _i32,
                                       _i32, _i32, _i32, _i64, _vp, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp, _vp, _vp,

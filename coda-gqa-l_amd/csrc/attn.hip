@@ -2907,8 +2907,8 @@ static size_t f3_split_bytes(const coda_attn_desc* d, int ns) {
 // whose 8-wave workgroups fill the CUs once (at least one a CU, fewer than
 // two): it keeps 8 waves and four stages, whose deeper prefetch serves a
 // grid that starts all at once (measured: a block-256 chunk at B = 4, 36 vs
-// 38 us; 4 waves win for grouped launches, small grids and configs[3]'s
-// 4096 workgroups)
+// 38 us; 4 waves win for grouped launches, small grids and, with two 8192-token
+// sequences of 32 heads, 4096 workgroups)
 template <int DH, int QM, bool TB>
 static int launch_f3_qm(const coda_attn_desc* d, hipStream_t st, int G, const ChunkGeom& cg) {
   if (cg.n == 0) {

@@ -1340,10 +1340,16 @@ __global__ __launch_bounds__(kApplyThreads) void block_apply_kernel(const coda_b
 // Ring write of the chunk's surviving block tokens (memory_banks.py:135-177)
 // for head h of sequence b, after the bank writes have read the evicted
 // ring rows; the lead head also writes the ring gates and visibility bytes.
-// Workgroup z takes the 16-byte pieces [z per, (z + 1) per) of the copy.
+// Workgroup z < nzr takes the 16-byte pieces [z per, (z + 1) per) of the
+// copy.  Workgroups z >= nzr (with a snapshot) copy head h's bank slots, and
+// the lead head's first one the visibility bytes: a chunk that evicts nothing
+// leaves the banks as they are, so ring write and snapshot are one launch
+// (as a launch and three copies they took 13 us and 35 us of host time: a
+// 1999-token prompt 467 -> 442 us).
 template <typename T, int DH>
 __global__ __launch_bounds__(kApplyThreads) void block_ring_kernel(const coda_bank_desc s, BlockGeom g, const T* kbk,
-                                                                   const T* vbk, const float* gb) {
+                                                                   const T* vbk, const float* gb, int nzr,
+                                                                   BankSnap snap) {
   constexpr int CH = DH / 8;
   const int h = blockIdx.x, b = blockIdx.y, t = threadIdx.x, NT = blockDim.x;
   const int W = s.W, Lbuf = W + s.Me + s.Ms;
@@ -1351,13 +1357,24 @@ __global__ __launch_bounds__(kApplyThreads) void block_ring_kernel(const coda_ba
   T* kb = (T*)s.k_buf + ((int64_t)b * s.Hkv + h) * Lbuf * DH;
   T* vb = (T*)s.v_buf + ((int64_t)b * s.Hkv + h) * Lbuf * DH;
   uint8_t* al = s.allowed + (int64_t)b * Lbuf;
+  if ((int)blockIdx.z >= nzr) {
+    const int M = s.Me + s.Ms, n = M * CH, step = ((int)gridDim.z - nzr) * NT;
+    const int64_t sb = ((int64_t)b * s.Hkv + h) * M * DH;
+    for (int i = ((int)blockIdx.z - nzr) * NT + t; i < n; i += step) {
+      st8<T>((T*)snap.k + sb + 8 * i, ld8<T>(kb + (int64_t)W * DH + 8 * i));
+      st8<T>((T*)snap.v + sb + 8 * i, ld8<T>(vb + (int64_t)W * DH + 8 * i));
+    }
+    if (lead && (int)blockIdx.z == nzr)
+      for (int i = t; i < M; i += NT) snap.allowed[(int64_t)b * M + i] = al[W + i];
+    return;
+  }
   auto blk_row = [&](const T* base, int jb) { return base + b * g.b_sb + h * g.b_sh + (int64_t)jb * g.b_sl; };
   const int Lr = g.ring_filled;
   const int first = max(Lr, g.n_ev);
   const int total = Lr + g.blk;
   const int rhead = (Lr == W) ? g.ring_head : 0;
   const int n_all = (total - first) * CH;  // pieces of 8 elements per plane (K and V each)
-  const int per = (n_all + (int)gridDim.z - 1) / (int)gridDim.z;
+  const int per = (n_all + nzr - 1) / nzr;
   const int p0 = min(n_all, (int)blockIdx.z * per), n_ring = min(n_all, p0 + per);
   auto ring_store = [&](int i, Piece8<T> xk, Piece8<T> xv) {
     const int r = first + i / CH, c = i % CH;
@@ -2706,6 +2723,20 @@ static int launch_fused(const coda_bank_desc* s, const void* kb, const void* vb,
   return check_launch("block_fused");
 }
 
+// The ring write, at most two 16-byte pieces per thread and plane in each
+// workgroup; with a snapshot, as many for the bank slots.
+template <typename T, int DH>
+static int launch_ring(const coda_bank_desc* s, const void* kb, const void* vb, const float* gb, const BlockGeom& g,
+                       hipStream_t st, BankSnap snap) {
+  const int first = std::max(g.ring_filled, g.n_ev);
+  const int n_all = (g.ring_filled + g.blk - first) * (DH / 8), n_bank = (s->Me + s->Ms) * (DH / 8);
+  const int nzr = std::max(1, (n_all + 2 * kApplyThreads - 1) / (2 * kApplyThreads));
+  const int nzs = snap.k ? (n_bank + 2 * kApplyThreads - 1) / (2 * kApplyThreads) : 0;
+  hipLaunchKernelGGL((block_ring_kernel<T, DH>), dim3(s->Hkv, s->B, nzr + nzs), dim3(kApplyThreads), 0, st, *s, g,
+                     (const T*)kb, (const T*)vb, gb, nzr, snap);
+  return check_launch("block_ring");
+}
+
 template <typename T, int DH>
 static int launch_block(const coda_bank_desc* s, const void* kb, const void* vb, const float* gb, BlockGeom g,
                         const int32_t* plan_c, float* ws, unsigned long long* tail, hipStream_t st,
@@ -2749,15 +2780,7 @@ static int launch_block(const coda_bank_desc* s, const void* kb, const void* vb,
     rc = check_launch("block_apply");
     if (rc) return rc;
   }
-  {
-    // at most two 16-byte pieces per thread and plane in each workgroup
-    const int first = std::max(g.ring_filled, g.n_ev);
-    const int n_all = (g.ring_filled + g.blk - first) * (DH / 8);
-    const int nzr = std::max(1, (n_all + 2 * kApplyThreads - 1) / (2 * kApplyThreads));
-    hipLaunchKernelGGL((block_ring_kernel<T, DH>), dim3(s->Hkv, s->B, nzr), dim3(kApplyThreads), 0, st, *s, g,
-                       (const T*)kb, (const T*)vb, gb);
-  }
-  return check_launch("block_ring");
+  return launch_ring<T, DH>(s, kb, vb, gb, g, st, BankSnap{nullptr, nullptr, nullptr});
 }
 
 extern "C" int coda_block_write_check(const coda_bank_desc* s, int Te, int Ts) {
@@ -2840,6 +2863,34 @@ extern "C" int coda_block_write_snapshot(const coda_bank_desc* s, const void* kb
                "coda_block_write_snapshot: snapshot rows must be 16-byte aligned");
   return block_write_impl(s, kb, vb, b_sb, b_sh, b_sl, gb, g_sb, blk, ring_head, ring_filled, pos0, plan_c, Kmax, Te,
                           Ts, workspace, workspace_bytes, stream, BankSnap{snap_k, snap_v, snap_allowed});
+}
+
+extern "C" int coda_block_ring_snapshot(const coda_bank_desc* s, const void* kb, const void* vb, int64_t b_sb,
+                                        int64_t b_sh, int64_t b_sl, const float* gb, int64_t g_sb, int blk,
+                                        int ring_filled, void* snap_k, void* snap_v, uint8_t* snap_allowed,
+                                        void* stream) {
+  const int rc = validate_bank(s, "coda_block_ring_snapshot");
+  if (rc) return rc;
+  CODA_REQUIRE(kb && vb && gb, "coda_block_ring_snapshot: block pointers missing");
+  CODA_REQUIRE(blk > 0 && ring_filled >= 0 && blk <= s->W && ring_filled <= s->W - blk,
+               "coda_block_ring_snapshot: %d tokens on top of %d evict from a ring of %d", blk, ring_filled, s->W);
+  CODA_REQUIRE(snap_k && snap_v && snap_allowed, "coda_block_ring_snapshot: snapshot pointers missing");
+  CODA_REQUIRE(((uintptr_t)snap_k % 16) == 0 && ((uintptr_t)snap_v % 16) == 0,
+               "coda_block_ring_snapshot: snapshot rows must be 16-byte aligned");
+  if (s->B == 0) return CODA_OK;
+  const BlockGeom g{blk, 0, ring_filled, 0, 0, 0, 0, 0, b_sb, b_sh, b_sl, g_sb};
+  const BankSnap snap{snap_k, snap_v, snap_allowed};
+  hipStream_t st = (hipStream_t)stream;
+  const bool bf = s->dtype == CODA_BF16;
+#define CODA_RING(D)                                                         \
+  return bf ? launch_ring<bf16_t, D>(s, kb, vb, gb, g, st, snap) \
+            : launch_ring<float, D>(s, kb, vb, gb, g, st, snap)
+  switch (s->Dh) {
+    case 32: CODA_RING(32);
+    case 64: CODA_RING(64);
+    default: CODA_RING(128);
+  }
+#undef CODA_RING
 }
 
 extern "C" int coda_block_write_chain(const coda_bank_desc* s, const void* kb, const void* vb, int64_t b_sb,

@@ -492,6 +492,16 @@ int coda_block_write_snapshot(const coda_bank_desc* s, const void* kb, const voi
                               void* workspace, size_t workspace_bytes, void* snap_k, void* snap_v,
                               uint8_t* snap_allowed, void* stream);
 
+/* coda_block_write with the snapshot of coda_block_write_snapshot, for a
+ * chunk that evicts nothing (ring_filled + blk <= W, else CODA_EINVAL): the
+ * ring write and the bank slots' copy in one launch.
+ * Replaces: the ring write of a prompt's first chunks
+ *   (src/coda_gqa_l/memory_banks.py:135-177). */
+int coda_block_ring_snapshot(const coda_bank_desc* s, const void* kb, const void* vb,
+                             int64_t b_sb, int64_t b_sh, int64_t b_sl, const float* gb, int64_t g_sb,
+                             int blk, int ring_filled, void* snap_k, void* snap_v, uint8_t* snap_allowed,
+                             void* stream);
+
 /* coda_block_write_snapshot for chunks c_first .. c_first + n_chunks - 1 of
  * a prefill call in one library call (the chunk loop on the host side of the
  * library): chunk c covers tokens [c blk, min(L, (c + 1) blk)) of kb / vb /

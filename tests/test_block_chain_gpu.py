@@ -82,3 +82,44 @@ def test_chain_is_the_chunks(monkeypatch, B, H, Hkv, W, Me, Ms, blk, L, warm, dt
         assert torch.equal(a, c), f"state {i}: chain and the four-kernel update differ"
     for i, (a, b) in enumerate(zip(snaps, snaps1)):
         assert torch.equal(a, b), f"snapshot {i} differs"
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("B,Hkv,W,Me,Ms,filled,blk,dtype", [
+    (1, 1, 16, 8, 8, 0, 1, torch.bfloat16), (2, 3, 300, 33, 45, 17, 283, torch.bfloat16),
+    (1, 2, 256, 0, 130, 100, 37, torch.float32), (3, 2, 64, 150, 0, 0, 64, torch.float32)])
+def test_ring_write_with_snapshot(B, Hkv, W, Me, Ms, filled, blk, dtype):
+    """coda_block_ring_snapshot: the ring of coda_block_write, the banks
+    copied and untouched; a chunk that evicts is refused."""
+    import coda_gqa_l
+    from coda_gqa_l import _hip
+    Dh, S = 64, Me + Ms
+    m = coda_gqa_l.CoDAGQALandmarkPerf2(embed_dim=Hkv * Dh, num_heads=Hkv, num_kv_heads=Hkv, window=W,
+                                        num_landmarks_exact=Me, num_landmarks_summary=Ms).to(DEV, dtype).eval()
+    g = torch.Generator(device=DEV).manual_seed(3)
+    states = []
+    for _ in range(2):
+        st = m.init_state(batch_size=B, device=DEV, dtype=dtype)
+        g.manual_seed(3)
+        st.k_buf.copy_(torch.randn(st.k_buf.shape, generator=g, device=DEV))
+        st.v_buf.copy_(torch.randn(st.k_buf.shape, generator=g, device=DEV))
+        st.allowed[:, W:] = torch.rand(B, S, generator=g, device=DEV) < 0.5
+        states.append(st)
+    k, v = (torch.randn(B, blk, Hkv, Dh, generator=g, device=DEV).to(dtype).permute(0, 2, 1, 3) for _ in range(2))
+    gates = torch.rand(B, blk, generator=g, device=DEV)
+    eta = m._eta_f32(torch.device(DEV), dtype) if Ms else None
+    kw = dict(k_blk=k, v_blk=v, g_blk=gates, pos0=filled, ring_head=0, ring_filled=filled, plan_c=None, kmax=1,
+              do_e=False, do_s=False, workspace=None, eta=eta)
+    snap = (torch.zeros(B, Hkv, S, Dh, dtype=dtype, device=DEV), torch.zeros(B, Hkv, S, Dh, dtype=dtype, device=DEV),
+            torch.full((B, S), 7, dtype=torch.uint8, device=DEV))
+    want = [states[0].k_buf[:, :, W:].clone(), states[0].v_buf[:, :, W:].clone(), states[0].allowed[:, W:].to(torch.uint8)]
+    assert m._write_block(states[0], snap=snap, **kw) == m._write_block(states[1], **kw)
+    for a, b in zip(snap, want):
+        assert torch.equal(a, b)
+    for f in ("k_buf", "v_buf", "allowed", "g_recent"):
+        assert torch.equal(getattr(states[0], f), getattr(states[1], f)), f
+    rc = _hip.lib().coda_block_ring_snapshot(
+        m._bank_desc(states[0], eta, None, None), k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1), k.stride(2),
+        gates.data_ptr(), gates.stride(0), blk, W - blk + 1, snap[0].data_ptr(), snap[1].data_ptr(), snap[2].data_ptr(),
+        _hip.stream_of(k))
+    assert rc not in (_hip.CODA_OK, _hip.CODA_EUNSUP)
