@@ -2652,23 +2652,8 @@ static bool fused_enabled() {
 
 // Launch shapes and dynamic LDS of a chunk's bank update with Te / Ts
 // candidates over `pairs` (sequence, head) pairs, shared by the launcher and
-// coda_block_write_check.  The one-launch kernel: each head over NZ
-// workgroups, about 256 in all (more where one workgroup's LDS would not
-// fit), at most 8 per head and 64 per sequence; nz = 0 when it cannot run.
-struct FusedShape {
-  int nz;
-  size_t lds;
-};
-static FusedShape fused_shape(const coda_bank_desc* s, int esz, int Te, int Ts, int pairs) {
-  FusedShape f{0, 0};
-  if (!(Te <= 64 && Ts <= 64 && Te + Ts > 0 && s->Hkv <= kFusedMaxGroup)) return f;
-  const int nz_max = std::max(1, std::min({kFusedMaxGroup / s->Hkv, 8, Te + Ts}));
-  int NZ = std::max(1, std::min((256 + pairs - 1) / pairs, nz_max));
-  size_t lds = fused_lds(s->Dh, esz, s->Me, s->Ms, Te, Ts, NZ).total;
-  while (lds + 1024 > kLdsMax && NZ < nz_max) lds = fused_lds(s->Dh, esz, s->Me, s->Ms, Te, Ts, ++NZ).total;
-  if (lds + 1024 <= kLdsMax) f = FusedShape{NZ, lds};  // the kernel's own static LDS is under 1 KiB
-  return f;
-}
+// coda_block_write_check.
+//
 // The four-kernel path: candidate rows split over nz_r route workgroups per
 // (sequence, head) (about 512 in all, at least 8 rows each); bank slots over
 // nz_a apply workgroups (about 512 in all), PS summary slots each.
@@ -2702,6 +2687,48 @@ static SplitShape split_shape(const coda_bank_desc* s, int Te, int Ts, int pairs
     p.lds_apply = apply_lds_bytes(s->Ms, Te, Ts, p.PS, LF);
   }
   return p;
+}
+
+// The bank sizes that a chunk update takes, by either path: the four-kernel
+// path fits, or all norm rows of one head in the element type fit a
+// workgroup beside the candidates, its share of the slots and the lists of a
+// decision.  The one-launch kernel keeps a share of the norm rows alone and
+// would fit larger banks; they stay refused, since the decode step and the
+// four-kernel path (CODA_BLOCK_FUSED=0) go on from the same state.
+static bool bank_sizes_fit(const coda_bank_desc* s, int esz, int Te, int Ts, int pairs) {
+  const size_t room = kLdsMax - 1024;
+  const SplitShape p = split_shape(s, Te, Ts, pairs);
+  if (p.lds_route <= room && p.lds_decide <= room && p.lds_apply <= room) return true;
+  if (!(Te <= 64 && Ts <= 64 && Te + Ts > 0 && s->Hkv <= kFusedMaxGroup)) return false;
+  const int NZ = std::max(1, std::min({kFusedMaxGroup / s->Hkv, 8, Te + Ts}));
+  const int DH = s->Dh, LF = DH / 2, Me = s->Me, Ms = s->Ms, TT = std::max(Te, Ts);
+  auto share = [&](int n) { return (n + NZ - 1) / NZ; };
+  size_t lds = 0;
+  for (int bytes : {TT * DH * esz, TT * DH * esz, share(Me) * DH * esz, share(Me) * DH * esz, share(Ms) * DH * esz,
+                    share(Ms) * DH * esz, 4 * TT, 4 * (Me + Ms), 8 * Me, 16 * Me, 4 * Me, 4 * TT, 4 * Te, 4 * Te,
+                    4 * Te, 4 * Te, 4 * Ts, 4 * Ts, 4 * Me, 8 * Ms, 4 * Ms, 4 * Ms, 4 * share(Ms) * LF,
+                    Me * (DH + 4) * esz, 4 * share(Te) * (DH + 4), Ms * (LF + 4) * esz, 4 * share(Ts) * (LF + 4)})
+    lds += al16(bytes);
+  return lds <= room;
+}
+
+// The one-launch kernel: each head over NZ
+// workgroups, about 256 in all (more where one workgroup's LDS would not
+// fit), at most 8 per head and 64 per sequence; nz = 0 when it cannot run.
+struct FusedShape {
+  int nz;
+  size_t lds;
+};
+static FusedShape fused_shape(const coda_bank_desc* s, int esz, int Te, int Ts, int pairs) {
+  FusedShape f{0, 0};
+  if (!(Te <= 64 && Ts <= 64 && Te + Ts > 0 && s->Hkv <= kFusedMaxGroup)) return f;
+  if (!bank_sizes_fit(s, esz, Te, Ts, pairs)) return f;
+  const int nz_max = std::max(1, std::min({kFusedMaxGroup / s->Hkv, 8, Te + Ts}));
+  int NZ = std::max(1, std::min((256 + pairs - 1) / pairs, nz_max));
+  size_t lds = fused_lds(s->Dh, esz, s->Me, s->Ms, Te, Ts, NZ).total;
+  while (lds + 1024 > kLdsMax && NZ < nz_max) lds = fused_lds(s->Dh, esz, s->Me, s->Ms, Te, Ts, ++NZ).total;
+  if (lds + 1024 <= kLdsMax) f = FusedShape{NZ, lds};  // the kernel's own static LDS is under 1 KiB
+  return f;
 }
 
 // Spin limit of the fused kernel's bounded waits (coda_block_sync_spin_limit)
