@@ -303,7 +303,8 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
             if not self._fused_front_ok(x):
                 raise NotImplementedError(
                     "the fused projection front end serves few token rows (decode: bf16 128, fp32 32); many rows "
-                    "take the torch linears: a many-row fused form (an in-place epilogue over a library GEMM, q / k / v / lambda as strided views of its output) faulted the GPU in a full-size run with no "
+                    "take the torch linears: a many-row fused form (an in-place epilogue over a library GEMM, "
+                    "q / k / v / lambda as strided views of its output) faulted the GPU in a full-size run with no "
                     "cause shown, and was removed")
             cos, sin = self._rope_rows(p0, L, x.device, x.dtype)
             d = self._proj_desc(x, M, L, cos, sin)

@@ -125,14 +125,14 @@ class RowsMixin:
             if gate:
                 ws.append(self.write_proj.weight)
                 bt.append(self.write_proj.bias)
-            w = torch.cat([t.detach() for t in ws]).to(dtype)
             b = torch.cat([t.detach().float() if t is not None else torch.zeros(wt.shape[0], device=dev)
                            for t, wt in zip(bt, ws)])
             b = torch.cat([b, torch.zeros((-b.numel()) % 4, device=dev)])
-            w = w.contiguous()
-            layout = 0
-            if w.is_cuda:
-                w, layout = self._rows_tiles(w), 1
+            ws = [t.detach().to(dtype) for t in ws]
+            if ws[0].is_cuda:
+                w, layout = self._rows_tiles(*ws), 1
+            else:
+                w, layout = torch.cat(ws).contiguous(), 0
         val = (w, b.contiguous(), layout)
         cache[("proj", dtype)] = (tag, val)
         if w.is_cuda:
@@ -140,13 +140,33 @@ class RowsMixin:
         return val
 
     @staticmethod
-    def _rows_tiles(w: torch.Tensor) -> torch.Tensor:
-        """(n, D) weights in the row kernel's fragment tiles (coda_rows_pack)."""
-        n, D = w.shape
-        wt = torch.empty((-(-n // 64) * 64, D), dtype=w.dtype, device=w.device)
-        _hip.check(_hip.lib().coda_rows_pack(_hip.dtype_code(w.dtype), w.data_ptr(), n, D, w.stride(0), wt.data_ptr(),
-                                             _hip.stream_of(wt)))
-        return wt
+    def _rows_tiles(*parts: torch.Tensor) -> torch.Tensor:
+        """(n, D) weights, the parts one after the other, in the row kernel's
+        fragment tiles (coda_rows_pack), n rounded up to a multiple of 64.  A
+        part that starts on a row block of 16 is packed from where it is (a
+        layer's first token paid a concatenation of all its weights
+        otherwise: 340 MB of traffic and a second buffer at 10305 x 8192);
+        rows that the loads of the kernel can't take are copied first."""
+        groups, n = [], 0
+        for t in parts:
+            if n % 16:
+                groups[-1].append(t)
+            else:
+                groups.append([t])
+            n += t.shape[0]
+        D, rows = parts[0].shape[1], -(-n // 64) * 64
+        # (each launch pads its rows to 64 and the next one writes over the
+        # padding; the last one's may end past `rows`)
+        wt = torch.empty((rows + 64, D), dtype=parts[0].dtype, device=parts[0].device)
+        wt[n // 64 * 64:].zero_()
+        at, fn, dt, stream = 0, _hip.lib().coda_rows_pack, _hip.dtype_code(wt.dtype), _hip.stream_of(wt)
+        for g in groups:
+            w = g[0].contiguous() if len(g) == 1 else torch.cat(g)
+            if w.data_ptr() % 16:
+                w = w.clone()
+            _hip.check(fn(dt, w.data_ptr(), w.shape[0], D, D, wt[at:].data_ptr(), stream))
+            at += w.shape[0]
+        return wt[:rows]
 
     @staticmethod
     def _plain_call(x: torch.Tensor, *lins: nn.Module) -> bool:
@@ -178,7 +198,7 @@ class RowsMixin:
         hit = self.__dict__.get("_o_rows")
         if hit is None or hit[0] != tag:
             with torch.no_grad():
-                tiles = self._rows_tiles(w.detach().contiguous())
+                tiles = self._rows_tiles(w.detach())
                 b = None if bias is None else bias.detach().float().contiguous()
             hit = self.__dict__["_o_rows"] = (tag, tiles, b, _Made(*(t for t in (tiles, b) if t is not None)))
         hit[3].use()

@@ -70,3 +70,24 @@ def test_step_equals_the_linears_route(B, D, H, Hkv, dtype):
         assert float((a.double() - b.double()).abs().max()) <= tol * float(b.double().abs().max())
     assert torch.equal(st.k_buf[:, :, 32:], st2.k_buf[:, :, 32:]) and torch.equal(st.allowed, st2.allowed)
     assert torch.equal(st.mem_last_exact, st2.mem_last_exact)
+
+
+@torch.no_grad()
+def test_weights_off_16_byte_addresses():
+    """Parameters that are views into a flat buffer, 2 bytes off: the step is
+    that of the same weights in storage of their own, bit for bit."""
+    torch.manual_seed(3)
+    m = coda_gqa_l.CoDAGQALandmarkPerf2(embed_dim=320, num_heads=5, num_kv_heads=5, window=32, num_landmarks_exact=16,
+                                        num_landmarks_summary=16).to(DEV, torch.bfloat16).eval()
+    st = m.init_state(batch_size=2, device=DEV, dtype=torch.bfloat16)
+    x = torch.randn(2, 1, 320, generator=torch.Generator(device=DEV).manual_seed(1), device=DEV).bfloat16()
+    st2 = state_io.deep_copy_state(st)
+    ya, _ = m.step(x, st)
+    for lin in (m.q_proj, m.k_proj, m.v_proj, m.lambda_proj, m.write_proj, m.o_proj):
+        w = lin.weight
+        flat = torch.empty(w.numel() + 1, dtype=w.dtype, device=DEV)
+        flat[1:].copy_(w.reshape(-1))
+        lin.weight = torch.nn.Parameter(flat[1:].view(w.shape))
+        assert lin.weight.data_ptr() % 16
+    yb, _ = m.step(x, st2)
+    assert torch.equal(ya, yb) and torch.equal(st.k_buf, st2.k_buf) and torch.equal(st.v_buf, st2.v_buf)
