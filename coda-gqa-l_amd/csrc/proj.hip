@@ -14,7 +14,6 @@
 #include "common.h"
 
 #include <climits>
-#include <type_traits>
 
 namespace coda {
 
@@ -119,24 +118,6 @@ struct LinearEpilogue {
       for (int e = 0; e < 4; ++e)
         if (f + e < n_feat) row[f + e] = Elt<T>::st(v[e]);
     }
-  }
-  __device__ __forceinline__ void once(int) const {}
-};
-
-// Epilogue of the lambda projection of many rows: sigmoid of the rounded
-// linear, rounded; `rows` token rows a blockIdx.y.
-template <typename T>
-struct SigmoidEpilogue {
-  T* out;
-  const float* bias;  // or null
-  int64_t o_sm;
-  int n_feat, rows;
-  __device__ __forceinline__ void operator()(int f, int m, pf32x4 v) const {
-    using E = Elt<T>;
-    T* row = out + ((int64_t)blockIdx.y * rows + m) * o_sm;
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (f + e < n_feat) row[f + e] = E::st(proj_sigmoid(E::rnd(v[e] + (bias ? bias[f + e] : 0.f))));
   }
   __device__ __forceinline__ void once(int) const {}
 };
@@ -299,13 +280,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const char* p, int n
 // writes and reads spread over the banks.  The slab is the wave's alone and
 // LDS serves a wave in order: no barrier.  The next chunk's weights load
 // while this chunk's products run.  Same sums in the same order as proj_rows.
-// blockIdx.y takes the next 16 MT token rows (coda_sigmoid_rows).
 template <typename T, int MT, int RB, int CS, typename Epi>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void proj_rows_lds(
     const T* __restrict__ W, int n_feat, int D, const T* __restrict__ X, int64_t x_sm, int M, const Epi epi) {
   extern __shared__ __attribute__((aligned(16))) char rows_smem[];
-  X += (int64_t)blockIdx.y * 16 * MT * x_sm;
-  M = min(M - (int)blockIdx.y * 16 * MT, 16 * MT);
   constexpr int RBY = CS * 64, PCS = RBY / 16, NI = 16 * PCS / 64, RPI = 64 / PCS;  // row bytes, pieces; loads a slab, rows a load
   const int f0 = blockIdx.x * 16 * RB;
   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), r16 = lane & 15, kq = lane >> 4;
@@ -413,8 +391,8 @@ static int launch_rows_lds(const T* W, int n_feat, int D, const T* X, int64_t x_
   constexpr size_t lds = slabs > RowsLds<MT, RB>::kBytes ? slabs : RowsLds<MT, RB>::kBytes;
   const int rc = lds_limit<proj_rows_lds<T, MT, RB, CS, Epi>>(lds, who);
   if (rc) return rc;
-  hipLaunchKernelGGL((proj_rows_lds<T, MT, RB, CS, Epi>),
-                     dim3((n_feat + 16 * RB - 1) / (16 * RB), (M + 16 * MT - 1) / (16 * MT)), dim3(512), lds, st, W, n_feat, D, X, x_sm, M, epi);
+  hipLaunchKernelGGL((proj_rows_lds<T, MT, RB, CS, Epi>), dim3((n_feat + 16 * RB - 1) / (16 * RB)), dim3(512), lds, st,
+                     W, n_feat, D, X, x_sm, M, epi);
   return check_launch("proj_rows_lds");
 }
 template <typename T, int MT, bool TILED, typename Epi>
@@ -550,31 +528,6 @@ extern "C" int coda_linear_rows(int dtype, const void* x, int64_t x_sm, int M, c
                                        "coda_linear_rows");
   return launch_rows_t<float, true>((const float*)w, D, n_feat, D, (const float*)x, x_sm, M,
                                     LinearEpilogue<float>{(float*)out, bias, o_sm, n_feat}, st, "coda_linear_rows");
-}
-
-// Token rows a workgroup: 32 while they leave CUs free or just fill them, 64
-// (half the weight reads) from there on.
-extern "C" int coda_sigmoid_rows(int dtype, const void* x, int64_t x_sm, int M, const void* w, int n_feat, int D,
-                                 const float* bias, void* out, int64_t o_sm, void* stream) {
-  CODA_REQUIRE(dtype == CODA_BF16, "coda_sigmoid_rows: bf16 only");
-  CODA_REQUIRE(M >= 0 && M <= (1 << 20) && n_feat > 0 && n_feat <= 128 && D > 0 && D <= (1 << 16) && D % 2048 == 0,
-               "coda_sigmoid_rows: bad sizes M=%d n_feat=%d D=%d (at most 2^20 rows, 128 features, D a multiple of 2048)",
-               M, n_feat, D);
-  CODA_REQUIRE(x && w && out, "coda_sigmoid_rows: null pointer");
-  CODA_REQUIRE(x_sm >= D && x_sm <= (1 << 20) && x_sm % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0,
-               "coda_sigmoid_rows: x / w rows must be 16-byte aligned");
-  if (M == 0) return CODA_OK;
-  hipStream_t st = (hipStream_t)stream;
-  auto run = [&](auto mt) {
-    constexpr int MT = decltype(mt)::value;
-    const SigmoidEpilogue<bf16_t> epi{(bf16_t*)out, bias, o_sm, n_feat, 16 * MT};
-    return n_feat <= 16 ? launch_rows_lds<bf16_t, MT, 1>((const bf16_t*)w, n_feat, D, (const bf16_t*)x, x_sm, M, epi, st,
-                                                         "coda_sigmoid_rows")
-                        : launch_rows_lds<bf16_t, MT, 2>((const bf16_t*)w, n_feat, D, (const bf16_t*)x, x_sm, M, epi, st,
-                                                         "coda_sigmoid_rows");
-  };
-  if (M <= 32 * device_cus()) return run(std::integral_constant<int, 2>{});
-  return run(std::integral_constant<int, 4>{});
 }
 
 extern "C" int coda_rows_pack(int dtype, const void* w, int n_feat, int D, int64_t w_sm, void* out, void* stream) {

@@ -126,14 +126,6 @@ int coda_project_rows(const coda_proj_desc* d, void* stream);
 int coda_linear_rows(int dtype, const void* x, int64_t x_sm, int M, const void* w, int n_feat, int D,
                      const float* bias, void* out, int64_t o_sm, void* stream);
 
-/* out (M, n_feat; row stride o_sm) = sigmoid(x W^T + bias), bf16, for the
- * many rows of a prompt (M <= 2^20) and few features (n_feat <= 128): x is
- * read once.  fp32 sums, the linear and its sigmoid rounded to bf16 each.  D a
- * multiple of 2048, the rest as coda_linear_rows.
- * Replaces: lambda_proj of a prefill (attention.py:404-407). */
-int coda_sigmoid_rows(int dtype, const void* x, int64_t x_sm, int M, const void* w, int n_feat, int D,
-                      const float* bias, void* out, int64_t o_sm, void* stream);
-
 /* The weights of coda_project in fragment tiles (w_layout 1): for row block
  * fb of 16 rows and k-step ks of 32 columns, a 1 KiB tile at element offset
  * (fb * D/32 + ks) * 512 holding W[16 fb + r][32 ks + 8 q + e] at element
