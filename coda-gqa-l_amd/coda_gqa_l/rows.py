@@ -187,14 +187,20 @@ class RowsMixin:
         """o_proj of decode-shaped heads (B, L, H*Dh): at most 32 token rows
         through the row kernel (bf16 4096 x 4096: 8.1 us at 1 row and 11.1 at
         32 against 12.0 and 12.4 for the library's GEMM, which is ahead at 64
-        with 12.8 against 14.5; and a shorter way through the host)."""
+        with 12.8 against 14.5).  Smaller bf16 layers take it up to 64 rows
+        (2048 x 2048) and 128 (1024 x 1024): the step waits for the host there
+        and this way is the shorter one (a token of 40 rows, 1024 x 1024: 32.6
+        us against 44.4 through the library)."""
         B, L, K = heads.shape
         o = self.o_proj
-        if B * L > 32 or K % 64 or heads.dtype not in (torch.bfloat16, torch.float32) or \
+        most = 32
+        if heads.dtype == torch.bfloat16 and type(o) is nn.Linear and o.weight.numel() <= 1 << 22:
+            most = 128 if o.weight.numel() <= 1 << 20 else 64
+        if B * L > most or K % 64 or heads.dtype not in (torch.bfloat16, torch.float32) or \
                 not self._plain_call(heads, o) or not heads.is_contiguous():
             return o(heads)
         w, bias = o.weight, o.bias
-        tag = (w._version, w.data_ptr(), w.device) + (() if bias is None else (bias._version, bias.data_ptr()))
+        tag = (w._version, w.data_ptr(), w.dtype, w.device) + (() if bias is None else (bias._version, bias.data_ptr()))
         hit = self.__dict__.get("_o_rows")
         if hit is None or hit[0] != tag:
             with torch.no_grad():
