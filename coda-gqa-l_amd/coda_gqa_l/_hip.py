@@ -79,6 +79,16 @@ class ProjDesc(ctypes.Structure):
     ]
 
 
+class ProjParams(ctypes.Structure):
+    """coda_proj_params (include/coda_mi355x.h)."""
+
+    _fields_ = [
+        ("w", _vp * 5), ("w_sm", _i64 * 5), ("b", _vp * 5), ("inv_freq", _vp), ("inv_dtype", _i32), ("p0", _i64),
+        ("rope_cos", _vp), ("rope_sin", _vp), ("theta", _vp), ("theta_dtype", _i32), ("theta_cos", _vp),
+        ("theta_sin", _vp),
+    ]
+
+
 _lock = threading.Lock()
 _lib: Optional[ctypes.CDLL] = None
 
@@ -127,6 +137,9 @@ _SIGS = {
     "coda_unit_rows": (_i32, [_i32, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _i32, _i32, _vp]),
     "coda_project": (_i32, [ctypes.POINTER(ProjDesc), _vp]),
     "coda_project_rows": (_i32, [ctypes.POINTER(ProjDesc), _vp]),
+    "coda_project_params": (_i32, [ctypes.POINTER(ProjDesc), ctypes.POINTER(ProjParams), _vp]),
+    "coda_linear_params": (_i32, [_i32, _vp, _i64, _i32, _vp, _i64, _i32, _i32, _vp, _vp, _i64, _vp]),
+    "coda_rope_tables": (_i32, [_i32, _vp, _i32, _i64, _i32, _i32, _vp, _vp, _vp]),
     "coda_linear_rows": (_i32, [_i32, _vp, _i64, _i32, _vp, _i32, _i32, _vp, _vp, _i64, _vp]),
     "coda_rows_pack": (_i32, [_i32, _vp, _i32, _i32, _i64, _vp, _vp]),
     "coda_project_workspace_bytes": (_i32, [ctypes.POINTER(ProjDesc), ctypes.POINTER(ctypes.c_size_t)]),

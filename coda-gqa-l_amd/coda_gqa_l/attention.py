@@ -289,7 +289,8 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         lam (B,H,L), and the RoPE tables (L, Dh/2) (attention.py:396-410,
         592-608).  fused (decode-shaped input, _fused_front_ok): one launch of
         the hand-written projection kernel with its RoPE and sigmoid
-        epilogues (coda_project), outputs in the torch path's layouts.
+        epilogues (on packed weights: coda_project_rows; on the parameters:
+        coda_project_params), outputs in the torch path's layouts.
         Otherwise the torch linears and the RoPE kernel.  A fused form for
         many token rows (a library GEMM over the packed weights, an epilogue
         kernel in place, q / k / v / lambda as strided views of its output)
@@ -306,33 +307,25 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
                     "take the torch linears: a many-row fused form (an in-place epilogue over a library GEMM, "
                     "q / k / v / lambda as strided views of its output) faulted the GPU in a full-size run with no "
                     "cause shown, and was removed")
-            cos, sin = self._rope_rows(p0, L, x.device, x.dtype)
+            rows = None if self._packed_front_ok(x) else self._front_rows(x)
+            cos, sin = (self._rope_rows if rows is None else self._rope_tables)(p0, L, x.device, x.dtype)
             d = self._proj_desc(x, M, L, cos, sin)
             g = torch.empty((B, L), dtype=torch.float32, device=x.device)
             d.g = g.data_ptr()
             xs = x if (x.is_contiguous() and x.data_ptr() % 16 == 0) else x.contiguous()
-            w, b, d.w_layout = self._proj_pack(x.dtype)
             q = torch.empty((B, L, Fq), dtype=x.dtype, device=x.device)
             k = torch.empty((B, L, Hkv, Dh), dtype=x.dtype, device=x.device)
             v = torch.empty((B, L, Fk), dtype=x.dtype, device=x.device)
             lam = torch.empty((B, L, H), dtype=x.dtype, device=x.device)
-            d.x, d.x_sm, d.w, d.bias = xs.data_ptr(), D, w.data_ptr(), b.data_ptr()
+            d.x, d.x_sm = xs.data_ptr(), D
             d.q, d.q_sm, d.k, d.k_sm, d.v, d.v_sm = q.data_ptr(), Fq, k.data_ptr(), Fk, v.data_ptr(), Fk
             d.lam, d.lam_sm = lam.data_ptr(), H
-            nb = self.__dict__.setdefault("_proj_ws_bytes", {})
-            key = (M, D, H, Hkv, Dh, d.gate)
-            if key not in nb:
-                n = ctypes.c_size_t(0)
-                _hip.check(_hip.lib().coda_project_workspace_bytes(d, n))
-                nb[key] = n.value
-            ws = None
-            if nb[key]:
-                cache = self.__dict__.setdefault("_proj_ws", {})
-                ws = cache.get(str(x.device))
-                if ws is None or ws.numel() < nb[key]:
-                    ws = cache[str(x.device)] = torch.empty(nb[key], dtype=torch.uint8, device=x.device)
-            d.workspace, d.workspace_bytes = _hip.ptr(ws), nb[key]
-            _hip.check(_hip.lib().coda_project_rows(d, _hip.stream_of(x)))
+            if rows is None:
+                w, b, d.w_layout = self._proj_pack(x.dtype)
+                d.w, d.bias = w.data_ptr(), b.data_ptr()
+                _hip.check(_hip.lib().coda_project_rows(d, _hip.stream_of(x)))
+            else:
+                _hip.check(_hip.lib().coda_project_params(d, self._proj_params(rows), _hip.stream_of(x)))
             return (q.view(B, L, H, Dh).permute(0, 2, 1, 3), k.permute(0, 2, 1, 3),
                     v.view(B, L, Hkv, Dh).permute(0, 2, 1, 3), g, lam.permute(0, 2, 1), cos, sin)
         cos, sin = self._rope_tables(p0, L, x.device, x.dtype)
@@ -445,38 +438,57 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         """A steady-state decode step (full ring, fixed bank sizes, no
         metrics or traces, decode-shaped input) from descriptors and
         buffers cached per state: per token the host sets the input and
-        RoPE-row pointers, makes two library calls (coda_project_rows,
-        then coda_decode_step on its outputs) and o_proj.  Returns None
-        when the general path must run; the cache is rebuilt whenever a
-        parameter, the state's tensors (object, storage or in-place version)
-        or the batch changes."""
-        if not self._fused_front_ok(x) or st.metrics is not None or st.recent_filled < self.window or \
+        RoPE-row pointers (packed weights) or the parameters' own addresses
+        and the position (few-row inputs that those don't serve), makes two
+        library calls (the projections, then coda_decode_step on their
+        outputs) and o_proj.  Returns None when the general path must run;
+        the cache is rebuilt whenever a parameter, the state's tensors
+        (object, storage or in-place version) or the batch changes."""
+        if st.metrics is not None or st.recent_filled < self.window or \
                 self._expandable() or (self.Me == 0 and self.Ms == 0) or self._tracing():
             return None
+        packed, rows, angles = self._packed_front_ok(x), None, None
+        if not packed:
+            rows = self._front_rows(x)
+            angles = None if rows is None else self._angles_rows(x.device, int(st.pos), 1)
+            if angles is None:
+                return None
         fp = self.__dict__.get("_fast")
         ts = (st.k_buf, st.v_buf, st.allowed, st.g_recent, st.mem_last_exact, st._exact_v_norm, st._sum_lf_k_norm)
         vers = tuple(-1 if t is None else t._version for t in ts)
         pvers = self._param_key()
         B = x.shape[0]
         if fp is None or fp["st"] is not st or fp["vers"] != vers or fp["pvers"] != pvers or fp["B"] != B or \
+                fp["packed"] != packed or \
                 fp["ptrs"] != tuple(-1 if t is None else t.data_ptr() for t in ts) or fp["dev"] != x.device:
-            fp = self._build_step_fast(x, st, ts, vers, pvers)
+            fp = self._build_step_fast(x, st, ts, vers, pvers, packed)
             if fp is None:
                 return None
         if not (x.is_contiguous() and x.data_ptr() % 16 == 0):
             x = x.contiguous()
         pos = int(st.pos)
-        cos_t, sin_t = fp["tab"]
-        if pos >= cos_t.shape[0]:
-            cos_t, sin_t = self._rope_rows(0, pos + 1, x.device, x.dtype)
-            fp["tab"] = (cos_t, sin_t)
-        row = fp["row_bytes"] * pos
         d, a = fp["proj"], fp["attn"]
         d.x = x.data_ptr()
-        d.rope_cos = a.rope_cos = cos_t.data_ptr() + row
-        d.rope_sin = a.rope_sin = sin_t.data_ptr() + row
         stream = _hip.stream_of(x)
-        _hip.check(fp["project"](fp["proj_ref"], stream))
+        cos_t, sin_t = fp["tab"]
+        if packed:
+            if pos >= cos_t.shape[0]:
+                cos_t, sin_t = self._rope_rows(0, pos + 1, x.device, x.dtype)
+                fp["tab"] = (cos_t, sin_t)
+            row = fp["row_bytes"] * pos
+            d.rope_cos = a.rope_cos = cos_t.data_ptr() + row
+            d.rope_sin = a.rope_sin = sin_t.data_ptr() + row
+            _hip.check(fp["project"](fp["proj_ref"], stream))
+        else:
+            # (the launch writes the token's RoPE row to fp["tab"])
+            if fp["rows"] != rows:
+                p = fp["params"] = self._proj_params(rows)
+                p.rope_cos, p.rope_sin = cos_t.data_ptr(), sin_t.data_ptr()
+                fp["rows"], fp["params_ref"] = rows, ctypes.byref(p)
+            p = fp["params"]
+            p.inv_freq, p.inv_dtype = angles
+            p.p0 = pos
+            _hip.check(fp["project"](fp["proj_ref"], fp["params_ref"], stream))
         routed = fp["routed"]
         routed.value = 1 if fp["record_pos"] == pos else 0
         j = int(st.recent_idx)
@@ -488,22 +500,22 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         fp["record_pos"] = pos + 1 if routed.value else -1
         # the general path's carried-record tag no longer matches this state
         self.__dict__["_route_tag"] = None
-        return self._out_rows(fp["heads_flat"])
+        return self._out_rows(fp["heads_flat"], kept=True)
 
     def _param_key(self) -> tuple:
-        """Identity and in-place version of every parameter of the layer and
-        of its (leaf) submodules, without the recursive module walk."""
+        """Identity, storage and in-place version of every parameter of the
+        layer and of its (leaf) submodules, without the recursive module walk."""
         out = []
         for p in self._parameters.values():
             if p is not None:
-                out += (id(p), p._version)
+                out += (id(p), p.data_ptr(), p._version)
         for mod in self._modules.values():
             for p in mod._parameters.values():
                 if p is not None:
-                    out += (id(p), p._version)
+                    out += (id(p), p.data_ptr(), p._version)
         return tuple(out)
 
-    def _build_step_fast(self, x, st, ts, vers, pvers):
+    def _build_step_fast(self, x, st, ts, vers, pvers, packed):
         """Descriptors and persistent buffers of _step_fast (see there)."""
         self.__dict__["_fast"] = None
         self._check_state(st)
@@ -522,22 +534,26 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         g = torch.empty((B, 1), dtype=torch.float32, device=dev)
         heads = torch.empty((B, 1, H, Dh), dtype=dt, device=dev)
         pos = int(st.pos)
-        cos_t, sin_t = self._rope_rows(0, pos + 1, dev, dt)
-        cos_t, sin_t = self.__dict__["_rope_cache"][(torch.device(dev), dt)]
+        w = b = None
+        if packed:
+            self._rope_rows(0, pos + 1, dev, dt)
+            cos_t, sin_t = self.__dict__["_rope_cache"][(torch.device(dev), dt)]
+            row = slice(pos, pos + 1)
+        else:
+            cos_t, sin_t = torch.empty((2, 1, Dh // 2), dtype=dt, device=dev)
+            row = slice(0, 1)
         d = self._proj_desc(x, B, 1, cos_t, sin_t)
-        w, b, d.w_layout = self._proj_pack(dt)
-        d.x_sm, d.w, d.bias = D, w.data_ptr(), b.data_ptr()
+        if packed:
+            w, b, d.w_layout = self._proj_pack(dt)
+            d.w, d.bias = w.data_ptr(), b.data_ptr()
+        d.x_sm = D
         d.q, d.q_sm, d.k, d.k_sm, d.v, d.v_sm = q.data_ptr(), Fq, k.data_ptr(), Fk, v.data_ptr(), Fk
         d.lam, d.lam_sm, d.g = lam.data_ptr(), H, g.data_ptr()
-        nb = ctypes.c_size_t(0)
-        _hip.check(_hip.lib().coda_project_workspace_bytes(d, nb))
-        pws = torch.empty(max(nb.value, 16), dtype=torch.uint8, device=dev) if nb.value else None
-        d.workspace, d.workspace_bytes = _hip.ptr(pws), nb.value
         qv = q.view(B, 1, H, Dh).permute(0, 2, 1, 3)
         lamv = lam.permute(0, 2, 1)
         ct, sn = self._theta_tables(dt)
         a, keep = ops.attention_desc(
-            q=qv, rope_cos=cos_t[pos:pos + 1], rope_sin=sin_t[pos:pos + 1], rope_interleaved=self.rope_interleaved,
+            q=qv, rope_cos=cos_t[row], rope_sin=sin_t[row], rope_interleaved=self.rope_interleaved,
             theta_cos=ct, theta_sin=sn, k_prefix=st.k_buf, v_prefix=st.v_buf,
             allowed=st.allowed if self.mask_unused_memory else None, k_block=None, v_block=None, lam=lamv,
             rms_weight=self._rms_weight(dt), eps=self._eps, out=heads.permute(0, 2, 1, 3))
@@ -551,15 +567,15 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         L_ = _hip.lib()
         routed = ctypes.c_int(0)
 
-        fp = {"st": st, "vers": vers, "pvers": pvers, "B": B, "dev": dev,
+        fp = {"st": st, "vers": vers, "pvers": pvers, "B": B, "dev": dev, "packed": packed, "rows": None,
               "ptrs": tuple(-1 if t is None else t.data_ptr() for t in ts),
               "tab": (cos_t, sin_t), "row_bytes": (Dh // 2) * cos_t.element_size(),
               "proj": d, "proj_ref": ctypes.byref(d), "attn": a, "attn_ref": ctypes.byref(a),
               "bank": bank, "bank_ref": ctypes.byref(bank),
-              "keep": (keep, q, k, v, lam, g, heads, w, b, pws, ws, ct, sn, eta, self._rms_weight(dt)),
+              "keep": (keep, q, k, v, lam, g, heads, w, b, ws, ct, sn, eta, self._rms_weight(dt)),
               "k_ptr": k.data_ptr(), "v_ptr": v.data_ptr(), "k_sb": Fk, "k_sh": Dh, "g_ptr": g.data_ptr(),
               "ws_ptr": _hip.ptr(ws), "ws_bytes": nb.value, "routed": routed, "routed_ref": ctypes.byref(routed),
-              "record_pos": routed_pos, "project": L_.coda_project_rows, "step": L_.coda_decode_step,
+              "record_pos": routed_pos, "project": L_.coda_project_rows if packed else L_.coda_project_params, "step": L_.coda_decode_step,
               "heads_flat": heads.view(B, 1, H * Dh)}
         self.__dict__["_fast"] = fp
         return fp

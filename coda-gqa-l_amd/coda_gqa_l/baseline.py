@@ -83,8 +83,10 @@ class CoDAGQA(RowsMixin, nn.Module):
         _hip.require_device(x)
         B, L, D = x.shape
         H, Hkv, Dh = self.num_heads, self.num_kv_heads, self.head_dim
-        if past_key_value is not None and self._decode_ok(x, past_key_value, is_causal):
-            return self._decode(x, *past_key_value)
+        if past_key_value is not None:
+            rows = self._decode_rows(x, past_key_value, is_causal)
+            if rows is not None:
+                return self._decode(x, rows, *past_key_value)
         q = self.q_proj(x).view(B, L, H, Dh).permute(0, 2, 1, 3)
         k = self.k_proj(x).view(B, L, Hkv, Dh).permute(0, 2, 1, 3)
         v = self.v_proj(x).view(B, L, Hkv, Dh).permute(0, 2, 1, 3)
@@ -101,61 +103,76 @@ class CoDAGQA(RowsMixin, nn.Module):
         heads = self.attention_core(q, k, v, lam, cos, sin, causal=2 if is_causal else 0)
         return self.o_proj(heads.view(B, L, D)), (k, v)
 
-    def _decode_ok(self, x: torch.Tensor, past: Tuple[torch.Tensor, torch.Tensor], is_causal: bool) -> bool:
-        """Whether _decode serves this call: few new tokens on top of a past,
-        no mask, bf16, at most 8 / G tokens a sequence, row-aligned K / V of
-        the layer's shape whose planes stay within the kernel's 31-bit offsets."""
+    def _decode_rows(self, x: torch.Tensor, past: Tuple[torch.Tensor, torch.Tensor], is_causal: bool):
+        """The parameters' addresses (_front_rows) where _decode serves this
+        call, else None: few new tokens on top of a past, no mask, bf16, at
+        most 8 / G tokens a sequence, row-aligned K / V of the layer's shape
+        whose planes stay within the kernel's 31-bit offsets."""
         B, L, _ = x.shape
         k, v = past
         if is_causal or L == 0 or x.dtype != torch.bfloat16 or k.dtype != x.dtype or v.dtype != x.dtype or \
                 2 * L * (self.num_heads // self.num_kv_heads) > 16 or self.head_dim not in (32, 64, 128):
-            return False
+            return None
         shape = (B, self.num_kv_heads, k.shape[2] if k.dim() == 4 else 0, self.head_dim)
         st = k.stride()
-        return (tuple(k.shape) == shape and tuple(v.shape) == shape and shape[2] > 0 and v.stride() == st and
+        if not (tuple(k.shape) == shape and tuple(v.shape) == shape and shape[2] > 0 and v.stride() == st and
                 st[3] == 1 and not (st[0] % 8 or st[1] % 8 or st[2] % 8) and
                 0 <= st[2] and (shape[2] + L + 16) * max(st[2], self.head_dim) < 1 << 30 and
                 not (k.data_ptr() % 16 or v.data_ptr() % 16) and k.device == v.device == x.device and
-                not (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad)) and
-                self._fused_front_ok(x) and self._plain_call(x, self.q_proj, self.k_proj, self.v_proj,
-                                                             self.lambda_proj))
+                not (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad))):
+            return None
+        return self._front_rows(x)
 
-    def _decode(self, x: torch.Tensor, k_past: torch.Tensor, v_past: torch.Tensor):
+    def _decode(self, x: torch.Tensor, rows: tuple, k_past: torch.Tensor, v_past: torch.Tensor):
         """forward() on top of a past for a few new tokens: one launch for the
-        projections and the RoPE of k (coda_project_rows), one for the
-        attention and the concatenated K / V (coda_attn_append, which reads
-        the past once for both), the merge of its splits, and o_proj."""
+        projections, the RoPE of k and the angle tables (coda_project_params),
+        one for the attention and the concatenated K / V (coda_attn_append,
+        which reads the past once for both), the merge of its splits, and
+        o_proj; all on the parameters as they stand at the call."""
         B, L, D = x.shape
         H, Hkv, Dh = self.num_heads, self.num_kv_heads, self.head_dim
-        G, past, M, e = H // Hkv, k_past.shape[2], B * L, x.element_size()
+        past, M, e, half = k_past.shape[2], B * L, x.element_size(), Dh // 2
         lib, stream, dev = _hip.lib(), _hip.stream_of(x), x.device
         xs = x if x.is_contiguous() and x.data_ptr() % 16 == 0 else x.contiguous()
-        cos, sin = self._rope_rows(past, L, dev, x.dtype)
-        th = self.theta
-        ct, st = self._derived("theta", th, x.dtype, lambda: (torch.cos(th).to(dtype=x.dtype).contiguous(),
-                                                              torch.sin(th).to(dtype=x.dtype).contiguous()))
         w = self.head_norm.weight.detach().to(x.dtype).contiguous() if self.head_norm_mode == "full" else None
         a = _hip.AttnDesc()
         a.dtype = _hip.dtype_code(x.dtype)
         a.B, a.H, a.Hkv, a.Lq, a.Dh = B, H, Hkv, L, Dh
-        # q | k | v | lambda | gate of the new tokens, then the heads, in one buffer
-        sizes = [M * D * e, M * Hkv * Dh * e, M * Hkv * Dh * e, M * H * e, M * 4]
+        # q | k | v | lambda | gate of the new tokens, RoPE cos | sin, theta
+        # cos | sin in one buffer
+        sizes = [M * D * e, M * Hkv * Dh * e, M * Hkv * Dh * e, M * H * e, M * 4, L * half * e, L * half * e,
+                 H * half * e, H * half * e]
         at = [0]
         for n in sizes:
             at.append(at[-1] + -(-n // 256) * 256)
         buf = torch.empty(at[-1], dtype=torch.uint8, device=dev)
         heads = torch.empty((B, L, D), dtype=x.dtype, device=dev)
         k, v = (torch.empty((B, Hkv, past + L, Dh), dtype=x.dtype, device=dev) for _ in range(2))
-        q_p, k_p, v_p, l_p, g_p = (buf.data_ptr() + o for o in at[:5])
-        d = self._proj_desc(x, M, L, cos, sin)
-        pw, pb, d.w_layout = self._proj_pack(x.dtype)
-        d.x, d.x_sm, d.w, d.bias = xs.data_ptr(), D, pw.data_ptr(), pb.data_ptr()
+        q_p, k_p, v_p, l_p, g_p, rc_p, rs_p, tc_p, ts_p = (buf.data_ptr() + o for o in at[:-1])
+        p = self._proj_params(rows)
+        angles, th, keep = self._angles_rows(dev, past, L), self.theta, ()
+        if angles is not None:
+            p.inv_freq, p.inv_dtype = angles
+            p.p0, p.rope_cos, p.rope_sin = past, rc_p, rs_p
+        else:
+            keep = self._rope_tables(past, L, dev, x.dtype)
+            rc_p, rs_p = (t.data_ptr() for t in keep)
+        if th.dtype in (torch.float32, torch.bfloat16) and th.device == dev and th.shape == (H, half) and \
+                th.is_contiguous():
+            p.theta, p.theta_dtype, p.theta_cos, p.theta_sin = th.data_ptr(), _hip.dtype_code(th.dtype), tc_p, ts_p
+        else:
+            tt = tuple(f(th).to(dtype=x.dtype).contiguous() for f in (torch.cos, torch.sin))
+            tc_p, ts_p = (t.data_ptr() for t in tt)
+            keep += tt
+        d = self._proj_desc(x, M, L)
+        d.rope_cos, d.rope_sin = rc_p, rs_p
+        d.x, d.x_sm = xs.data_ptr(), D
         d.q, d.q_sm, d.k, d.k_sm, d.v, d.v_sm = q_p, D, k_p, Hkv * Dh, v_p, Hkv * Dh
         d.lam, d.lam_sm, d.g = l_p, H, g_p
-        _hip.check(lib.coda_project_rows(d, stream))
+        _hip.check(lib.coda_project_params(d, p, stream))
         a.q, a.q_sb, a.q_sh, a.q_sl = q_p, L * D, Dh, D
-        a.theta_cos, a.theta_sin = ct.data_ptr(), st.data_ptr()
-        a.rope_cos, a.rope_sin, a.rope_interleaved = cos.data_ptr(), sin.data_ptr(), int(self.rope_interleaved)
+        a.theta_cos, a.theta_sin = tc_p, ts_p
+        a.rope_cos, a.rope_sin, a.rope_interleaved = rc_p, rs_p, int(self.rope_interleaved)
         a.kp, a.vp, a.Lp = k_p, v_p, L
         a.p_sb, a.p_sh, a.p_sl = L * Hkv * Dh, Dh, Hkv * Dh
         a.kb, a.vb, a.Lb = k_past.data_ptr(), v_past.data_ptr(), past

@@ -1,5 +1,5 @@
-"""Few-row projections shared by the bounded and unbounded layers: the packed
-weights, RoPE rows and descriptors of coda_project_rows / coda_linear_rows
+"""Few-row projections shared by the bounded and unbounded layers: parameters
+(as they lie, or packed), RoPE tables and descriptors of the row kernels
 (csrc/proj.hip) for decode-shaped inputs."""
 
 from __future__ import annotations
@@ -80,17 +80,21 @@ class RowsMixin:
         return tab[0][p0:need], tab[1][p0:need]
 
     def _rope_tables(self, p0: int, L: int, device, dtype: torch.dtype) -> Tuple[torch.Tensor, torch.Tensor]:
-        """RoPE tables (L, Dh/2) of a prompt: rows of the cached table (made
-        for the call alone they are seven small kernels, 20 us, and 45 us of
-        host time), but for positions past 65536 (tables of at most 32 MiB
-        are kept), under capture (a graph must not hold rows of a table that
-        a later call replaces) and where self.rope is not the plain module."""
-        r = self.rope
-        if p0 + L > 65536 or type(r) is not RotaryEmbedding or r._forward_hooks or r._forward_pre_hooks or \
-                nn.modules.module._has_any_global_hook() or torch.cuda.is_current_stream_capturing():
-            c, s_ = r(seq_len=L, offset=p0, device=device, dtype=dtype)
+        """RoPE tables (L, Dh/2): made for the call, by one launch in place of
+        the module's seven where the module is the plain one (nothing is kept,
+        so nothing can go stale, be freed under a captured graph or be read
+        before it is written)."""
+        a = None
+        if dtype in (torch.float32, torch.bfloat16) and not nn.modules.module._has_any_global_hook():
+            a = self._angles_rows(device, p0, L)
+        if a is None:
+            c, s_ = self.rope(seq_len=L, offset=p0, device=device, dtype=dtype)
             return c.contiguous(), s_.contiguous()
-        return self._rope_rows(p0, L, device, dtype)
+        half = self.head_dim // 2
+        t = torch.empty((2, L, half), dtype=dtype, device=device)
+        _hip.check(_hip.lib().coda_rope_tables(_hip.dtype_code(dtype), a[0], a[1], p0, L, half, t[0].data_ptr(),
+                                               t[1].data_ptr(), _hip.stream_of(t)))
+        return t[0], t[1]
 
     def _proj_pack(self, dtype: torch.dtype):
         """Packed [q | k | v | lambda | write] weights (n_feat, D) in `dtype`,
@@ -168,71 +172,134 @@ class RowsMixin:
             at += w.shape[0]
         return wt[:rows]
 
-    @staticmethod
-    def _plain_call(x: torch.Tensor, *lins: nn.Module) -> bool:
-        """Whether calling these modules on x is no more than their matrix
-        product: nn.Linear in x's dtype, no hooks, no autocast, no gradient."""
+    def _plain_rows(self, x: torch.Tensor, *names: str) -> Optional[tuple]:
+        """(address, row stride, bias address) of each of these linears' own
+        parameters, one after the other, where calling the module on x is no
+        more than its matrix product and the row kernels can take that: an
+        nn.Linear in x's dtype on x's device, no hooks, no forward of the
+        instance's own, no autocast, no gradient.  Else None.  Asked at every
+        call: nothing about a parameter is remembered."""
         if torch.is_autocast_enabled(x.device.type) or nn.modules.module._has_any_global_hook():
-            return False
+            return None
         grad = torch.is_grad_enabled()
         if grad and x.requires_grad:
-            return False
-        for m in lins:
-            if type(m) is not nn.Linear or m.weight.dtype != x.dtype or m._forward_hooks or m._forward_pre_hooks or \
-                    grad and m.weight.requires_grad:
-                return False
-        return True
+            return None
+        dt, dev, K, mods, out = x.dtype, x.device, x.shape[-1], self._modules, []
+        for name in names:
+            m = mods[name]
+            d = m.__dict__
+            if type(m) is not nn.Linear or m._forward_hooks or m._forward_pre_hooks or "forward" in d:
+                return None
+            ps = d["_parameters"]
+            w, b = ps.get("weight"), ps.get("bias")
+            if type(w) is not nn.Parameter or w.dtype is not dt or w.device != dev or w.dim() != 2:
+                return None
+            n, k = w.shape
+            if k != K or n != m.out_features or w.stride(1) != 1 or w.stride(0) < K or grad and w.requires_grad:
+                return None
+            pb = None
+            if b is not None:
+                if type(b) is not nn.Parameter or b.dtype is not dt or b.device != dev or b.shape != (n,) or \
+                        b.stride(0) != 1 or grad and b.requires_grad:
+                    return None
+                pb = b.data_ptr()
+            out += (w.data_ptr(), w.stride(0), pb)
+        return tuple(out)
 
-    def _out_rows(self, heads: torch.Tensor) -> torch.Tensor:
-        """o_proj of decode-shaped heads (B, L, H*Dh): at most 32 token rows
-        through the row kernel (bf16 4096 x 4096: 8.1 us at 1 row and 11.1 at
-        32 against 12.0 and 12.4 for the library's GEMM, which is ahead at 64
-        with 12.8 against 14.5).  Smaller bf16 layers take it up to 64 rows
-        (2048 x 2048) and 128 (1024 x 1024): the step waits for the host there
-        and this way is the shorter one (a token of 40 rows, 1024 x 1024: 32.6
-        us against 44.4 through the library)."""
+    def _out_rows(self, heads: torch.Tensor, kept: bool = False) -> torch.Tensor:
+        """o_proj of decode-shaped heads (B, L, H*Dh): few token rows of not too
+        large a layer through the row kernel, on the parameter itself.  kept:
+        the caller writes over heads later, so a module that may hold on to
+        its input (hooks, autograd) gets a copy.
+
+        The kernel against the library's GEMM, us, bf16: 4096 x 4096 8.7 and
+        14.9 at 1 row, 12.9 and 12.7 at 32, 16.2 and 14.4 at 64; 2048 x 2048
+        4.2 and 5.2, 6.3 and 7.3 at 64; 1024 x 1024 3.1 and 4.2, 6.6 and 6.5
+        at 64, 10.3 and 5.2 at 128, where the step still waits for the host
+        and this way is the shorter one (a token of 128 rows 39.9 us among
+        others and 71.5 alone against 54.1 and 71.8 through the module); 8192
+        x 8192 29.4 and 28.9 at 1 row, 31.5 and 28.8 at 16: the library's.
+        fp32: 1024 x 1024 4.5 and 5.5 at 1 row, 5.8 and 6.8 at 32; a token of
+        32 rows, 2048 x 2048, 53.5 us against 61.1; 4096 x 4096 15.8 and 15.4
+        at 1 row, 22.8 and 18.5 at 32: the library's."""
         B, L, K = heads.shape
         o = self.o_proj
-        most = 32
-        if heads.dtype == torch.bfloat16 and type(o) is nn.Linear and o.weight.numel() <= 1 << 22:
-            most = 128 if o.weight.numel() <= 1 << 20 else 64
-        if B * L > most or K % 64 or heads.dtype not in (torch.bfloat16, torch.float32) or \
-                not self._plain_call(heads, o) or not heads.is_contiguous():
-            return o(heads)
-        w, bias = o.weight, o.bias
-        tag = (w._version, w.data_ptr(), w.dtype, w.device) + (() if bias is None else (bias._version, bias.data_ptr()))
-        hit = self.__dict__.get("_o_rows")
-        if hit is None or hit[0] != tag:
-            with torch.no_grad():
-                tiles = self._rows_tiles(w.detach())
-                b = None if bias is None else bias.detach().float().contiguous()
-            hit = self.__dict__["_o_rows"] = (tag, tiles, b, _Made(*(t for t in (tiles, b) if t is not None)))
-        hit[3].use()
+        rows, most = B * L, 0
+        if type(o) is nn.Linear:
+            n = o.out_features * K
+            if heads.dtype == torch.bfloat16:
+                most = 128 if n <= 1 << 20 else 64 if n <= 1 << 22 else 32 if n <= 1 << 24 else 0
+            elif heads.dtype == torch.float32:
+                most = 32 if n <= 1 << 22 else 0
+        fits = 0 < rows <= most and K % 64 == 0 and heads.is_contiguous()
+        p = self._plain_rows(heads, "o_proj") if fits or kept else None
+        if p is None or not fits:
+            return o(heads.clone() if kept and p is None else heads)
         y = torch.empty((B, L, o.out_features), dtype=heads.dtype, device=heads.device)
-        _hip.check(_hip.lib().coda_linear_rows(
-            _hip.dtype_code(heads.dtype), heads.data_ptr(), K, B * L, hit[1].data_ptr(), o.out_features, K, _hip.ptr(hit[2]),
-            y.data_ptr(), o.out_features, _hip.stream_of(heads)))
+        _hip.check(_hip.lib().coda_linear_params(
+            _hip.dtype_code(heads.dtype), heads.data_ptr(), K, rows, p[0], p[1], o.out_features, K, p[2], y.data_ptr(),
+            o.out_features, _hip.stream_of(heads)))
         return y
 
-    def _proj_desc(self, x: torch.Tensor, M: int, L: int, cos: torch.Tensor, sin: torch.Tensor):
+    def _proj_desc(self, x: torch.Tensor, M: int, L: int, cos: Optional[torch.Tensor] = None,
+                   sin: Optional[torch.Tensor] = None):
         d = _hip.ProjDesc()
         d.dtype, d.M, d.D, d.L = _hip.dtype_code(x.dtype), M, self.embed_dim, L
         d.H, d.Hkv, d.Dh = self.num_heads, self.num_kv_heads, self.head_dim
         d.rope_interleaved, d.gate = int(self.rope_interleaved), int(self._has_gate())
-        d.rope_cos, d.rope_sin = cos.data_ptr(), sin.data_ptr()
+        d.rope_cos, d.rope_sin = _hip.ptr(cos), _hip.ptr(sin)
         return d
 
-    def _fused_front_ok(self, x: torch.Tensor) -> bool:
-        """Whether coda_project_rows serves x: D a multiple of 64, head_dim a
-        multiple of 4, and few token rows.  bf16: at most 64, or 128 (5 library
-        GEMMs with their sigmoids and RoPE take 103 us at 10305 x 8192 and 128
-        rows, the one launch 53); fp32: at most 32 (at 64 the library's GEMMs
-        are ahead)."""
+    def _packed_front_ok(self, x: torch.Tensor) -> bool:
+        """Whether the front end on packed weights serves x: bf16, at most 64
+        token rows, D a multiple of 64, head_dim a multiple of 4.  (6177 x
+        4096, weights not in cache: 12.2 us at 1 row and 18.2 at 64, on the
+        parameters 13.3 and 22.3; 10305 x 8192 31.3 against 36.1.)"""
         B, L, D = x.shape
-        if D % 64 or self.head_dim % 4:
-            return False
-        if x.dtype == torch.bfloat16 and B * L <= 64:
-            return True
+        return x.dtype == torch.bfloat16 and B * L <= 64 and D % 64 == 0 and self.head_dim % 4 == 0 and \
+            D == self.embed_dim
+
+    def _front_rows(self, x: torch.Tensor) -> Optional[tuple]:
+        """The parameters' addresses (_plain_rows) where coda_project_params
+        serves x: D a multiple of 64, head_dim a multiple of 4, and few token
+        rows.  bf16: at most 128 (5 library GEMMs with their sigmoids and
+        RoPE take 103 us at 10305 x 8192 and 128 rows, this launch 64); fp32: at most 32 (at
+        64 the library's GEMMs are ahead)."""
+        B, L, D = x.shape
         most = 128 if x.dtype == torch.bfloat16 else 32 if x.dtype == torch.float32 else 0
-        gate = (self.write_proj,) if self._has_gate() else ()
-        return B * L <= most and self._plain_call(x, self.q_proj, self.k_proj, self.v_proj, self.lambda_proj, *gate)
+        if not 0 < B * L <= most or D % 64 or D != self.embed_dim or self.head_dim % 4:
+            return None
+        names = ("q_proj", "k_proj", "v_proj", "lambda_proj")
+        p = self._plain_rows(x, *names, *(("write_proj",) if self._has_gate() else ()))
+        if p is None:
+            return None
+        H, F, mods = self.num_heads, self.num_heads * self.head_dim, self._modules
+        Fk = self.num_kv_heads * self.head_dim
+        if tuple(mods[n].out_features for n in names) != (F, Fk, Fk, H) or \
+                self._has_gate() and mods["write_proj"].out_features != 1:
+            return None
+        return p
+
+    def _fused_front_ok(self, x: torch.Tensor) -> bool:
+        """Whether one launch of the row kernel serves x's projections."""
+        return self._packed_front_ok(x) or self._front_rows(x) is not None
+
+    def _angles_rows(self, device, p0: int, L: int) -> Optional[tuple]:
+        """(address, type code) of the RoPE frequencies where the kernels can
+        make the tables of positions p0 .. p0 + L - 1 as self.rope would."""
+        r = self._modules["rope"]
+        if type(r) is not RotaryEmbedding or r._forward_hooks or r._forward_pre_hooks or "forward" in r.__dict__ or \
+                not 0 <= p0 <= (1 << 24) - L:
+            return None
+        inv = r._buffers.get("inv_freq")
+        if inv is None or inv.dtype not in (torch.float32, torch.bfloat16) or inv.device != device or \
+                inv.shape != (self.head_dim // 2,) or inv.stride(0) != 1:
+            return None
+        return inv.data_ptr(), _hip.dtype_code(inv.dtype)
+
+    @staticmethod
+    def _proj_params(rows: tuple) -> "_hip.ProjParams":
+        p = _hip.ProjParams()
+        for i in range(len(rows) // 3):
+            p.w[i], p.w_sm[i], p.b[i] = rows[3 * i:3 * i + 3]
+        return p

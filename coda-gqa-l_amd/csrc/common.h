@@ -117,6 +117,30 @@ __device__ __forceinline__ void rope_pair_t(float e, float o, float c, float s, 
   }
 }
 
+// Angle tables as the torch ops make them (primitives.py:30-55): positions
+// and products in the frequencies' type, cos and sin rounded to it, then to T.
+// (angles of CODA_F32 or CODA_BF16)
+__device__ __forceinline__ float angle_ld(const void* p, int dtype, int i) {
+  return dtype == CODA_BF16 ? bf2f(((const bf16_t*)p)[i]) : ((const float*)p)[i];
+}
+template <typename T>
+__device__ __forceinline__ float2 cos_sin_of(float a, int dtype) {
+  float c = cosf(a), s = sinf(a);
+  if (dtype == CODA_BF16) {
+    c = Elt<bf16_t>::rnd(c);
+    s = Elt<bf16_t>::rnd(s);
+  }
+  return float2{Elt<T>::rnd(c), Elt<T>::rnd(s)};
+}
+// (positions up to 2^24: exact in fp32)
+template <typename T>
+__device__ __forceinline__ float2 rope_angle(const void* inv_freq, int dtype, int64_t pos, int pair) {
+  const bool bf = dtype == CODA_BF16;
+  const float t = bf ? Elt<bf16_t>::rnd((float)pos) : (float)pos;
+  const float f = t * angle_ld(inv_freq, dtype, pair);
+  return cos_sin_of<T>(bf ? Elt<bf16_t>::rnd(f) : f, dtype);
+}
+
 // The new token's K handed to a decode-step kernel before RoPE: the kernel
 // ropes it with the token's own tables (cs / sn: Dh/2 entries of the
 // element type) as it writes and reads it.  mode 0: K already roped,

@@ -14,6 +14,7 @@
 #include "common.h"
 
 #include <climits>
+#include <type_traits>
 
 namespace coda {
 
@@ -39,23 +40,112 @@ __device__ __forceinline__ void proj_put4(bf16_t* p, const pf32x4& v) {
 }
 __device__ __forceinline__ void proj_put4(float* p, const pf32x4& v) { *reinterpret_cast<pf4u*>(p) = v; }
 
+// The layer's own parameters (coda_proj_params) as sections of the packed
+// feature order: q, k, v, lambda, gate
+template <typename T>
+struct ParamRows {
+  const T* w[5];
+  const T* b[5];
+  int64_t sm[5];
+  int start[5];  // first feature of a section; INT_MAX: not there
+  int Dh;
+  int halves;  // k rows of a head in the order (0, half, 1, half + 1, ..): half-split RoPE
+  __device__ __forceinline__ int section(int f) const {
+    int s = 0;
+#pragma unroll
+    for (int i = 1; i < 5; ++i) s = f >= start[i] ? i : s;
+    return s;
+  }
+  // a[s], from registers
+  template <typename V>
+  __device__ __forceinline__ V pick(const V (&a)[5], int s) const {
+    V v = a[0];
+#pragma unroll
+    for (int i = 1; i < 5; ++i) v = s == i ? a[i] : v;
+    return v;
+  }
+  // row of section s that feature f is
+  __device__ __forceinline__ int row_in(int s, int f) const {
+    int r = f - pick(start, s);
+    if (halves && s == 1) {
+      const int c = r % Dh;
+      r = r - c + (c >> 1) + (c & 1) * (Dh / 2);
+    }
+    return r;
+  }
+  // row of feature f0 + r16, at most last; f0, last the same in every lane:
+  // in most blocks of 16 the section is too (200 vector instructions before
+  // the first load cost 0.4 us)
+  __device__ __forceinline__ const T* row16(int f0, int r16, int last) const {
+    const int s0 = section(min(f0, last)), f = min(f0 + r16, last);
+    if (s0 == section(min(f0 + 15, last))) return pick(w, s0) + row_in(s0, f) * pick(sm, s0);
+    const int s = section(f);
+    return pick(w, s) + row_in(s, f) * pick(sm, s);
+  }
+  // biases of features f .. f + 3 (f a multiple of 4; past the last: any)
+  __device__ __forceinline__ pf32x4 bias4(int f, int last) const {
+    const int s = section(f);
+    pf32x4 v{0.f, 0.f, 0.f, 0.f};
+    if (s < 3) {
+      const T* p = pick(b, s);
+      if (!p) return v;
+      const int r = row_in(s, f), hs = halves && s == 1 ? Dh / 2 : 0;
+      const int o1 = hs ? hs : 1, o2 = hs ? 1 : 2, o3 = hs ? hs + 1 : 3;
+      return pf32x4{Elt<T>::ld(p[r]), Elt<T>::ld(p[r + o1]), Elt<T>::ld(p[r + o2]), Elt<T>::ld(p[r + o3])};
+    }
+    const T* lb = b[3];
+    const T* gb = b[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int ff = min(f + e, last);
+      const bool gate = ff >= start[4];
+      const T* p = gate ? gb : lb;
+      if (p) v[e] = Elt<T>::ld(p[ff - (gate ? start[4] : start[3])]);
+    }
+    return v;
+  }
+};
+// Angle tables made by the launch itself (pointers null: given in the
+// descriptor, or not asked for)
+struct FrontTables {
+  const void* inv_freq;
+  int inv_dtype;
+  int64_t p0;
+  void* rope_cos;
+  void* rope_sin;
+  const void* theta;
+  int theta_dtype, n_theta;
+  void* theta_cos;
+  void* theta_sin;
+};
+
 // Epilogue of features f .. f + 3 (f a multiple of 4) of token row m:
 // the fp32 accumulators plus bias, rounded and routed to q / k (RoPE) / v /
 // lambda / gate
-template <typename T>
+// PARAMS: biases from the parameters, the launch's own tables; else one
+// packed fp32 bias vector (zero where a linear has none) and given tables
+template <typename T, bool PARAMS>
 struct FrontEpilogue {
   coda_proj_desc d;
-  __device__ __forceinline__ void operator()(int f, int m, pf32x4 v) const {
+  FrontTables tab;
+  template <typename Src>
+  __device__ __forceinline__ pf32x4 bias4(const Src& W, int f, int last) const {
+    if constexpr (PARAMS) {
+      return W.bias4(f, last);
+    } else {
+      if (f + 3 <= last) {
+        const float4 v = *reinterpret_cast<const float4*>(d.bias + f);
+        return pf32x4{v.x, v.y, v.z, v.w};
+      }
+      return pf32x4{d.bias[f], d.bias[min(f + 1, last)], d.bias[min(f + 2, last)], d.bias[min(f + 3, last)]};
+    }
+  }
+  template <typename Src>
+  __device__ __forceinline__ void operator()(const Src& W, int f, int m, pf32x4 v) const {
     using E = Elt<T>;
     const int Fq = d.H * d.Dh, Fk = d.Hkv * d.Dh, half = d.Dh / 2;
     const int o_k = Fq, o_v = Fq + Fk, o_l = Fq + 2 * Fk, o_g = o_l + d.H;
-    if (f + 3 < o_l) {  // q / k / v: the linear's bias (zero where it has none)
-      const float4 bb = *reinterpret_cast<const float4*>(d.bias + f);
-      v[0] += bb.x;
-      v[1] += bb.y;
-      v[2] += bb.z;
-      v[3] += bb.w;
-    }
+    v += bias4(W, f, o_g - (d.gate ? 0 : 1));
     if (f + 3 < o_k) {  // q
       proj_put4((T*)d.q + (int64_t)m * d.q_sm + f, v);
     } else if (f >= o_k && f + 3 < o_v) {  // k: two RoPE pairs
@@ -68,7 +158,18 @@ struct FrontEpilogue {
 #pragma unroll
       for (int pp = 0; pp < 2; ++pp) {
         const int p = c / 2 + pp;  // pair index
-        const float cc = E::ld(cs[(int64_t)prow * half + p]), ss = E::ld(sn[(int64_t)prow * half + p]);
+        float cc, ss;
+        if constexpr (!PARAMS) {
+          cc = E::ld(cs[(int64_t)prow * half + p]);
+          ss = E::ld(sn[(int64_t)prow * half + p]);
+        } else if (tab.inv_freq) {
+          const float2 t = rope_angle<T>(tab.inv_freq, tab.inv_dtype, tab.p0 + prow, p);
+          cc = t.x;
+          ss = t.y;
+        } else {
+          cc = E::ld(cs[(int64_t)prow * half + p]);
+          ss = E::ld(sn[(int64_t)prow * half + p]);
+        }
         rope_pair_t<T>(E::rnd(v[2 * pp]), E::rnd(v[2 * pp + 1]), cc, ss, inter, r[2 * pp], r[2 * pp + 1]);
       }
       if (inter) {
@@ -87,30 +188,46 @@ struct FrontEpilogue {
       for (int rr = 0; rr < 4; ++rr) {
         const int ff = f + rr;
         if (ff < o_l || ff >= o_g + (d.gate ? 1 : 0)) continue;
-        const float lin = E::rnd(v[rr] + d.bias[ff]);
+        const float lin = E::rnd(v[rr]);
         const float sg = E::rnd(proj_sigmoid(lin));
         if (ff < o_g) ((T*)d.lam)[(int64_t)m * d.lam_sm + (ff - o_l)] = E::st(sg);
         else d.g[m] = sg;
       }
     }
   }
-  // no gate column: the gate is 1
+  // no gate column: the gate is 1; the tables that the launch leaves
   __device__ __forceinline__ void once(int t) const {
     if (!d.gate && t < d.M) d.g[t] = 1.f;
+    if constexpr (PARAMS) {
+      const int half = d.Dh / 2;
+      if (tab.inv_freq)
+        for (int i = t; i < d.L * half; i += 512) {
+          const float2 a = rope_angle<T>(tab.inv_freq, tab.inv_dtype, tab.p0 + i / half, i % half);
+          ((T*)tab.rope_cos)[i] = Elt<T>::st(a.x);
+          ((T*)tab.rope_sin)[i] = Elt<T>::st(a.y);
+        }
+      if (tab.theta)
+        for (int i = t; i < tab.n_theta; i += 512) {
+          const float2 a = cos_sin_of<T>(angle_ld(tab.theta, tab.theta_dtype, i), tab.theta_dtype);
+          ((T*)tab.theta_cos)[i] = Elt<T>::st(a.x);
+          ((T*)tab.theta_sin)[i] = Elt<T>::st(a.y);
+        }
+    }
   }
 };
 
 // Epilogue of a plain linear layer: out = acc + bias, one rounding
-template <typename T>
+template <typename T, typename BT>
 struct LinearEpilogue {
   T* out;
-  const float* bias;  // or null
+  const BT* bias;  // or null
   int64_t o_sm;
   int n_feat;
-  __device__ __forceinline__ void operator()(int f, int m, pf32x4 v) const {
+  template <typename Src>
+  __device__ __forceinline__ void operator()(const Src&, int f, int m, pf32x4 v) const {
     T* row = out + (int64_t)m * o_sm;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] += bias && f + e < n_feat ? bias[f + e] : 0.f;
+    for (int e = 0; e < 4; ++e) v[e] += bias && f + e < n_feat ? Elt<BT>::ld(bias[f + e]) : 0.f;
     if (f + 3 < n_feat) {
       proj_put4(row + f, v);
     } else {
@@ -131,12 +248,32 @@ struct LinearEpilogue {
 // HBM once; the token rows are read by every workgroup from L2.
 // K goes in pairs of 64-byte steps: a lane's two 16-byte pieces of a row
 // come from the two halves of one 128-byte line, requested back to back.
-// Measured (bf16, weights not in cache): 6184 x 4096 M = 1 12.5 us, M = 16
-// 14.1 us (4.0 / 3.6 TB/s), 4096 x 4096 M = 1 8.1 us (the library 12.0),
-// 10305 x 8192 M = 1 30.4 us (5.5 TB/s).
-// TILED: W in fragment tiles (coda_project_pack), where the operand of row
-// block fb at k-step ks is the KiB at (fb D/32 + ks) 512 elements (bf16),
-// lane l's 16 bytes at 16 l; else row-major with row stride w_sm.
+// Measured (bf16, tiles, weights not in cache): 6177 x 4096 M = 1 12.2 us, M
+// = 16 13.3 us (4.1 / 3.8 TB/s), 10305 x 8192 M = 1 31.3 us (5.4 TB/s).
+// The weights: in fragment tiles (TileRows; coda_project_pack), where the
+// operand of row block fb at k-step ks is the KiB at (fb D/32 + ks) 512
+// elements (bf16), lane l's 16 bytes at 16 l; or rows as they lie (MatRows:
+// one matrix; ParamRows: the layer's own parameters), at any element address.
+// A load of tiles is a KiB in one piece, one of rows 16 pieces of 64 bytes:
+// 6177 x 4096 M = 1 13.3 us (tiles 12.2), M = 64 22.3 (18.2), 10305 x 8192 M =
+// 128 63.3 (53.7), 4096 x 4096 M = 1 8.7 (7.9; the library 14.9).
+template <typename T>
+struct TileRows {
+  static constexpr bool kTiles = true;
+  const T* w;
+};
+template <typename T>
+struct MatRows {
+  const T* w;
+  int64_t sm;
+  __device__ __forceinline__ const T* row16(int f0, int r16, int last) const { return w + min(f0 + r16, last) * sm; }
+};
+template <typename Src>
+struct IsTiles : std::false_type {};
+template <typename T>
+struct IsTiles<TileRows<T>> : std::true_type {};
+// a row's 16 bytes at any element address
+typedef uint32_t pu32x4u __attribute__((ext_vector_type(4), aligned(2)));
 template <typename T>
 __device__ __forceinline__ pf32x4 rows_mfma(const pu32x4& a, const pu32x4& b, pf32x4 c) {
   if constexpr (sizeof(T) == 2) {
@@ -156,10 +293,20 @@ struct RowsLds {
   static constexpr int kWaves = RB * MT <= 8 ? 8 : 4;
   static constexpr size_t kBytes = (size_t)kWaves * RB * MT * 64 * sizeof(pf32x4);
 };
+// One dword of each 64 bytes of the epilogue's arguments, read before the
+// products: the compiler loads them where they are used, after the products,
+// in several dependent rounds, each a miss of the scalar cache then
+template <typename V>
+__device__ __forceinline__ void touch_args(const V& v) {
+  const int* p = reinterpret_cast<const int*>(&v);
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(V) / 4); i += 16) asm volatile("" ::"s"(p[i]));
+}
 // The waves' partials (accumulators of 16 features x 16 tokens each), summed in
 // wave order, and the epilogue
-template <int MT, int RB, typename Epi>
-__device__ __forceinline__ void rows_finish(pf32x4 (&acc)[RB][MT], char* smem, int n_feat, int M, const Epi& epi) {
+template <int MT, int RB, typename Src, typename Epi>
+__device__ __forceinline__ void rows_finish(pf32x4 (&acc)[RB][MT], char* smem, int n_feat, int M, const Src& W,
+                                            const Epi& epi) {
   pf32x4* part = reinterpret_cast<pf32x4*>(smem);
   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), f0 = blockIdx.x * 16 * RB;
   constexpr int NWv = RowsLds<MT, RB>::kWaves;
@@ -192,14 +339,14 @@ __device__ __forceinline__ void rows_finish(pf32x4 (&acc)[RB][MT], char* smem, i
 #pragma unroll
     for (int w = 1; w < NWv; ++w) sum += part[(w * RB * MT + ij) * 64 + l];
     const int m = 16 * (ij % MT) + (l & 15), f = f0 + 16 * (ij / MT) + 4 * (l >> 4);
-    if (m < M && f < n_feat) epi(f, m, sum);
+    if (m < M && f < n_feat) epi(W, f, m, sum);
   }
 }
 
-template <typename T, int MT, int RB, bool TILED, typename Epi>
+template <typename T, int MT, int RB, typename Src, typename Epi>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void proj_rows(
-    const T* __restrict__ W, int64_t w_sm, int n_feat, int D, const T* __restrict__ X, int64_t x_sm, int M,
-    const Epi epi) {
+    const Src W, int n_feat, int D, const T* __restrict__ X, int64_t x_sm, int M, const Epi epi) {
+  constexpr bool TILED = IsTiles<Src>::value;
   extern __shared__ __attribute__((aligned(16))) char rows_smem[];
   // pairs of k-steps in flight ahead of the products
   constexpr int LP = RB * MT <= 3 ? 4 : RB * MT <= 12 ? 2 : 1;
@@ -212,8 +359,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   const char* wr[RB];
 #pragma unroll
   for (int i = 0; i < RB; ++i)
-    wr[i] = TILED ? (const char*)W + ((int64_t)min(f0 / 16 + i, (n_feat + 15) / 16 - 1) * pairs + p0) * 2048 + 16 * lane
-                  : (const char*)(W + (int64_t)min(f0 + 16 * i + r16, n_feat - 1) * w_sm) + 128 * p0 + 16 * kq;
+    if constexpr (TILED)
+      wr[i] = (const char*)W.w + ((int64_t)min(f0 / 16 + i, (n_feat + 15) / 16 - 1) * pairs + p0) * 2048 + 16 * lane;
+    else
+      wr[i] = (const char*)W.row16(f0 + 16 * i, r16, n_feat - 1) + 128 * p0 + 16 * kq;
   const char* xr[MT];
 #pragma unroll
   for (int j = 0; j < MT; ++j) xr[j] = (const char*)(X + (int64_t)min(16 * j + r16, M - 1) * x_sm) + 128 * p0 + 16 * kq;
@@ -222,7 +371,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
 #pragma unroll
     for (int i = 0; i < RB; ++i)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) a[u][i][h] = *reinterpret_cast<const pu32x4*>(wr[i] + WP * p + WH * h);
+      for (int h = 0; h < 2; ++h)
+        a[u][i][h] = *reinterpret_cast<const typename std::conditional<TILED, pu32x4, pu32x4u>::type*>(wr[i] + WP * p + WH * h);
 #pragma unroll
     for (int j = 0; j < MT; ++j)
 #pragma unroll
@@ -236,6 +386,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
 #pragma unroll
   for (int u = 0; u < LP; ++u)
     if (u < np) load(u, u);
+  touch_args(epi);
   auto products = [&](const pu32x4 (&as)[RB][2], const pu32x4 (&bs)[MT][2]) {
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -258,7 +409,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
     products(a[u % LP], b[u % LP]);
     if (p + u + LP < np) load(u % LP, p + u + LP);
   }
-  rows_finish<MT, RB>(acc, rows_smem, n_feat, M, epi);
+  rows_finish<MT, RB>(acc, rows_smem, n_feat, M, W, epi);
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const char* p, int nbytes) {
@@ -280,23 +431,32 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const char* p, int n
 // writes and reads spread over the banks.  The slab is the wave's alone and
 // LDS serves a wave in order: no barrier.  The next chunk's weights load
 // while this chunk's products run.  Same sums in the same order as proj_rows.
-template <typename T, int MT, int RB, int CS, typename Epi>
+template <typename T, int MT, int RB, int CS, typename Src, typename Epi>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void proj_rows_lds(
-    const T* __restrict__ W, int n_feat, int D, const T* __restrict__ X, int64_t x_sm, int M, const Epi epi) {
+    const Src W, int n_feat, int D, const T* __restrict__ X, int64_t x_sm, int M, const Epi epi) {
+  constexpr bool TILED = IsTiles<Src>::value;
   extern __shared__ __attribute__((aligned(16))) char rows_smem[];
   constexpr int RBY = CS * 64, PCS = RBY / 16, NI = 16 * PCS / 64, RPI = 64 / PCS;  // row bytes, pieces; loads a slab, rows a load
   const int f0 = blockIdx.x * 16 * RB;
   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), r16 = lane & 15, kq = lane >> 4;
   const int steps = D * (int)sizeof(T) / 64, nc = steps / (8 * CS), s0 = nc * CS * wv;
   char* slab = rows_smem + wv * 16 * RBY;
-  // weights and token rows through raw buffer resources: 32-bit offsets, and
+  // tiles and token rows through raw buffer resources: 32-bit offsets, and
   // token rows past the last read 0 without touching memory
   const int nfb = (n_feat + 15) / 16;
-  const __amdgpu_buffer_rsrc_t rw = rows_rsrc((const char*)W + (int64_t)(f0 / 16) * steps * 1024, RB * steps * 1024);
   const __amdgpu_buffer_rsrc_t rx = rows_rsrc((const char*)X, (int)(((M - 1) * x_sm + D) * (int)sizeof(T)));
+  __amdgpu_buffer_rsrc_t rw;
   int wo[RB];
+  const char* wr[RB];
+  if constexpr (TILED) {
+    rw = rows_rsrc((const char*)W.w + (int64_t)(f0 / 16) * steps * 1024, RB * steps * 1024);
 #pragma unroll
-  for (int i = 0; i < RB; ++i) wo[i] = (min(f0 / 16 + i, nfb - 1) - f0 / 16) * steps * 1024 + s0 * 1024;
+    for (int i = 0; i < RB; ++i) wo[i] = (min(f0 / 16 + i, nfb - 1) - f0 / 16) * steps * 1024 + s0 * 1024;
+  } else {
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+      wr[i] = (const char*)W.row16(f0 + 16 * i, r16, n_feat - 1) + 64 * s0 + 16 * kq;
+  }
   const int lr = lane / PCS, lp = lane % PCS, xrow = (int)x_sm * (int)sizeof(T);
   const int xo = 64 * s0 + 16 * lp + lr * xrow;
   pu32x4 a0[CS][RB], a1[CS][RB], x0[NI], x1[NI];
@@ -304,8 +464,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
 #pragma unroll
     for (int s = 0; s < CS; ++s)
 #pragma unroll
-      for (int i = 0; i < RB; ++i)
-        w[s][i] = __builtin_amdgcn_raw_buffer_load_b128(rw, 16 * lane, wo[i] + (c * CS + s) * 1024, 0);
+      for (int i = 0; i < RB; ++i) {
+        if constexpr (TILED) w[s][i] = __builtin_amdgcn_raw_buffer_load_b128(rw, 16 * lane, wo[i] + (c * CS + s) * 1024, 0);
+        else w[s][i] = *reinterpret_cast<const pu32x4u*>(wr[i] + c * RBY + 64 * s);
+      }
   };
   // slab (chunk c, tokens 16 j ..)
   auto load_x = [&](pu32x4 (&v)[NI], int c, int j) {
@@ -347,6 +509,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   load_w(a0, 0);
   load_x(x0, 0, 0);
   load_x(x1, 0, 1);
+  touch_args(epi);
   int c = 0;
   for (; c + 1 < nc; c += 2) {
     chunk(c, a0, a1);
@@ -354,17 +517,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   }
   if (c < nc) chunk(c, a0, a1);
   __syncthreads();
-  rows_finish<MT, RB>(acc, rows_smem, n_feat, M, epi);
+  rows_finish<MT, RB>(acc, rows_smem, n_feat, M, W, epi);
 }
 
-template <typename T, int MT, int RB, bool TILED, typename Epi>
-static int launch_rows_k(const T* W, int64_t w_sm, int n_feat, int D, const T* X, int64_t x_sm, int M, const Epi& epi,
+template <typename T, int MT, int RB, typename Src, typename Epi>
+static int launch_rows_k(const Src& W, int n_feat, int D, const T* X, int64_t x_sm, int M, const Epi& epi,
                          hipStream_t st, const char* who) {
   constexpr size_t lds = RowsLds<MT, RB>::kBytes;
-  const int rc = lds_limit<proj_rows<T, MT, RB, TILED, Epi>>(lds, who);
+  const int rc = lds_limit<proj_rows<T, MT, RB, Src, Epi>>(lds, who);
   if (rc) return rc;
-  hipLaunchKernelGGL((proj_rows<T, MT, RB, TILED, Epi>), dim3((n_feat + 16 * RB - 1) / (16 * RB)), dim3(512), lds, st, W,
-                     w_sm, n_feat, D, X, x_sm, M, epi);
+  hipLaunchKernelGGL((proj_rows<T, MT, RB, Src, Epi>), dim3((n_feat + 16 * RB - 1) / (16 * RB)), dim3(512), lds, st, W,
+                     n_feat, D, X, x_sm, M, epi);
   return check_launch("proj_rows");
 }
 // Features a workgroup: the RB (1 .. 3) of the fewest 16-feature turns, ceil
@@ -382,23 +545,24 @@ static int rows_rb(int n_feat) {
   }
   return best;
 }
-template <typename T, int MT, int RB, typename Epi>
-static int launch_rows_lds(const T* W, int n_feat, int D, const T* X, int64_t x_sm, int M, const Epi& epi,
+template <typename T, int MT, int RB, typename Src, typename Epi>
+static int launch_rows_lds(const Src& W, int n_feat, int D, const T* X, int64_t x_sm, int M, const Epi& epi,
                            hipStream_t st, const char* who) {
-  // steps a chunk: as many as the accumulators leave registers for
-  constexpr int CS = RB * MT <= 4 ? 8 : RB * MT <= 16 ? 4 : 2;
+  // steps a chunk: as many as the accumulators (and the row addresses of
+  // weights that are not tiles) leave registers for
+  constexpr int CS = RB * MT <= (IsTiles<Src>::value ? 4 : 3) || RB == 1 && MT == 4 ? 8 : RB * MT <= 16 ? 4 : 2;
   constexpr size_t slabs = (size_t)8 * 16 * CS * 64;
   constexpr size_t lds = slabs > RowsLds<MT, RB>::kBytes ? slabs : RowsLds<MT, RB>::kBytes;
-  const int rc = lds_limit<proj_rows_lds<T, MT, RB, CS, Epi>>(lds, who);
+  const int rc = lds_limit<proj_rows_lds<T, MT, RB, CS, Src, Epi>>(lds, who);
   if (rc) return rc;
-  hipLaunchKernelGGL((proj_rows_lds<T, MT, RB, CS, Epi>), dim3((n_feat + 16 * RB - 1) / (16 * RB)), dim3(512), lds, st,
-                     W, n_feat, D, X, x_sm, M, epi);
+  hipLaunchKernelGGL((proj_rows_lds<T, MT, RB, CS, Src, Epi>), dim3((n_feat + 16 * RB - 1) / (16 * RB)), dim3(512), lds,
+                     st, W, n_feat, D, X, x_sm, M, epi);
   return check_launch("proj_rows_lds");
 }
-template <typename T, int MT, bool TILED, typename Epi>
-static int launch_rows_mt(const T* W, int64_t w_sm, int n_feat, int D, const T* X, int64_t x_sm, int M, const Epi& epi,
+template <typename T, int MT, typename Src, typename Epi>
+static int launch_rows_mt(const Src& W, int n_feat, int D, const T* X, int64_t x_sm, int M, const Epi& epi,
                           hipStream_t st, const char* who) {
-  if constexpr (TILED && MT > 1) {
+  if constexpr (MT > 1) {
     // (token rows within a 31-bit offset)
     if (D * sizeof(T) % 4096 == 0 && x_sm >= 0 && (M * x_sm + D) * (int64_t)sizeof(T) < INT_MAX) {
       switch (rows_rb(n_feat)) {
@@ -409,24 +573,18 @@ static int launch_rows_mt(const T* W, int64_t w_sm, int n_feat, int D, const T* 
     }
   }
   switch (rows_rb(n_feat)) {
-    case 1: return launch_rows_k<T, MT, 1, TILED>(W, w_sm, n_feat, D, X, x_sm, M, epi, st, who);
-    case 2: return launch_rows_k<T, MT, 2, TILED>(W, w_sm, n_feat, D, X, x_sm, M, epi, st, who);
-    default: return launch_rows_k<T, MT, 3, TILED>(W, w_sm, n_feat, D, X, x_sm, M, epi, st, who);
+    case 1: return launch_rows_k<T, MT, 1>(W, n_feat, D, X, x_sm, M, epi, st, who);
+    case 2: return launch_rows_k<T, MT, 2>(W, n_feat, D, X, x_sm, M, epi, st, who);
+    default: return launch_rows_k<T, MT, 3>(W, n_feat, D, X, x_sm, M, epi, st, who);
   }
 }
-template <typename T, bool TILED, typename Epi>
-static int launch_rows_t(const T* W, int64_t w_sm, int n_feat, int D, const T* X, int64_t x_sm, int M, const Epi& epi,
-                         hipStream_t st, const char* who) {
-  if (M <= 16) return launch_rows_mt<T, 1, TILED>(W, w_sm, n_feat, D, X, x_sm, M, epi, st, who);
-  if (M <= 32) return launch_rows_mt<T, 2, TILED>(W, w_sm, n_feat, D, X, x_sm, M, epi, st, who);
-  if (M <= 64) return launch_rows_mt<T, 4, TILED>(W, w_sm, n_feat, D, X, x_sm, M, epi, st, who);
-  return launch_rows_mt<T, 8, TILED>(W, w_sm, n_feat, D, X, x_sm, M, epi, st, who);
-}
-template <typename T, typename Epi>
-static int launch_rows(const void* W, int64_t w_sm, int tiled, int n_feat, int D, const void* X, int64_t x_sm, int M,
-                       const Epi& epi, hipStream_t st, const char* who) {
-  return tiled ? launch_rows_t<T, true>((const T*)W, w_sm, n_feat, D, (const T*)X, x_sm, M, epi, st, who)
-               : launch_rows_t<T, false>((const T*)W, w_sm, n_feat, D, (const T*)X, x_sm, M, epi, st, who);
+template <typename T, typename Src, typename Epi>
+static int launch_rows(const Src& W, int n_feat, int D, const T* X, int64_t x_sm, int M, const Epi& epi,
+                       hipStream_t st, const char* who) {
+  if (M <= 16) return launch_rows_mt<T, 1>(W, n_feat, D, X, x_sm, M, epi, st, who);
+  if (M <= 32) return launch_rows_mt<T, 2>(W, n_feat, D, X, x_sm, M, epi, st, who);
+  if (M <= 64) return launch_rows_mt<T, 4>(W, n_feat, D, X, x_sm, M, epi, st, who);
+  return launch_rows_mt<T, 8>(W, n_feat, D, X, x_sm, M, epi, st, who);
 }
 // one thread per 16-byte piece of the tiled copy; row_pieces: 16-byte pieces
 // of a row
@@ -458,26 +616,50 @@ static bool rows_path(int D) {
   return D >= 512 && D <= 8192 && D % 256 == 0 && ((D / 256) & (D / 256 - 1)) == 0;
 }
 
-// What both front-end entries ask of a descriptor
-static int check_project(const coda_proj_desc* d, const char* who) {
+// What the front-end entries ask of a descriptor (packed: of its w and bias too)
+static int check_project(const coda_proj_desc* d, const char* who, bool packed) {
   CODA_REQUIRE(d->D > 0 && d->D % kProjKT == 0, "%s: D=%d must be a positive multiple of %d", who, d->D, kProjKT);
   CODA_REQUIRE(d->H > 0 && d->Hkv > 0 && d->Dh > 0 && d->Dh % 4 == 0 && d->L > 0,
                "%s: bad sizes H=%d Hkv=%d Dh=%d L=%d", who, d->H, d->Hkv, d->Dh, d->L);
-  CODA_REQUIRE(d->x && d->w && d->bias && d->rope_cos && d->rope_sin && d->q && d->k && d->v && d->lam && d->g,
-               "%s: pointer missing", who);
-  CODA_REQUIRE(((uintptr_t)d->bias % 16) == 0, "%s: bias must be 16-byte aligned", who);
+  CODA_REQUIRE(d->x && d->q && d->k && d->v && d->lam && d->g, "%s: pointer missing", who);
+  CODA_REQUIRE(!packed || (d->w && d->bias && d->rope_cos && d->rope_sin), "%s: pointer missing", who);
+  CODA_REQUIRE(!packed || ((uintptr_t)d->bias % 16) == 0, "%s: bias must be 16-byte aligned", who);
   const int pc = d->dtype == CODA_BF16 ? 8 : 4;  // elements of a 16-byte piece
-  CODA_REQUIRE(d->x_sm % pc == 0 && ((uintptr_t)d->x % 16) == 0 && ((uintptr_t)d->w % 16) == 0,
+  CODA_REQUIRE(d->x_sm % pc == 0 && ((uintptr_t)d->x % 16) == 0 && (!packed || ((uintptr_t)d->w % 16) == 0),
                "%s: x / w rows must be 16-byte aligned", who);
   CODA_REQUIRE(d->q_sm % 4 == 0 && d->k_sm % 4 == 0 && d->v_sm % 4 == 0 && ((uintptr_t)d->q % 8) == 0 &&
                    ((uintptr_t)d->k % 8) == 0 && ((uintptr_t)d->v % 8) == 0,
                "%s: q / k / v rows must be 8-byte aligned", who);
   return CODA_OK;
 }
+static int front_features(const coda_proj_desc* d) {
+  return d->H * d->Dh + 2 * d->Hkv * d->Dh + d->H + (d->gate ? 1 : 0);
+}
 template <typename T>
 static int run_project(const coda_proj_desc* d, hipStream_t st, const char* who) {
-  const int n_feat = d->H * d->Dh + 2 * d->Hkv * d->Dh + d->H + (d->gate ? 1 : 0);
-  return launch_rows<T>(d->w, d->D, d->w_layout, n_feat, d->D, d->x, d->x_sm, d->M, FrontEpilogue<T>{*d}, st, who);
+  const FrontEpilogue<T, false> epi{*d, FrontTables{}};
+  const T *w = (const T*)d->w, *x = (const T*)d->x;
+  const int n = front_features(d);
+  return d->w_layout ? launch_rows<T>(TileRows<T>{w}, n, d->D, x, d->x_sm, d->M, epi, st, who)
+                     : launch_rows<T>(MatRows<T>{w, d->D}, n, d->D, x, d->x_sm, d->M, epi, st, who);
+}
+template <typename T>
+static int run_project_params(const coda_proj_desc* d, const coda_proj_params* p, hipStream_t st, const char* who) {
+  ParamRows<T> r;
+  const int sizes[5] = {d->H * d->Dh, d->Hkv * d->Dh, d->Hkv * d->Dh, d->H, d->gate ? 1 : 0};
+  int f = 0;
+  for (int i = 0; i < 5; ++i) {
+    r.w[i] = (const T*)p->w[i];
+    r.b[i] = (const T*)p->b[i];
+    r.sm[i] = p->w_sm[i];
+    r.start[i] = sizes[i] ? f : INT_MAX;
+    f += sizes[i];
+  }
+  r.Dh = d->Dh;
+  r.halves = !d->rope_interleaved;
+  const FrontTables t{p->inv_freq,  p->inv_dtype, p->p0,        p->rope_cos, p->rope_sin,
+                      p->theta, p->theta_dtype, d->H * (d->Dh / 2), p->theta_cos, p->theta_sin};
+  return launch_rows<T>(r, f, d->D, (const T*)d->x, d->x_sm, d->M, FrontEpilogue<T, true>{*d, t}, st, who);
 }
 
 }  // namespace coda
@@ -489,7 +671,7 @@ extern "C" int coda_project(const coda_proj_desc* d, void* stream) {
   CODA_REQUIRE(d->dtype == CODA_BF16, "coda_project: bf16 only");
   CODA_REQUIRE(d->M >= 0 && d->M <= 64, "coda_project: %d token rows; the front end serves decode-shaped inputs "
                "(at most 64 rows), many rows are library GEMMs", d->M);
-  const int rc = check_project(d, "coda_project");
+  const int rc = check_project(d, "coda_project", true);
   if (rc) return rc;
   if (d->M == 0) return CODA_OK;
   CODA_REQUIRE(d->w_layout == 0 || (d->w_layout == 1 && rows_path(d->D)),
@@ -501,7 +683,7 @@ extern "C" int coda_project_rows(const coda_proj_desc* d, void* stream) {
   CODA_REQUIRE(d != nullptr, "coda_project_rows: null descriptor");
   CODA_REQUIRE(d->dtype == CODA_BF16 || d->dtype == CODA_F32, "coda_project_rows: dtype must be CODA_F32 or CODA_BF16");
   CODA_REQUIRE(d->M >= 0 && d->M <= 128, "coda_project_rows: %d token rows (at most 128)", d->M);
-  const int rc = check_project(d, "coda_project_rows");
+  const int rc = check_project(d, "coda_project_rows", true);
   if (rc) return rc;
   if (d->M == 0) return CODA_OK;
   CODA_REQUIRE(d->w_layout == 0 || d->w_layout == 1, "coda_project_rows: weight layout %d", d->w_layout);
@@ -509,25 +691,71 @@ extern "C" int coda_project_rows(const coda_proj_desc* d, void* stream) {
                                : run_project<float>(d, (hipStream_t)stream, "coda_project_rows");
 }
 
+extern "C" int coda_project_params(const coda_proj_desc* d, const coda_proj_params* p, void* stream) {
+  const char* who = "coda_project_params";
+  CODA_REQUIRE(d != nullptr && p != nullptr, "%s: null descriptor", who);
+  CODA_REQUIRE(d->dtype == CODA_BF16 || d->dtype == CODA_F32, "%s: dtype must be CODA_F32 or CODA_BF16", who);
+  CODA_REQUIRE(d->M >= 0 && d->M <= 128, "%s: %d token rows (at most 128)", who, d->M);
+  const int rc = check_project(d, who, false);
+  if (rc) return rc;
+  const size_t esz = d->dtype == CODA_BF16 ? 2 : 4;
+  for (int i = 0; i < (d->gate ? 5 : 4); ++i) {
+    CODA_REQUIRE(p->w[i] && p->w_sm[i] >= d->D, "%s: weight %d missing or its rows shorter than D", who, i);
+    CODA_REQUIRE((uintptr_t)p->w[i] % esz == 0 && (uintptr_t)p->b[i] % esz == 0, "%s: weight or bias %d off its type",
+                 who, i);
+  }
+  const auto angle = [](int t) { return t == CODA_F32 || t == CODA_BF16; };
+  CODA_REQUIRE(p->inv_freq ? p->rope_cos && p->rope_sin && angle(p->inv_dtype) && p->p0 >= 0 && p->p0 + d->L <= 1 << 24
+                           : d->rope_cos && d->rope_sin,
+               "%s: RoPE tables missing, or positions past 2^24", who);
+  CODA_REQUIRE(!p->theta || (p->theta_cos && p->theta_sin && angle(p->theta_dtype)), "%s: theta tables missing", who);
+  if (d->M == 0) return CODA_OK;
+  return d->dtype == CODA_BF16 ? run_project_params<bf16_t>(d, p, (hipStream_t)stream, who)
+                               : run_project_params<float>(d, p, (hipStream_t)stream, who);
+}
+
+static int check_linear(int dtype, const void* x, int64_t x_sm, int M, const void* w, int n_feat, int D, const void* out,
+                        int64_t o_sm, const char* who) {
+  CODA_REQUIRE(dtype == CODA_BF16 || dtype == CODA_F32, "%s: dtype must be CODA_F32 or CODA_BF16", who);
+  CODA_REQUIRE(M >= 0 && M <= 128 && n_feat > 0 && D > 0 && D % kProjKT == 0,
+               "%s: bad sizes M=%d n_feat=%d D=%d (at most 128 rows, D a multiple of %d)", who, M, n_feat, D, kProjKT);
+  CODA_REQUIRE(x && w && out, "%s: null pointer", who);
+  const int pc = dtype == CODA_BF16 ? 8 : 4;
+  CODA_REQUIRE(x_sm % pc == 0 && ((uintptr_t)x % 16) == 0, "%s: x / w rows must be 16-byte aligned", who);
+  CODA_REQUIRE(o_sm % 4 == 0 && ((uintptr_t)out % 8) == 0, "%s: out rows must be 8-byte aligned", who);
+  return CODA_OK;
+}
+template <typename T, typename BT, typename Src>
+static int run_linear(const Src& w, const void* x, int64_t x_sm, int M, int n_feat, int D, const void* bias, void* out,
+                      int64_t o_sm, void* stream, const char* who) {
+  return launch_rows<T>(w, n_feat, D, (const T*)x, x_sm, M,
+                        LinearEpilogue<T, BT>{(T*)out, (const BT*)bias, o_sm, n_feat}, (hipStream_t)stream, who);
+}
+
 extern "C" int coda_linear_rows(int dtype, const void* x, int64_t x_sm, int M, const void* w, int n_feat, int D,
                                 const float* bias, void* out, int64_t o_sm, void* stream) {
-  CODA_REQUIRE(dtype == CODA_BF16 || dtype == CODA_F32, "coda_linear_rows: dtype must be CODA_F32 or CODA_BF16");
-  CODA_REQUIRE(M >= 0 && M <= 128 && n_feat > 0 && D > 0 && D % kProjKT == 0,
-               "coda_linear_rows: bad sizes M=%d n_feat=%d D=%d (at most 128 rows, D a multiple of %d)", M, n_feat, D,
-               kProjKT);
-  CODA_REQUIRE(x && w && out, "coda_linear_rows: null pointer");
-  const int pc = dtype == CODA_BF16 ? 8 : 4;
-  CODA_REQUIRE(x_sm % pc == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0,
-               "coda_linear_rows: x / w rows must be 16-byte aligned");
-  CODA_REQUIRE(o_sm % 4 == 0 && ((uintptr_t)out % 8) == 0, "coda_linear_rows: out rows must be 8-byte aligned");
+  const char* who = "coda_linear_rows";
+  const int rc = check_linear(dtype, x, x_sm, M, w, n_feat, D, out, o_sm, who);
+  if (rc) return rc;
+  CODA_REQUIRE(((uintptr_t)w % 16) == 0, "%s: x / w rows must be 16-byte aligned", who);
   if (M == 0) return CODA_OK;
-  hipStream_t st = (hipStream_t)stream;
-  if (dtype == CODA_BF16)
-    return launch_rows_t<bf16_t, true>((const bf16_t*)w, D, n_feat, D, (const bf16_t*)x, x_sm, M,
-                                       LinearEpilogue<bf16_t>{(bf16_t*)out, bias, o_sm, n_feat}, st,
-                                       "coda_linear_rows");
-  return launch_rows_t<float, true>((const float*)w, D, n_feat, D, (const float*)x, x_sm, M,
-                                    LinearEpilogue<float>{(float*)out, bias, o_sm, n_feat}, st, "coda_linear_rows");
+  return dtype == CODA_BF16
+             ? run_linear<bf16_t, float>(TileRows<bf16_t>{(const bf16_t*)w}, x, x_sm, M, n_feat, D, bias, out, o_sm, stream, who)
+             : run_linear<float, float>(TileRows<float>{(const float*)w}, x, x_sm, M, n_feat, D, bias, out, o_sm, stream, who);
+}
+
+extern "C" int coda_linear_params(int dtype, const void* x, int64_t x_sm, int M, const void* w, int64_t w_sm, int n_feat,
+                                  int D, const void* bias, void* out, int64_t o_sm, void* stream) {
+  const char* who = "coda_linear_params";
+  const int rc = check_linear(dtype, x, x_sm, M, w, n_feat, D, out, o_sm, who);
+  if (rc) return rc;
+  const size_t esz = dtype == CODA_BF16 ? 2 : 4;
+  CODA_REQUIRE(w_sm >= D && (uintptr_t)w % esz == 0 && (uintptr_t)bias % esz == 0,
+               "%s: weight rows shorter than D, or off their type", who);
+  if (M == 0) return CODA_OK;
+  return dtype == CODA_BF16
+             ? run_linear<bf16_t, bf16_t>(MatRows<bf16_t>{(const bf16_t*)w, w_sm}, x, x_sm, M, n_feat, D, bias, out, o_sm, stream, who)
+             : run_linear<float, float>(MatRows<float>{(const float*)w, w_sm}, x, x_sm, M, n_feat, D, bias, out, o_sm, stream, who);
 }
 
 extern "C" int coda_rows_pack(int dtype, const void* w, int n_feat, int D, int64_t w_sm, void* out, void* stream) {

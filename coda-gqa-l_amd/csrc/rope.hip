@@ -96,9 +96,44 @@ __global__ __launch_bounds__(256) void rope_bf16_vec(bf16_t* __restrict__ out, i
   }
 }
 
+// cos / sin tables of positions p0 .. p0 + L - 1: one thread per entry.  In
+// place of the seven element-wise launches of the torch ops (20 us and 45 us
+// of host time a prompt); made for the call, so that no table outlives the
+// frequencies it came from, or a captured graph's use of it.
+template <typename T>
+__global__ __launch_bounds__(256) void rope_tables_kernel(const void* __restrict__ inv_freq, int inv_dtype, int64_t p0,
+                                                          int half, int64_t total, T* __restrict__ cos_t,
+                                                          T* __restrict__ sin_t) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= total) return;
+  const float2 a = rope_angle<T>(inv_freq, inv_dtype, p0 + i / half, (int)(i % half));
+  cos_t[i] = Elt<T>::st(a.x);
+  sin_t[i] = Elt<T>::st(a.y);
+}
+
 }  // namespace coda
 
 using namespace coda;
+
+extern "C" int coda_rope_tables(int dtype, const void* inv_freq, int inv_dtype, int64_t p0, int L, int half, void* cos_t,
+                                void* sin_t, void* stream) {
+  const auto ok = [](int t) { return t == CODA_F32 || t == CODA_BF16; };
+  CODA_REQUIRE(ok(dtype) && ok(inv_dtype), "coda_rope_tables: dtypes must be CODA_F32 or CODA_BF16");
+  CODA_REQUIRE(L >= 0 && half > 0 && p0 >= 0 && p0 + L <= 1 << 24, "coda_rope_tables: bad sizes p0=%lld L=%d half=%d",
+               (long long)p0, L, half);
+  if (L == 0) return CODA_OK;
+  CODA_REQUIRE(inv_freq && cos_t && sin_t, "coda_rope_tables: null pointer");
+  const int64_t total = (int64_t)L * half;
+  const dim3 grid((unsigned)((total + 255) / 256)), block(256);
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == CODA_F32)
+    hipLaunchKernelGGL(rope_tables_kernel<float>, grid, block, 0, st, inv_freq, inv_dtype, p0, half, total, (float*)cos_t,
+                       (float*)sin_t);
+  else
+    hipLaunchKernelGGL(rope_tables_kernel<bf16_t>, grid, block, 0, st, inv_freq, inv_dtype, p0, half, total,
+                       (bf16_t*)cos_t, (bf16_t*)sin_t);
+  return check_launch("rope_tables");
+}
 
 extern "C" int coda_rope_fwd(int dtype, void* out, int64_t o_sb, int64_t o_sh, int64_t o_sl, const void* x,
                              int64_t x_sb, int64_t x_sh, int64_t x_sl, const void* cos_t, const void* sin_t,

@@ -118,6 +118,33 @@ int coda_project(const coda_proj_desc* d, void* stream);
  * tiles (coda_rows_pack) for every D that is a multiple of 64. */
 int coda_project_rows(const coda_proj_desc* d, void* stream);
 
+/* The parameters of a layer where they lie: q, k, v, lambda and write-gate
+ * linears (the gate's unused with gate 0) in the descriptor's dtype, at any
+ * element address. */
+typedef struct {
+  const void* w[5];        /* (features, D), unit column stride */
+  int64_t w_sm[5];         /* row strides in elements, at least D */
+  const void* b[5];        /* (features) or NULL */
+  const void* inv_freq;    /* (Dh/2) RoPE frequencies, or NULL: the descriptor's tables */
+  int inv_dtype;           /* CODA_F32 or CODA_BF16 */
+  int64_t p0;              /* position of table row 0; p0 + L at most 2^24 */
+  void* rope_cos;          /* with inv_freq: written, (L, Dh/2) */
+  void* rope_sin;
+  const void* theta;       /* (H, Dh/2) noise angles, or NULL */
+  int theta_dtype;
+  void* theta_cos;         /* with theta: written, (H, Dh/2) */
+  void* theta_sin;
+} coda_proj_params;
+
+/* coda_project_rows on the parameters themselves: no packed copy stands
+ * between the call and a parameter, so an edit of one, by whatever means, is
+ * seen by the next call, and a captured graph reads what the module holds.
+ * With inv_freq / theta the launch makes those tables too (as the torch ops
+ * do: products, cos and sin in the angles' type, then the dtype), and leaves
+ * them for the attention that follows.  The descriptor's w, bias, w_layout
+ * are unused. */
+int coda_project_params(const coda_proj_desc* d, const coda_proj_params* p, void* stream);
+
 /* out (M, n_feat; row stride o_sm) = x (M, D; row stride x_sm) W^T + bias
  * for M <= 128 token rows: fp32 accumulation, one rounding.  w: the (n_feat,
  * D) weights in fragment tiles (coda_rows_pack); bias: (n_feat) float32 or
@@ -125,6 +152,11 @@ int coda_project_rows(const coda_proj_desc* d, void* stream);
  * Replaces: o_proj of CoDAGQALandmarkPerf2.step (attention.py:538). */
 int coda_linear_rows(int dtype, const void* x, int64_t x_sm, int M, const void* w, int n_feat, int D,
                      const float* bias, void* out, int64_t o_sm, void* stream);
+
+/* The same on a linear's own weight (n_feat, D; row stride w_sm) and bias
+ * (n_feat, in dtype, or NULL), at any element address. */
+int coda_linear_params(int dtype, const void* x, int64_t x_sm, int M, const void* w, int64_t w_sm, int n_feat, int D,
+                       const void* bias, void* out, int64_t o_sm, void* stream);
 
 /* The weights of coda_project in fragment tiles (w_layout 1): for row block
  * fb of 16 rows and k-step ks of 32 columns, a 1 KiB tile at element offset
@@ -308,6 +340,13 @@ int coda_rope_fwd(int dtype, void* out, int64_t o_sb, int64_t o_sh, int64_t o_sl
                   const void* x, int64_t x_sb, int64_t x_sh, int64_t x_sl,
                   const void* cos_t, const void* sin_t, int B, int Hx, int L, int Dh,
                   int interleaved, void* stream);
+
+/* RoPE tables (L, half) of positions p0 .. p0 + L - 1 (p0 + L at most 2^24)
+ * in dtype from inv_freq (half): products, cos and sin in inv_dtype, as the
+ * torch ops take them.
+ * Replaces: RotaryEmbedding.forward (src/coda_gqa_l/primitives.py:44-55). */
+int coda_rope_tables(int dtype, const void* inv_freq, int inv_dtype, int64_t p0, int L, int half, void* cos_t,
+                     void* sin_t, void* stream);
 
 /* ------------------------------------------------------------------------
  * Bounded-cache state (CoDAGQALandmarkStatePerf2, src/coda_gqa_l/state.py:24-54)
