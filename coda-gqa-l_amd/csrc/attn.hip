@@ -2794,15 +2794,17 @@ static int rows_nsplit(const coda_attn_desc* d) {
 // attn_f32's launch: 16-row query tiles; 8 waves a workgroup where the tiles
 // fill the CUs at most twice, and the keys over several workgroups where they
 // leave CUs idle, each with at least four tiles a wave (a decode token over
-// 384 keys: two workgroups a head and the merge 8.9 + 4.1 us, one launch 9 us)
+// 384 keys: two workgroups a head and the merge 8.9 + 4.1 us, one launch 9 us).
+// chunks > 0: a grouped launch, of however many chunks, keeps each chunk's keys
+// in one workgroup (the merge sees one descriptor, not each chunk's own rows)
 struct F32Shape {
   int qt, ntile, nw, nsplit, per;
 };
-static F32Shape f32_shape(const coda_attn_desc* d, int cus, int chunks = 1) {
+static F32Shape f32_shape(const coda_attn_desc* d, int cus, int chunks = 0) {
   F32Shape f;
   f.qt = std::max(1, 8 / (d->H / d->Hkv));
   f.ntile = (d->Lq + f.qt - 1) / f.qt;
-  const int64_t wgs = (int64_t)f.ntile * d->Hkv * d->B * chunks;
+  const int64_t wgs = (int64_t)f.ntile * d->Hkv * d->B * std::max(chunks, 1);
   const int Lk = d->Lp + d->Lb;
   f.nw = wgs <= 2 * cus ? 8 : 4;
   const int64_t want = wgs > 0 ? std::min<int64_t>(std::min<int64_t>(cus / wgs, Lk / (64 * f.nw)),
@@ -2810,7 +2812,7 @@ static F32Shape f32_shape(const coda_attn_desc* d, int cus, int chunks = 1) {
   f.per = ((Lk + (int)std::max<int64_t>(want, 1) - 1) / (int)std::max<int64_t>(want, 1) + 15) / 16 * 16;
   f.per = std::max(f.per, 16);
   f.nsplit = std::max(1, (Lk + f.per - 1) / f.per);
-  if (chunks > 1) {  // (each chunk has keys of its own)
+  if (chunks > 0) {
     f.nsplit = 1;
     f.per = std::max(Lk, 16);
   }
@@ -2949,7 +2951,7 @@ static int launch_merge(const coda_attn_desc* d, hipStream_t st, int qt, int nti
 template <int DH>
 static int launch_f32(const coda_attn_desc* d, hipStream_t st, const ChunkGeom& cg) {
   const int n = cg.n > 0 ? cg.n : 1;
-  F32Shape f = f32_shape(d, device_cus(), n);
+  const F32Shape f = f32_shape(d, device_cus(), cg.n);
   if (f.nsplit > 1) {
     const size_t need = (size_t)d->B * d->Hkv * f.ntile * f.nsplit * 16 * (DH + 2) * sizeof(float);
     if (!d->workspace || d->workspace_bytes < need)
