@@ -2951,11 +2951,12 @@ static int launch_merge(const coda_attn_desc* d, hipStream_t st, int qt, int nti
 template <int DH>
 static int launch_f32(const coda_attn_desc* d, hipStream_t st, const ChunkGeom& cg) {
   const int n = cg.n > 0 ? cg.n : 1;
-  const F32Shape f = f32_shape(d, device_cus(), cg.n);
-  if (f.nsplit > 1) {
-    const size_t need = (size_t)d->B * d->Hkv * f.ntile * f.nsplit * 16 * (DH + 2) * sizeof(float);
-    if (!d->workspace || d->workspace_bytes < need)
-      return fail(CODA_ESMALL, "coda_diff_attn_fwd: workspace %zu < %zu bytes", d->workspace_bytes, need);
+  F32Shape f = f32_shape(d, device_cus(), cg.n);
+  // (a caller's workspace too small for the splits: one launch)
+  if (f.nsplit > 1 && (!d->workspace || (uintptr_t)d->workspace % 4 ||
+                       d->workspace_bytes < (size_t)d->B * d->Hkv * f.ntile * f.nsplit * 16 * (DH + 2) * sizeof(float))) {
+    f.nsplit = 1;
+    f.per = std::max((d->Lp + d->Lb + 15) / 16 * 16, 16);
   }
   const size_t lds = (size_t)f.nw * 16 * (DH + 4) * sizeof(float);
   const dim3 grid(f.ntile * f.nsplit, d->Hkv, d->B * n);
