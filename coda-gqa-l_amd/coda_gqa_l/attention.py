@@ -459,7 +459,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         pvers = self._param_key()
         B = x.shape[0]
         if fp is None or fp["st"] is not st or fp["vers"] != vers or fp["pvers"] != pvers or fp["B"] != B or \
-                fp["packed"] != packed or \
+                fp["packed"] != packed or fp["dtype"] is not x.dtype or \
                 fp["ptrs"] != tuple(-1 if t is None else t.data_ptr() for t in ts) or fp["dev"] != x.device:
             fp = self._build_step_fast(x, st, ts, vers, pvers, packed)
             if fp is None:
@@ -567,7 +567,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         L_ = _hip.lib()
         routed = ctypes.c_int(0)
 
-        fp = {"st": st, "vers": vers, "pvers": pvers, "B": B, "dev": dev, "packed": packed, "rows": None,
+        fp = {"st": st, "vers": vers, "pvers": pvers, "B": B, "dev": dev, "dtype": dt, "packed": packed, "rows": None,
               "ptrs": tuple(-1 if t is None else t.data_ptr() for t in ts),
               "tab": (cos_t, sin_t), "row_bytes": (Dh // 2) * cos_t.element_size(),
               "proj": d, "proj_ref": ctypes.byref(d), "attn": a, "attn_ref": ctypes.byref(a),
