@@ -31,7 +31,7 @@ import torch.nn as nn
 from . import _hip, ops
 from .memory_banks import METRIC_KEYS, DeviceMetrics, MemoryBankMixin
 from .primitives import HeadwiseRMSNorm, RotaryEmbedding, apply_rope
-from .rows import RowsMixin
+from .rows import RowsMixin, _aligned
 from .state import CoDAGQALandmarkStatePerf2
 
 __all__ = ["CoDAGQALandmarkPerf2", "CoDAGQALandmarkStatePerf2"]
@@ -312,7 +312,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
             d = self._proj_desc(x, M, L, cos, sin)
             g = torch.empty((B, L), dtype=torch.float32, device=x.device)
             d.g = g.data_ptr()
-            xs = x if (x.is_contiguous() and x.data_ptr() % 16 == 0) else x.contiguous()
+            xs = _aligned(x)
             q = torch.empty((B, L, Fq), dtype=x.dtype, device=x.device)
             k = torch.empty((B, L, Hkv, Dh), dtype=x.dtype, device=x.device)
             v = torch.empty((B, L, Fk), dtype=x.dtype, device=x.device)
@@ -464,8 +464,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
             fp = self._build_step_fast(x, st, ts, vers, pvers, packed)
             if fp is None:
                 return None
-        if not (x.is_contiguous() and x.data_ptr() % 16 == 0):
-            x = x.contiguous()
+        x = _aligned(x)
         pos = int(st.pos)
         d, a = fp["proj"], fp["attn"]
         d.x = x.data_ptr()

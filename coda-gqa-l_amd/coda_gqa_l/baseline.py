@@ -18,7 +18,7 @@ import torch.nn as nn
 
 from . import _hip, ops
 from .primitives import HeadwiseRMSNorm, RotaryEmbedding, apply_rope
-from .rows import RowsMixin
+from .rows import RowsMixin, _aligned
 
 
 class CoDAGQA(RowsMixin, nn.Module):
@@ -133,7 +133,7 @@ class CoDAGQA(RowsMixin, nn.Module):
         H, Hkv, Dh = self.num_heads, self.num_kv_heads, self.head_dim
         past, M, e, half = k_past.shape[2], B * L, x.element_size(), Dh // 2
         lib, stream, dev = _hip.lib(), _hip.stream_of(x), x.device
-        xs = x if x.is_contiguous() and x.data_ptr() % 16 == 0 else x.contiguous()
+        xs = _aligned(x)
         w = self.head_norm.weight.detach().to(x.dtype).contiguous() if self.head_norm_mode == "full" else None
         a = _hip.AttnDesc()
         a.dtype = _hip.dtype_code(x.dtype)

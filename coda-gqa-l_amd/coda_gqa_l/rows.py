@@ -36,6 +36,12 @@ class _Made:
                 t.record_stream(cur)
 
 
+def _aligned(x: torch.Tensor) -> torch.Tensor:
+    """x, or a copy of it where the row kernels can't read it in place
+    (contiguous() returns a contiguous x off a 16-byte address as it is)."""
+    return x if x.is_contiguous() and x.data_ptr() % 16 == 0 else x.clone(memory_format=torch.contiguous_format)
+
+
 class RowsMixin:
     """Needs q_proj, k_proj, v_proj, lambda_proj, o_proj, rope, num_heads,
     num_kv_heads, head_dim, embed_dim and rope_interleaved; a write gate where
