@@ -307,8 +307,9 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
                     "take the torch linears: a many-row fused form (an in-place epilogue over a library GEMM, "
                     "q / k / v / lambda as strided views of its output) faulted the GPU in a full-size run with no "
                     "cause shown, and was removed")
-            rows = None if self._packed_front_ok(x) else self._front_rows(x)
-            cos, sin = (self._rope_rows if rows is None else self._rope_tables)(p0, L, x.device, x.dtype)
+            capturing = torch.cuda.is_current_stream_capturing()
+            rows = None if self._packed_front_ok(x) and not capturing else self._front_rows(x)
+            cos, sin = (self._rope_rows if rows is None and not capturing else self._rope_tables)(p0, L, x.device, x.dtype)
             d = self._proj_desc(x, M, L, cos, sin)
             g = torch.empty((B, L), dtype=torch.float32, device=x.device)
             d.g = g.data_ptr()
@@ -441,11 +442,12 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         RoPE-row pointers (packed weights) or the parameters' own addresses
         and the position (few-row inputs that those don't serve), makes two
         library calls (the projections, then coda_decode_step on their
-        outputs) and o_proj.  Returns None when the general path must run;
-        the cache is rebuilt whenever a parameter, the state's tensors
+        outputs) and o_proj.  Returns None when the general path must run
+        (under capture too: a graph reads no buffer of the cache); it is rebuilt whenever a parameter, the state's tensors
         (object, storage or in-place version) or the batch changes."""
         if st.metrics is not None or st.recent_filled < self.window or \
-                self._expandable() or (self.Me == 0 and self.Ms == 0) or self._tracing():
+                self._expandable() or (self.Me == 0 and self.Ms == 0) or self._tracing() or \
+                torch.cuda.is_current_stream_capturing():
             return None
         packed, rows, angles = self._packed_front_ok(x), None, None
         if not packed:

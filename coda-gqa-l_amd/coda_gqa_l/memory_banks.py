@@ -481,7 +481,7 @@ class MemoryBankMixin:
                     "ws": ws, "ws_ptr": _hip.ptr(ws), "ws_bytes": nb.value, "routed": ctypes.c_int(0),
                     "fn": _hip.lib().coda_decode_step, "fn_raw_k": _hip.lib().coda_decode_step_raw_k}
             self.__dict__["_dplan"] = plan
-        a = plan["attn"]
+        a = self._handed(plan)["attn"]
         a.q = q.data_ptr()
         a.q_sb, a.q_sh, a.q_sl = q.stride()[:3]
         a.rope_cos, a.rope_sin = rope_cos.data_ptr(), rope_sin.data_ptr()
@@ -527,7 +527,7 @@ class MemoryBankMixin:
         if buf is None or buf.numel() < nbytes:
             buf = torch.empty(max(nbytes, 1 << 16), dtype=torch.uint8, device=device)
             cache[key] = buf
-        return buf
+        return self._handed(buf)
 
     def _workspace(self, device, nbytes: int) -> Optional[torch.Tensor]:
         """Device scratch reused across calls (grown on demand); calls on one

@@ -58,16 +58,28 @@ class RowsMixin:
         tag = (src._version, src.data_ptr(), src.dtype, src.device)
         hit = cache.get((name, key))
         if hit is not None and hit[0] == tag:
-            return hit[1]
+            return self._handed(hit[1])
         with torch.no_grad():
             val = fn()
-        cache[(name, key)] = (tag, val)
+        if not torch.cuda.is_current_stream_capturing():
+            cache[(name, key)] = (tag, val)
+        return val
+
+    def _handed(self, val):
+        """val, a tensor or several kept across calls, on its way to a caller:
+        under capture it stays alive with the layer (a graph goes on reading
+        it when the layer has replaced it).  What is made under capture is not
+        kept at all: nothing has run yet."""
+        if torch.cuda.is_current_stream_capturing():
+            held = self.__dict__.setdefault("_graph_held", {})
+            held[id(val)] = val
         return val
 
     def _rope_rows(self, p0: int, L: int, device, dtype: torch.dtype) -> Tuple[torch.Tensor, torch.Tensor]:
         """RoPE tables (L, Dh/2) of positions p0 .. p0 + L - 1: rows of one
         cached table, grown by doubling; every element is the same fp32
-        product and cos / sin as in a table made for these positions alone."""
+        product and cos / sin as in a table made for these positions alone.
+        (Not under capture: a larger table replaces and frees it.)"""
         cache = self.__dict__.setdefault("_rope_cache", {})
         made = self.__dict__.setdefault("_rope_made", {})
         key = (torch.device(device), dtype)
@@ -119,7 +131,7 @@ class RowsMixin:
             made = self.__dict__.get("_proj_made", {}).get(dtype)
             if made is not None:
                 made.use()
-            return hit[1]
+            return self._handed(hit[1])
         H, Hkv, Dh = self.num_heads, self.num_kv_heads, self.head_dim
         with torch.no_grad():
             dev = self.q_proj.weight.device
@@ -144,6 +156,8 @@ class RowsMixin:
             else:
                 w, layout = torch.cat(ws).contiguous(), 0
         val = (w, b.contiguous(), layout)
+        if w.is_cuda and torch.cuda.is_current_stream_capturing():
+            return val
         cache[("proj", dtype)] = (tag, val)
         if w.is_cuda:
             self.__dict__.setdefault("_proj_made", {})[dtype] = _Made(*val[:2])
