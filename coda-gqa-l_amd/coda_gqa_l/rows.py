@@ -42,10 +42,23 @@ def _aligned(x: torch.Tensor) -> torch.Tensor:
     return x if x.is_contiguous() and x.data_ptr() % 16 == 0 else x.clone(memory_format=torch.contiguous_format)
 
 
+# What a layer keeps between calls: copies derived from parameters; and
+# workspaces, plans and buffers
+_PARAM_COPIES = ("_derived_cache", "_rope_cache", "_rope_made", "_proj_made", "_fast", "_dplan")
+_KEPT = _PARAM_COPIES + ("_graph_held", "_step_ws_bytes", "_route_ws", "_route_tag", "_ws_cache", "_block_ws",
+                         "_block_checked", "_status_pending", "_snap_cache", "_last_chunk_group")
+
+
 class RowsMixin:
     """Needs q_proj, k_proj, v_proj, lambda_proj, o_proj, rope, num_heads,
     num_kv_heads, head_dim, embed_dim and rope_interleaved; a write gate where
     _has_gate() says so."""
+
+    def __getstate__(self) -> dict:
+        """For copies and saves of the layer: without what it keeps between
+        calls (events and descriptors that can't travel, addresses that would
+        name the original's memory)."""
+        return {k: v for k, v in self.__dict__.items() if k not in _KEPT}
 
     def _has_gate(self) -> bool:
         return getattr(self, "write_policy", "none") != "none"
