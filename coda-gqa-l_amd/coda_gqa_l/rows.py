@@ -36,6 +36,14 @@ class _Made:
                 t.record_stream(cur)
 
 
+def _version(t: torch.Tensor) -> Optional[int]:
+    """t's in-place version; None for an inference tensor, which counts none."""
+    try:
+        return t._version
+    except RuntimeError:
+        return None
+
+
 def _aligned(x: torch.Tensor) -> torch.Tensor:
     """x, or a copy of it where the row kernels can't read it in place
     (contiguous() returns a contiguous x off a 16-byte address as it is)."""
@@ -101,11 +109,11 @@ class RowsMixin:
         inv = self.rope.inv_freq
         hit = made.get(key)
         if tab is None or tab[0].shape[0] < need or hit is None or hit[0] is not inv or \
-                hit[1] != (inv._version, inv.data_ptr()):
+                hit[1] != (_version(inv), inv.data_ptr()):
             n = 1 << max(12, (need - 1).bit_length())
             c, s_ = self.rope(seq_len=n, offset=0, device=device, dtype=dtype)
             tab = cache[key] = (c.contiguous(), s_.contiguous())
-            made[key] = (inv, (inv._version, inv.data_ptr()), _Made(*tab) if tab[0].is_cuda else None)
+            made[key] = (inv, (_version(inv), inv.data_ptr()), _Made(*tab) if tab[0].is_cuda else None)
         elif hit[2] is not None:
             hit[2].use()
         return tab[0][p0:need], tab[1][p0:need]

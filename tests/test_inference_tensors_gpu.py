@@ -40,7 +40,7 @@ def test_bounded_moved_inside(B, dtype):
     m, n = make(), make().to(DEV, dtype).eval()
     with torch.inference_mode():
         m = m.to(DEV, dtype).eval()
-    print([k for k, t in (*m.named_parameters(), *m.named_buffers()) if t.is_inference()])
+    assert m.rope.inv_freq.is_inference()
     x = torch.randn(B, 60, 256, generator=torch.Generator(device=DEV).manual_seed(1), device=DEV).to(dtype)
     with torch.no_grad():
         out = []
@@ -48,6 +48,8 @@ def test_bounded_moved_inside(B, dtype):
             torch.manual_seed(9)
             st = layer.init_state(batch_size=B, device=DEV, dtype=dtype)
             ys = [layer.prefill_chunked(x[:, :50], st, block_size=16)[0]]
-            out.append(ys + [layer.step(x[:, 50 + t:51 + t], st)[0] for t in range(3)] + [st.k_buf, st.v_buf])
+            out.append(ys + [layer.step(x[:, 50 + t:51 + t], st)[0].clone() for t in range(3)] + [st.k_buf, st.v_buf])
+        # (torch takes another GEMM for such weights: sums in another order)
+        tol = 1e-5 if dtype == torch.float32 else 2e-2
         for a, b in zip(*out):
-            assert torch.equal(a, b)
+            assert float((a.float() - b.float()).abs().max()) <= tol * float(b.float().abs().max())
