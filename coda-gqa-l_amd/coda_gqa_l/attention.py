@@ -31,7 +31,7 @@ import torch.nn as nn
 from . import _hip, ops
 from .memory_banks import METRIC_KEYS, DeviceMetrics, MemoryBankMixin
 from .primitives import HeadwiseRMSNorm, RotaryEmbedding, apply_rope
-from .rows import RowsMixin, _aligned
+from .rows import RowsMixin, _aligned, _capturing
 from .state import CoDAGQALandmarkStatePerf2
 
 __all__ = ["CoDAGQALandmarkPerf2", "CoDAGQALandmarkStatePerf2"]
@@ -307,7 +307,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
                     "take the torch linears: a many-row fused form (an in-place epilogue over a library GEMM, "
                     "q / k / v / lambda as strided views of its output) faulted the GPU in a full-size run with no "
                     "cause shown, and was removed")
-            capturing = torch.cuda.is_current_stream_capturing()
+            capturing = _capturing()
             rows = None if self._packed_front_ok(x) and not capturing else self._front_rows(x)
             cos, sin = (self._rope_rows if rows is None and not capturing else self._rope_tables)(p0, L, x.device, x.dtype)
             d = self._proj_desc(x, M, L, cos, sin)
@@ -322,7 +322,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
             d.q, d.q_sm, d.k, d.k_sm, d.v, d.v_sm = q.data_ptr(), Fq, k.data_ptr(), Fk, v.data_ptr(), Fk
             d.lam, d.lam_sm = lam.data_ptr(), H
             if rows is None:
-                w, b, d.w_layout = self._proj_pack(x.dtype)
+                w, b, d.w_layout = self._packed_weights(x)
                 d.w, d.bias = w.data_ptr(), b.data_ptr()
                 _hip.check(_hip.lib().coda_project_rows(d, _hip.stream_of(x)))
             else:
@@ -447,7 +447,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         (object, storage or in-place version) or the batch changes."""
         if st.metrics is not None or st.recent_filled < self.window or \
                 self._expandable() or (self.Me == 0 and self.Ms == 0) or self._tracing() or \
-                torch.cuda.is_current_stream_capturing():
+                _capturing():
             return None
         packed, rows, angles = self._packed_front_ok(x), None, None
         if not packed:
@@ -545,7 +545,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
             row = slice(0, 1)
         d = self._proj_desc(x, B, 1, cos_t, sin_t)
         if packed:
-            w, b, d.w_layout = self._proj_pack(dt)
+            w, b, d.w_layout = self._packed_weights(x)
             d.w, d.bias = w.data_ptr(), b.data_ptr()
         d.x_sm = D
         d.q, d.q_sm, d.k, d.k_sm, d.v, d.v_sm = q.data_ptr(), Fq, k.data_ptr(), Fk, v.data_ptr(), Fk

@@ -22,7 +22,7 @@ class _Made:
     def __init__(self, *tensors: torch.Tensor):
         self.tensors = tensors
         self.stream, self.event = _hip.stream_of(tensors[0]), None
-        if not torch.cuda.is_current_stream_capturing():
+        if not _capturing():
             self.event = torch.cuda.Event()
             self.event.record(torch.cuda.current_stream(tensors[0].device))
 
@@ -30,10 +30,14 @@ class _Made:
         if self.event is None:
             return
         cur = torch.cuda.current_stream(self.tensors[0].device)
-        if cur.cuda_stream != self.stream and not torch.cuda.is_current_stream_capturing():
+        if cur.cuda_stream != self.stream and not _capturing():
             cur.wait_event(self.event)
             for t in self.tensors:
                 t.record_stream(cur)
+
+
+def _capturing() -> bool:
+    return torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing()
 
 
 def _version(t: torch.Tensor) -> Optional[int]:
@@ -82,7 +86,7 @@ class RowsMixin:
             return self._handed(hit[1])
         with torch.no_grad():
             val = fn()
-        if not torch.cuda.is_current_stream_capturing():
+        if not _capturing():
             cache[(name, key)] = (tag, val)
         return val
 
@@ -91,7 +95,7 @@ class RowsMixin:
         under capture it stays alive with the layer (a graph goes on reading
         it when the layer has replaced it).  What is made under capture is not
         kept at all: nothing has run yet."""
-        if torch.cuda.is_current_stream_capturing():
+        if _capturing():
             held = self.__dict__.setdefault("_graph_held", {})
             held[id(val)] = val
         return val
@@ -164,10 +168,15 @@ class RowsMixin:
                 wk = wk[perm]
                 bk = bk[perm] if bk is not None else None
             ws = [self.q_proj.weight, wk, self.v_proj.weight, self.lambda_proj.weight]
+            sizes = [H * Dh, Hkv * Dh, Hkv * Dh, H]
             bt = [self.q_proj.bias, bk, self.v_proj.bias, self.lambda_proj.bias]
             if gate:
                 ws.append(self.write_proj.weight)
                 bt.append(self.write_proj.bias)
+                sizes.append(1)
+            for t, u, n in zip(ws, bt, sizes):
+                if tuple(t.shape) != (n, self.embed_dim) or u is not None and tuple(u.shape) != (n,):
+                    raise RuntimeError(f"projection weight {tuple(t.shape)} is not ({n}, {self.embed_dim})")
             b = torch.cat([t.detach().float() if t is not None else torch.zeros(wt.shape[0], device=dev)
                            for t, wt in zip(bt, ws)])
             b = torch.cat([b, torch.zeros((-b.numel()) % 4, device=dev)])
@@ -177,11 +186,18 @@ class RowsMixin:
             else:
                 w, layout = torch.cat(ws).contiguous(), 0
         val = (w, b.contiguous(), layout)
-        if w.is_cuda and torch.cuda.is_current_stream_capturing():
+        if w.is_cuda and _capturing():
             return val
         cache[("proj", dtype)] = (tag, val)
         if w.is_cuda:
             self.__dict__.setdefault("_proj_made", {})[dtype] = _Made(*val[:2])
+        return val
+
+    def _packed_weights(self, x: torch.Tensor):
+        """_proj_pack for x's projections: the kernel reads x's device alone."""
+        val = self._proj_pack(x.dtype)
+        if val[0].device != x.device:
+            raise RuntimeError(f"projection weights on {val[0].device}, input on {x.device}")
         return val
 
     @staticmethod
