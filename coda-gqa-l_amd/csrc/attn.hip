@@ -646,7 +646,7 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // then m [R], l [R]; row st * GL + orow of a tile of qt queries, GL = G * qt,
 // orow = g * qt + query.  FLASH: the epilogue of attn_f3_bf16 (fp32, the noise
 // output rounded once) instead of the eager ops' rounding.
-static constexpr int kMaxSplits = 512, kFewSplits = 64;
+static constexpr int kMaxSplits = 512;
 template <typename T, int DH, bool FLASH>
 __device__ __forceinline__ void merge_store(const coda_attn_desc& a, int b, int h, int qi, int lane,
                                             const float (&os)[(DH + 63) / 64], const float (&on)[(DH + 63) / 64]) {
@@ -682,10 +682,10 @@ __device__ __forceinline__ void merge_store(const coda_attn_desc& a, int b, int 
     if (act[i]) orow_p[dd[i]] = E::st(y[i]);
 }
 
-// At most kFewSplits splits: a wave per output row, four rows a workgroup, a
-// lane per split for the weights, no barrier.  Two dependent round trips and
-// the partials' bytes (a workgroup a row and its barriers: 18 us for 8192
-// rows of two splits, about 8 here).
+// Few splits (at most 64) of many rows: a wave per output row, four rows a
+// workgroup, a lane per split for the weights, no barrier.  Two dependent round
+// trips, the walk over the splits and the partials' bytes (a workgroup a row
+// and its barriers: 18 us for 8192 rows of two splits, about 8 here).
 template <typename T, int DH, bool FLASH>
 __global__ __launch_bounds__(256) void attn_merge_few(const coda_attn_desc a, int qt, int R, int nsplit, const float* ws) {
   constexpr int NV = (DH + 63) / 64;
@@ -720,9 +720,9 @@ __global__ __launch_bounds__(256) void attn_merge_few(const coda_attn_desc a, in
   merge_store<T, DH, FLASH>(a, b, hk * G + g, qi, lane, o[0], o[1]);
 }
 
-// More splits (few query rows over very many keys): a workgroup per output
-// row, its two streams' maxima and sums over the splits on 128 threads each,
-// then 256 / DH groups of threads sum the splits' channels.
+// More splits (few query rows over many keys): a workgroup per output row,
+// its two streams' maxima and sums over the splits on 128 threads each, then
+// 256 / DH groups of threads sum the splits' channels.
 template <typename T, int DH>
 __global__ __launch_bounds__(256) void attn_merge(const coda_attn_desc a, int qt, int R, int nsplit, const float* ws) {
   constexpr int NG = 256 / DH, NV = (DH + 63) / 64;
@@ -2941,9 +2941,16 @@ static int launch_f3(const coda_attn_desc* d, hipStream_t st, int G, const Chunk
   if (d->q_noise && !d->rope_cos) return launch_f3_qm<DH, 2, false>(d, st, G, cg);
   return launch_f3_qm<DH, 3, false>(d, st, G, cg);
 }
+// A wave a row walks the splits one after the other, a workgroup a row pays
+// its barriers: attention and merge of 4096 keys, 8 KV heads of 128, 1 query of
+// 4 heads each, with the two: 64 splits of 32 rows 41.2 and 17.7 us, 16 of
+// 128 28.6 and 22.0, 8 of 256 33.9 and 30.8, 4 of 512 52.1 and 51.3, 2 of 1024
+// 104.9 and 105.1; 3 splits of 1920 rows 51.3 and 52.0.  (Four splits or more
+// means few rows: keys are split where rows leave the chip idle.)
+static constexpr int kWalkSplits = 3;
 template <typename T, int DH>
 static int launch_merge(const coda_attn_desc* d, hipStream_t st, int qt, int ntile, int nsplit) {
-  if (nsplit <= kFewSplits) return launch_merge_few<T, DH, false>(d, st, qt, 16, nsplit);
+  if (nsplit <= kWalkSplits) return launch_merge_few<T, DH, false>(d, st, qt, 16, nsplit);
   hipLaunchKernelGGL((attn_merge<T, DH>), dim3(ntile * (d->H / d->Hkv) * qt, d->Hkv * d->B), dim3(256), 0, st, *d, qt, 16,
                      nsplit, (const float*)d->workspace);
   return check_launch("attn_merge");
