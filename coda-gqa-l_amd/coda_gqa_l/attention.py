@@ -700,8 +700,8 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         Hkv, W, S = self.num_kv_heads, self.window, self.Me + self.Ms
         blk = int(block_size)
         n_chunks = -(-L // blk)
-        # snapshot buffers of up to 256 MiB (at most 1024 chunks), made once
-        # per shape and kept: calls of any length reuse them
+        # snapshot buffers for the largest group so far, of up to 256 MiB (at
+        # most 1024 chunks), kept per shape
         per_chunk = 2 * B * Hkv * S * Dh * q.element_size()
         cap = max(1, min(1024, 65535 // max(B, 1), (256 << 20) // max(per_chunk, 1)))
         if self.pipelined_group_chunks is not None:
@@ -710,11 +710,11 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         cache = self.__dict__.setdefault("_snap_cache", {})
         key = (str(q.device), q.dtype, B, Hkv, S, Dh)
         buf = cache.get(key)
-        if buf is None or buf[0].shape[0] != cap:
-            buf = cache[key] = (torch.empty((cap, B, Hkv, S, Dh), dtype=q.dtype, device=q.device),
-                                torch.empty((cap, B, Hkv, S, Dh), dtype=q.dtype, device=q.device),
-                                torch.empty((cap, B, S), dtype=torch.uint8, device=q.device))
-        sk, sv, sa = buf
+        if buf is None or buf[0].shape[0] < group:
+            buf = cache[key] = (torch.empty((group, B, Hkv, S, Dh), dtype=q.dtype, device=q.device),
+                                torch.empty((group, B, Hkv, S, Dh), dtype=q.dtype, device=q.device),
+                                torch.empty((group, B, S), dtype=torch.uint8, device=q.device))
+        sk, sv, sa = self._handed(buf)
         # chunks that evict run as one chain call when no metrics, flags or
         # traces are collected per chunk
         chain = (state.metrics is None and not (self._expandable() and not self.training) and
