@@ -72,6 +72,17 @@ class RowsMixin:
         name the original's memory)."""
         return {k: v for k, v in self.__dict__.items() if k not in _KEPT}
 
+    def drop_parameter_copies(self) -> None:
+        """Forget everything derived from parameters: for after a change of
+        one that torch does not count (through .data, or from outside torch).
+        Counted changes need no such call.  Prompts, unbounded layers, o_proj,
+        fp32 steps and steps of more than 64 rows read the projections' own
+        values in any case; kept are the packed q / k / v / lambda / gate
+        weights and RoPE rows of bf16 steps of up to 64 rows, and a bounded
+        layer's noise angles, head norm weight and summary rates."""
+        for k in _PARAM_COPIES:
+            self.__dict__.pop(k, None)
+
     def _has_gate(self) -> bool:
         return getattr(self, "write_policy", "none") != "none"
 

@@ -79,3 +79,28 @@ def test_bounded_step(B, dtype, every, steady):
         assert torch.equal(a, b) and st.pos == before + 1
         for f in ("k_buf", "v_buf", "g_recent", "allowed", "mem_last_exact"):
             assert torch.equal(getattr(st, f), getattr(st2, f)), f
+
+
+@pytest.mark.parametrize("B,dtype", [(2, torch.bfloat16), (70, torch.bfloat16), (2, torch.float32)])
+@torch.no_grad()
+def test_dropped_copies(B, dtype):
+    """Every parameter and buffer of a bounded layer changed through .data,
+    then drop_parameter_copies()."""
+    def make():
+        return coda_gqa_l.CoDAGQALandmarkPerf2(embed_dim=256, num_heads=4, num_kv_heads=2, window=16, num_landmarks_exact=8,
+                                               num_landmarks_summary=8).to(DEV, dtype).eval()
+
+    torch.manual_seed(2)
+    m, g = make(), torch.Generator(device=DEV).manual_seed(4)
+    st = m.init_state(batch_size=B, device=DEV, dtype=dtype)
+    xs = torch.randn(B, 60, 256, generator=g, device=DEV).to(dtype)
+    m.prefill_chunked(xs[:, :50], st, block_size=16, return_outputs=False)
+    m.step(xs[:, 50:51], st)
+    m.step(xs[:, 51:52], st)
+    _edit([*m.parameters(), *m.buffers()], g)
+    m.drop_parameter_copies()
+    n, st2 = _given(make, _values(m)), state_io.deep_copy_state(st)
+    for part in (xs[:, 52:53], xs[:, 53:54]):
+        assert torch.equal(m.step(part, st)[0], n.step(part, st2)[0])
+    assert torch.equal(m.prefill_chunked(xs[:, :30], st, block_size=16)[0], n.prefill_chunked(xs[:, :30], st2, block_size=16)[0])
+    assert torch.equal(st.k_buf, st2.k_buf) and torch.equal(st.v_buf, st2.v_buf)
