@@ -443,8 +443,10 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         and the position (few-row inputs that those don't serve), makes two
         library calls (the projections, then coda_decode_step on their
         outputs) and o_proj.  Returns None when the general path must run
-        (under capture too: a graph reads no buffer of the cache); it is rebuilt whenever a parameter, the state's tensors
-        (object, storage or in-place version) or the batch changes."""
+        (under capture too: a graph reads no buffer of the cache); the
+        cache is rebuilt whenever a parameter, the state's tensors (object, storage or in-place
+        version), the batch, the dtype or the stream changes (its buffers
+        belong to the stream that they were made on)."""
         if st.metrics is not None or st.recent_filled < self.window or \
                 self._expandable() or (self.Me == 0 and self.Ms == 0) or self._tracing() or \
                 _capturing():
@@ -459,9 +461,9 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         ts = (st.k_buf, st.v_buf, st.allowed, st.g_recent, st.mem_last_exact, st._exact_v_norm, st._sum_lf_k_norm)
         vers = tuple(-1 if t is None else t._version for t in ts)
         pvers = self._param_key()
-        B = x.shape[0]
+        B, stream = x.shape[0], _hip.stream_of(x)
         if fp is None or fp["st"] is not st or fp["vers"] != vers or fp["pvers"] != pvers or fp["B"] != B or \
-                fp["packed"] != packed or fp["dtype"] is not x.dtype or \
+                fp["packed"] != packed or fp["dtype"] is not x.dtype or fp["stream"] != stream or \
                 fp["ptrs"] != tuple(-1 if t is None else t.data_ptr() for t in ts) or fp["dev"] != x.device:
             fp = self._build_step_fast(x, st, ts, vers, pvers, packed)
             if fp is None:
@@ -470,7 +472,6 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         pos = int(st.pos)
         d, a = fp["proj"], fp["attn"]
         d.x = x.data_ptr()
-        stream = _hip.stream_of(x)
         cos_t, sin_t = fp["tab"]
         if packed:
             if pos >= cos_t.shape[0]:
@@ -568,7 +569,7 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         L_ = _hip.lib()
         routed = ctypes.c_int(0)
 
-        fp = {"st": st, "vers": vers, "pvers": pvers, "B": B, "dev": dev, "dtype": dt, "packed": packed, "rows": None,
+        fp = {"st": st, "vers": vers, "pvers": pvers, "B": B, "dev": dev, "dtype": dt, "stream": _hip.stream_of(x), "packed": packed, "rows": None,
               "ptrs": tuple(-1 if t is None else t.data_ptr() for t in ts),
               "tab": (cos_t, sin_t), "row_bytes": (Dh // 2) * cos_t.element_size(),
               "proj": d, "proj_ref": ctypes.byref(d), "attn": a, "attn_ref": ctypes.byref(a),
