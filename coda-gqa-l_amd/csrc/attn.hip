@@ -639,6 +639,7 @@ __global__ __launch_bounds__(256) void attn_rows_bf16(const coda_attn_desc a, in
   }
 }
 
+// v_exp_f32 (2^x; -inf -> 0)
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // Merge of the per-split partials of attn_rows_bf16, attn_f32 and attn_f3_bf16,
@@ -860,8 +861,6 @@ __device__ __forceinline__ int fa_vswz(int k) {
   return DH == 128 ? 2 * (k & 7) : 2 * ((k >> 1) & 3);
 }
 
-// v_exp_f32 (2^x; -inf -> 0)
-
 __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
   typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
   bf16x2_t v;
@@ -899,7 +898,7 @@ __device__ __forceinline__ void unpack4(const uint2& u, float x[4]) {
   x[3] = bf2f((bf16_t)(u.y >> 16));
 }
 
-// ------------------------------------------------------------ fused decode step
+// ------------------------------------------------------------ grouped chunks
 // Chunks of a prefill call in one launch (coda_prefill_attn_chunks):
 // y = chunk c_first + y (blockIdx.y; attn_f32: blockIdx.z / B), covering queries [t0, t0 + Lq) of the
 // call, t0 = c blk, Lq = min(blk, L - t0); its block keys are the call's
@@ -1145,6 +1144,7 @@ __global__ __launch_bounds__(NW * 64) void attn_f32(const coda_attn_desc a_, int
   }
 }
 
+// ------------------------------------------------------------ fused decode step
 static constexpr int kFusedMaxBank = 256;  // exact + summary slots of the fused step
 // decode_step_bf16: one workgroup per (KV head hk, sequence b) runs the
 // whole decode step of that pair once the ring is full (the same work as
