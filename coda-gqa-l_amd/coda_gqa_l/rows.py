@@ -145,10 +145,10 @@ class RowsMixin:
             c, s_ = self.rope(seq_len=L, offset=p0, device=device, dtype=dtype)
             return c.contiguous(), s_.contiguous()
         half = self.head_dim // 2
-        t = torch.empty((2, L, half), dtype=dtype, device=device)
-        _hip.check(_hip.lib().coda_rope_tables(_hip.dtype_code(dtype), a[0], a[1], p0, L, half, t[0].data_ptr(),
-                                               t[1].data_ptr(), _hip.stream_of(t)))
-        return t[0], t[1]
+        c, s_ = torch.empty((L, half), dtype=dtype, device=device), torch.empty((L, half), dtype=dtype, device=device)
+        _hip.check(_hip.lib().coda_rope_tables(_hip.dtype_code(dtype), a[0], a[1], p0, L, half, c.data_ptr(), s_.data_ptr(),
+                                               _hip.stream_of(c)))
+        return c, s_
 
     def _proj_pack(self, dtype: torch.dtype):
         """Packed [q | k | v | lambda | write] weights (n_feat, D) in `dtype`,
