@@ -138,6 +138,7 @@ _SIGS = {
     "coda_project": (_i32, [ctypes.POINTER(ProjDesc), _vp]),
     "coda_project_rows": (_i32, [ctypes.POINTER(ProjDesc), _vp]),
     "coda_project_params": (_i32, [ctypes.POINTER(ProjDesc), ctypes.POINTER(ProjParams), _vp]),
+    "coda_project_pack_params": (_i32, [ctypes.POINTER(ProjDesc), ctypes.POINTER(ProjParams), _vp, _vp, _vp]),
     "coda_linear_params": (_i32, [_i32, _vp, _i64, _i32, _vp, _i64, _i32, _i32, _vp, _vp, _i64, _vp]),
     "coda_rope_tables": (_i32, [_i32, _vp, _i32, _i64, _i32, _i32, _vp, _vp, _vp]),
     "coda_linear_rows": (_i32, [_i32, _vp, _i64, _i32, _vp, _i32, _i32, _vp, _vp, _i64, _vp]),

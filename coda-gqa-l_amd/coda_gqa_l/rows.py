@@ -156,7 +156,8 @@ class RowsMixin:
         layout code for coda_project, per parameter version; with half-split
         RoPE each k head's rows are reordered to the pairs (i, i + Dh/2) on
         adjacent rows.  On a HIP device the weights are kept in the row
-        kernel's fragment tiles (coda_rows_pack, layout 1)."""
+        kernel's fragment tiles (layout 1), made in one launch where they have
+        that dtype already."""
         gate = self._has_gate()
         lins = (self.q_proj, self.k_proj, self.v_proj, self.lambda_proj) + ((self.write_proj,) if gate else ())
         ps = [t for lin in lins for t in (lin.weight, lin.bias) if t is not None]
@@ -168,35 +169,39 @@ class RowsMixin:
             if made is not None:
                 made.use()
             return self._handed(hit[1])
-        H, Hkv, Dh = self.num_heads, self.num_kv_heads, self.head_dim
-        with torch.no_grad():
-            dev = self.q_proj.weight.device
-            wk, bk = self.k_proj.weight, self.k_proj.bias
-            if not self.rope_interleaved:
-                half = Dh // 2
-                pair = torch.stack([torch.arange(half), torch.arange(half) + half], 1).reshape(-1)
-                perm = (torch.arange(Hkv)[:, None] * Dh + pair[None]).reshape(-1).to(dev)
-                wk = wk[perm]
-                bk = bk[perm] if bk is not None else None
-            ws = [self.q_proj.weight, wk, self.v_proj.weight, self.lambda_proj.weight]
-            sizes = [H * Dh, Hkv * Dh, Hkv * Dh, H]
-            bt = [self.q_proj.bias, bk, self.v_proj.bias, self.lambda_proj.bias]
-            if gate:
-                ws.append(self.write_proj.weight)
-                bt.append(self.write_proj.bias)
-                sizes.append(1)
-            for t, u, n in zip(ws, bt, sizes):
-                if tuple(t.shape) != (n, self.embed_dim) or u is not None and tuple(u.shape) != (n,):
-                    raise RuntimeError(f"projection weight {tuple(t.shape)} is not ({n}, {self.embed_dim})")
-            b = torch.cat([t.detach().float() if t is not None else torch.zeros(wt.shape[0], device=dev)
-                           for t, wt in zip(bt, ws)])
-            b = torch.cat([b, torch.zeros((-b.numel()) % 4, device=dev)])
-            ws = [t.detach().to(dtype) for t in ws]
-            if ws[0].is_cuda:
-                w, layout = self._rows_tiles(*ws), 1
-            else:
-                w, layout = torch.cat(ws).contiguous(), 0
-        val = (w, b.contiguous(), layout)
+        H, Hkv, Dh, D = self.num_heads, self.num_kv_heads, self.head_dim, self.embed_dim
+        sizes = (H * Dh, Hkv * Dh, Hkv * Dh, H, 1)
+        for lin, n in zip(lins, sizes):
+            if tuple(lin.weight.shape) != (n, D) or lin.bias is not None and tuple(lin.bias.shape) != (n,):
+                raise RuntimeError(f"projection weight {tuple(lin.weight.shape)} is not ({n}, {D})")
+        n_feat = sum(sizes[:len(lins)])
+        dev, layout = self.q_proj.weight.device, 0
+        if all(t.is_cuda and t.device == dev and t.dtype == dtype and t.stride(-1) == 1 for t in ps):
+            w, layout = torch.empty((-(-n_feat // 64) * 64, D), dtype=dtype, device=dev), 1
+            b = torch.empty(-(-n_feat // 4) * 4, dtype=torch.float32, device=dev)
+            d, rows = self._proj_desc(w, 0, 1), []
+            for lin in lins:
+                rows += (lin.weight.data_ptr(), lin.weight.stride(0), _hip.ptr(lin.bias))
+            _hip.check(_hip.lib().coda_project_pack_params(d, self._proj_params(rows), w.data_ptr(), b.data_ptr(),
+                                                           _hip.stream_of(w)))
+        else:
+            with torch.no_grad():
+                ws, bs = [lin.weight.detach() for lin in lins], []
+                for lin in lins:
+                    bs.append(lin.bias.detach().float() if lin.bias is not None
+                              else torch.zeros(lin.out_features, device=dev))
+                if not self.rope_interleaved:
+                    pair = torch.stack([torch.arange(Dh // 2), torch.arange(Dh // 2) + Dh // 2], 1).reshape(-1)
+                    perm = (torch.arange(Hkv)[:, None] * Dh + pair[None]).reshape(-1).to(dev)
+                    ws[1], bs[1] = ws[1][perm], bs[1][perm]
+                w = torch.cat(ws).to(dtype).contiguous()
+                b = torch.cat(bs + [torch.zeros((-n_feat) % 4, device=dev)])
+                if w.is_cuda:
+                    tiles, layout = torch.empty((-(-n_feat // 64) * 64, D), dtype=dtype, device=dev), 1
+                    _hip.check(_hip.lib().coda_rows_pack(_hip.dtype_code(dtype), w.data_ptr(), n_feat, D, D,
+                                                         tiles.data_ptr(), _hip.stream_of(w)))
+                    w = tiles
+        val = (w, b, layout)
         if w.is_cuda and _capturing():
             return val
         cache[("proj", dtype)] = (tag, val)
@@ -210,35 +215,6 @@ class RowsMixin:
         if val[0].device != x.device:
             raise RuntimeError(f"projection weights on {val[0].device}, input on {x.device}")
         return val
-
-    @staticmethod
-    def _rows_tiles(*parts: torch.Tensor) -> torch.Tensor:
-        """(n, D) weights, the parts one after the other, in the row kernel's
-        fragment tiles (coda_rows_pack), n rounded up to a multiple of 64.  A
-        part that starts on a row block of 16 is packed from where it is (a
-        layer's first token paid a concatenation of all its weights
-        otherwise: 340 MB of traffic and a second buffer at 10305 x 8192);
-        rows that the loads of the kernel can't take are copied first."""
-        groups, n = [], 0
-        for t in parts:
-            if n % 16:
-                groups[-1].append(t)
-            else:
-                groups.append([t])
-            n += t.shape[0]
-        D, rows = parts[0].shape[1], -(-n // 64) * 64
-        # (each launch pads its rows to 64 and the next one writes over the
-        # padding; the last one's may end past `rows`)
-        wt = torch.empty((rows + 64, D), dtype=parts[0].dtype, device=parts[0].device)
-        wt[n // 64 * 64:].zero_()
-        at, fn, dt, stream = 0, _hip.lib().coda_rows_pack, _hip.dtype_code(wt.dtype), _hip.stream_of(wt)
-        for g in groups:
-            w = g[0].contiguous() if len(g) == 1 else torch.cat(g)
-            if w.data_ptr() % 16:
-                w = w.clone()
-            _hip.check(fn(dt, w.data_ptr(), w.shape[0], D, D, wt[at:].data_ptr(), stream))
-            at += w.shape[0]
-        return wt[:rows]
 
     def _plain_rows(self, x: torch.Tensor, *names: str) -> Optional[tuple]:
         """(address, row stride, bias address) of each of these linears' own

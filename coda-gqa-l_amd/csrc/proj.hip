@@ -82,6 +82,11 @@ struct ParamRows {
     const int s = section(f);
     return pick(w, s) + row_in(s, f) * pick(sm, s);
   }
+  __device__ __forceinline__ float bias1(int f) const {
+    const int s = section(f);
+    const T* p = pick(b, s);
+    return p ? Elt<T>::ld(p[row_in(s, f)]) : 0.f;
+  }
   // biases of features f .. f + 3 (f a multiple of 4; past the last: any)
   __device__ __forceinline__ pf32x4 bias4(int f, int last) const {
     const int s = section(f);
@@ -644,7 +649,7 @@ static int run_project(const coda_proj_desc* d, hipStream_t st, const char* who)
                      : launch_rows<T>(MatRows<T>{w, d->D}, n, d->D, x, d->x_sm, d->M, epi, st, who);
 }
 template <typename T>
-static int run_project_params(const coda_proj_desc* d, const coda_proj_params* p, hipStream_t st, const char* who) {
+static ParamRows<T> param_rows(const coda_proj_desc* d, const coda_proj_params* p) {
   ParamRows<T> r;
   const int sizes[5] = {d->H * d->Dh, d->Hkv * d->Dh, d->Hkv * d->Dh, d->H, d->gate ? 1 : 0};
   int f = 0;
@@ -657,9 +662,42 @@ static int run_project_params(const coda_proj_desc* d, const coda_proj_params* p
   }
   r.Dh = d->Dh;
   r.halves = !d->rope_interleaved;
+  return r;
+}
+template <typename T>
+static int run_project_params(const coda_proj_desc* d, const coda_proj_params* p, hipStream_t st, const char* who) {
+  const ParamRows<T> r = param_rows<T>(d, p);
   const FrontTables t{p->inv_freq,  p->inv_dtype, p->p0,        p->rope_cos, p->rope_sin,
                       p->theta, p->theta_dtype, d->H * (d->Dh / 2), p->theta_cos, p->theta_sin};
-  return launch_rows<T>(r, f, d->D, (const T*)d->x, d->x_sm, d->M, FrontEpilogue<T, true>{*d, t}, st, who);
+  return launch_rows<T>(r, front_features(d), d->D, (const T*)d->x, d->x_sm, d->M, FrontEpilogue<T, true>{*d, t}, st,
+                        who);
+}
+// The packed form of a layer's parameters, tiles and fp32 biases, in one
+// launch: one thread per 16-byte piece of the tiles (a concatenation and its
+// packing moved the weights twice and took a dozen launches of a layer's
+// first token)
+template <typename T>
+__global__ __launch_bounds__(256) void proj_pack_params_kernel(const ParamRows<T> W, int n_feat, int row_pieces,
+                                                               uint4* __restrict__ out, int64_t n_pieces,
+                                                               float* __restrict__ bias) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < (n_feat + 3) / 4 * 4) bias[i] = i < n_feat ? W.bias1((int)i) : 0.f;
+  if (i >= n_pieces) return;
+  const int l = (int)(i & 63), ksteps = row_pieces / 4;
+  const int64_t tile = i >> 6, fb = tile / ksteps;
+  const int ks = (int)(tile % ksteps);
+  pu32x4 v{0u, 0u, 0u, 0u};
+  if (fb * 16 + (l & 15) < n_feat)
+    v = *reinterpret_cast<const pu32x4u*>((const char*)W.row16((int)fb * 16, l & 15, n_feat - 1) + 64 * ks + 16 * (l >> 4));
+  out[i] = make_uint4(v[0], v[1], v[2], v[3]);
+}
+template <typename T>
+static int run_pack_params(const coda_proj_desc* d, const coda_proj_params* p, void* out, float* bias, hipStream_t st) {
+  const int n = front_features(d), row_pieces = d->D * (int)sizeof(T) / 16;
+  const int64_t n_pieces = (int64_t)((n + 63) / 64) * 64 * row_pieces;
+  hipLaunchKernelGGL(proj_pack_params_kernel<T>, dim3((unsigned)((n_pieces + 255) / 256)), dim3(256), 0, st,
+                     param_rows<T>(d, p), n, row_pieces, (uint4*)out, n_pieces, bias);
+  return check_launch("proj_pack_params_kernel");
 }
 
 }  // namespace coda
@@ -691,19 +729,39 @@ extern "C" int coda_project_rows(const coda_proj_desc* d, void* stream) {
                                : run_project<float>(d, (hipStream_t)stream, "coda_project_rows");
 }
 
-extern "C" int coda_project_params(const coda_proj_desc* d, const coda_proj_params* p, void* stream) {
-  const char* who = "coda_project_params";
-  CODA_REQUIRE(d != nullptr && p != nullptr, "%s: null descriptor", who);
-  CODA_REQUIRE(d->dtype == CODA_BF16 || d->dtype == CODA_F32, "%s: dtype must be CODA_F32 or CODA_BF16", who);
-  CODA_REQUIRE(d->M >= 0 && d->M <= 128, "%s: %d token rows (at most 128)", who, d->M);
-  const int rc = check_project(d, who, false);
-  if (rc) return rc;
+// What both entries on parameters ask of them
+static int check_params(const coda_proj_desc* d, const coda_proj_params* p, const char* who) {
   const size_t esz = d->dtype == CODA_BF16 ? 2 : 4;
   for (int i = 0; i < (d->gate ? 5 : 4); ++i) {
     CODA_REQUIRE(p->w[i] && p->w_sm[i] >= d->D, "%s: weight %d missing or its rows shorter than D", who, i);
     CODA_REQUIRE((uintptr_t)p->w[i] % esz == 0 && (uintptr_t)p->b[i] % esz == 0, "%s: weight or bias %d off its type",
                  who, i);
   }
+  return CODA_OK;
+}
+
+extern "C" int coda_project_pack_params(const coda_proj_desc* d, const coda_proj_params* p, void* out, float* bias,
+                                        void* stream) {
+  const char* who = "coda_project_pack_params";
+  CODA_REQUIRE(d != nullptr && p != nullptr && out && bias, "%s: null pointer", who);
+  CODA_REQUIRE(d->dtype == CODA_BF16 || d->dtype == CODA_F32, "%s: dtype must be CODA_F32 or CODA_BF16", who);
+  CODA_REQUIRE(d->D > 0 && d->D % kProjKT == 0 && d->H > 0 && d->Hkv > 0 && d->Dh > 0 && d->Dh % 4 == 0,
+               "%s: bad sizes D=%d H=%d Hkv=%d Dh=%d", who, d->D, d->H, d->Hkv, d->Dh);
+  CODA_REQUIRE((uintptr_t)out % 16 == 0 && (uintptr_t)bias % 16 == 0, "%s: outputs must be 16-byte aligned", who);
+  const int rc = check_params(d, p, who);
+  if (rc) return rc;
+  return d->dtype == CODA_BF16 ? run_pack_params<bf16_t>(d, p, out, bias, (hipStream_t)stream)
+                               : run_pack_params<float>(d, p, out, bias, (hipStream_t)stream);
+}
+
+extern "C" int coda_project_params(const coda_proj_desc* d, const coda_proj_params* p, void* stream) {
+  const char* who = "coda_project_params";
+  CODA_REQUIRE(d != nullptr && p != nullptr, "%s: null descriptor", who);
+  CODA_REQUIRE(d->dtype == CODA_BF16 || d->dtype == CODA_F32, "%s: dtype must be CODA_F32 or CODA_BF16", who);
+  CODA_REQUIRE(d->M >= 0 && d->M <= 128, "%s: %d token rows (at most 128)", who, d->M);
+  int rc = check_project(d, who, false);
+  if (!rc) rc = check_params(d, p, who);
+  if (rc) return rc;
   const auto angle = [](int t) { return t == CODA_F32 || t == CODA_BF16; };
   CODA_REQUIRE(p->inv_freq ? p->rope_cos && p->rope_sin && angle(p->inv_dtype) && p->p0 >= 0 && p->p0 + d->L <= 1 << 24
                            : d->rope_cos && d->rope_sin,

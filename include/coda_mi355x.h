@@ -145,6 +145,13 @@ typedef struct {
  * are unused. */
 int coda_project_params(const coda_proj_desc* d, const coda_proj_params* p, void* stream);
 
+/* The packed form of the same parameters for coda_project_rows (w_layout 1):
+ * fragment tiles (ceil64(n_feat) * D elements, rows past the last zero) and
+ * fp32 biases (n_feat rounded up to 4, zero where there is none), in one
+ * launch.  Of d: dtype, D, H, Hkv, Dh, gate, rope_interleaved. */
+int coda_project_pack_params(const coda_proj_desc* d, const coda_proj_params* p, void* out, float* bias,
+                             void* stream);
+
 /* out (M, n_feat; row stride o_sm) = x (M, D; row stride x_sm) W^T + bias
  * for M <= 128 token rows: fp32 accumulation, one rounding.  w: the (n_feat,
  * D) weights in fragment tiles (coda_rows_pack); bias: (n_feat) float32 or

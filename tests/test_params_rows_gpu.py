@@ -7,7 +7,6 @@ import torch
 
 import coda_gqa_l
 from coda_gqa_l import _hip
-from coda_gqa_l.rows import RowsMixin
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -34,7 +33,8 @@ def test_linear_params_equals_tiles(M, N, D, bias, apart, off, dtype):
     x = torch.randn(M, D + 8, generator=g, device=DEV).to(dtype)[:, :D]
     b = torch.randn(N, generator=g, device=DEV).to(dtype) if bias else None
     code, st, L = _hip.dtype_code(dtype), _hip.stream_of(x), _hip.lib()
-    tiles = RowsMixin._rows_tiles(w)
+    tiles = torch.empty(-(-N // 64) * 64, D, device=DEV, dtype=dtype)
+    _hip.check(L.coda_rows_pack(code, w.data_ptr(), N, D, D, tiles.data_ptr(), st))
     ld = N + (-N) % 4 + 4
     want, got = (torch.full((M + 1, ld), 7.0, device=DEV, dtype=dtype) for _ in range(2))
     bf = b.float() if bias else None
@@ -106,3 +106,27 @@ def test_tables_equal_the_module(dtype, inv):
     for p0, L in ((0, 1), (0, 65536), (4095, 3), (1 << 20, 777), ((1 << 24) - 9, 9), ((1 << 24) - 8, 9)):
         for got, want in zip(m._rope_tables(p0, L, dev, dtype), m.rope(seq_len=L, offset=p0, device=dev, dtype=dtype)):
             assert got.shape == want.shape and got.is_contiguous() and torch.equal(got, want), (p0, L)
+
+
+@pytest.mark.parametrize("B,D,H,Hkv,inter,gate", [(1, 512, 8, 2, True, True), (9, 320, 5, 5, False, True),
+                                                  (33, 256, 4, 2, False, False), (2, 4096, 32, 8, False, True)])
+@pytest.mark.parametrize("half_bias", [False, True])
+@torch.no_grad()
+def test_pack_in_one_launch(B, D, H, Hkv, inter, gate, half_bias):
+    """The packed form from the parameters, any address, against the one from
+    a concatenation (taken where a dtype differs: here fp32 copies of the same
+    values)."""
+    torch.manual_seed(D)
+    m = coda_gqa_l.CoDAGQALandmarkPerf2(
+        embed_dim=D, num_heads=H, num_kv_heads=Hkv, window=16, num_landmarks_exact=8, num_landmarks_summary=8,
+        rope_interleaved=inter, **({} if gate else {"write_policy": "none"})).to(DEV, torch.bfloat16).eval()
+    lins = [m.q_proj, m.k_proj, m.v_proj, m.lambda_proj] + ([m.write_proj] if gate else [])
+    for i, lin in enumerate(lins):
+        lin.weight = torch.nn.Parameter(_off(lin.weight, i, i))
+        lin.bias = torch.nn.Parameter(torch.randn(lin.out_features, device=DEV).bfloat16()) if (i % 2) != half_bias else None
+    w, b, layout = m._proj_pack(torch.bfloat16)
+    for lin in lins:
+        lin.float()
+    m.drop_parameter_copies()
+    w2, b2, layout2 = m._proj_pack(torch.bfloat16)
+    assert layout == layout2 == 1 and torch.equal(w, w2) and torch.equal(b, b2)
