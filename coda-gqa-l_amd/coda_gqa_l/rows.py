@@ -221,9 +221,11 @@ class RowsMixin:
         parameters, one after the other, where calling the module on x is no
         more than its matrix product and the row kernels can take that: an
         nn.Linear in x's dtype on x's device, no hooks, no forward of the
-        instance's own, no autocast, no gradient.  Else None.  Asked at every
-        call: nothing about a parameter is remembered."""
-        if torch.is_autocast_enabled(x.device.type) or nn.modules.module._has_any_global_hook():
+        instance's own or put in the class's place, no autocast, no gradient,
+        no tensor subclass.  Else None.  Asked at every call: nothing about a
+        parameter is remembered."""
+        if torch.is_autocast_enabled(x.device.type) or nn.modules.module._has_any_global_hook() or \
+                type(x) not in (torch.Tensor, nn.Parameter) or nn.Linear.forward.__module__ != "torch.nn.modules.linear":
             return None
         grad = torch.is_grad_enabled()
         if grad and x.requires_grad:

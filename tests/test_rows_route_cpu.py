@@ -81,6 +81,10 @@ def test_inputs():
     w, lam = m.k_proj.weight, m.lambda_proj
     got = m._front_rows(_x())
     assert got[3:6] == (w.data_ptr(), D, None) and got[9:] == (lam.weight.data_ptr(), D, lam.bias.data_ptr())
+    assert m._front_rows(_x().as_subclass(type("T", (torch.Tensor,), {}))) is None
+    with pytest.MonkeyPatch.context() as mp:
+        mp.setattr(nn.Linear, "forward", lambda self, x: x)
+        assert m._front_rows(_x()) is None
     with torch.autocast("cpu", dtype=torch.bfloat16):
         assert m._front_rows(_x()) is None
     with torch.enable_grad():
