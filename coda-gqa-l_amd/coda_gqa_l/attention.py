@@ -31,7 +31,7 @@ import torch.nn as nn
 from . import _hip, ops
 from .memory_banks import METRIC_KEYS, DeviceMetrics, MemoryBankMixin
 from .primitives import HeadwiseRMSNorm, RotaryEmbedding, apply_rope
-from .rows import RowsMixin, _aligned, _capturing
+from .rows import RowsMixin, _aligned, _capturing, _version
 from .state import CoDAGQALandmarkStatePerf2
 
 __all__ = ["CoDAGQALandmarkPerf2", "CoDAGQALandmarkStatePerf2"]
@@ -506,8 +506,10 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
 
     def _param_key(self) -> tuple:
         """Identity, storage and in-place version of every parameter of the
-        layer and of its (leaf) submodules, without the recursive module walk."""
-        out = []
+        layer and of its (leaf) submodules, and of the RoPE frequencies,
+        without the recursive module walk."""
+        inv = self._modules["rope"]._buffers.get("inv_freq")
+        out = [] if inv is None else [id(inv), inv.data_ptr(), _version(inv)]
         for p in self._parameters.values():
             if p is not None:
                 out += (id(p), p.data_ptr(), p._version)

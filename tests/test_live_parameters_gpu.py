@@ -104,3 +104,32 @@ def test_dropped_copies(B, dtype):
         assert torch.equal(m.step(part, st)[0], n.step(part, st2)[0])
     assert torch.equal(m.prefill_chunked(xs[:, :30], st, block_size=16)[0], n.prefill_chunked(xs[:, :30], st2, block_size=16)[0])
     assert torch.equal(st.k_buf, st2.k_buf) and torch.equal(st.v_buf, st2.v_buf)
+
+
+@pytest.mark.parametrize("change", ["mul_", "replaced", "data replaced"])
+@torch.no_grad()
+def test_counted_changes(change):
+    """Packed weights and kept RoPE rows (bf16, few rows): changes that torch
+    counts need no call."""
+    def make():
+        return coda_gqa_l.CoDAGQALandmarkPerf2(embed_dim=256, num_heads=4, num_kv_heads=2, window=16, num_landmarks_exact=8,
+                                               num_landmarks_summary=8).to(DEV, torch.bfloat16).eval()
+
+    torch.manual_seed(2)
+    m, g = make(), torch.Generator(device=DEV).manual_seed(4)
+    st = m.init_state(batch_size=2, device=DEV, dtype=torch.bfloat16)
+    xs = torch.randn(2, 60, 256, generator=g, device=DEV).bfloat16()
+    m.prefill_chunked(xs[:, :50], st, block_size=16, return_outputs=False)
+    for t in range(50, 56, 2):
+        m.step(xs[:, t:t + 1], st)
+        if change == "mul_":
+            m.k_proj.weight.mul_(1.25)
+            m.rope.inv_freq.mul_(0.5)
+        elif change == "replaced":
+            m.k_proj.weight = torch.nn.Parameter(m.k_proj.weight * 1.25)
+            m.rope.inv_freq = m.rope.inv_freq * 0.5
+        else:
+            m.k_proj.weight.data = m.k_proj.weight * 1.25
+        n, st2 = _given(make, _values(m)), state_io.deep_copy_state(st)
+        assert torch.equal(m.step(xs[:, t + 1:t + 2], st)[0], n.step(xs[:, t + 1:t + 2], st2)[0])
+        assert torch.equal(st.k_buf, st2.k_buf)
