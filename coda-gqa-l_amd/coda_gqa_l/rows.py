@@ -121,16 +121,16 @@ class RowsMixin:
         key = (torch.device(device), dtype)
         tab = cache.get(key)
         need = int(p0) + int(L)
-        inv = self.rope.inv_freq
-        hit = made.get(key)
-        if tab is None or tab[0].shape[0] < need or hit is None or hit[0] is not inv or \
-                hit[1] != (_version(inv), inv.data_ptr()):
+        inv = getattr(self.rope, "inv_freq", None)  # (a module of the user's own may have none)
+        tag, hit = None if inv is None else (_version(inv), inv.data_ptr()), made.get(key)
+        if tab is None or tab[0].shape[0] < need or hit is None or hit[0] is not self.rope or hit[1] is not inv or \
+                hit[2] != tag:
             n = 1 << max(12, (need - 1).bit_length())
             c, s_ = self.rope(seq_len=n, offset=0, device=device, dtype=dtype)
             tab = cache[key] = (c.contiguous(), s_.contiguous())
-            made[key] = (inv, (_version(inv), inv.data_ptr()), _Made(*tab) if tab[0].is_cuda else None)
-        elif hit[2] is not None:
-            hit[2].use()
+            made[key] = (self.rope, inv, tag, _Made(*tab) if tab[0].is_cuda else None)
+        elif hit[3] is not None:
+            hit[3].use()
         return tab[0][p0:need], tab[1][p0:need]
 
     def _rope_tables(self, p0: int, L: int, device, dtype: torch.dtype) -> Tuple[torch.Tensor, torch.Tensor]:
