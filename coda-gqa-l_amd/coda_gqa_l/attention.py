@@ -309,7 +309,8 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
                     "cause shown, and was removed")
             capturing = _capturing()
             rows = None if self._packed_front_ok(x) and not capturing else self._front_rows(x)
-            cos, sin = (self._rope_rows if rows is None and not capturing else self._rope_tables)(p0, L, x.device, x.dtype)
+            tables = self._rope_rows if rows is None and not capturing else self._rope_tables
+            cos, sin = tables(p0, L, x.device, x.dtype)
             d = self._proj_desc(x, M, L, cos, sin)
             g = torch.empty((B, L), dtype=torch.float32, device=x.device)
             d.g = g.data_ptr()
@@ -571,7 +572,8 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
         L_ = _hip.lib()
         routed = ctypes.c_int(0)
 
-        fp = {"st": st, "vers": vers, "pvers": pvers, "B": B, "dev": dev, "dtype": dt, "stream": _hip.stream_of(x), "packed": packed, "rows": None,
+        fp = {"st": st, "vers": vers, "pvers": pvers, "B": B, "dev": dev, "dtype": dt, "stream": _hip.stream_of(x),
+              "packed": packed, "rows": None, "step": L_.coda_decode_step,
               "ptrs": tuple(-1 if t is None else t.data_ptr() for t in ts),
               "tab": (cos_t, sin_t), "row_bytes": (Dh // 2) * cos_t.element_size(),
               "proj": d, "proj_ref": ctypes.byref(d), "attn": a, "attn_ref": ctypes.byref(a),
@@ -579,7 +581,8 @@ class CoDAGQALandmarkPerf2(MemoryBankMixin, RowsMixin, nn.Module):
               "keep": (keep, q, k, v, lam, g, heads, w, b, ws, ct, sn, eta, self._rms_weight(dt)),
               "k_ptr": k.data_ptr(), "v_ptr": v.data_ptr(), "k_sb": Fk, "k_sh": Dh, "g_ptr": g.data_ptr(),
               "ws_ptr": _hip.ptr(ws), "ws_bytes": nb.value, "routed": routed, "routed_ref": ctypes.byref(routed),
-              "record_pos": routed_pos, "project": L_.coda_project_rows if packed else L_.coda_project_params, "step": L_.coda_decode_step,
+              "record_pos": routed_pos,
+              "project": L_.coda_project_rows if packed else L_.coda_project_params,
               "heads_flat": heads.view(B, 1, H * Dh)}
         self.__dict__["_fast"] = fp
         return fp

@@ -146,8 +146,8 @@ class RowsMixin:
             return c.contiguous(), s_.contiguous()
         half = self.head_dim // 2
         c, s_ = torch.empty((L, half), dtype=dtype, device=device), torch.empty((L, half), dtype=dtype, device=device)
-        _hip.check(_hip.lib().coda_rope_tables(_hip.dtype_code(dtype), a[0], a[1], p0, L, half, c.data_ptr(), s_.data_ptr(),
-                                               _hip.stream_of(c)))
+        _hip.check(_hip.lib().coda_rope_tables(_hip.dtype_code(dtype), a[0], a[1], p0, L, half, c.data_ptr(),
+                                               s_.data_ptr(), _hip.stream_of(c)))
         return c, s_
 
     def _proj_pack(self, dtype: torch.dtype):
